@@ -6,6 +6,7 @@ Usage: python bd-simulations_amd/build.py [--param-header path/to/parameter.h]
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -21,19 +22,31 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contra
              "-I" + os.path.join(ROOT, "include")]
 
 
+# device sources, compiled side by side and joined (ld -r) into one object,
+# bdk_kernels.hip.o; then the rest
+KERNELS = ("bdk_kernels.hip", "bdk_obs.hip")
+SOURCES = KERNELS + ("bdk_noalloc.hip", "bdk_api.cpp", "bdk_serve.cpp")
+
+
 def run(cmd):
     print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
 
 
 def build_lib():
-    objs = []
     os.makedirs(os.path.join(HERE, "_build"), exist_ok=True)
-    for src in ("bdk_kernels.hip", "bdk_noalloc.hip", "bdk_api.cpp", "bdk_serve.cpp"):
-        obj = os.path.join(HERE, "_build", src + ".o")
+
+    def compile_one(src):
+        obj = os.path.join(HERE, "_build", ("part_" if src in KERNELS else "") + src + ".o")
         extra = ["-x", "hip"] if src.endswith(".hip") else []
         run([HIPCC] + HIP_FLAGS + extra + ["-c", os.path.join(CSRC, src), "-o", obj])
-        objs.append(obj)
+        return obj
+
+    with ThreadPoolExecutor(min(8, len(SOURCES))) as pool:  # one compiler process each
+        objs = list(pool.map(compile_one, SOURCES))
+    joined = os.path.join(HERE, "_build", "bdk_kernels.hip.o")
+    run(["ld", "-r", "-o", joined] + objs[:len(KERNELS)])
+    objs = [joined] + objs[len(KERNELS):]
     tmp = LIB + ".tmp"
     run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp] + objs)
     os.replace(tmp, LIB)

@@ -209,6 +209,8 @@ namespace bdkx {
 hipError_t launch_wca(bdk_t *h, hipStream_t st = nullptr);  // WCA forces -> fwca (default: h->stream)
 hipError_t launch_deposit(bdk_t *h, int reset, int slot = 0, hipStream_t st = nullptr);  // charges -> rho
                                                   // (reset: re-arm per-step scalars; slot: during a rebuild)
+hipError_t launch_species_deposit(bdk_t *h, int species);  // number density of one species -> rho
+hipError_t launch_zero_ints(int *p, int n, hipStream_t st);
 hipError_t launch_rearm(bdk_t *h);                // per-step scalars when no deposit runs
 size_t deposit_lds_bytes(const bdk_t *h);          // LDS of one deposit block
 hipError_t launch_fft(bdk_t *h);                  // rho -> fmesh (r2c, multiply, c2r)

@@ -35,329 +35,13 @@
 // build; cell indices are therefore bit-exact.
 #pragma clang fp contract(off)
 
-#include <hip/hip_runtime.h>
-
-#include <algorithm>
-#include <cmath>
-#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
-#include <type_traits>
 
-#include "bdk_internal.hpp"
+#include "bdk_device.hpp"
+#include "bdk_fft.hpp"
 
 namespace bdkx {
-
-template <typename R> struct V2;
-template <> struct V2<float> { using T = float2; };
-template <> struct V2<double> { using T = double2; };
-template <typename R> struct V4;
-template <> struct V4<float> { using T = float4; };
-template <> struct V4<double> { using T = double4; };
-
-// Complex helpers of the FFT and spectral arithmetic.  The complex product
-// uses explicit fused multiply-adds (the file compiles without automatic
-// contraction, so every kernel that inlines it rounds the same way).
-template <typename C> __device__ __forceinline__ C cm(decltype(C::x) a, decltype(C::x) b) {
-    C r;
-    r.x = a;
-    r.y = b;
-    return r;
-}
-template <typename C> __device__ __forceinline__ C cadd(C a, C b) { return cm<C>(a.x + b.x, a.y + b.y); }
-template <typename C> __device__ __forceinline__ C csub(C a, C b) { return cm<C>(a.x - b.x, a.y - b.y); }
-template <typename C> __device__ __forceinline__ C cconj(C a) { return cm<C>(a.x, -a.y); }
-template <typename C> __device__ __forceinline__ C cmul(C a, C b) {
-    return cm<C>(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
-}
-template <typename C> __device__ __forceinline__ C cmul_i(C a) { return cm<C>(-a.y, a.x); }    // i*a
-template <typename C> __device__ __forceinline__ C cmul_mi(C a) { return cm<C>(a.y, -a.x); }   // -i*a
-template <typename C> __device__ __forceinline__ C cscale(C a, decltype(C::x) s) { return cm<C>(a.x * s, a.y * s); }
-
-__device__ __forceinline__ double dbits(unsigned long long b) { return __longlong_as_double((long long)b); }
-__device__ __forceinline__ unsigned long long bitsd(double v) { return (unsigned long long)__double_as_longlong(v); }
-
-// ------------------------------------------------------------------ Philox
-// Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11).
-__device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32_t k1) {
-#pragma unroll
-    for (int r = 0; r < 10; ++r) {
-        if (r) {
-            k0 += 0x9E3779B9u;
-            k1 += 0xBB67AE85u;
-        }
-        // one 32x32 -> 64-bit product each (a single multiply instruction
-        // instead of separate low and high halves)
-        const uint64_t p0 = (uint64_t)0xD2511F53u * c[0], p1 = (uint64_t)0xCD9E8D57u * c[2];
-        const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0;
-        const uint32_t hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
-        uint32_t n0 = hi1 ^ c[1] ^ k0;
-        uint32_t n2 = hi0 ^ c[3] ^ k1;
-        c[0] = n0;
-        c[1] = lo1;
-        c[2] = n2;
-        c[3] = lo0;
-    }
-}
-
-// noise of particle `pid` at step `step`: disc of radius sqrt 5 (variance
-// 5/4 per component, the distribution of dm:1321-1325) or Gaussian.
-__device__ __forceinline__ double2 philox_noise(unsigned long long seed, uint32_t pid, unsigned long long step,
-                                                int gauss, double var) {
-    uint32_t c[4] = {pid, (uint32_t)step, (uint32_t)(step >> 32), 0x4244u};
-    philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
-    const double inv53 = 1.0 / 9007199254740992.0;
-    double u1 = (double)(((((unsigned long long)c[1]) << 32) | c[0]) >> 11) * inv53;
-    double u2 = (double)(((((unsigned long long)c[3]) << 32) | c[2]) >> 11) * inv53;
-    double r = gauss ? sqrt(-2.0 * var * log(1.0 - u1)) : sqrt(5.0 * u1);
-    double a = 2.0 * M_PI * u2;
-    double sa, ca;
-    sincos(a, &sa, &ca);
-    double2 o;
-    o.x = r * ca;
-    o.y = r * sa;
-    return o;
-}
-
-// The same draws in FP32 (FP32 force mode: the random force is a force):
-// u1, u2 are the high words of the FP64 path's 64-bit draws rounded to FP32
-// (relative error <= 2^-24 + 2^-32/u), r and the angle in FP32.
-__device__ __forceinline__ double2 philox_noise_f32(unsigned long long seed, uint32_t pid, unsigned long long step,
-                                                    int gauss, double var) {
-    uint32_t c[4] = {pid, (uint32_t)step, (uint32_t)(step >> 32), 0x4244u};
-    philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
-    const float u1 = fminf((float)c[1] * 2.3283064365386963e-10f, 0.99999994f);  // 2^-32, below 1
-    const float u2 = (float)c[3] * 2.3283064365386963e-10f;
-    const float r = gauss ? sqrtf(-2.0f * (float)var * logf(1.0f - u1)) : sqrtf(5.0f * u1);
-    float sa, ca;
-    sincospif(2.0f * u2, &sa, &ca);
-    double2 o;
-    o.x = (double)(r * ca);
-    o.y = (double)(r * sa);
-    return o;
-}
-
-// ------------------------------------------------------------------ launch order
-// Workgroups are dispatched round-robin over the 8 XCDs, each with its own
-// L2.  Renumbered so that every XCD runs one contiguous range of the logical
-// grid, neighbouring tiles (whose inputs overlap) share an L2.
-__device__ __forceinline__ int xcd_block(int on) {
-    const int b = blockIdx.x + blockIdx.y * gridDim.x;
-    if (!on) return b;
-    const int nb = gridDim.x * gridDim.y;
-    const int x = b & 7, i = b >> 3, base = nb >> 3, rem = nb & 7;
-    return x < rem ? x * (base + 1) + i : rem * (base + 1) + (x - rem) * base + i;
-}
-
-// ------------------------------------------------------------------ geometry
-__device__ __forceinline__ int wrapc(int u, int n) {
-    int v = u % n;
-    return v < 0 ? v + n : v;
-}
-// u in [-n, 2n)
-__device__ __forceinline__ int wrap1(int u, int n) { return u < 0 ? u + n : (u >= n ? u - n : u); }
-// Mesh code is compiled for two kinds of mesh size: P2 (Z a power of two:
-// masks and shifts) and the other even sizes.  The kind is a template
-// parameter of every mesh kernel, chosen by its launcher, so the
-// power-of-two instruction stream carries no test of the other.
-__device__ __forceinline__ bool zpow2(int Z) { return (Z & (Z - 1)) == 0; }
-// mesh index u in [-Z, 2Z) into [0, Z)
-template <bool P2> __device__ __forceinline__ int wrapz(int u, int Z) { return P2 ? (u & (Z - 1)) : wrap1(u, Z); }
-// x / d and x % d for 0 <= x < 2^22: a shift when d is a power of two, else
-// the float reciprocal corrected to the exact quotient
-struct Dv {
-    int d, sh;
-    float inv;
-    __device__ explicit Dv(int d_)
-        : d(d_), sh((d_ & (d_ - 1)) == 0 ? __ffs(d_) - 1 : -1), inv(__builtin_amdgcn_rcpf((float)d_)) {}
-    __device__ int q(int x) const {
-        if (sh >= 0) return x >> sh;
-        int v = (int)((float)x * inv);
-        const int r = x - v * d;
-        v += (r >= d) - (r < 0);
-        return v;
-    }
-    __device__ int r(int x) const { return sh >= 0 ? (x & (d - 1)) : x - q(x) * d; }
-};
-// the same with the kind of d known at compile time (P2: a power of two)
-template <bool P2> struct DvT : Dv {
-    __device__ explicit DvT(int d_) : Dv(d_) {}
-};
-template <> struct DvT<true> {
-    int d, sh;
-    __device__ explicit DvT(int d_) : d(d_), sh(__ffs(d_) - 1) {}
-    __device__ int q(int x) const { return x >> sh; }
-    __device__ int r(int x) const { return x & (d - 1); }
-};
-// c / nc for 0 <= c < 2^24 (float reciprocal, corrected to the exact quotient)
-__device__ __forceinline__ int div_nc(int c, const Geo &g) {
-    int q = (int)((float)c * g.ncinv);
-    const int r = c - q * g.nc;
-    q += (r >= g.nc) - (r < 0);
-    return q;
-}
-
-// mesh index and weights along one axis (NGP gr:44-54, CIC gr:154-190,
-// TSC gr:435-459), evaluated in FP64 in the reference's operation order
-template <int SCHEME>
-__device__ __forceinline__ void weights1d(double x, double h, int &k, double w[3]) {
-    int kk = (int)(x / h);
-    k = kk;
-    if (SCHEME == 0) {
-        w[0] = 0.0;
-        w[1] = 1.0;
-        w[2] = 0.0;
-    } else if (SCHEME == 1) {
-        double tmp = x / h - (kk + 0.5);
-        w[1] = 1.0 - fabs(tmp);
-        if (tmp < 0.0) {
-            w[0] = -tmp;
-            w[2] = 0.0;
-        } else {
-            w[0] = 0.0;
-            w[2] = tmp;
-        }
-    } else {
-        double d = x - (kk + 0.5) * h;
-        w[1] = 0.75 - d * d / h / h;
-        double tmp = fabs((d + h) / h);
-        w[0] = 0.5 * (1.5 - tmp) * (1.5 - tmp);
-        tmp = fabs((d - h) / h);
-        w[2] = 0.5 * (1.5 - tmp) * (1.5 - tmp);
-    }
-}
-
-// Weights in the precision of the forces: FP64 follows the reference's
-// operations exactly; FP32 takes the index from x/h in FP64 and evaluates
-// the offset t = x/h - k - 1/2 and the textbook weights (CIC: 1-|t|, -t, t;
-// TSC: 3/4-t^2, (1/2-t)^2/2, (1/2+t)^2/2) in FP32.
-template <typename R, int SCHEME>
-__device__ __forceinline__ void weights_r(double x, const Geo &g, int &k, R w[3]) {
-    if (std::is_same<R, double>::value) {
-        double wd[3];
-        weights1d<SCHEME>(x, g.h, k, wd);
-        w[0] = (R)wd[0];
-        w[1] = (R)wd[1];
-        w[2] = (R)wd[2];
-        return;
-    }
-    if (SCHEME == 0) {
-        k = (int)(x / g.h);
-        w[0] = 0;
-        w[1] = 1;
-        w[2] = 0;
-        return;
-    }
-    // CIC/TSC weights are continuous across a cell edge, so x * (1/h) may
-    // pick the neighbouring index at an exact edge without changing the sum
-    const double u = x * g.hinv;
-    const int kk = (int)u;
-    k = kk;
-    const float t = (float)(u - (kk + 0.5));
-    if (SCHEME == 1) {
-        w[1] = 1.0f - fabsf(t);
-        w[0] = t < 0.0f ? -t : 0.0f;
-        w[2] = t < 0.0f ? 0.0f : t;
-    } else {
-        const float a = 0.5f - t, b = 0.5f + t;
-        w[1] = 0.75f - t * t;
-        w[0] = 0.5f * a * a;
-        w[2] = 0.5f * b * b;
-    }
-}
-
-// One WCA pair, the arithmetic of dm:640-698 (type 0, pair 11), dm:815-868
-// (type 1, pair 22) and dm:987-1040 (type 2, pair 12): force on particle a
-// at (xa,ya) from b at (xb,yb).  Minimum image as abstand2 (am:100-166) and
-// the shift logic of dm:663-676.  Returns false outside the cutoff.
-template <typename R>
-__device__ __forceinline__ bool wca_pair(double xa, double ya, double xb, double yb, int type, const Geo &g,
-                                         R &fx, R &fy) {
-    const double L = g.L;
-    double t1 = xa - xb, t2 = xa - xb + L, t3 = xa - xb - L;
-    double m23 = (t3 * t3 < t2 * t2) ? t3 * t3 : t2 * t2;
-    double dx2 = (m23 < t1 * t1) ? m23 : t1 * t1;
-    t1 = ya - yb;
-    t2 = ya - yb + L;
-    t3 = ya - yb - L;
-    m23 = (t3 * t3 < t2 * t2) ? t3 * t3 : t2 * t2;
-    double dy2 = (m23 < t1 * t1) ? m23 : t1 * t1;
-    double a2 = dx2 + dy2;
-    double sig = type == 1 ? g.s22 : g.s12;
-    if (type == 0) {
-        if (a2 > g.cut2) return false;
-    } else {
-        if (a2 * sig * sig > g.cut2) return false;
-    }
-    double x2 = xb, y2 = yb;
-    double dx = xa - x2, dy = ya - y2;
-    if (dx * dx + dy * dy > a2) {
-        if ((dx - L) * (dx - L) < dx * dx)
-            x2 += L;
-        else if ((dx + L) * (dx + L) < dx * dx)
-            x2 -= L;
-        dx = xa - x2;
-        if ((dy - L) * (dy - L) < dy * dy)
-            y2 += L;
-        else if ((dy + L) * (dy + L) < dy * dy)
-            y2 -= L;
-        dy = ya - y2;
-    }
-    if (type != 0) {
-        a2 *= sig * sig;
-        dx *= sig;
-        dy *= sig;
-    }
-    const R ra2 = (R)a2;
-    const R a_8 = (R)1.0 / (ra2 * ra2 * ra2 * ra2);
-    const R a_14 = (R)1.0 / (ra2 * ra2 * ra2 * ra2 * ra2 * ra2 * ra2);
-    R absF;
-    if (type == 0)
-        absF = (R)4.0 * (R)6.0 * ((R)2.0 * a_14 - a_8);
-    else
-        absF = (R)(type == 1 ? g.e22f : g.e12f) * (R)4.0 * (R)6.0 * ((R)2.0 * a_14 - a_8);
-    if (absF > (R)g.maxpair) absF = (R)g.maxpair;
-    fx = absF * (R)dx;
-    fy = absF * (R)dy;
-    return true;
-}
-
-// ------------------------------------------------------------------ block scan
-// exclusive scan of a[0..n) in LDS (n <= 4*blockDim.x, blockDim.x <= 1024),
-// returns the total; all threads must call it
-__device__ int block_exscan4(int *a, int n, int *wsum) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nw = (blockDim.x + 63) >> 6;
-    int v[4];
-    int s = 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        int idx = 4 * tid + q;
-        v[q] = idx < n ? a[idx] : 0;
-        s += v[q];
-    }
-    int x = s;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) wsum[w] = x;
-    __syncthreads();
-    int woff = 0, total = 0;
-    for (int q = 0; q < nw; ++q) {
-        if (q < w) woff += wsum[q];
-        total += wsum[q];
-    }
-    int e = woff + x - s;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        int idx = 4 * tid + q;
-        if (idx < n) a[idx] = e;
-        e += v[q];
-    }
-    __syncthreads();
-    return total;
-}
 
 // ------------------------------------------------------------------ WCA
 // One thread per list position.  Neighbours come from the cell list of
@@ -992,433 +676,6 @@ __global__ void k_rearm(Geo g, DevBufs d) {
         d.sc->exc_bits[(step + 1) & 1] = 0ull;
     }
 }
-// ------------------------------------------------------------------ FFT in LDS
-// tw[k] = exp(-2 pi i k / Z), k < Z; the inverse transforms use the conjugates.
-// radix-4 butterfly in place, y = DFT4(v) (inverse: conjugate kernel)
-template <typename C>
-__device__ __forceinline__ void dft4(C *v, bool inv) {
-    C t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
-    C t2 = cadd(v[1], v[3]), t3 = csub(v[1], v[3]);
-    C r3 = inv ? cmul_i(t3) : cmul_mi(t3);
-    v[0] = cadd(t0, t2);
-    v[2] = csub(t0, t2);
-    v[1] = cadd(t1, r3);
-    v[3] = csub(t1, r3);
-}
-
-// radix-8 butterfly: y[2m] = DFT4(v[t] + v[t+4])[m],
-// y[2m+1] = DFT4((v[t] - v[t+4]) W^t)[m], W = exp(-+2 pi i / 8)
-template <typename C>
-__device__ __forceinline__ void dft8(const C *v, C *y, bool inv) {
-    using R = decltype(C::x);
-    const R c = (R)0.70710678118654752440;
-    C a[4], b[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        a[t] = cadd(v[t], v[t + 4]);
-        b[t] = csub(v[t], v[t + 4]);
-    }
-    // b[1] *= W, b[2] *= W^2, b[3] *= W^3
-    if (!inv) {
-        b[1] = cm<C>(c * (b[1].x + b[1].y), c * (b[1].y - b[1].x));
-        b[2] = cmul_mi(b[2]);
-        b[3] = cm<C>(c * (b[3].y - b[3].x), -c * (b[3].x + b[3].y));
-    } else {
-        b[1] = cm<C>(c * (b[1].x - b[1].y), c * (b[1].x + b[1].y));
-        b[2] = cmul_i(b[2]);
-        b[3] = cm<C>(-c * (b[3].x + b[3].y), c * (b[3].x - b[3].y));
-    }
-    dft4(a, inv);
-    dft4(b, inv);
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        y[2 * m] = a[m];
-        y[2 * m + 1] = b[m];
-    }
-}
-
-// radix-16 butterfly: y[2m] = DFT8(v[t] + v[t+8])[m],
-// y[2m+1] = DFT8((v[t] - v[t+8]) W^t)[m], W = exp(-+2 pi i / 16)
-template <typename C>
-__device__ __forceinline__ void dft16(const C *v, C *y, bool inv) {
-    using R = decltype(C::x);
-    const R c1 = (R)0.92387953251128675613, s1 = (R)0.38268343236508977173;  // cos, sin of pi/8
-    const R h = (R)0.70710678118654752440;
-    // W^t = cos(t pi/8) -+ i sin(t pi/8), t = 1..7
-    const R wr[8] = {(R)1, c1, h, s1, (R)0, -s1, -h, -c1};
-    const R wi[8] = {(R)0, s1, h, c1, (R)1, c1, h, s1};
-    C a[8], b[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        a[t] = cadd(v[t], v[t + 8]);
-        b[t] = csub(v[t], v[t + 8]);
-    }
-    b[4] = inv ? cmul_i(b[4]) : cmul_mi(b[4]);
-#pragma unroll
-    for (int t = 1; t < 8; ++t) {
-        if (t == 4) continue;
-        const R si = inv ? wi[t] : -wi[t];
-        b[t] = cm<C>(b[t].x * wr[t] - b[t].y * si, b[t].x * si + b[t].y * wr[t]);
-    }
-    C ya[8], yb[8];
-    dft8(a, ya, inv);
-    dft8(b, yb, inv);
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        y[2 * m] = ya[m];
-        y[2 * m + 1] = yb[m];
-    }
-}
-
-// LDS layout of the FFT rows: element i of a row sits at lp(i), one padding
-// element after every 8.  The output strides of the first Stockham passes
-// (8 and 64 elements) then spread over the banks instead of piling onto a
-// few (measured: half the LDS cycles of the unpadded passes were bank
-// conflicts).  A row of n elements takes n + n/8 + 1 (odd) elements.
-__device__ __forceinline__ int lp(int i) { return i + (i >> 3); }
-__host__ __device__ __forceinline__ int lds_row(int n) { return n + n / 8 + 1; }
-
-// One Stockham pass of radix RAD (2, 4 or 8) over nrows rows of length
-// n = 2^logn held in LDS (row stride `stride`, layout lp), in place: every thread reads
-// its butterflies' inputs (and, for small register footprints, their
-// twiddles: powers 1, 2, 4 from the FP64-built table, 3, 5, 6, 7 as
-// products) before the barrier and writes the outputs after it.  Twiddle of input t of butterfly j: tw[(t k) << twsh],
-// k = j mod Ns (conjugated for the inverse transform).
-// Output index ((j - k) << LR) + k + t Ns with Ns a power of 8 maps to
-// lp(base) + t (Ns + Ns/8); input index j + t nb to lp(j) + t (nb + nb/8)
-// when nb is a multiple of 8 (SMALL: nb < 8, mapped per element).
-template <typename R, int EPT, int RAD, bool SMALL>
-__device__ __forceinline__ void fft_pass(typename V2<R>::T *buf, int logn, int nrows, int stride, int logNs,
-                                         const typename V2<R>::T *__restrict__ tw, int logZ, bool inv) {
-    using C = typename V2<R>::T;
-    constexpr int LR = RAD == 16 ? 4 : (RAD == 8 ? 3 : (RAD == 4 ? 2 : 1));
-    // butterflies per thread (radix 16 at 8 elements per thread: one, on half
-    // of the threads)
-    constexpr int NB = EPT >= RAD ? EPT / RAD : 1;
-    constexpr bool PRE = sizeof(R) == 4 && NB * (RAD - 1) <= 16;  // twiddles fetched before the barrier
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int lognb = logn - LR, nb = 1 << lognb;
-    const int tot = nb * nrows;
-    const int Ns = 1 << logNs;
-    const int twsh = logZ - (logNs + LR);
-    const int nbp = nb + (nb >> 3), Nsp = Ns + (Ns >> 3);
-    C v[NB][RAD];
-    C w[PRE ? NB : 1][RAD - 1];
-    // twiddles of butterfly k: tw^1, tw^2, tw^4 (and tw^8) from the table,
-    // the other powers as products (one to three roundings deeper; 3 loads
-    // instead of 7 for radix 8, 4 instead of 15 for radix 16).  Every tiling
-    // forms them the same way -- before the barrier when the registers allow
-    // (PRE), else after it -- so the transform's rounding does not depend on
-    // the elements per thread.
-    auto twiddles = [&](int k, C *ww) {
-        ww[0] = tw[k << twsh];
-        if (RAD >= 4) {
-            ww[1] = tw[(2 * k) << twsh];
-            ww[2] = cmul(ww[0], ww[1]);
-        }
-        if (RAD >= 8) {
-            ww[3] = tw[(4 * k) << twsh];
-            ww[4] = cmul(ww[3], ww[0]);
-            ww[5] = cmul(ww[3], ww[1]);
-            ww[6] = cmul(ww[3], ww[2]);
-        }
-        if (RAD == 16) {
-            ww[7] = tw[(8 * k) << twsh];
-#pragma unroll
-            for (int t = 8; t < 15; ++t) ww[t] = cmul(ww[7], ww[t - 8]);
-        }
-    };
-#pragma unroll
-    for (int e = 0; e < NB; ++e) {
-        const int b = tid + e * nt;
-        if (b < tot) {
-            const int row = b >> lognb, j = b & (nb - 1);
-            const C *p = buf + row * stride;
-            if (SMALL) {
-#pragma unroll
-                for (int t = 0; t < RAD; ++t) v[e][t] = p[lp(j + t * nb)];
-            } else {
-                p += lp(j);
-#pragma unroll
-                for (int t = 0; t < RAD; ++t) v[e][t] = p[t * nbp];
-            }
-            if (PRE) twiddles(j & (Ns - 1), w[PRE ? e : 0]);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < NB; ++e) {
-        const int b = tid + e * nt;
-        if (b < tot) {
-            const int row = b >> lognb, j = b & (nb - 1);
-            const int k = j & (Ns - 1);
-            C wl[RAD - 1];
-            if (!PRE) twiddles(k, wl);
-#pragma unroll
-            for (int t = 1; t < RAD; ++t) {
-                C ww = PRE ? w[PRE ? e : 0][t - 1] : wl[t - 1];
-                if (inv) ww.y = -ww.y;
-                v[e][t] = cmul(v[e][t], ww);
-            }
-            C y[RAD];
-            if (RAD == 2) {
-                y[0] = cadd(v[e][0], v[e][1]);
-                y[1] = csub(v[e][0], v[e][1]);
-            } else if (RAD == 4) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) y[t] = v[e][t];
-                dft4(y, inv);
-            } else if (RAD == 8) {
-                dft8(v[e], y, inv);
-            } else {
-                dft16(v[e], y, inv);
-            }
-            if (RAD == 16 && Ns < 8) {
-                // the first radix-16 pass (Ns = 1): outputs 16 j + t straddle a
-                // padding element, so each takes its own padded index
-                C *q = buf + row * stride;
-                const int base = (j - k) << LR;
-#pragma unroll
-                for (int t = 0; t < RAD; ++t) q[lp(base + k + t * Ns)] = y[t];
-            } else {
-                C *q = buf + row * stride + lp(((j - k) << LR) + k);
-#pragma unroll
-                for (int t = 0; t < RAD; ++t) q[t * Nsp] = y[t];
-            }
-        }
-    }
-    __syncthreads();
-}
-
-// radix-3 butterfly, y = DFT3(v): W = exp(-+2 pi i / 3) = -1/2 -+ i sqrt(3)/2
-template <typename C>
-__device__ __forceinline__ void dft3(const C *v, C *y, bool inv) {
-    using R = decltype(C::x);
-    const R h = (R)0.86602540378443864676;  // sqrt(3)/2
-    const C s = cadd(v[1], v[2]), d = csub(v[1], v[2]);
-    const C m = cm<C>(v[0].x - (R)0.5 * s.x, v[0].y - (R)0.5 * s.y);
-    const C r = inv ? cm<C>(-h * d.y, h * d.x) : cm<C>(h * d.y, -h * d.x);  // (+-i) sqrt(3)/2 (v1 - v2)
-    y[0] = cadd(v[0], s);
-    y[1] = cadd(m, r);
-    y[2] = csub(m, r);
-}
-
-// radix-P butterfly for P = 5, 7 as the P-point DFT, y[u] = sum_t v[t] W^(tu
-// mod P), W = exp(-+2 pi i / P) = tw[Z / P] (conjugated for the inverse);
-// P divides Z.
-template <typename C, int P>
-__device__ __forceinline__ void dftp(const C *v, C *y, const C *__restrict__ tw, int Z, bool inv) {
-    const int zp = Z / P;
-    C w[P];
-#pragma unroll
-    for (int k = 0; k < P; ++k) {
-        w[k] = tw[k * zp];
-        if (inv) w[k].y = -w[k].y;
-    }
-#pragma unroll
-    for (int u = 0; u < P; ++u) {
-        C acc = v[0];
-#pragma unroll
-        for (int t = 1; t < P; ++t) acc = cadd(acc, cmul(v[t], w[(t * u) % P]));
-        y[u] = acc;
-    }
-}
-
-// One Stockham pass of radix RAD (2, 3, 4, 5, 7 or 8) over rows of any
-// length n divisible by RAD (the meshes whose size is not a power of two).
-// The same butterflies as fft_pass, with per-element LDS addresses (lp of
-// every index), exact integer division for the butterfly and row indices,
-// and every twiddle power loaded from the table: tw[t k Z / (Ns RAD)].
-// Inputs are read before the barrier, outputs written after it (in place).
-template <typename R, int EPT, int RAD>
-__device__ __forceinline__ void fft_pass_g(typename V2<R>::T *buf, int n, int nrows, int stride, int Ns,
-                                           const typename V2<R>::T *__restrict__ tw, int Z, bool inv) {
-    using C = typename V2<R>::T;
-    constexpr int NB = (EPT + RAD - 1) / RAD;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int nb = n / RAD, tot = nb * nrows;
-    const int twm = Z / (Ns * RAD);
-    const Dv dnb(nb), dns(Ns);
-    C v[NB][RAD];
-#pragma unroll
-    for (int e = 0; e < NB; ++e) {
-        const int b = tid + e * nt;
-        if (b < tot) {
-            const int row = dnb.q(b), j = b - row * nb;
-            const C *p = buf + row * stride;
-#pragma unroll
-            for (int t = 0; t < RAD; ++t) v[e][t] = p[lp(j + t * nb)];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < NB; ++e) {
-        const int b = tid + e * nt;
-        if (b < tot) {
-            const int row = dnb.q(b), j = b - row * nb;
-            const int k = dns.r(j);
-#pragma unroll
-            for (int t = 1; t < RAD; ++t) {
-                C ww = tw[t * k * twm];
-                if (inv) ww.y = -ww.y;
-                v[e][t] = cmul(v[e][t], ww);
-            }
-            C y[RAD];
-            if constexpr (RAD == 2) {
-                y[0] = cadd(v[e][0], v[e][1]);
-                y[1] = csub(v[e][0], v[e][1]);
-            } else if constexpr (RAD == 3) {
-                dft3(v[e], y, inv);
-            } else if constexpr (RAD == 4) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) y[t] = v[e][t];
-                dft4(y, inv);
-            } else if constexpr (RAD == 8) {
-                dft8(v[e], y, inv);
-            } else {
-                dftp<C, RAD>(v[e], y, tw, Z, inv);
-            }
-            C *q = buf + row * stride;
-            const int base = (j - k) * RAD + k;
-#pragma unroll
-            for (int t = 0; t < RAD; ++t) q[lp(base + t * Ns)] = y[t];
-        }
-    }
-    __syncthreads();
-}
-
-// Transform of rows of length n = 2^p 3^c 5^d 7^f: radix-8 passes over the
-// factor 2^p, one radix-4 or radix-2 pass for its remaining bits, then one
-// radix-3, -5 or -7 pass per odd factor.  A power-of-two n takes fft_pass
-// (below).
-template <typename R, int EPT>
-__device__ __forceinline__ void lds_fft_g(typename V2<R>::T *buf, int n, int nrows, int stride,
-                                          const typename V2<R>::T *__restrict__ tw, int Z, bool inv) {
-    int m = n, c3 = 0, c5 = 0, c7 = 0;
-    while (m % 3 == 0) {
-        m /= 3;
-        ++c3;
-    }
-    while (m % 5 == 0) {
-        m /= 5;
-        ++c5;
-    }
-    while (m % 7 == 0) {
-        m /= 7;
-        ++c7;
-    }
-    int Ns = 1;
-    while (m >= 8) {
-        fft_pass_g<R, EPT, 8>(buf, n, nrows, stride, Ns, tw, Z, inv);
-        Ns *= 8;
-        m /= 8;
-    }
-    if (m == 4) {
-        fft_pass_g<R, EPT, 4>(buf, n, nrows, stride, Ns, tw, Z, inv);
-        Ns *= 4;
-    } else if (m == 2) {
-        fft_pass_g<R, EPT, 2>(buf, n, nrows, stride, Ns, tw, Z, inv);
-        Ns *= 2;
-    }
-    for (; c3 > 0; --c3) {
-        fft_pass_g<R, EPT, 3>(buf, n, nrows, stride, Ns, tw, Z, inv);
-        Ns *= 3;
-    }
-    for (; c5 > 0; --c5) {
-        fft_pass_g<R, EPT, 5>(buf, n, nrows, stride, Ns, tw, Z, inv);
-        Ns *= 5;
-    }
-    for (; c7 > 0; --c7) {
-        fft_pass_g<R, EPT, 7>(buf, n, nrows, stride, Ns, tw, Z, inv);
-        Ns *= 7;
-    }
-}
-
-// rows of length n: the power-of-two passes below, or lds_fft_g when n has an
-// odd factor (tw holds exp(-2 pi i k / Z), k < Z; n divides Z).  R16: the
-// kernel's power-of-two rows take radix-16 passes (FP32); a kernel's choice
-// does not depend on its elements per thread, so neither does its rounding.
-template <typename R, int EPT, bool R16 = false, bool R16T = false>
-__device__ __forceinline__ void lds_fft_pow2(typename V2<R>::T *buf, int logn, int nrows, int stride,
-                                             const typename V2<R>::T *__restrict__ tw, int logZ, bool inv);
-template <typename R, int EPT>
-__device__ __forceinline__ void lds_fft(typename V2<R>::T *buf, int n, int nrows, int stride,
-                                        const typename V2<R>::T *__restrict__ tw, int Z, bool inv) {
-    if ((n & (n - 1)) == 0 && (Z & (Z - 1)) == 0)
-        lds_fft_pow2<R, EPT>(buf, __ffs(n) - 1, nrows, stride, tw, __ffs(Z) - 1, inv);
-    else
-        lds_fft_g<R, EPT>(buf, n, nrows, stride, tw, Z, inv);
-}
-// the same with the mesh kind known at compile time (P2: n and Z powers of two)
-template <typename R, int EPT, bool P2, bool R16 = false, bool R16T = false>
-__device__ __forceinline__ void lds_fft_t(typename V2<R>::T *buf, int n, int nrows, int stride,
-                                          const typename V2<R>::T *__restrict__ tw, int Z, bool inv) {
-    if (P2)
-        lds_fft_pow2<R, EPT, R16, R16T>(buf, __ffs(n) - 1, nrows, stride, tw, __ffs(Z) - 1, inv);
-    else
-        lds_fft_g<R, EPT>(buf, n, nrows, stride, tw, Z, inv);
-}
-
-// radix-8 passes (radix-16 passes with R16), then one pass of a smaller radix
-// for the remaining bits
-template <typename R, int EPT, bool R16, bool R16T>
-__device__ __forceinline__ void lds_fft_pow2(typename V2<R>::T *buf, int logn, int nrows, int stride,
-                                             const typename V2<R>::T *__restrict__ tw, int logZ, bool inv) {
-    int logNs = 0;
-    if constexpr (R16T && sizeof(R) == 4) {
-        // radix-8 passes, with the last 4 bits (when radix 8 would leave one
-        // bit for a radix-2 pass) in one radix-16 pass: 1024 points in passes
-        // of 8, 8 and 16
-        if (logn >= 7 && logn % 3 == 1) {
-            while (logn - logNs > 4) {
-                fft_pass<R, EPT, 8, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-                logNs += 3;
-            }
-            fft_pass<R, EPT, 16, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-            return;
-        }
-    }
-    if constexpr (R16 && sizeof(R) == 4) {
-        // FP32 rows of at least 128: radix-16 passes, then one pass of radix
-        // 8, 4 or 2 for the remaining bits (2048 points in 3 passes instead
-        // of 4)
-        if (logn >= 7) {
-            while (logn - logNs >= 4) {
-                fft_pass<R, EPT, 16, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-                logNs += 4;
-            }
-            const int rem = logn - logNs;
-            if (rem == 3)
-                fft_pass<R, EPT, 8, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-            else if (rem == 2)
-                fft_pass<R, EPT, 4, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-            else if (rem == 1)
-                fft_pass<R, EPT, 2, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-            return;
-        }
-    }
-    const bool small8 = logn - 3 < 3;  // nb = n/8 below 8
-    while (logn - logNs >= 3) {
-        if (small8)
-            fft_pass<R, EPT, 8, true>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-        else
-            fft_pass<R, EPT, 8, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-        logNs += 3;
-    }
-    if (logn - logNs == 2) {
-        if (logn - 2 < 3)
-            fft_pass<R, EPT, 4, true>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-        else
-            fft_pass<R, EPT, 4, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-    } else if (logn - logNs == 1) {
-        if (logn - 1 < 3)
-            fft_pass<R, EPT, 2, true>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-        else
-            fft_pass<R, EPT, 2, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-    }
-}
-
-constexpr int FFT_THREADS = 256;
 
 // Row r2c: rows k0..k0+RB-1 of the real mesh -> half spectrum X[m], m<Z/2,
 // with X[0] packing (DC, Nyquist) (both real), written transposed:
@@ -2431,12 +1688,6 @@ static const int *fft_ept_default() {
     return v;
 }
 
-static int ept_for(int want, int need) {
-    int e = want;
-    while (e * FFT_THREADS < need && e < 32) e *= 2;
-    return e;
-}
-
 // the largest divisor of m not above cap (at least 1)
 static int div_at_most(int m, int cap) {
     cap = std::max(1, std::min(m, cap));
@@ -2651,17 +1902,30 @@ hipError_t launch_deposit(bdk_t *h, int reset, int slot, hipStream_t st) {
     return hipGetLastError();
 }
 
+// number density of one species (charges 1 and 0) -> rho, from the list order
+hipError_t launch_species_deposit(bdk_t *h, int species) {
+    DepPlan pl = dep_plan(h, 0);
+    pl.a.q1 = species == 1 ? 1.0 : 0.0;
+    pl.a.q2 = species == 2 ? 1.0 : 0.0;
+    hipStream_t st = h->stream;
+    const bool f32 = h->p.precision != BDK_FP64;
+    switch (h->g.scheme) {
+    case 0: f32 ? launch_deposit_t<float, 0>(h, pl, st) : launch_deposit_t<double, 0>(h, pl, st); break;
+    case 1: f32 ? launch_deposit_t<float, 1>(h, pl, st) : launch_deposit_t<double, 1>(h, pl, st); break;
+    default: f32 ? launch_deposit_t<float, 2>(h, pl, st) : launch_deposit_t<double, 2>(h, pl, st); break;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_zero_ints(int *p, int n, hipStream_t st) {
+    hipLaunchKernelGGL(k_zero_int, dim3(nblk(n, 256)), dim3(256), 0, st, p, n);
+    return hipGetLastError();
+}
+
 hipError_t launch_rearm(bdk_t *h) {
     hipLaunchKernelGGL(k_rearm, dim3(1), dim3(64), 0, h->stream, h->g, h->d);
     return hipGetLastError();
 }
-
-#define BDK_EPT_SWITCH(E, CALL) \
-    switch (E) {                \
-    case 8: CALL(8); break;     \
-    case 16: CALL(16); break;   \
-    default: CALL(32); break;   \
-    }
 
 template <typename R, bool Q, bool R16> static void launch_fft_tq(bdk_t *h, int only, hipStream_t st, int end_step) {
     using C = typename V2<R>::T;
@@ -2798,439 +2062,6 @@ hipError_t launch_refresh(bdk_t *h) {
 hipError_t launch_noise_out(bdk_t *h) {
     hipLaunchKernelGGL(k_noise_out, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d);
     return hipGetLastError();
-}
-
-// rho(k) of one species (record_rhoFFTW, auswertung.cpp:529-626): the
-// species' number density (weights drho, gridRoutinen.cpp:672-1040) is
-// transformed (r2c rows + this column pass), multiplied by (-1)^(i+j)
-// (the origin moved to the box centre) and the real parts are summed over
-// shells bin = (int)(dq_dqFT |k|/dq + 1/2) of the full Z x Z plane: a
-// column m of the half spectrum stands for itself and its mirror
-// (Z-j, Z-m), whose conjugate adds the same real part (the imaginary parts
-// cancel).  One thread per column sums in a fixed order into that column's
-// partial row; k_rhok_final adds the partial rows in order.
-template <typename R, int EPT>
-__global__ __launch_bounds__(FFT_THREADS) void k_col_rhok(const typename V2<R>::T *__restrict__ ht,
-                                                          const typename V2<R>::T *__restrict__ tw, int Z,
-                                                          double dqr, int nbins, double *part) {
-    using C = typename V2<R>::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    const int m = blockIdx.x, tid = threadIdx.x, Zh = Z >> 1;
-    for (int k = tid; k < Z; k += blockDim.x) s[lp(k)] = ht[(size_t)m * Z + k];
-    double *p0 = part + (size_t)m * nbins, *pn = part + (size_t)Zh * nbins;
-    for (int b = tid; b < nbins; b += blockDim.x) {
-        p0[b] = 0.0;
-        if (m == 0) pn[b] = 0.0;
-    }
-    __syncthreads();
-    lds_fft<R, EPT>(s, Z, 1, lds_row(Z), tw, Z, false);
-    if (tid != 0) return;
-    for (int j = 0; j < Z; ++j) {
-        const double xq = (double)(wrap1(j + Zh, Z) - Zh);
-        const double sg = ((j + m) & 1) ? -1.0 : 1.0;
-        if (m > 0) {
-            const int bin = (int)(dqr * sqrt(xq * xq + (double)m * m) + 0.5);
-            if (bin < nbins) p0[bin] += 2.0 * sg * (double)s[lp(j)].x;
-        } else {
-            const C P = s[lp(j)], Q = s[lp(j == 0 ? 0 : Z - j)];
-            const double dc = 0.5 * ((double)P.x + (double)Q.x);  // Re of the DC column
-            const double ny = 0.5 * ((double)P.y + (double)Q.y);  // Re of the Nyquist column
-            int bin = (int)(dqr * sqrt(xq * xq) + 0.5);
-            if (bin < nbins) p0[bin] += sg * dc;
-            bin = (int)(dqr * sqrt(xq * xq + (double)Zh * Zh) + 0.5);
-            if (bin < nbins) pn[bin] += sg * ny;  // (-1)^(j + Z/2) = (-1)^j
-        }
-    }
-}
-
-__global__ void k_rhok_final(const double *part, int ncol, int nbins, double *out) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbins) return;
-    double v = 0.0;
-    for (int m = 0; m < ncol; ++m) v += part[(size_t)m * nbins + b];
-    out[b] = v;
-}
-
-template <typename R> static void launch_rhok_t(bdk_t *h, double dqr, int nbins, double *part, double *out) {
-    using C = typename V2<R>::T;
-    const int Z = h->g.Z;
-    const int ept = ept_for(8, Z);
-    const size_t lds = (size_t)lds_row(Z) * sizeof(C);
-#define RHOK(E)                                                                                              \
-    (void)hipFuncSetAttribute((const void *)k_col_rhok<R, E>, hipFuncAttributeMaxDynamicSharedMemorySize,      \
-                              160 * 1024);                                                                     \
-    hipLaunchKernelGGL((k_col_rhok<R, E>), dim3(Z / 2), dim3(FFT_THREADS), lds, h->stream, (const C *)h->d.ht, \
-                       (const C *)h->d.tw, Z, dqr, nbins, part)
-    BDK_EPT_SWITCH(ept, RHOK)
-#undef RHOK
-    hipLaunchKernelGGL(k_rhok_final, dim3(nblk(nbins, 256)), dim3(256), 0, h->stream, part, Z / 2 + 1, nbins, out);
-}
-
-// species density (weights q1, q2 per species) -> rho, r2c rows, column pass + shells
-hipError_t launch_rhok(bdk_t *h, int species, double dqr, int nbins, double *part, double *out) {
-    DepPlan pl = dep_plan(h, 0);
-    pl.a.q1 = species == 1 ? 1.0 : 0.0;
-    pl.a.q2 = species == 2 ? 1.0 : 0.0;
-    hipStream_t st = h->stream;
-    const bool f32 = h->p.precision != BDK_FP64;
-    switch (h->g.scheme) {
-    case 0: f32 ? launch_deposit_t<float, 0>(h, pl, st) : launch_deposit_t<double, 0>(h, pl, st); break;
-    case 1: f32 ? launch_deposit_t<float, 1>(h, pl, st) : launch_deposit_t<double, 1>(h, pl, st); break;
-    default: f32 ? launch_deposit_t<float, 2>(h, pl, st) : launch_deposit_t<double, 2>(h, pl, st); break;
-    }
-    hipError_t e = launch_fft_pass(h, 0);
-    if (e != hipSuccess) return e;
-    if (f32)
-        launch_rhok_t<float>(h, dqr, nbins, part, out);
-    else
-        launch_rhok_t<double>(h, dqr, nbins, part, out);
-    return hipGetLastError();
-}
-
-// Pair correlation g11, g12, g22 (record_korrelationsfunktion11/12/22,
-// auswertung.cpp:110-188): minimum-image distances (abstand2, am:100-166)
-// of all pairs closer than nbins*dr, found through the cells within R cells,
-// binned by (int)(r/dr).  Ordered pairs (12 pairs from the species-1 side)
-// are counted with integer atomics in LDS per block, then added to the
-// global histograms: the counts are exact and deterministic.
-__global__ __launch_bounds__(256) void k_pair_hist(Geo g, DevBufs d, int nbins, double dr, int R,
-                                                   unsigned long long *hist) {
-    extern __shared__ unsigned int shist[];  // [3][nbins]
-    for (int b = threadIdx.x; b < 3 * nbins; b += blockDim.x) shist[b] = 0u;
-    __syncthreads();
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < g.N) {
-        const int nc = g.nc, c = d.lcell[q];
-        const int cx = div_nc(c, g), cy = c - cx * nc;
-        const double2 ri = d.lrel[q];
-        const double xi = cx * g.B + ri.x, yi = cy * g.B + ri.y, L = g.L;
-        const bool s2i = d.lpid[q] >= g.n1;
-        const bool all = 2 * R + 1 >= nc;
-        const int a0 = all ? 0 : cx - R, a1 = all ? nc - 1 : cx + R;
-        const int b0 = all ? 0 : cy - R, b1 = all ? nc - 1 : cy + R;
-        for (int a = a0; a <= a1; ++a) {
-            const int ux = wrapc(a, nc);
-            for (int b = b0; b <= b1; ++b) {
-                const int uy = wrapc(b, nc), cc = ux * nc + uy;
-                const int qe = d.start[cc + 1];
-                for (int j = d.start[cc]; j < qe; ++j) {
-                    if (j == q) continue;
-                    const bool s2j = d.lpid[j] >= g.n1;
-                    if (s2i && !s2j) continue;
-                    const double2 rj = d.lrel[j];
-                    double t1 = xi - (ux * g.B + rj.x), t2 = t1 + L, t3 = t1 - L;
-                    double m = t3 * t3 < t2 * t2 ? t3 * t3 : t2 * t2;
-                    const double dx2 = m < t1 * t1 ? m : t1 * t1;
-                    t1 = yi - (uy * g.B + rj.y);
-                    t2 = t1 + L;
-                    t3 = t1 - L;
-                    m = t3 * t3 < t2 * t2 ? t3 * t3 : t2 * t2;
-                    const double dy2 = m < t1 * t1 ? m : t1 * t1;
-                    const int idx = (int)(sqrt(dx2 + dy2) / dr);
-                    if (idx < 0 || idx >= nbins) continue;
-                    const int type = s2i ? 2 : (s2j ? 1 : 0);
-                    atomicAdd(&shist[type * nbins + idx], 1u);
-                }
-            }
-        }
-    }
-    __syncthreads();
-    for (int b = threadIdx.x; b < 3 * nbins; b += blockDim.x)
-        if (shist[b]) atomicAdd(&hist[b], (unsigned long long)shist[b]);
-}
-
-hipError_t launch_pair_hist(bdk_t *h, int nbins, double dr, unsigned long long *hist) {
-    int R = (int)ceil(nbins * dr / h->g.B);
-    if (R < 1) R = 1;
-    const size_t lds = (size_t)3 * nbins * sizeof(unsigned int);
-    (void)hipFuncSetAttribute((const void *)k_pair_hist, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-    hipLaunchKernelGGL(k_pair_hist, dim3(nblk(h->g.N, 256)), dim3(256), lds, h->stream, h->g, h->d, nbins, dr, R,
-                       hist);
-    return hipGetLastError();
-}
-
-// ------------------------------------------------------------------ observables
-// Radial density profiles of the blob (berechne_dichteprofile,
-// observablen_auswertung.cpp:227-330) around the circular-mean centres of
-// the species (berechne_mittelpunkte, observablen_auswertung.cpp:140-223).
-// Sums use a fixed-order reduction (per-block tree, then one block over the
-// block partials in order) and the histograms integer atomics, so the
-// result is deterministic.
-constexpr int OBS_THREADS = 256;
-
-// block partial sums of cos/sin(2 pi x / L), cos/sin(2 pi y / L) per species
-__global__ __launch_bounds__(OBS_THREADS) void k_circ_partial(Geo g, DevBufs d, double *part) {
-    __shared__ double sm[OBS_THREADS][8];
-    const int q = blockIdx.x * OBS_THREADS + threadIdx.x;
-    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (q < g.N) {
-        const int c = d.lcell[q];
-        const int gx = div_nc(c, g), gy = c - gx * g.nc;
-        const double2 r = d.lrel[q];
-        const double k = 2.0 * M_PI / g.L;
-        const double x = gx * g.B + r.x, y = gy * g.B + r.y;
-        const int o = d.lpid[q] >= g.n1 ? 4 : 0;
-        v[o + 0] = cos(x * k);
-        v[o + 1] = sin(x * k);
-        v[o + 2] = cos(y * k);
-        v[o + 3] = sin(y * k);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sm[threadIdx.x][i] = v[i];
-    __syncthreads();
-    for (int w = OBS_THREADS / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) sm[threadIdx.x][i] += sm[threadIdx.x + w][i];
-        __syncthreads();
-    }
-    if (threadIdx.x < 8) part[blockIdx.x * 8 + threadIdx.x] = sm[0][threadIdx.x];
-}
-
-// centres S1, S2, Sgamma = (S1+S2)/2 from the block partials (one block)
-__global__ __launch_bounds__(OBS_THREADS) void k_circ_final(Geo g, const double *part, int nb, double *centers) {
-    __shared__ double sm[OBS_THREADS][8];
-    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int b = threadIdx.x; b < nb; b += OBS_THREADS)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] += part[b * 8 + i];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sm[threadIdx.x][i] = v[i];
-    __syncthreads();
-    for (int w = OBS_THREADS / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) sm[threadIdx.x][i] += sm[threadIdx.x + w][i];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const double k = 2.0 * M_PI / g.L;
-        double S[4];
-        for (int a = 0; a < 4; ++a)  // (S1x, S1y, S2x, S2y)
-            S[a] = (atan2(-sm[0][2 * a + 1], -sm[0][2 * a]) + M_PI) / k;
-        centers[0] = S[0];
-        centers[1] = S[1];
-        centers[2] = S[2];
-        centers[3] = S[3];
-        centers[4] = 0.5 * (S[0] + S[2]);
-        centers[5] = 0.5 * (S[1] + S[3]);
-    }
-}
-
-// counts per bin: rho1ring (Sgamma), rho2ring (S2), rho1zen1, rho1zen2,
-// rho2zen1, rho2zen2; distances without periodic images, beyond the last
-// bin into the last bin (as the reference)
-__global__ __launch_bounds__(OBS_THREADS) void k_radial_hist(Geo g, DevBufs d, const double *centers, int nbins,
-                                                             double dr, int *hist) {
-    const int q = blockIdx.x * OBS_THREADS + threadIdx.x;
-    if (q >= g.N) return;
-    const int c = d.lcell[q];
-    const int gx = div_nc(c, g), gy = c - gx * g.nc;
-    const double2 r = d.lrel[q];
-    const double x = gx * g.B + r.x, y = gy * g.B + r.y;
-    const bool s2 = d.lpid[q] >= g.n1;
-    // (histogram, centre index) pairs of this species
-    const int hs[3] = {s2 ? 1 : 0, s2 ? 4 : 2, s2 ? 5 : 3};
-    const int cs[3] = {s2 ? 1 : 2, 0, 1};  // 0: S1, 1: S2, 2: Sgamma
-    for (int i = 0; i < 3; ++i) {
-        const double dx = x - centers[2 * cs[i]], dy = y - centers[2 * cs[i] + 1];
-        const double rr = sqrt(dx * dx + dy * dy);
-        int bin = (int)(rr / dr);
-        if (bin < 0 || bin >= nbins) bin = nbins - 1;
-        atomicAdd(&hist[hs[i] * nbins + bin], 1);
-    }
-}
-
-hipError_t launch_radial(bdk_t *h, int nbins, double dr, double *part, double *centers, int *hist) {
-    const int nb = (int)nblk(h->g.N, OBS_THREADS);
-    hipLaunchKernelGGL(k_circ_partial, dim3(nb), dim3(OBS_THREADS), 0, h->stream, h->g, h->d, part);
-    hipLaunchKernelGGL(k_circ_final, dim3(1), dim3(OBS_THREADS), 0, h->stream, h->g, part, nb, centers);
-    hipLaunchKernelGGL(k_zero_int, dim3(nblk(6 * nbins, 256)), dim3(256), 0, h->stream, hist, 6 * nbins);
-    hipLaunchKernelGGL(k_radial_hist, dim3(nb), dim3(OBS_THREADS), 0, h->stream, h->g, h->d, centers, nbins, dr,
-                       hist);
-    return hipGetLastError();
-}
-
-// ------------------------------------------------------------------ snapshot grid
-// Local densities on an m x m grid of width w = L/m (main_auswertung.cpp:
-// 214-320): each particle adds its TSC weights times 1/w^2 to the nine cells
-// around cell (int)(x/w) mod m of its species' grid.  The weight products are
-// summed as 2^-40 fixed point in 64-bit integers, so the grid does not depend
-// on the order of the additions.  The offset d from the cell centre uses the
-// unwrapped cell index (the reference wraps first, which only differs when
-// x/w rounds up to m).
-constexpr double SNAP_SCALE = 1099511627776.0;  // 2^40
-
-__device__ __forceinline__ void snap_tsc(double x, double w, int m, int &k, double wt[3]) {
-    const int k0 = (int)(x / w);
-    k = k0 % m;
-    const double dd = x - (k0 + 0.5) * w;
-    wt[1] = 0.75 - dd * dd / (w * w);
-    double t = fabs((dd + w) / w);
-    wt[0] = 0.5 * (1.5 - t) * (1.5 - t);
-    t = fabs((dd - w) / w);
-    wt[2] = 0.5 * (1.5 - t) * (1.5 - t);
-}
-
-__global__ __launch_bounds__(256) void k_snap_grid(Geo g, DevBufs d, int m, double w, unsigned long long *acc) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= g.N) return;
-    const int c = d.lcell[q];
-    const int gx = div_nc(c, g), gy = c - gx * g.nc;
-    const double2 r = d.lrel[q];
-    int k, l;
-    double wx[3], wy[3];
-    snap_tsc(gx * g.B + r.x, w, m, k, wx);
-    snap_tsc(gy * g.B + r.y, w, m, l, wy);
-    unsigned long long *a = acc + (d.lpid[q] >= g.n1 ? (size_t)m * m : 0);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const size_t row = (size_t)((k - 1 + i + m) % m) * m;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const long long v = __double2ll_rn(wx[i] * wy[j] * SNAP_SCALE);
-            atomicAdd(&a[row + (l - 1 + j + m) % m], (unsigned long long)v);
-        }
-    }
-}
-
-// fixed point -> densities; with stats: the histograms of rho1, rho2,
-// rho = rho1 + rho2 and rho1 - rho2 and the cells over the thresholds
-// (main_auswertung.cpp:324-375), counted per block in LDS.
-// cnt: [4][nbins] histograms, then 7 threshold counts.
-__device__ __forceinline__ int snap_bin(double t, int nbins) {
-    if (!(t > -1.0)) return 0;  // (int) truncates toward zero; below 0 clamps to 0
-    if (t >= (double)nbins) return nbins - 1;
-    const int b = (int)t;
-    return b < 0 ? 0 : (b >= nbins ? nbins - 1 : b);
-}
-
-__global__ __launch_bounds__(256) void k_snap_final(int m, double drho, const unsigned long long *acc, double *rho,
-                                                    int stats, int nbins, double dbin, SnapThresh th,
-                                                    unsigned int *cnt) {
-    extern __shared__ unsigned int sh[];  // [4 * nbins + 7]
-    const int nsh = 4 * nbins + 7;
-    if (stats)
-        for (int i = threadIdx.x; i < nsh; i += blockDim.x) sh[i] = 0u;
-    __syncthreads();
-    const size_t mm = (size_t)m * m;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < mm; i += stride) {
-        const double r1 = ((double)acc[i] / SNAP_SCALE) * drho;
-        const double r2 = ((double)acc[mm + i] / SNAP_SCALE) * drho;
-        rho[i] = r1;
-        rho[mm + i] = r2;
-        if (!stats) continue;
-        const double rs = r1 + r2, dr = r1 - r2;
-        for (int t = 0; t < 3; ++t)
-            if (rs > th.rho[t]) atomicAdd(&sh[4 * nbins + t], 1u);
-        const double f = rs > 0.0 ? fabs(dr) / rs : 0.0;  // 0/0 passes no threshold
-        for (int t = 0; t < 4; ++t)
-            if (rs > 0.0 && f > th.drho[t]) atomicAdd(&sh[4 * nbins + 3 + t], 1u);
-        atomicAdd(&sh[snap_bin(r1 / dbin - 0.5, nbins)], 1u);
-        atomicAdd(&sh[nbins + snap_bin(r2 / dbin - 0.5, nbins)], 1u);
-        atomicAdd(&sh[2 * nbins + snap_bin(rs / dbin - 0.5, nbins)], 1u);
-        atomicAdd(&sh[3 * nbins + snap_bin(dr / dbin - 0.5 + (double)(nbins / 2), nbins)], 1u);
-    }
-    if (!stats) return;
-    __syncthreads();
-    for (int i = threadIdx.x; i < nsh; i += blockDim.x)
-        if (sh[i]) atomicAdd(&cnt[i], sh[i]);
-}
-
-hipError_t launch_snap(bdk_t *h, int m, unsigned long long *acc, double *rho, int stats, int nbins, double dbin,
-                       SnapThresh th, unsigned int *cnt) {
-    const double w = h->p.L / m;
-    hipLaunchKernelGGL(k_snap_grid, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d, m, w, acc);
-    const size_t mm = (size_t)m * m;
-    const int nb = (int)std::min<size_t>(nblk(mm, 256), 4096);
-    const size_t lds = stats ? (size_t)(4 * nbins + 7) * sizeof(unsigned int) : 0;
-    hipLaunchKernelGGL(k_snap_final, dim3(nb), dim3(256), lds, h->stream, m, 1.0 / (w * w), acc, rho, stats, nbins,
-                       dbin, th, cnt);
-    return hipGetLastError();
-}
-
-// ------------------------------------------------------------------ direct rho(k)
-// record_ftrho_unkorrigiert (au:307-360): for each wave-vector index pair
-// (i, j) the sums over one species of cos and sin(dq (x i + y j)).  For
-// species 1 the reference takes y = git_y B + rel_x (au:333), unless the
-// parameters ask for rel_y (ftrho_fix); species 2 uses rel_y.  Block (chunk,
-// pair): a fixed-order tree sum over the chunk's particles into
-// partial[pair][chunk]; k_ftrho_final adds the chunks in order.
-constexpr int FT_THREADS = 256, FT_PER_THREAD = 16, FT_MAX_CHUNKS = 64;
-
-// chunk `chunk` of nchunk covers list positions [chunk per, (chunk + 1) per);
-// per is a multiple of FT_THREADS, and nchunk is at most FT_MAX_CHUNKS, so
-// the partial sums stay small at any N.  fix: species 1 takes rel_y.
-__global__ __launch_bounds__(FT_THREADS) void k_ftrho(Geo g, DevBufs d, const int2 *ij, int species, int fix,
-                                                      double dq, double2 *partial, int nchunk, int per) {
-    __shared__ double sc[FT_THREADS], ss[FT_THREADS];
-    const int p = blockIdx.y, chunk = blockIdx.x, tid = threadIdx.x;
-    const int2 q = ij[p];
-    double c = 0.0, s = 0.0;
-    const int q0 = chunk * per, q1 = min(q0 + per, g.N);
-    for (int t = q0 + tid; t < q1; t += FT_THREADS) {
-        const bool s2 = d.lpid[t] >= g.n1;
-        if (s2 != (species == 2)) continue;
-        const int cell = d.lcell[t];
-        const int gx = div_nc(cell, g), gy = cell - gx * g.nc;
-        const double2 r = d.lrel[t];
-        const double x = gx * g.B + r.x;
-        const double y = gy * g.B + ((species == 1 && !fix) ? r.x : r.y);
-        double sn, cs;
-        sincos(dq * (x * q.x + y * q.y), &sn, &cs);
-        c += cs;
-        s += sn;
-    }
-    sc[tid] = c;
-    ss[tid] = s;
-    __syncthreads();
-    for (int w = FT_THREADS / 2; w > 0; w >>= 1) {
-        if (tid < w) {
-            sc[tid] += sc[tid + w];
-            ss[tid] += ss[tid + w];
-        }
-        __syncthreads();
-    }
-    if (tid == 0) partial[(size_t)p * nchunk + chunk] = make_double2(sc[0], ss[0]);
-}
-
-__global__ void k_ftrho_final(const double2 *partial, int nchunk, int npairs, double *re, double *im) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npairs) return;
-    double c = 0.0, s = 0.0;
-    for (int k = 0; k < nchunk; ++k) {
-        const double2 v = partial[(size_t)p * nchunk + k];
-        c += v.x;
-        s += v.y;
-    }
-    re[p] = c;
-    im[p] = s;
-}
-
-// chunks of at least FT_THREADS * FT_PER_THREAD positions, at most FT_MAX_CHUNKS
-static void ftrho_split(const bdk_t *h, int &nchunk, int &per) {
-    nchunk = std::min((int)nblk(h->g.N, FT_THREADS * FT_PER_THREAD), FT_MAX_CHUNKS);
-    per = (int)nblk(h->g.N, nchunk * FT_THREADS) * FT_THREADS;
-    nchunk = std::max(1, (int)nblk(h->g.N, per));
-}
-
-hipError_t launch_ftrho(bdk_t *h, const int2 *ij, int npairs, int species, double dq, double2 *partial, double *re,
-                        double *im) {
-    int nchunk, per;
-    ftrho_split(h, nchunk, per);
-    hipLaunchKernelGGL(k_ftrho, dim3(nchunk, npairs), dim3(FT_THREADS), 0, h->stream, h->g, h->d, ij, species,
-                       h->p.ftrho_fix ? 1 : 0, dq, partial, nchunk, per);
-    hipLaunchKernelGGL(k_ftrho_final, dim3(nblk(npairs, 256)), dim3(256), 0, h->stream, partial, nchunk, npairs, re,
-                       im);
-    return hipGetLastError();
-}
-
-int ftrho_chunks(const bdk_t *h) {
-    int nchunk, per;
-    ftrho_split(h, nchunk, per);
-    return nchunk;
 }
 
 // ------------------------------------------------------------------ step counters

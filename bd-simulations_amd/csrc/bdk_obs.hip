@@ -1,0 +1,437 @@
+// Device observables: rho(k) by FFT and by direct sums, pair correlations,
+// radial profiles, the snapshot density grid.
+#pragma clang fp contract(off)
+
+#include "bdk_device.hpp"
+#include "bdk_fft.hpp"
+
+namespace bdkx {
+
+static inline unsigned nblk(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
+
+// rho(k) of one species (record_rhoFFTW, auswertung.cpp:529-626): the
+// species' number density (weights drho, gridRoutinen.cpp:672-1040) is
+// transformed (r2c rows + this column pass), multiplied by (-1)^(i+j)
+// (the origin moved to the box centre) and the real parts are summed over
+// shells bin = (int)(dq_dqFT |k|/dq + 1/2) of the full Z x Z plane: a
+// column m of the half spectrum stands for itself and its mirror
+// (Z-j, Z-m), whose conjugate adds the same real part (the imaginary parts
+// cancel).  One thread per column sums in a fixed order into that column's
+// partial row; k_rhok_final adds the partial rows in order.
+template <typename R, int EPT>
+__global__ __launch_bounds__(FFT_THREADS) void k_col_rhok(const typename V2<R>::T *__restrict__ ht,
+                                                          const typename V2<R>::T *__restrict__ tw, int Z,
+                                                          double dqr, int nbins, double *part) {
+    using C = typename V2<R>::T;
+    extern __shared__ unsigned char smem_raw[];
+    C *s = (C *)smem_raw;
+    const int m = blockIdx.x, tid = threadIdx.x, Zh = Z >> 1;
+    for (int k = tid; k < Z; k += blockDim.x) s[lp(k)] = ht[(size_t)m * Z + k];
+    double *p0 = part + (size_t)m * nbins, *pn = part + (size_t)Zh * nbins;
+    for (int b = tid; b < nbins; b += blockDim.x) {
+        p0[b] = 0.0;
+        if (m == 0) pn[b] = 0.0;
+    }
+    __syncthreads();
+    lds_fft<R, EPT>(s, Z, 1, lds_row(Z), tw, Z, false);
+    if (tid != 0) return;
+    for (int j = 0; j < Z; ++j) {
+        const double xq = (double)(wrap1(j + Zh, Z) - Zh);
+        const double sg = ((j + m) & 1) ? -1.0 : 1.0;
+        if (m > 0) {
+            const int bin = (int)(dqr * sqrt(xq * xq + (double)m * m) + 0.5);
+            if (bin < nbins) p0[bin] += 2.0 * sg * (double)s[lp(j)].x;
+        } else {
+            const C P = s[lp(j)], Q = s[lp(j == 0 ? 0 : Z - j)];
+            const double dc = 0.5 * ((double)P.x + (double)Q.x);  // Re of the DC column
+            const double ny = 0.5 * ((double)P.y + (double)Q.y);  // Re of the Nyquist column
+            int bin = (int)(dqr * sqrt(xq * xq) + 0.5);
+            if (bin < nbins) p0[bin] += sg * dc;
+            bin = (int)(dqr * sqrt(xq * xq + (double)Zh * Zh) + 0.5);
+            if (bin < nbins) pn[bin] += sg * ny;  // (-1)^(j + Z/2) = (-1)^j
+        }
+    }
+}
+
+__global__ void k_rhok_final(const double *part, int ncol, int nbins, double *out) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= nbins) return;
+    double v = 0.0;
+    for (int m = 0; m < ncol; ++m) v += part[(size_t)m * nbins + b];
+    out[b] = v;
+}
+
+template <typename R> static void launch_rhok_t(bdk_t *h, double dqr, int nbins, double *part, double *out) {
+    using C = typename V2<R>::T;
+    const int Z = h->g.Z;
+    const int ept = ept_for(8, Z);
+    const size_t lds = (size_t)lds_row(Z) * sizeof(C);
+#define RHOK(E)                                                                                              \
+    (void)hipFuncSetAttribute((const void *)k_col_rhok<R, E>, hipFuncAttributeMaxDynamicSharedMemorySize,      \
+                              160 * 1024);                                                                     \
+    hipLaunchKernelGGL((k_col_rhok<R, E>), dim3(Z / 2), dim3(FFT_THREADS), lds, h->stream, (const C *)h->d.ht, \
+                       (const C *)h->d.tw, Z, dqr, nbins, part)
+    BDK_EPT_SWITCH(ept, RHOK)
+#undef RHOK
+    hipLaunchKernelGGL(k_rhok_final, dim3(nblk(nbins, 256)), dim3(256), 0, h->stream, part, Z / 2 + 1, nbins, out);
+}
+
+// species density -> rho, r2c rows, column pass + shells
+hipError_t launch_rhok(bdk_t *h, int species, double dqr, int nbins, double *part, double *out) {
+    hipError_t e = launch_species_deposit(h, species);
+    if (e == hipSuccess) e = launch_fft_pass(h, 0);
+    if (e != hipSuccess) return e;
+    if (h->p.precision != BDK_FP64)
+        launch_rhok_t<float>(h, dqr, nbins, part, out);
+    else
+        launch_rhok_t<double>(h, dqr, nbins, part, out);
+    return hipGetLastError();
+}
+
+// Pair correlation g11, g12, g22 (record_korrelationsfunktion11/12/22,
+// auswertung.cpp:110-188): minimum-image distances (abstand2, am:100-166)
+// of all pairs closer than nbins*dr, found through the cells within R cells,
+// binned by (int)(r/dr).  Ordered pairs (12 pairs from the species-1 side)
+// are counted with integer atomics in LDS per block, then added to the
+// global histograms: the counts are exact and deterministic.
+__global__ __launch_bounds__(256) void k_pair_hist(Geo g, DevBufs d, int nbins, double dr, int R,
+                                                   unsigned long long *hist) {
+    extern __shared__ unsigned int shist[];  // [3][nbins]
+    for (int b = threadIdx.x; b < 3 * nbins; b += blockDim.x) shist[b] = 0u;
+    __syncthreads();
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < g.N) {
+        const int nc = g.nc, c = d.lcell[q];
+        const int cx = div_nc(c, g), cy = c - cx * nc;
+        const double2 ri = d.lrel[q];
+        const double xi = cx * g.B + ri.x, yi = cy * g.B + ri.y, L = g.L;
+        const bool s2i = d.lpid[q] >= g.n1;
+        const bool all = 2 * R + 1 >= nc;
+        const int a0 = all ? 0 : cx - R, a1 = all ? nc - 1 : cx + R;
+        const int b0 = all ? 0 : cy - R, b1 = all ? nc - 1 : cy + R;
+        for (int a = a0; a <= a1; ++a) {
+            const int ux = wrapc(a, nc);
+            for (int b = b0; b <= b1; ++b) {
+                const int uy = wrapc(b, nc), cc = ux * nc + uy;
+                const int qe = d.start[cc + 1];
+                for (int j = d.start[cc]; j < qe; ++j) {
+                    if (j == q) continue;
+                    const bool s2j = d.lpid[j] >= g.n1;
+                    if (s2i && !s2j) continue;
+                    const double2 rj = d.lrel[j];
+                    double t1 = xi - (ux * g.B + rj.x), t2 = t1 + L, t3 = t1 - L;
+                    double m = t3 * t3 < t2 * t2 ? t3 * t3 : t2 * t2;
+                    const double dx2 = m < t1 * t1 ? m : t1 * t1;
+                    t1 = yi - (uy * g.B + rj.y);
+                    t2 = t1 + L;
+                    t3 = t1 - L;
+                    m = t3 * t3 < t2 * t2 ? t3 * t3 : t2 * t2;
+                    const double dy2 = m < t1 * t1 ? m : t1 * t1;
+                    const int idx = (int)(sqrt(dx2 + dy2) / dr);
+                    if (idx < 0 || idx >= nbins) continue;
+                    const int type = s2i ? 2 : (s2j ? 1 : 0);
+                    atomicAdd(&shist[type * nbins + idx], 1u);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < 3 * nbins; b += blockDim.x)
+        if (shist[b]) atomicAdd(&hist[b], (unsigned long long)shist[b]);
+}
+
+hipError_t launch_pair_hist(bdk_t *h, int nbins, double dr, unsigned long long *hist) {
+    int R = (int)ceil(nbins * dr / h->g.B);
+    if (R < 1) R = 1;
+    const size_t lds = (size_t)3 * nbins * sizeof(unsigned int);
+    (void)hipFuncSetAttribute((const void *)k_pair_hist, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
+    hipLaunchKernelGGL(k_pair_hist, dim3(nblk(h->g.N, 256)), dim3(256), lds, h->stream, h->g, h->d, nbins, dr, R,
+                       hist);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------ observables
+// Radial density profiles of the blob (berechne_dichteprofile,
+// observablen_auswertung.cpp:227-330) around the circular-mean centres of
+// the species (berechne_mittelpunkte, observablen_auswertung.cpp:140-223).
+// Sums use a fixed-order reduction (per-block tree, then one block over the
+// block partials in order) and the histograms integer atomics, so the
+// result is deterministic.
+constexpr int OBS_THREADS = 256;
+
+// block partial sums of cos/sin(2 pi x / L), cos/sin(2 pi y / L) per species
+__global__ __launch_bounds__(OBS_THREADS) void k_circ_partial(Geo g, DevBufs d, double *part) {
+    __shared__ double sm[OBS_THREADS][8];
+    const int q = blockIdx.x * OBS_THREADS + threadIdx.x;
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (q < g.N) {
+        const int c = d.lcell[q];
+        const int gx = div_nc(c, g), gy = c - gx * g.nc;
+        const double2 r = d.lrel[q];
+        const double k = 2.0 * M_PI / g.L;
+        const double x = gx * g.B + r.x, y = gy * g.B + r.y;
+        const int o = d.lpid[q] >= g.n1 ? 4 : 0;
+        v[o + 0] = cos(x * k);
+        v[o + 1] = sin(x * k);
+        v[o + 2] = cos(y * k);
+        v[o + 3] = sin(y * k);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sm[threadIdx.x][i] = v[i];
+    __syncthreads();
+    for (int w = OBS_THREADS / 2; w > 0; w >>= 1) {
+        if (threadIdx.x < w)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sm[threadIdx.x][i] += sm[threadIdx.x + w][i];
+        __syncthreads();
+    }
+    if (threadIdx.x < 8) part[blockIdx.x * 8 + threadIdx.x] = sm[0][threadIdx.x];
+}
+
+// centres S1, S2, Sgamma = (S1+S2)/2 from the block partials (one block)
+__global__ __launch_bounds__(OBS_THREADS) void k_circ_final(Geo g, const double *part, int nb, double *centers) {
+    __shared__ double sm[OBS_THREADS][8];
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < nb; b += OBS_THREADS)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] += part[b * 8 + i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sm[threadIdx.x][i] = v[i];
+    __syncthreads();
+    for (int w = OBS_THREADS / 2; w > 0; w >>= 1) {
+        if (threadIdx.x < w)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sm[threadIdx.x][i] += sm[threadIdx.x + w][i];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        const double k = 2.0 * M_PI / g.L;
+        double S[4];
+        for (int a = 0; a < 4; ++a)  // (S1x, S1y, S2x, S2y)
+            S[a] = (atan2(-sm[0][2 * a + 1], -sm[0][2 * a]) + M_PI) / k;
+        centers[0] = S[0];
+        centers[1] = S[1];
+        centers[2] = S[2];
+        centers[3] = S[3];
+        centers[4] = 0.5 * (S[0] + S[2]);
+        centers[5] = 0.5 * (S[1] + S[3]);
+    }
+}
+
+// counts per bin: rho1ring (Sgamma), rho2ring (S2), rho1zen1, rho1zen2,
+// rho2zen1, rho2zen2; distances without periodic images, beyond the last
+// bin into the last bin (as the reference)
+__global__ __launch_bounds__(OBS_THREADS) void k_radial_hist(Geo g, DevBufs d, const double *centers, int nbins,
+                                                             double dr, int *hist) {
+    const int q = blockIdx.x * OBS_THREADS + threadIdx.x;
+    if (q >= g.N) return;
+    const int c = d.lcell[q];
+    const int gx = div_nc(c, g), gy = c - gx * g.nc;
+    const double2 r = d.lrel[q];
+    const double x = gx * g.B + r.x, y = gy * g.B + r.y;
+    const bool s2 = d.lpid[q] >= g.n1;
+    // (histogram, centre index) pairs of this species
+    const int hs[3] = {s2 ? 1 : 0, s2 ? 4 : 2, s2 ? 5 : 3};
+    const int cs[3] = {s2 ? 1 : 2, 0, 1};  // 0: S1, 1: S2, 2: Sgamma
+    for (int i = 0; i < 3; ++i) {
+        const double dx = x - centers[2 * cs[i]], dy = y - centers[2 * cs[i] + 1];
+        const double rr = sqrt(dx * dx + dy * dy);
+        int bin = (int)(rr / dr);
+        if (bin < 0 || bin >= nbins) bin = nbins - 1;
+        atomicAdd(&hist[hs[i] * nbins + bin], 1);
+    }
+}
+
+hipError_t launch_radial(bdk_t *h, int nbins, double dr, double *part, double *centers, int *hist) {
+    const int nb = (int)nblk(h->g.N, OBS_THREADS);
+    hipLaunchKernelGGL(k_circ_partial, dim3(nb), dim3(OBS_THREADS), 0, h->stream, h->g, h->d, part);
+    hipLaunchKernelGGL(k_circ_final, dim3(1), dim3(OBS_THREADS), 0, h->stream, h->g, part, nb, centers);
+    hipError_t e = launch_zero_ints(hist, 6 * nbins, h->stream);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_radial_hist, dim3(nb), dim3(OBS_THREADS), 0, h->stream, h->g, h->d, centers, nbins, dr,
+                       hist);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------ snapshot grid
+// Local densities on an m x m grid of width w = L/m (main_auswertung.cpp:
+// 214-320): each particle adds its TSC weights times 1/w^2 to the nine cells
+// around cell (int)(x/w) mod m of its species' grid.  The weight products are
+// summed as 2^-40 fixed point in 64-bit integers, so the grid does not depend
+// on the order of the additions.  The offset d from the cell centre uses the
+// unwrapped cell index (the reference wraps first, which only differs when
+// x/w rounds up to m).
+constexpr double SNAP_SCALE = 1099511627776.0;  // 2^40
+
+__device__ __forceinline__ void snap_tsc(double x, double w, int m, int &k, double wt[3]) {
+    const int k0 = (int)(x / w);
+    k = k0 % m;
+    const double dd = x - (k0 + 0.5) * w;
+    wt[1] = 0.75 - dd * dd / (w * w);
+    double t = fabs((dd + w) / w);
+    wt[0] = 0.5 * (1.5 - t) * (1.5 - t);
+    t = fabs((dd - w) / w);
+    wt[2] = 0.5 * (1.5 - t) * (1.5 - t);
+}
+
+__global__ __launch_bounds__(256) void k_snap_grid(Geo g, DevBufs d, int m, double w, unsigned long long *acc) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= g.N) return;
+    const int c = d.lcell[q];
+    const int gx = div_nc(c, g), gy = c - gx * g.nc;
+    const double2 r = d.lrel[q];
+    int k, l;
+    double wx[3], wy[3];
+    snap_tsc(gx * g.B + r.x, w, m, k, wx);
+    snap_tsc(gy * g.B + r.y, w, m, l, wy);
+    unsigned long long *a = acc + (d.lpid[q] >= g.n1 ? (size_t)m * m : 0);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const size_t row = (size_t)((k - 1 + i + m) % m) * m;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const long long v = __double2ll_rn(wx[i] * wy[j] * SNAP_SCALE);
+            atomicAdd(&a[row + (l - 1 + j + m) % m], (unsigned long long)v);
+        }
+    }
+}
+
+// fixed point -> densities; with stats: the histograms of rho1, rho2,
+// rho = rho1 + rho2 and rho1 - rho2 and the cells over the thresholds
+// (main_auswertung.cpp:324-375), counted per block in LDS.
+// cnt: [4][nbins] histograms, then 7 threshold counts.
+__device__ __forceinline__ int snap_bin(double t, int nbins) {
+    if (!(t > -1.0)) return 0;  // (int) truncates toward zero; below 0 clamps to 0
+    if (t >= (double)nbins) return nbins - 1;
+    const int b = (int)t;
+    return b < 0 ? 0 : (b >= nbins ? nbins - 1 : b);
+}
+
+__global__ __launch_bounds__(256) void k_snap_final(int m, double drho, const unsigned long long *acc, double *rho,
+                                                    int stats, int nbins, double dbin, SnapThresh th,
+                                                    unsigned int *cnt) {
+    extern __shared__ unsigned int sh[];  // [4 * nbins + 7]
+    const int nsh = 4 * nbins + 7;
+    if (stats)
+        for (int i = threadIdx.x; i < nsh; i += blockDim.x) sh[i] = 0u;
+    __syncthreads();
+    const size_t mm = (size_t)m * m;
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < mm; i += stride) {
+        const double r1 = ((double)acc[i] / SNAP_SCALE) * drho;
+        const double r2 = ((double)acc[mm + i] / SNAP_SCALE) * drho;
+        rho[i] = r1;
+        rho[mm + i] = r2;
+        if (!stats) continue;
+        const double rs = r1 + r2, dr = r1 - r2;
+        for (int t = 0; t < 3; ++t)
+            if (rs > th.rho[t]) atomicAdd(&sh[4 * nbins + t], 1u);
+        const double f = rs > 0.0 ? fabs(dr) / rs : 0.0;  // 0/0 passes no threshold
+        for (int t = 0; t < 4; ++t)
+            if (rs > 0.0 && f > th.drho[t]) atomicAdd(&sh[4 * nbins + 3 + t], 1u);
+        atomicAdd(&sh[snap_bin(r1 / dbin - 0.5, nbins)], 1u);
+        atomicAdd(&sh[nbins + snap_bin(r2 / dbin - 0.5, nbins)], 1u);
+        atomicAdd(&sh[2 * nbins + snap_bin(rs / dbin - 0.5, nbins)], 1u);
+        atomicAdd(&sh[3 * nbins + snap_bin(dr / dbin - 0.5 + (double)(nbins / 2), nbins)], 1u);
+    }
+    if (!stats) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < nsh; i += blockDim.x)
+        if (sh[i]) atomicAdd(&cnt[i], sh[i]);
+}
+
+hipError_t launch_snap(bdk_t *h, int m, unsigned long long *acc, double *rho, int stats, int nbins, double dbin,
+                       SnapThresh th, unsigned int *cnt) {
+    const double w = h->p.L / m;
+    hipLaunchKernelGGL(k_snap_grid, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d, m, w, acc);
+    const size_t mm = (size_t)m * m;
+    const int nb = (int)std::min<size_t>(nblk(mm, 256), 4096);
+    const size_t lds = stats ? (size_t)(4 * nbins + 7) * sizeof(unsigned int) : 0;
+    hipLaunchKernelGGL(k_snap_final, dim3(nb), dim3(256), lds, h->stream, m, 1.0 / (w * w), acc, rho, stats, nbins,
+                       dbin, th, cnt);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------ direct rho(k)
+// record_ftrho_unkorrigiert (au:307-360): for each wave-vector index pair
+// (i, j) the sums over one species of cos and sin(dq (x i + y j)).  For
+// species 1 the reference takes y = git_y B + rel_x (au:333), unless the
+// parameters ask for rel_y (ftrho_fix); species 2 uses rel_y.  Block (chunk,
+// pair): a fixed-order tree sum over the chunk's particles into
+// partial[pair][chunk]; k_ftrho_final adds the chunks in order.
+constexpr int FT_THREADS = 256, FT_PER_THREAD = 16, FT_MAX_CHUNKS = 64;
+
+// chunk `chunk` of nchunk covers list positions [chunk per, (chunk + 1) per);
+// per is a multiple of FT_THREADS, and nchunk is at most FT_MAX_CHUNKS, so
+// the partial sums stay small at any N.  fix: species 1 takes rel_y.
+__global__ __launch_bounds__(FT_THREADS) void k_ftrho(Geo g, DevBufs d, const int2 *ij, int species, int fix,
+                                                      double dq, double2 *partial, int nchunk, int per) {
+    __shared__ double sc[FT_THREADS], ss[FT_THREADS];
+    const int p = blockIdx.y, chunk = blockIdx.x, tid = threadIdx.x;
+    const int2 q = ij[p];
+    double c = 0.0, s = 0.0;
+    const int q0 = chunk * per, q1 = min(q0 + per, g.N);
+    for (int t = q0 + tid; t < q1; t += FT_THREADS) {
+        const bool s2 = d.lpid[t] >= g.n1;
+        if (s2 != (species == 2)) continue;
+        const int cell = d.lcell[t];
+        const int gx = div_nc(cell, g), gy = cell - gx * g.nc;
+        const double2 r = d.lrel[t];
+        const double x = gx * g.B + r.x;
+        const double y = gy * g.B + ((species == 1 && !fix) ? r.x : r.y);
+        double sn, cs;
+        sincos(dq * (x * q.x + y * q.y), &sn, &cs);
+        c += cs;
+        s += sn;
+    }
+    sc[tid] = c;
+    ss[tid] = s;
+    __syncthreads();
+    for (int w = FT_THREADS / 2; w > 0; w >>= 1) {
+        if (tid < w) {
+            sc[tid] += sc[tid + w];
+            ss[tid] += ss[tid + w];
+        }
+        __syncthreads();
+    }
+    if (tid == 0) partial[(size_t)p * nchunk + chunk] = make_double2(sc[0], ss[0]);
+}
+
+__global__ void k_ftrho_final(const double2 *partial, int nchunk, int npairs, double *re, double *im) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= npairs) return;
+    double c = 0.0, s = 0.0;
+    for (int k = 0; k < nchunk; ++k) {
+        const double2 v = partial[(size_t)p * nchunk + k];
+        c += v.x;
+        s += v.y;
+    }
+    re[p] = c;
+    im[p] = s;
+}
+
+// chunks of at least FT_THREADS * FT_PER_THREAD positions, at most FT_MAX_CHUNKS
+static void ftrho_split(const bdk_t *h, int &nchunk, int &per) {
+    nchunk = std::min((int)nblk(h->g.N, FT_THREADS * FT_PER_THREAD), FT_MAX_CHUNKS);
+    per = (int)nblk(h->g.N, nchunk * FT_THREADS) * FT_THREADS;
+    nchunk = std::max(1, (int)nblk(h->g.N, per));
+}
+
+hipError_t launch_ftrho(bdk_t *h, const int2 *ij, int npairs, int species, double dq, double2 *partial, double *re,
+                        double *im) {
+    int nchunk, per;
+    ftrho_split(h, nchunk, per);
+    hipLaunchKernelGGL(k_ftrho, dim3(nchunk, npairs), dim3(FT_THREADS), 0, h->stream, h->g, h->d, ij, species,
+                       h->p.ftrho_fix ? 1 : 0, dq, partial, nchunk, per);
+    hipLaunchKernelGGL(k_ftrho_final, dim3(nblk(npairs, 256)), dim3(256), 0, h->stream, partial, nchunk, npairs, re,
+                       im);
+    return hipGetLastError();
+}
+
+int ftrho_chunks(const bdk_t *h) {
+    int nchunk, per;
+    ftrho_split(h, nchunk, per);
+    return nchunk;
+}
+
+}  // namespace bdkx
