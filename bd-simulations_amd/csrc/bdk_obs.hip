@@ -90,14 +90,112 @@ hipError_t launch_rhok(bdk_t *h, int species, double dqr, int nbins, double *par
 
 // Pair correlation g11, g12, g22 (record_korrelationsfunktion11/12/22,
 // auswertung.cpp:110-188): minimum-image distances (abstand2, am:100-166)
-// of all pairs closer than nbins*dr, found through the cells within R cells,
-// binned by (int)(r/dr).  Ordered pairs (12 pairs from the species-1 side)
-// are counted with integer atomics in LDS per block, then added to the
-// global histograms: the counts are exact and deterministic.
-__global__ __launch_bounds__(256) void k_pair_hist(Geo g, DevBufs d, int nbins, double dr, int R,
-                                                   unsigned long long *hist) {
+// of all pairs closer than nbins*dr, binned by (int)(r/dr).  Every unordered
+// pair is visited once and counted with integer atomics in LDS per block, a
+// same-species pair as two (both orders) and a 12 pair as one, then added to
+// the global histograms: the counts are exact and deterministic.
+//
+// Bound by the pair arithmetic (FP64 distances; 8.0M pairs at N = 4000).
+// The bin comes from an FP32 square root and a multiplication; only a value
+// within its error of a bin edge (a fraction 1e-6 to 1e-3 of the pairs) takes
+// the FP64 square root and division that define it.
+//
+// A call at N = 4000, r up to L/2 (751 bins): 12.56 ms -> 67 us.  One thread
+// per particle over all 71,000 cells had 16 blocks on the chip and read two
+// list starts per mostly empty cell.
+constexpr int PH_THREADS = 512;   // particles i per job, one per thread
+constexpr int PH_J = 64;          // particles j per job, staged in LDS
+constexpr long long PH_JOB_MAX = (1LL << 30) / (PH_THREADS * PH_J);  // jobs per block: 2 counts each in 32 bits
+
+struct PairBins {
+    int nbins;
+    double dr;
+    float inv;   // 1/dr
+    float umax;  // beyond it no bin
+};
+
+// counts one pair with squared distance d2 (FP64); type 0: 11, 1: 12, 2: 22
+__device__ __forceinline__ void pair_count(double d2, int type, const PairBins &pb, unsigned int *sh) {
+    const float u = __builtin_amdgcn_sqrtf((float)d2) * pb.inv;
+    if (!(u < pb.umax)) return;
+    int b = (int)u;
+    // u is within 2^-21 u of sqrt(d2)/dr (three roundings and a 1-ulp root):
+    // away from the bin's edges its integer part is the exact one
+    const float fr = u - (float)b, eps = 1e-6f + 5e-7f * u;
+    if (fr < eps || fr > 1.0f - eps) b = (int)(sqrt(d2) / pb.dr);
+    if (b < pb.nbins) atomicAdd(&sh[type * pb.nbins + b], type == 1 ? 1u : 2u);
+}
+
+// min over the images of t, t + L, t - L of the square (|t| below 2 L: the
+// nearer image is |t| - L)
+__device__ __forceinline__ double image2(double t, double L) {
+    const double u = fabs(t), v = u - L;
+    const double a = u * u, b = v * v;
+    return b < a ? b : a;
+}
+
+__device__ __forceinline__ void pair_flush(const unsigned int *sh, int nbins, unsigned long long *hist) {
+    for (int b = threadIdx.x; b < 3 * nbins; b += blockDim.x)
+        if (sh[b]) atomicAdd(&hist[b], (unsigned long long)sh[b]);
+}
+
+// All pairs (the cells within R cells cover the box): jobs of PH_THREADS
+// particles i (one per thread) times PH_J particles j > i in LDS; tile I of
+// particles i meets the j tiles from its own first position on.
+__global__ __launch_bounds__(PH_THREADS) void k_pair_hist_all(Geo g, DevBufs d, PairBins pb,
+                                                              unsigned long long *hist) {
     extern __shared__ unsigned int shist[];  // [3][nbins]
-    for (int b = threadIdx.x; b < 3 * nbins; b += blockDim.x) shist[b] = 0u;
+    __shared__ double2 sx[PH_J];
+    __shared__ int ss[PH_J];
+    const int tid = threadIdx.x;
+    for (int b = tid; b < 3 * pb.nbins; b += PH_THREADS) shist[b] = 0u;
+    const int nj = (g.N + PH_J - 1) / PH_J;
+    constexpr int STEP = PH_THREADS / PH_J;
+    auto load = [&](int q, double2 &x, int &s2) {
+        const int c = d.lcell[q], cx = div_nc(c, g), cy = c - cx * g.nc;
+        const double2 r = d.lrel[q];
+        x.x = cx * g.B + r.x;
+        x.y = cy * g.B + r.y;
+        s2 = d.lpid[q] >= g.n1 ? 1 : 0;
+    };
+    long long job = blockIdx.x;
+    int I = 0, have = -1;
+    double2 xi = make_double2(0.0, 0.0);
+    int s2i = 0;
+    for (;;) {
+        while (I * STEP < nj && job >= nj - I * STEP) {
+            job -= nj - I * STEP;
+            ++I;
+        }
+        if (I * STEP >= nj) break;
+        const int qi = I * PH_THREADS + tid;
+        if (have != I) {
+            have = I;
+            if (qi < g.N) load(qi, xi, s2i);
+        }
+        const int j0 = (I * STEP + (int)job) * PH_J, jn = min(PH_J, g.N - j0);
+        __syncthreads();
+        if (tid < jn) load(j0 + tid, sx[tid], ss[tid]);
+        __syncthreads();
+        if (qi < g.N)
+            for (int k = max(0, qi + 1 - j0); k < jn; ++k) {
+                const double2 xj = sx[k];
+                pair_count(image2(xi.x - xj.x, g.L) + image2(xi.y - xj.y, g.L), s2i + ss[k], pb, shist);
+            }
+        job += gridDim.x;
+    }
+    __syncthreads();
+    pair_flush(shist, pb.nbins, hist);
+}
+
+// Pairs within R cells, 2 R + 1 < nc: one thread per particle (list
+// position) and range of row offsets.  The cells (cx + a, cy - R .. cy + R)
+// of a row are one range of the list, two where y wraps; rows a > 0 hold
+// each pair once, row 0 is taken from the particle on.
+__global__ __launch_bounds__(256) void k_pair_hist_near(Geo g, DevBufs d, PairBins pb, int R, int rows_per,
+                                                        unsigned long long *hist) {
+    extern __shared__ unsigned int shist[];  // [3][nbins]
+    for (int b = threadIdx.x; b < 3 * pb.nbins; b += blockDim.x) shist[b] = 0u;
     __syncthreads();
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q < g.N) {
@@ -105,48 +203,65 @@ __global__ __launch_bounds__(256) void k_pair_hist(Geo g, DevBufs d, int nbins, 
         const int cx = div_nc(c, g), cy = c - cx * nc;
         const double2 ri = d.lrel[q];
         const double xi = cx * g.B + ri.x, yi = cy * g.B + ri.y, L = g.L;
-        const bool s2i = d.lpid[q] >= g.n1;
-        const bool all = 2 * R + 1 >= nc;
-        const int a0 = all ? 0 : cx - R, a1 = all ? nc - 1 : cx + R;
-        const int b0 = all ? 0 : cy - R, b1 = all ? nc - 1 : cy + R;
-        for (int a = a0; a <= a1; ++a) {
-            const int ux = wrapc(a, nc);
-            for (int b = b0; b <= b1; ++b) {
-                const int uy = wrapc(b, nc), cc = ux * nc + uy;
-                const int qe = d.start[cc + 1];
-                for (int j = d.start[cc]; j < qe; ++j) {
-                    if (j == q) continue;
-                    const bool s2j = d.lpid[j] >= g.n1;
-                    if (s2i && !s2j) continue;
+        const int s2i = d.lpid[q] >= g.n1 ? 1 : 0;
+        const int a0 = blockIdx.y * rows_per, a1 = min(a0 + rows_per, R + 1);
+        for (int a = a0; a < a1; ++a) {
+            const int ux = wrap1(cx + a, nc), row = ux * nc;
+            const double xr = ux * g.B;
+            // row 0: the rest of the own cell, then the cells above it
+            const int lo = a == 0 ? cy : cy - R, hi = cy + R;
+            for (int part = 0; part < 2; ++part) {
+                int y0, y1;  // inclusive cells of this part
+                if (part == 0) {
+                    y0 = max(lo, 0);
+                    y1 = min(hi, nc - 1);
+                } else if (lo < 0) {
+                    y0 = lo + nc;
+                    y1 = nc - 1;
+                } else if (hi >= nc) {
+                    y0 = 0;
+                    y1 = hi - nc;
+                } else {
+                    break;
+                }
+                const int je = d.start[row + y1 + 1];
+                int j = d.start[row + y0];
+                if (a == 0 && part == 0) j = q + 1;
+                for (; j < je; ++j) {
                     const double2 rj = d.lrel[j];
-                    double t1 = xi - (ux * g.B + rj.x), t2 = t1 + L, t3 = t1 - L;
-                    double m = t3 * t3 < t2 * t2 ? t3 * t3 : t2 * t2;
-                    const double dx2 = m < t1 * t1 ? m : t1 * t1;
-                    t1 = yi - (uy * g.B + rj.y);
-                    t2 = t1 + L;
-                    t3 = t1 - L;
-                    m = t3 * t3 < t2 * t2 ? t3 * t3 : t2 * t2;
-                    const double dy2 = m < t1 * t1 ? m : t1 * t1;
-                    const int idx = (int)(sqrt(dx2 + dy2) / dr);
-                    if (idx < 0 || idx >= nbins) continue;
-                    const int type = s2i ? 2 : (s2j ? 1 : 0);
-                    atomicAdd(&shist[type * nbins + idx], 1u);
+                    const int uy = d.lcell[j] - row;
+                    const int s2j = d.lpid[j] >= g.n1 ? 1 : 0;
+                    pair_count(image2(xi - (xr + rj.x), L) + image2(yi - (uy * g.B + rj.y), L), s2i + s2j, pb, shist);
                 }
             }
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < 3 * nbins; b += blockDim.x)
-        if (shist[b]) atomicAdd(&hist[b], (unsigned long long)shist[b]);
+    pair_flush(shist, pb.nbins, hist);
 }
 
+// All pairs where the cells within R cover the box, else the rows of cells.
 hipError_t launch_pair_hist(bdk_t *h, int nbins, double dr, unsigned long long *hist) {
-    int R = (int)ceil(nbins * dr / h->g.B);
+    const Geo &g = h->g;
+    int R = (int)std::min(ceil(nbins * dr / g.B), (double)g.nc);
     if (R < 1) R = 1;
+    // (outside FP32's comfortable range 1/dr is left 0: every bin from FP64)
+    const PairBins pb = {nbins, dr, dr > 1e-12 && dr < 1e12 ? (float)(1.0 / dr) : 0.0f,
+                         (float)nbins * 1.00001f + 1.0f};
     const size_t lds = (size_t)3 * nbins * sizeof(unsigned int);
-    (void)hipFuncSetAttribute((const void *)k_pair_hist, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-    hipLaunchKernelGGL(k_pair_hist, dim3(nblk(h->g.N, 256)), dim3(256), lds, h->stream, h->g, h->d, nbins, dr, R,
-                       hist);
+    if (2 * R + 1 >= g.nc) {
+        const long long nj = nblk(g.N, PH_J), ni = nblk(g.N, PH_THREADS);
+        const long long jobs = ni * nj - (PH_THREADS / PH_J) * (ni * (ni - 1) / 2);
+        // one block per compute unit, more where the 32-bit counts need it
+        const long long grid = std::max(std::min(jobs, 256LL), (jobs + PH_JOB_MAX - 1) / PH_JOB_MAX);
+        hipLaunchKernelGGL(k_pair_hist_all, dim3((unsigned)grid), dim3(PH_THREADS), lds, h->stream, g, h->d, pb, hist);
+    } else {
+        // rows split over blocks while the particles alone leave the chip idle
+        const int nb = (int)nblk(g.N, 256), want = std::max(1, std::min(R + 1, 1024 / nb));
+        const int per = (int)nblk(R + 1, want);
+        hipLaunchKernelGGL(k_pair_hist_near, dim3(nb, nblk(R + 1, per)), dim3(256), lds, h->stream, g, h->d, pb, R,
+                           per, hist);
+    }
     return hipGetLastError();
 }
 

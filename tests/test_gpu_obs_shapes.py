@@ -1,0 +1,44 @@
+"""Device observables at the sizes where their kernels can go wrong: edges of
+tiles, remainders, the smallest inputs, both sides of each choice of kernel."""
+import math
+
+import numpy as np
+import pytest
+
+import bdk
+from common import params
+from helpers import pair_correlation_ref, to_git_rel
+
+pytestmark = pytest.mark.gpu
+
+
+def random_sim(n1, n2, L, seed, **kw):
+    """Uncorrelated positions (pairs at every distance down to ~0)."""
+    bp, _ = params(n1=n1, n2=n2, L=L, seed=seed, **dict(dict(Z=64, precision=bdk.FP64), **kw))
+    x = np.random.default_rng(seed).uniform(0.0, L, (n1 + n2, 2))
+    d = bdk.derived(bp)
+    s = bdk.RunDynamik(bp)
+    s.set_positions(*to_git_rel(x, d["B"], d["nc"]))
+    return s
+
+
+@pytest.mark.parametrize("n1,n2", [(2, 2), (31, 33), (300, 212), (511, 2), (500, 77), (1100, 900)])
+@pytest.mark.parametrize("rmax,nbins", [(2.0, 7), (8.5, 400), (13.4, 61), (15.2, 4096), (40.0, 33)])
+def test_pair_counts_at_tile_edges(n1, n2, rmax, nbins):
+    """Both kernels of the pair histogram (cells within the range, all pairs)
+    against every pair by brute force, as whole counts: numbers of particles
+    around the tiles of 64 and 512, ranges up to and across half the box
+    (nc = 27: 12 cells are the last range that does not cover it)."""
+    print("case: pair counts n=%d+%d rmax=%g nbins=%d" % (n1, n2, rmax, nbins), flush=True)
+    L = 30.5
+    s = random_sim(n1, n2, L, 11 + n1)
+    assert s.nc == 27
+    dr = rmax / nbins
+    g = s.pair_correlation(nbins, dr)
+    noalloc = s.pair_correlation_noalloc(nbins, dr)
+    x = s.absolute()
+    want = pair_correlation_ref(x[:n1], x[n1:], L, nbins, dr)
+    for got, same, ref in zip(g, noalloc, want):
+        assert np.allclose(got, ref, rtol=1e-12, atol=0)
+        assert np.array_equal(got, same)
+    s.close()
