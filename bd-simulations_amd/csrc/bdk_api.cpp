@@ -145,6 +145,9 @@ void free_dev(bdk_t *h) {
                     h->d.qvf, h->d.sc};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
+    if (h->ws) (void)hipFree(h->ws);
+    h->ws = nullptr;
+    h->ws_cap = 0;
     if (h->info_dev) (void)hipFree(h->info_dev);
     h->info_dev = nullptr;
     h->d = bdkx::DevBufs();
@@ -158,6 +161,40 @@ template <typename T> hipError_t dalloc(T *&p, size_t n) {
 }
 
 hipError_t dalloc_v(void *&p, size_t bytes) { return hipMalloc(&p, bytes > 0 ? bytes : 16); }
+
+// Device scratch of one observable call, taken from the handle.  It is kept
+// for the next call up to kKeepScratch (a hipMalloc and hipFree pair and the
+// synchronisation they imply cost more than a small observable's kernels);
+// more is given back when the call ends.
+constexpr size_t kKeepScratch = 64u << 20;
+struct Scratch {
+    bdk_t *h;
+    size_t used = 0;
+    explicit Scratch(bdk_t *h_) : h(h_) {}
+    ~Scratch() {
+        if (h->ws_cap <= kKeepScratch) return;
+        (void)hipFree(h->ws);  // waits for the device
+        h->ws = nullptr;
+        h->ws_cap = 0;
+    }
+    static size_t pad(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+    // room for parts of `bytes` in all (each padded); then take() them in turn
+    hipError_t reserve(size_t bytes) {
+        used = 0;
+        if (bytes <= h->ws_cap) return hipSuccess;
+        if (h->ws) (void)hipFree(h->ws);
+        h->ws = nullptr;
+        h->ws_cap = 0;
+        const hipError_t e = hipMalloc(&h->ws, bytes);
+        if (e == hipSuccess) h->ws_cap = bytes;
+        return e;
+    }
+    template <typename T> T *take(size_t n) {
+        T *p = (T *)((char *)h->ws + used);
+        used += pad(n * sizeof(T));
+        return p;
+    }
+};
 
 // spectral tables (dm:578-594, dm:1384-1394), built in FP64 on the host
 int build_tables_host(bdk_t *h) {
@@ -1918,29 +1955,20 @@ int bdk_rho_k(bdk_t *h, int32_t species, double dq_ratio, int32_t nbins, double 
     if ((species != 1 && species != 2) || !(dq_ratio > 0.0) || nbins < 1 || !re)
         return fail(h, BDK_ERR_ARG, "need species 1 or 2, dq_ratio > 0, nbins >= 1, re");
     const int Z = h->g.Z;
-    double *part = nullptr, *out = nullptr;
-    hipError_t e = hipMalloc((void **)&part, (size_t)(Z / 2 + 1) * nbins * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc((void **)&out, (size_t)nbins * sizeof(double));
-    if (e == hipSuccess) e = bdkx::launch_rhok(h, species, dq_ratio, nbins, part, out);
-    std::vector<double> sum(nbins);
-    if (e == hipSuccess) e = hipMemcpyAsync(sum.data(), out, nbins * 8, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (part) (void)hipFree(part);
-    if (out) (void)hipFree(out);
-    if (e != hipSuccess) return hipfail(h, e, "bdk_rho_k");
-    // lattice points per shell over the full plane (auswertung.cpp:497-510)
-    std::vector<int64_t> cnt(nbins, 0);
-    for (int i = 0; i < Z; ++i) {
-        const double xq = ((i + Z / 2) % Z) - Z / 2;
-        for (int j = 0; j < Z; ++j) {
-            const double yq = ((j + Z / 2) % Z) - Z / 2;
-            const int bin = (int)(dq_ratio * std::sqrt(xq * xq + yq * yq) + 0.5);
-            if (bin >= 0 && bin < nbins) ++cnt[bin];
-        }
+    const size_t np = (size_t)(Z / 2 + 1) * 2 * nbins;
+    Scratch ws(h);
+    hipError_t e = ws.reserve(Scratch::pad(np * 8) + Scratch::pad((size_t)2 * nbins * 8));
+    std::vector<double> sum((size_t)2 * nbins);  // shell sums, then lattice points per shell (auswertung.cpp:497-510)
+    if (e == hipSuccess) {
+        double *part = ws.take<double>(np), *out = ws.take<double>((size_t)2 * nbins);
+        e = bdkx::launch_rhok(h, species, dq_ratio, nbins, part, out);
+        if (e == hipSuccess) e = hipMemcpyAsync(sum.data(), out, sum.size() * 8, hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     }
-    const double L = h->p.L;
+    if (e != hipSuccess) return hipfail(h, e, "bdk_rho_k");
+    const double L = h->p.L, *cnt = sum.data() + nbins;
     for (int b = 0; b < nbins; ++b) {  // auswertung.cpp:572-576
-        re[b] = cnt[b] ? sum[b] * (L * L / ((double)Z * Z)) / cnt[b] : 0.0;
+        re[b] = cnt[b] > 0.0 ? sum[b] * (L * L / ((double)Z * Z)) / cnt[b] : 0.0;
         if (im) im[b] = 0.0;
     }
     return BDK_OK;

@@ -200,6 +200,8 @@ struct bdk {
     std::string err;
     int64_t host_step = 0;
     bdkx::StepInfoDev *info_dev = nullptr;  // step counters (bdk_step_info), allocated on first use
+    void *ws = nullptr;            // scratch of the observables (bdk_api.cpp: Scratch), kept up to kKeepScratch
+    size_t ws_cap = 0;
     bdkx::PosWriter writer;
 };
 
@@ -225,7 +227,8 @@ hipError_t launch_refresh(bdk_t *h);              // refresh only (no motion)
 hipError_t launch_noise_out(bdk_t *h);            // noise of the next step, by pid
 // ordered-pair distance histograms [3][nbins] (11, 12, 22), zeroed by the caller
 hipError_t launch_pair_hist(bdk_t *h, int nbins, double dr, unsigned long long *hist);
-// rho(k) of one species: part [(Z/2+1)*nbins] scratch, out[nbins] shell sums
+// rho(k) of one species: part [(Z/2+1) * 2 nbins] scratch, out[2 nbins] = shell sums, then the lattice points of
+// each shell
 hipError_t launch_rhok(bdk_t *h, int species, double dqr, int nbins, double *part, double *out);
 // radial density profiles: part [ceil(N/256)*8] scratch, centers[6], hist[6*nbins]
 hipError_t launch_radial(bdk_t *h, int nbins, double dr, double *part, double *centers, int *hist);

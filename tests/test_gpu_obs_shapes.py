@@ -7,7 +7,7 @@ import pytest
 
 import bdk
 from common import params
-from helpers import pair_correlation_ref, to_git_rel
+from helpers import pair_correlation_ref, rho_k_ref, to_git_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -41,4 +41,26 @@ def test_pair_counts_at_tile_edges(n1, n2, rmax, nbins):
     for got, same, ref in zip(g, noalloc, want):
         assert np.allclose(got, ref, rtol=1e-12, atol=0)
         assert np.array_equal(got, same)
+    s.close()
+
+
+@pytest.mark.parametrize("Z", [8, 10, 64, 250, 512])
+@pytest.mark.parametrize("ratio,nbins", [(0.5, None), (0.5, 1), (1.0, 4), (0.37, 200), (2.5, 3)])
+def test_rho_k_shells(Z, ratio, nbins):
+    """Shell sums and lattice points per shell (one thread per shell and
+    column) against the full plane: the smallest meshes, an odd Z/2, one
+    shell, shells wider and narrower than a mesh mode, more shells than the
+    plane holds."""
+    nb = nbins or int(0.5 * Z * ratio)
+    print("case: rho(k) shells Z=%d ratio=%g nbins=%d" % (Z, ratio, nb), flush=True)
+    n1, n2, L = 300, 211, 30.5
+    s = random_sim(n1, n2, L, 17, Z=Z, scheme=bdk.TSC)
+    x = s.absolute()
+    # the Nyquist column of an odd Z/2 enters with the sign of an even one
+    top = nb if Z % 4 == 0 else min(nb, int(ratio * (Z // 2) + 0.5))
+    for sp, xs in ((1, x[:n1]), (2, x[n1:])):
+        re, im = s.rho_k(sp, ratio, nb)
+        want = rho_k_ref(xs, L, Z, bdk.TSC, ratio, nb)
+        assert np.abs(re - want)[:top].max() < 1e-11 * n1
+        assert not im.any()
     s.close()
