@@ -1834,15 +1834,17 @@ int bdk_pair_correlation(bdk_t *h, int32_t nbins, double dr, double *g11, double
     int rc = ensure(h);
     if (rc) return rc;
     if (nbins < 1 || nbins > 4096 || !(dr > 0.0)) return fail(h, BDK_ERR_ARG, "need 1 <= nbins <= 4096, dr > 0");
-    unsigned long long *hist = nullptr;
     const size_t hb = (size_t)3 * nbins * sizeof(unsigned long long);
-    hipError_t e = hipMalloc((void **)&hist, hb);
-    if (e == hipSuccess) e = hipMemsetAsync(hist, 0, hb, h->stream);
-    if (e == hipSuccess) e = bdkx::launch_pair_hist(h, nbins, dr, hist);
+    Scratch ws(h);
+    hipError_t e = ws.reserve(Scratch::pad(hb));
     std::vector<unsigned long long> cnt((size_t)3 * nbins);
-    if (e == hipSuccess) e = hipMemcpyAsync(cnt.data(), hist, hb, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (hist) (void)hipFree(hist);
+    if (e == hipSuccess) {
+        unsigned long long *hist = ws.take<unsigned long long>((size_t)3 * nbins);
+        e = hipMemsetAsync(hist, 0, hb, h->stream);
+        if (e == hipSuccess) e = bdkx::launch_pair_hist(h, nbins, dr, hist);
+        if (e == hipSuccess) e = hipMemcpyAsync(cnt.data(), hist, hb, hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    }
     if (e != hipSuccess) return hipfail(h, e, "bdk_pair_correlation");
     // auswertung.cpp:120-121, 149-150, 173-174 (g12 keeps the reference's N1-1)
     const double L = h->p.L, n1 = h->p.n1, n2 = h->p.n2;

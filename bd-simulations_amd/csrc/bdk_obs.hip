@@ -137,10 +137,13 @@ hipError_t launch_rhok(bdk_t *h, int species, double dqr, int nbins, double *par
 // within its error of a bin edge (a fraction 1e-6 to 1e-3 of the pairs) takes
 // the FP64 square root and division that define it.
 //
-// A call at N = 4000, r up to L/2 (751 bins): 12.56 ms -> 67 us.  One thread
-// per particle over all 71,000 cells had 16 blocks on the chip and read two
-// list starts per mostly empty cell.
-constexpr int PH_THREADS = 512;   // particles i per job, one per thread
+// N = 4000, r up to L/2 (751 bins): 12.5 ms -> 24 us for the kernel.  One
+// thread per particle over all 71,000 cells had 16 blocks on the chip and
+// read two list starts per mostly empty cell.  Jobs of 1024 x 64 pairs on 256
+// blocks, four pairs of a thread in flight: 24 us; one at a time 36; 512 x 64
+// 30, 256 x 64 on 512 blocks 27 (more bins cleared and added per pair), 256 x
+// 128 49.
+constexpr int PH_THREADS = 1024;   // particles i per job, one per thread
 constexpr int PH_J = 64;          // particles j per job, staged in LDS
 constexpr long long PH_JOB_MAX = (1LL << 30) / (PH_THREADS * PH_J);  // jobs per block: 2 counts each in 32 bits
 
@@ -151,15 +154,20 @@ struct PairBins {
     float umax;  // beyond it no bin
 };
 
-// counts one pair with squared distance d2 (FP64); type 0: 11, 1: 12, 2: 22
-__device__ __forceinline__ void pair_count(double d2, int type, const PairBins &pb, unsigned int *sh) {
+// bin of a squared distance d2 (FP64); nbins or more: none
+__device__ __forceinline__ int pair_bin(double d2, const PairBins &pb) {
     const float u = __builtin_amdgcn_sqrtf((float)d2) * pb.inv;
-    if (!(u < pb.umax)) return;
-    int b = (int)u;
+    if (!(u < pb.umax)) return pb.nbins;
+    const int b = (int)u;
     // u is within 2^-21 u of sqrt(d2)/dr (three roundings and a 1-ulp root):
     // away from the bin's edges its integer part is the exact one
     const float fr = u - (float)b, eps = 1e-6f + 5e-7f * u;
-    if (fr < eps || fr > 1.0f - eps) b = (int)(sqrt(d2) / pb.dr);
+    if (fr < eps || fr > 1.0f - eps) return (int)(sqrt(d2) / pb.dr);
+    return b;
+}
+// counts one pair; type 0: 11, 1: 12, 2: 22
+__device__ __forceinline__ void pair_count(double d2, int type, const PairBins &pb, unsigned int *sh) {
+    const int b = pair_bin(d2, pb);
     if (b < pb.nbins) atomicAdd(&sh[type * pb.nbins + b], type == 1 ? 1u : 2u);
 }
 
@@ -214,11 +222,30 @@ __global__ __launch_bounds__(PH_THREADS) void k_pair_hist_all(Geo g, DevBufs d, 
         __syncthreads();
         if (tid < jn) load(j0 + tid, sx[tid], ss[tid]);
         __syncthreads();
-        if (qi < g.N)
-            for (int k = max(0, qi + 1 - j0); k < jn; ++k) {
+        if (qi < g.N) {
+            // four pairs at a time: their LDS reads and square roots overlap
+            int k = max(0, qi + 1 - j0);
+            for (; k + 4 <= jn; k += 4) {
+                double d2[4];
+                int ty[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const double2 xj = sx[k + e];
+                    ty[e] = s2i + ss[k + e];
+                    d2[e] = image2(xi.x - xj.x, g.L) + image2(xi.y - xj.y, g.L);
+                }
+                int b[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) b[e] = pair_bin(d2[e], pb);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (b[e] < pb.nbins) atomicAdd(&shist[ty[e] * pb.nbins + b[e]], ty[e] == 1 ? 1u : 2u);
+            }
+            for (; k < jn; ++k) {
                 const double2 xj = sx[k];
                 pair_count(image2(xi.x - xj.x, g.L) + image2(xi.y - xj.y, g.L), s2i + ss[k], pb, shist);
             }
+        }
         job += gridDim.x;
     }
     __syncthreads();

@@ -22,12 +22,12 @@ def random_sim(n1, n2, L, seed, **kw):
     return s
 
 
-@pytest.mark.parametrize("n1,n2", [(2, 2), (31, 33), (300, 212), (511, 2), (500, 77), (1100, 900)])
+@pytest.mark.parametrize("n1,n2", [(2, 2), (31, 33), (300, 212), (511, 2), (500, 77), (525, 499), (1100, 1013)])
 @pytest.mark.parametrize("rmax,nbins", [(2.0, 7), (8.5, 400), (13.4, 61), (15.2, 4096), (40.0, 33)])
 def test_pair_counts_at_tile_edges(n1, n2, rmax, nbins):
     """Both kernels of the pair histogram (cells within the range, all pairs)
     against every pair by brute force, as whole counts: numbers of particles
-    around the tiles of 64 and 512, ranges up to and across half the box
+    around the tiles of 64 and 1024, ranges up to and across half the box
     (nc = 27: 12 cells are the last range that does not cover it)."""
     print("case: pair counts n=%d+%d rmax=%g nbins=%d" % (n1, n2, rmax, nbins), flush=True)
     L = 30.5
