@@ -1803,22 +1803,22 @@ int bdk_radial_profile(bdk_t *h, int32_t nbins, double dr, double *centers, doub
     int rc = ensure(h);
     if (rc) return rc;
     if (nbins < 1 || !(dr > 0.0) || !profiles) return fail(h, BDK_ERR_ARG, "need nbins >= 1, dr > 0, profiles");
-    const int nb = (h->g.N + 255) / 256;
-    double *part = nullptr, *cen = nullptr;
-    int *hist = nullptr;
-    hipError_t e = hipMalloc((void **)&part, (size_t)nb * 8 * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc((void **)&cen, 6 * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc((void **)&hist, (size_t)6 * nbins * sizeof(int));
-    if (e == hipSuccess) e = bdkx::launch_radial(h, nbins, dr, part, cen, hist);
-    std::vector<int> cnt((size_t)6 * nbins);
-    double c6[6] = {0, 0, 0, 0, 0, 0};
-    if (e == hipSuccess) e = hipMemcpyAsync(cnt.data(), hist, cnt.size() * 4, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(c6, cen, sizeof(c6), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (part) (void)hipFree(part);
-    if (cen) (void)hipFree(cen);
-    if (hist) (void)hipFree(hist);
+    const size_t np = (size_t)bdkx::radial_blocks(h) * 8, ncnt = (size_t)6 * nbins, ncopy = (size_t)bdkx::radial_copies(nbins);
+    Scratch ws(h);
+    hipError_t e = ws.reserve(Scratch::pad(np * 8) + Scratch::pad(6 * 8 + ncopy * ncnt * 4));
+    std::vector<char> got(6 * 8 + ncopy * ncnt * 4);  // centres, then the copies of the counts
+    if (e == hipSuccess) {
+        double *part = ws.take<double>(np), *cen = (double *)ws.take<char>(got.size());
+        e = bdkx::launch_radial(h, nbins, dr, part, cen, (int *)(cen + 6));
+        if (e == hipSuccess) e = hipMemcpyAsync(got.data(), cen, got.size(), hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    }
     if (e != hipSuccess) return hipfail(h, e, "bdk_radial_profile");
+    const double *c6 = (const double *)got.data();
+    const int *copies = (const int *)(got.data() + 6 * 8);
+    std::vector<int> cnt(copies, copies + ncnt);
+    for (size_t k = 1; k < ncopy; ++k)
+        for (size_t i = 0; i < ncnt; ++i) cnt[i] += copies[k * ncnt + i];
     const double L = h->p.L;
     const double v1 = h->p.n1 ? L * L / (h->p.n1 * dr * dr * M_PI) : 0.0;  // observablen_auswertung.cpp:268
     const double v2 = h->p.n2 ? L * L / (h->p.n2 * dr * dr * M_PI) : 0.0;
@@ -1826,7 +1826,7 @@ int bdk_radial_profile(bdk_t *h, int32_t nbins, double dr, double *centers, doub
     for (int k = 0; k < 6; ++k)
         for (int b = 0; b < nbins; ++b)
             profiles[(size_t)k * nbins + b] = cnt[(size_t)k * nbins + b] * (vf[k] / (2 * b + 1));
-    if (centers) std::memcpy(centers, c6, sizeof(c6));
+    if (centers) std::memcpy(centers, c6, 6 * sizeof(double));
     return BDK_OK;
 }
 

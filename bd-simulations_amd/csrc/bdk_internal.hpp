@@ -230,7 +230,10 @@ hipError_t launch_pair_hist(bdk_t *h, int nbins, double dr, unsigned long long *
 // rho(k) of one species: part [(Z/2+1) * 2 nbins] scratch, out[2 nbins] = shell sums, then the lattice points of
 // each shell
 hipError_t launch_rhok(bdk_t *h, int species, double dqr, int nbins, double *part, double *out);
-// radial density profiles: part [ceil(N/256)*8] scratch, centers[6], hist[6*nbins]
+// radial density profiles: part [radial_blocks * 8] scratch, centers[6],
+// hist[radial_copies][6*nbins] (to be added up)
+int radial_blocks(const bdk_t *h);
+int radial_copies(int nbins);
 hipError_t launch_radial(bdk_t *h, int nbins, double dr, double *part, double *centers, int *hist);
 // snapshot density grid (main_auswertung.cpp:214-375): acc [2][m*m] zeroed by
 // the caller, rho [2][m*m]; stats: cnt [4*nbins + 7] zeroed by the caller

@@ -7,7 +7,7 @@ import pytest
 
 import bdk
 from common import params
-from helpers import pair_correlation_ref, rho_k_ref, to_git_rel
+from helpers import pair_correlation_ref, radial_profile_ref, rho_k_ref, to_git_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -63,4 +63,23 @@ def test_rho_k_shells(Z, ratio, nbins):
         want = rho_k_ref(xs, L, Z, bdk.TSC, ratio, nb)
         assert np.abs(re - want)[:top].max() < 1e-11 * n1
         assert not im.any()
+    s.close()
+
+
+@pytest.mark.parametrize("n1,n2", [(1, 1), (130, 126), (1100, 949), (2048, 1), (9000, 8000)])
+@pytest.mark.parametrize("nbins,dr", [(1, 3.0), (60, 0.5), (2048, 0.01), (2049, 0.01)])
+def test_radial_profile_at_block_edges(n1, n2, nbins, dr):
+    """One block and several, species of one particle, and both homes of the
+    histogram (LDS up to 2048 bins)."""
+    print("case: radial profile n=%d+%d nbins=%d" % (n1, n2, nbins), flush=True)
+    L = 60.5
+    s = random_sim(n1, n2, L, 23 + n1)
+    cen, prof = s.radial_profile(nbins, dr)
+    x = s.absolute()
+    cref, pref = radial_profile_ref(x[:n1], x[n1:], L, nbins, dr)
+    assert np.allclose(cen, cref, rtol=0, atol=1e-9 * L)
+    # whole counts: a value within rounding of a bin edge may differ
+    assert np.isclose(prof, pref, rtol=1e-12, atol=0).mean() > 0.999
+    ring = np.pi * dr * dr * (2 * np.arange(nbins) + 1)
+    assert np.allclose((prof * ring).sum(1), L * L, rtol=1e-12)
     s.close()
