@@ -1876,26 +1876,25 @@ static int density_snapshot(bdk_t *h, int32_t m, double *rho1, double *rho2, int
         for (int t = 0; t < 3; ++t) th.rho[t] = rho_thresh[t];
         for (int t = 0; t < 4; ++t) th.drho[t] = drho_thresh[t];
     }
-    unsigned long long *acc = nullptr;
-    double *rho = nullptr;
-    unsigned int *cnt = nullptr;
-    const size_t nc = stats ? (size_t)4 * nbins + 7 : 1;
-    hipError_t e = hipMalloc((void **)&acc, 2 * mm * sizeof(unsigned long long));
-    if (e == hipSuccess) e = hipMalloc((void **)&rho, 2 * mm * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc((void **)&cnt, nc * sizeof(unsigned int));
-    if (e == hipSuccess) e = hipMemsetAsync(acc, 0, 2 * mm * sizeof(unsigned long long), h->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(cnt, 0, nc * sizeof(unsigned int), h->stream);
-    if (e == hipSuccess) e = bdkx::launch_snap(h, m, acc, rho, stats, nbins, dbin, th, cnt);
-    std::vector<unsigned int> c(nc);
-    if (e == hipSuccess && rho1) e = hipMemcpyAsync(rho1, rho, mm * 8, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess && rho2) e = hipMemcpyAsync(rho2, rho + mm, mm * 8, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess && stats)
-        e = hipMemcpyAsync(c.data(), cnt, nc * sizeof(unsigned int), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (acc) (void)hipFree(acc);
-    if (rho) (void)hipFree(rho);
-    if (cnt) (void)hipFree(cnt);
+    const size_t nc = stats ? (size_t)4 * nbins + 7 : 0, ncopy = (size_t)bdkx::snap_copies();
+    const bool grid = rho1 || rho2;
+    Scratch ws(h);
+    hipError_t e = ws.reserve(Scratch::pad(grid ? 2 * mm * 8 : 0) + Scratch::pad(ncopy * nc * sizeof(unsigned int)));
+    std::vector<unsigned int> c(ncopy * nc);
+    if (e == hipSuccess) {
+        double *rho = grid ? ws.take<double>(2 * mm) : nullptr;
+        unsigned int *cnt = stats ? ws.take<unsigned int>(ncopy * nc) : nullptr;
+        if (stats) e = hipMemsetAsync(cnt, 0, ncopy * nc * sizeof(unsigned int), h->stream);
+        if (e == hipSuccess) e = bdkx::launch_snap(h, m, rho, stats, nbins, dbin, th, cnt);
+        if (e == hipSuccess && rho1) e = hipMemcpyAsync(rho1, rho, mm * 8, hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess && rho2) e = hipMemcpyAsync(rho2, rho + mm, mm * 8, hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess && stats)
+            e = hipMemcpyAsync(c.data(), cnt, c.size() * sizeof(unsigned int), hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    }
     if (e != hipSuccess) return hipfail(h, e, what);
+    for (size_t k = 1; k < ncopy; ++k)
+        for (size_t i = 0; i < nc; ++i) c[i] += c[k * nc + i];
     if (stats) {
         const double pre = 1.0 / (double)mm;  // main_auswertung.cpp:328
         if (hist)

@@ -235,14 +235,16 @@ hipError_t launch_rhok(bdk_t *h, int species, double dqr, int nbins, double *par
 int radial_blocks(const bdk_t *h);
 int radial_copies(int nbins);
 hipError_t launch_radial(bdk_t *h, int nbins, double dr, double *part, double *centers, int *hist);
-// snapshot density grid (main_auswertung.cpp:214-375): acc [2][m*m] zeroed by
-// the caller, rho [2][m*m]; stats: cnt [4*nbins + 7] zeroed by the caller
+// snapshot density grid (main_auswertung.cpp:214-375): rho [2][m*m] (null:
+// not wanted); stats: cnt [snap_copies][4*nbins + 7] zeroed by the caller (to
+// be added up)
+int snap_copies();
 struct SnapThresh {
     double rho[3];
     double drho[4];
 };
-hipError_t launch_snap(bdk_t *h, int m, unsigned long long *acc, double *rho, int stats, int nbins, double dbin,
-                       SnapThresh th, unsigned int *cnt);
+hipError_t launch_snap(bdk_t *h, int m, double *rho, int stats, int nbins, double dbin, SnapThresh th,
+                       unsigned int *cnt);
 // direct rho(k) sums (au:307-360) of one species for npairs index pairs ij;
 // partial [npairs][ftrho_chunks(h)]
 hipError_t launch_ftrho(bdk_t *h, const int2 *ij, int npairs, int species, double dq, double2 *partial, double *re,

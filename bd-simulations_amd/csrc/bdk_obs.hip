@@ -481,11 +481,23 @@ hipError_t launch_radial(bdk_t *h, int nbins, double dr, double *part, double *c
 // on the order of the additions.  The offset d from the cell centre uses the
 // unwrapped cell index (the reference wraps first, which only differs when
 // x/w rounds up to m).
+//
+// A block owns a tile of ts x ts grid cells and sums both species' weights
+// there in LDS: it visits the particles of the list cells around the tile
+// (each row of them is one range of the list, two where y wraps) and keeps
+// what falls into the tile.  Then it turns its cells into densities and
+// counts their statistics at once.  2M particles on 1414^2: 427 -> 62 us,
+// against nine global 64-bit atomics per particle, a cleared accumulator and
+// a second pass over it.
 constexpr double SNAP_SCALE = 1099511627776.0;  // 2^40
+constexpr int SNAP_TILE = 32;                   // grid cells per tile side, at most
+constexpr int SNAP_CELLS = 48;                  // list cells under a tile's side, about, at most
+constexpr int SNAP_SEG = 512;                   // list ranges per round
+constexpr int SNAP_COPIES = 8;                  // copies of the counters, added on the host
 
 __device__ __forceinline__ void snap_tsc(double x, double w, int m, int &k, double wt[3]) {
     const int k0 = (int)(x / w);
-    k = k0 % m;
+    k = k0 >= m || k0 <= -m ? k0 % m : k0;
     const double dd = x - (k0 + 0.5) * w;
     wt[1] = 0.75 - dd * dd / (w * w);
     double t = fabs((dd + w) / w);
@@ -494,32 +506,7 @@ __device__ __forceinline__ void snap_tsc(double x, double w, int m, int &k, doub
     wt[2] = 0.5 * (1.5 - t) * (1.5 - t);
 }
 
-__global__ __launch_bounds__(256) void k_snap_grid(Geo g, DevBufs d, int m, double w, unsigned long long *acc) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= g.N) return;
-    const int c = d.lcell[q];
-    const int gx = div_nc(c, g), gy = c - gx * g.nc;
-    const double2 r = d.lrel[q];
-    int k, l;
-    double wx[3], wy[3];
-    snap_tsc(gx * g.B + r.x, w, m, k, wx);
-    snap_tsc(gy * g.B + r.y, w, m, l, wy);
-    unsigned long long *a = acc + (d.lpid[q] >= g.n1 ? (size_t)m * m : 0);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const size_t row = (size_t)((k - 1 + i + m) % m) * m;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const long long v = __double2ll_rn(wx[i] * wy[j] * SNAP_SCALE);
-            atomicAdd(&a[row + (l - 1 + j + m) % m], (unsigned long long)v);
-        }
-    }
-}
-
-// fixed point -> densities; with stats: the histograms of rho1, rho2,
-// rho = rho1 + rho2 and rho1 - rho2 and the cells over the thresholds
-// (main_auswertung.cpp:324-375), counted per block in LDS.
-// cnt: [4][nbins] histograms, then 7 threshold counts.
+// bin of a histogram value (main_auswertung.cpp:324-375)
 __device__ __forceinline__ int snap_bin(double t, int nbins) {
     if (!(t > -1.0)) return 0;  // (int) truncates toward zero; below 0 clamps to 0
     if (t >= (double)nbins) return nbins - 1;
@@ -527,48 +514,155 @@ __device__ __forceinline__ int snap_bin(double t, int nbins) {
     return b < 0 ? 0 : (b >= nbins ? nbins - 1 : b);
 }
 
-__global__ __launch_bounds__(256) void k_snap_final(int m, double drho, const unsigned long long *acc, double *rho,
-                                                    int stats, int nbins, double dbin, SnapThresh th,
-                                                    unsigned int *cnt) {
-    extern __shared__ unsigned int sh[];  // [4 * nbins + 7]
-    const int nsh = 4 * nbins + 7;
-    if (stats)
-        for (int i = threadIdx.x; i < nsh; i += blockDim.x) sh[i] = 0u;
-    __syncthreads();
-    const size_t mm = (size_t)m * m;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < mm; i += stride) {
-        const double r1 = ((double)acc[i] / SNAP_SCALE) * drho;
-        const double r2 = ((double)acc[mm + i] / SNAP_SCALE) * drho;
-        rho[i] = r1;
-        rho[mm + i] = r2;
-        if (!stats) continue;
-        const double rs = r1 + r2, dr = r1 - r2;
-        for (int t = 0; t < 3; ++t)
-            if (rs > th.rho[t]) atomicAdd(&sh[4 * nbins + t], 1u);
-        const double f = rs > 0.0 ? fabs(dr) / rs : 0.0;  // 0/0 passes no threshold
-        for (int t = 0; t < 4; ++t)
-            if (rs > 0.0 && f > th.drho[t]) atomicAdd(&sh[4 * nbins + 3 + t], 1u);
-        atomicAdd(&sh[snap_bin(r1 / dbin - 0.5, nbins)], 1u);
-        atomicAdd(&sh[nbins + snap_bin(r2 / dbin - 0.5, nbins)], 1u);
-        atomicAdd(&sh[2 * nbins + snap_bin(rs / dbin - 0.5, nbins)], 1u);
-        atomicAdd(&sh[3 * nbins + snap_bin(dr / dbin - 0.5 + (double)(nbins / 2), nbins)], 1u);
+// one count at sh[i] by every active lane; lanes that share one i (most grid
+// cells of a dilute state are empty) count together
+__device__ __forceinline__ void snap_count(unsigned int *sh, int i) {
+    const int first = __builtin_amdgcn_readfirstlane(i);
+    if (__all(i == first)) {
+        const unsigned long long act = __ballot(1);
+        if ((int)(threadIdx.x & 63) == __ffsll((unsigned long long)act) - 1) atomicAdd(&sh[first], (unsigned)__popcll(act));
+    } else {
+        atomicAdd(&sh[i], 1u);
     }
-    if (!stats) return;
-    __syncthreads();
-    for (int i = threadIdx.x; i < nsh; i += blockDim.x)
-        if (sh[i]) atomicAdd(&cnt[i], sh[i]);
 }
 
-hipError_t launch_snap(bdk_t *h, int m, unsigned long long *acc, double *rho, int stats, int nbins, double dbin,
-                       SnapThresh th, unsigned int *cnt) {
-    const double w = h->p.L / m;
-    hipLaunchKernelGGL(k_snap_grid, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d, m, w, acc);
+// list cells that hold every particle which can reach grid cells [p0, p1) of
+// an axis: those of x / w in [p0 - 1, p1 + 1), widened by the excursion e of
+// offsets outside their cell and a cell of margin
+__device__ __forceinline__ void snap_span(int p0, int p1, double w, double e, const Geo &g, int &c0, int &n) {
+    const int lo = (int)floor(((p0 - 1) * w - e) / g.B) - 1, hi = (int)floor(((p1 + 1) * w + e) / g.B) + 1;
+    n = hi - lo + 1;
+    c0 = lo;
+    if (n >= g.nc) {
+        n = g.nc;
+        c0 = 0;
+    }
+}
+
+struct SnapArgs {
+    int m, ts, tiles;  // grid cells per side, per tile side, tiles per side
+    double w, drho;
+    int stats, nbins;
+    double dbin;
+    SnapThresh th;
+};
+
+__global__ __launch_bounds__(256) void k_snap_tiles(Geo g, DevBufs d, SnapArgs a, double *rho, unsigned int *cnt) {
+    extern __shared__ unsigned int sh[];  // [4 * nbins + 7] counts
+    __shared__ unsigned long long acc[2 * SNAP_TILE * SNAP_TILE];
+    __shared__ int seg_q[SNAP_SEG], seg_pre[SNAP_SEG + 1], wsum[4];
+    const int tid = threadIdx.x, nsh = 4 * a.nbins + 7, nc = g.nc, m = a.m;
+    if (a.stats)
+        for (int i = tid; i < nsh; i += 256) sh[i] = 0u;
+    // excursion bound of the current state
+    const double e = dbits(d.sc->exc_bits[d.sc->step & 1]) + 1e-9 * g.L;
     const size_t mm = (size_t)m * m;
-    const int nb = (int)std::min<size_t>(nblk(mm, 256), 4096);
+    for (int tile = blockIdx.x; tile < a.tiles * a.tiles; tile += gridDim.x) {
+        const int k0 = (tile / a.tiles) * a.ts, l0 = (tile % a.tiles) * a.ts;
+        const int nk = min(a.ts, m - k0), nl = min(a.ts, m - l0), nown = nk * nl;
+        __syncthreads();
+        for (int i = tid; i < 2 * nown; i += 256) acc[i] = 0ull;
+        int cx0, nx, cy0, ny;
+        snap_span(k0, k0 + nk, a.w, e, g, cx0, nx);
+        snap_span(l0, l0 + nl, a.w, e, g, cy0, ny);
+        cx0 = wrapc(cx0, nc);
+        cy0 = wrapc(cy0, nc);
+        const int parts = cy0 + ny > nc ? 2 : 1;  // a row's y range wraps
+        const int nseg = nx * parts;
+        for (int s0 = 0; s0 < nseg; s0 += SNAP_SEG) {
+            const int ns = min(SNAP_SEG, nseg - s0);
+            __syncthreads();
+            for (int i = tid; i < ns; i += 256) {
+                const int r = (s0 + i) / parts, part = (s0 + i) - r * parts;
+                int ux = cx0 + r;
+                if (ux >= nc) ux -= nc;
+                const int ya = part == 0 ? cy0 : 0, yb = part == 0 ? min(cy0 + ny, nc) : cy0 + ny - nc;
+                const int q = d.start[ux * nc + ya];
+                seg_q[i] = q;
+                seg_pre[i] = max(d.start[ux * nc + yb] - q, 0);
+            }
+            __syncthreads();
+            const int total = block_exscan4(seg_pre, ns, wsum);
+            for (int t = tid; t < total; t += 256) {
+                int lo = 0, hi = ns - 1;  // last range that begins at or before t
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (seg_pre[mid] <= t) lo = mid;
+                    else hi = mid - 1;
+                }
+                const int q = seg_q[lo] + (t - seg_pre[lo]);
+                bool s2;
+                const double2 x = list_position(g, d, q, s2);
+                int k, l;
+                double wx[3], wy[3];
+                snap_tsc(x.x, a.w, m, k, wx);
+                snap_tsc(x.y, a.w, m, l, wy);
+                unsigned long long *p = acc + (s2 ? nown : 0);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const int kk = wrap1(k - 1 + i, m) - k0;
+                    if ((unsigned)kk >= (unsigned)nk) continue;
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) {
+                        const int ll = wrap1(l - 1 + j, m) - l0;
+                        if ((unsigned)ll >= (unsigned)nl) continue;
+                        const long long v = __double2ll_rn(wx[i] * wy[j] * SNAP_SCALE);
+                        atomicAdd(&p[kk * nl + ll], (unsigned long long)v);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < nown; i += 256) {
+            const double r1 = ((double)acc[i] / SNAP_SCALE) * a.drho;
+            const double r2 = ((double)acc[nown + i] / SNAP_SCALE) * a.drho;
+            if (rho) {
+                const int kk = i / nl;
+                const size_t o = (size_t)(k0 + kk) * m + l0 + (i - kk * nl);
+                rho[o] = r1;
+                rho[mm + o] = r2;
+            }
+            if (!a.stats) continue;
+            const int nbins = a.nbins;
+            const double rs = r1 + r2, dr = r1 - r2;
+            for (int t = 0; t < 3; ++t)
+                if (rs > a.th.rho[t]) snap_count(sh, 4 * nbins + t);
+            const double f = rs > 0.0 ? fabs(dr) / rs : 0.0;  // 0/0 passes no threshold
+            for (int t = 0; t < 4; ++t)
+                if (rs > 0.0 && f > a.th.drho[t]) snap_count(sh, 4 * nbins + 3 + t);
+            snap_count(sh, snap_bin(r1 / a.dbin - 0.5, nbins));
+            snap_count(sh, nbins + snap_bin(r2 / a.dbin - 0.5, nbins));
+            snap_count(sh, 2 * nbins + snap_bin(rs / a.dbin - 0.5, nbins));
+            snap_count(sh, 3 * nbins + snap_bin(dr / a.dbin - 0.5 + (double)(nbins / 2), nbins));
+        }
+    }
+    if (!a.stats) return;
+    __syncthreads();
+    unsigned int *out = cnt + (size_t)(blockIdx.x % SNAP_COPIES) * nsh;
+    for (int i = tid; i < nsh; i += 256)
+        if (sh[i]) atomicAdd(&out[i], sh[i]);
+}
+
+int snap_copies() { return SNAP_COPIES; }
+
+hipError_t launch_snap(bdk_t *h, int m, double *rho, int stats, int nbins, double dbin, SnapThresh th,
+                       unsigned int *cnt) {
+    SnapArgs a = {};
+    a.m = m;
+    a.w = h->p.L / m;
+    a.drho = 1.0 / (a.w * a.w);
+    // a wide grid cell covers many list cells: smaller tiles, so that a coarse
+    // grid still spreads over the chip
+    a.ts = std::max(1, std::min(SNAP_TILE, (int)std::min(SNAP_CELLS * h->g.B / a.w, 1e6)));
+    a.tiles = (int)nblk(m, a.ts);
+    a.stats = stats;
+    a.nbins = stats ? nbins : 0;
+    a.dbin = dbin;
+    a.th = th;
     const size_t lds = stats ? (size_t)(4 * nbins + 7) * sizeof(unsigned int) : 0;
-    hipLaunchKernelGGL(k_snap_final, dim3(nb), dim3(256), lds, h->stream, m, 1.0 / (w * w), acc, rho, stats, nbins,
-                       dbin, th, cnt);
+    (void)hipFuncSetAttribute((const void *)k_snap_tiles, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+    const unsigned grid = (unsigned)std::min((long long)a.tiles * a.tiles, 2048LL);
+    hipLaunchKernelGGL(k_snap_tiles, dim3(grid), dim3(256), lds, h->stream, h->g, h->d, a, rho, cnt);
     return hipGetLastError();
 }
 

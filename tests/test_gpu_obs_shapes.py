@@ -7,7 +7,8 @@ import pytest
 
 import bdk
 from common import params
-from helpers import pair_correlation_ref, radial_profile_ref, rho_k_ref, to_git_rel
+from helpers import (density_stats_ref, pair_correlation_ref, radial_profile_ref, rho_k_ref, to_git_rel,
+                     tsc_snapshot_ref)
 
 pytestmark = pytest.mark.gpu
 
@@ -82,4 +83,37 @@ def test_radial_profile_at_block_edges(n1, n2, nbins, dr):
     assert np.isclose(prof, pref, rtol=1e-12, atol=0).mean() > 0.999
     ring = np.pi * dr * dr * (2 * np.arange(nbins) + 1)
     assert np.allclose((prof * ring).sum(1), L * L, rtol=1e-12)
+    s.close()
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 5, 31, 32, 33, 64, 97, 300])
+@pytest.mark.parametrize("outside", [False, True])
+def test_snapshot_tiles(m, outside):
+    """Tiles of the snapshot grid: one cell to several tiles with remainders,
+    grid cells wider and narrower than list cells, list ranges that wrap, and
+    (outside) offsets beyond their list cell, as the reference's random start
+    leaves them.  Same bound as the whole-grid test: every contribution is
+    rounded to 2^-41 of a weight."""
+    print("case: snapshot tiles m=%d outside=%d" % (m, outside), flush=True)
+    n1, n2, L = 900, 700, 61.3
+    s = random_sim(n1, n2, L, 29)
+    if outside:
+        s.set_positions(*bdk.MT(31).init_positions(s.p))
+        assert s.positions()[1].max() > s.B
+    r1, r2 = s.density_grid(m)
+    x = s.absolute()
+    w1, w2 = tsc_snapshot_ref(x[:n1], x[n1:], L, m)
+    w = L / m
+    for got, ref, xs in ((r1, w1, x[:n1]), (r2, w2, x[n1:])):
+        k = np.floor(xs / w).astype(np.int64)
+        cnt = np.zeros((m, m))
+        for a in (-1, 0, 1):
+            for b in (-1, 0, 1):
+                np.add.at(cnt, ((k[:, 0] + a) % m, (k[:, 1] + b) % m), 1.0)
+        assert np.all(np.abs(got - ref) <= cnt * (2.0 ** -41 + 1e-15) / (w * w))
+    th, dth = (0.1, 0.2, 0.5), (0.1, 0.2, 0.5, 0.99)
+    for nbins, dbin in ((100, 0.01), (1, 1.0), (4096, 0.001)):
+        hist, over = s.density_stats(m, nbins, dbin, th, dth)
+        hr, orf = density_stats_ref(r1, r2, nbins, dbin, th, dth)
+        assert np.array_equal(hist, hr) and np.array_equal(over, orf)
     s.close()
