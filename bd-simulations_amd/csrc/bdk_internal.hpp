@@ -245,11 +245,13 @@ struct SnapThresh {
 };
 hipError_t launch_snap(bdk_t *h, int m, double *rho, int stats, int nbins, double dbin, SnapThresh th,
                        unsigned int *cnt);
-// direct rho(k) sums (au:307-360) of one species for npairs index pairs ij;
-// partial [npairs][ftrho_chunks(h)]
-hipError_t launch_ftrho(bdk_t *h, const int2 *ij, int npairs, int species, double dq, double2 *partial, double *re,
-                        double *im);
-int ftrho_chunks(const bdk_t *h);
+// direct rho(k) sums (au:307-360) of one species over the index pairs i, j < qbins:
+// part [parts][2][side][side] scratch, out [2][side][side] (cos, then sin sums)
+struct FtPlan {
+    int side, per, parts;
+};
+FtPlan ftrho_plan(const bdk_t *h, int qbins);
+hipError_t launch_ftrho(bdk_t *h, const FtPlan &f, int qbins, int species, double dq, double *part, double *out);
 hipError_t set_kernel_attributes();
 // device address of the allocation-free entry's scratch array on device
 // `dev` (current), looked up once per device (bdk_noalloc.hip)

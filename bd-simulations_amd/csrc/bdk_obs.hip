@@ -670,82 +670,142 @@ hipError_t launch_snap(bdk_t *h, int m, double *rho, int stats, int nbins, doubl
 // record_ftrho_unkorrigiert (au:307-360): for each wave-vector index pair
 // (i, j) the sums over one species of cos and sin(dq (x i + y j)).  For
 // species 1 the reference takes y = git_y B + rel_x (au:333), unless the
-// parameters ask for rel_y (ftrho_fix); species 2 uses rel_y.  Block (chunk,
-// pair): a fixed-order tree sum over the chunk's particles into
-// partial[pair][chunk]; k_ftrho_final adds the chunks in order.
-constexpr int FT_THREADS = 256, FT_PER_THREAD = 16, FT_MAX_CHUNKS = 64;
+// parameters ask for rel_y (ftrho_fix); species 2 uses rel_y.
+//
+// exp(i dq (x i + y j)) is a product of a factor of x and a factor of y, so
+// the sums over the particles are one complex product X^T Y of the factors
+// of all i and all j, taken by the FP64 matrix units: 2 q sine/cosine pairs
+// per particle instead of one per (i, j).  Each angle is reduced to
+// [-pi, pi] before the sine and cosine without rounding (i u - 2 rint(i u / 2)
+// with u = x dq / pi kept in two doubles), so the sums come out nearer to
+// exact arithmetic than with one rounded angle per pair (against extended
+// precision: 1e-16 to 7e-16 of their norm, before 3e-15 to 2e-14).
+//
+// A block takes a tile of 32 x 32 index pairs and a part of the list: it
+// queues the species' particles in list order, and for every 32 of them
+// writes both factors to LDS and each of its four waves multiplies a 16 x 16
+// quarter.  The parts are added in order (k_sum_rows).  Bound by the FP64
+// sine/cosine evaluations.  20,000 particles, 30 x 30: 2 x 58 -> 2 x 15 us.
+constexpr int FT_THREADS = 256, FT_TILE = 32, FT_K = 32;
+// LDS row of one particle's factors: 32 cosines, 32 sines, padded so that two
+// consecutive rows' quarters read by half a wave lie in different banks
+constexpr int FT_ROW = 80;
 
-// chunk `chunk` of nchunk covers list positions [chunk per, (chunk + 1) per);
-// per is a multiple of FT_THREADS, and nchunk is at most FT_MAX_CHUNKS, so
-// the partial sums stay small at any N.  fix: species 1 takes rel_y.
-__global__ __launch_bounds__(FT_THREADS) void k_ftrho(Geo g, DevBufs d, const int2 *ij, int species, int fix,
-                                                      double dq, double2 *partial, int nchunk, int per) {
-    __shared__ double sc[FT_THREADS], ss[FT_THREADS];
-    const int p = blockIdx.y, chunk = blockIdx.x, tid = threadIdx.x;
-    const int2 q = ij[p];
-    double c = 0.0, s = 0.0;
-    const int q0 = chunk * per, q1 = min(q0 + per, g.N);
-    for (int t = q0 + tid; t < q1; t += FT_THREADS) {
-        const bool s2 = d.lpid[t] >= g.n1;
-        if (s2 != (species == 2)) continue;
-        const int cell = d.lcell[t];
-        const int gx = div_nc(cell, g), gy = cell - gx * g.nc;
-        const double2 r = d.lrel[t];
-        const double x = gx * g.B + r.x;
-        const double y = gy * g.B + ((species == 1 && !fix) ? r.x : r.y);
-        double sn, cs;
-        sincos(dq * (x * q.x + y * q.y), &sn, &cs);
-        c += cs;
-        s += sn;
-    }
-    sc[tid] = c;
-    ss[tid] = s;
-    __syncthreads();
-    for (int w = FT_THREADS / 2; w > 0; w >>= 1) {
-        if (tid < w) {
-            sc[tid] += sc[tid + w];
-            ss[tid] += ss[tid + w];
+typedef double ft_acc __attribute__((ext_vector_type(4)));
+
+// cos and sin of (k u) pi, u = uh + ul
+__device__ __forceinline__ void ft_factor(int k, double uh, double ul, double *cs, double *sn) {
+    const double t = k * uh, te = fma((double)k, uh, -t) + k * ul;
+    sincospi((t - 2.0 * rint(0.5 * t)) + te, sn, cs);
+}
+
+__global__ __launch_bounds__(FT_THREADS) void k_ftrho(Geo g, DevBufs d, int species, int fix, int qbins, int nt,
+                                                      double ch, double cl, int per, double *part) {
+    __shared__ double X[FT_K * FT_ROW], Y[FT_K * FT_ROW];
+    __shared__ double2 queue[FT_THREADS + FT_K];
+    __shared__ int wcnt[FT_THREADS / 64];
+    const int ti = (int)blockIdx.y / nt, tj = (int)blockIdx.y - ti * nt;
+    if (FT_TILE * FT_TILE * (ti * ti + tj * tj) > qbins * qbins) return;  // beyond the quarter circle
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wi = (wave >> 1) * 16, wj = (wave & 1) * 16;
+    const int q0 = blockIdx.x * per, q1 = min(q0 + per, g.N);
+    const double ydrop = species == 1 && !fix ? 1.0 : 0.0;
+    ft_acc re = {0.0, 0.0, 0.0, 0.0}, im = {0.0, 0.0, 0.0, 0.0};
+    int n = 0;  // queued particles
+    for (int base = q0; base < q1; base += FT_THREADS) {
+        const int t = base + tid;
+        bool want = false;
+        double2 x;
+        if (t < q1) {
+            want = (d.lpid[t] >= g.n1) == (species == 2);
+            const int cell = d.lcell[t], gx = div_nc(cell, g), gy = cell - gx * g.nc;
+            const double2 r = d.lrel[t];
+            x.x = gx * g.B + r.x;
+            x.y = gy * g.B + (ydrop != 0.0 ? r.x : r.y);
         }
+        const unsigned long long mask = __ballot(want);
+        if (lane == 0) wcnt[wave] = __popcll(mask);
         __syncthreads();
+        int pos = n + __popcll(mask & ((1ull << lane) - 1ull));
+        for (int w = 0; w < FT_THREADS / 64; ++w) {
+            if (w < wave) pos += wcnt[w];
+            n += wcnt[w];
+        }
+        if (want) queue[pos] = x;
+        __syncthreads();
+        int head = 0;
+        const bool last = base + FT_THREADS >= q1;
+        while (n - head >= FT_K || (last && n > head)) {
+            const int m = min(FT_K, n - head);
+            // factors: index tid % 32, particles tid / 32 + 8 e
+            for (int e = 0; e < FT_K / 8; ++e) {
+                const int i = tid & 31, k = (tid >> 5) + 8 * e;
+                double cx = 0.0, sx = 0.0, cy = 0.0, sy = 0.0;
+                if (k < m) {
+                    const double2 p = queue[head + k];
+                    const double ux = p.x * ch, uy = p.y * ch;
+                    ft_factor(FT_TILE * ti + i, ux, fma(p.x, ch, -ux) + p.x * cl, &cx, &sx);
+                    ft_factor(FT_TILE * tj + i, uy, fma(p.y, ch, -uy) + p.y * cl, &cy, &sy);
+                }
+                X[k * FT_ROW + i] = cx;
+                X[k * FT_ROW + 32 + i] = sx;
+                Y[k * FT_ROW + i] = cy;
+                Y[k * FT_ROW + 32 + i] = sy;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < FT_K; k += 4) {
+                // operands: row (column) lane % 16 of particle k + lane / 16
+                const int o = (k + (lane >> 4)) * FT_ROW + (lane & 15);
+                const double xc = X[o + wi], xs = X[o + wi + 32], yc = Y[o + wj], ys = Y[o + wj + 32];
+                re = __builtin_amdgcn_mfma_f64_16x16x4f64(xc, yc, re, 0, 0, 0);
+                re = __builtin_amdgcn_mfma_f64_16x16x4f64(-xs, ys, re, 0, 0, 0);
+                im = __builtin_amdgcn_mfma_f64_16x16x4f64(xs, yc, im, 0, 0, 0);
+                im = __builtin_amdgcn_mfma_f64_16x16x4f64(xc, ys, im, 0, 0, 0);
+            }
+            __syncthreads();
+            head += m;
+        }
+        // what is left (fewer than FT_K) moves to the front
+        n -= head;
+        double2 keep;
+        if (tid < n) keep = queue[head + tid];
+        __syncthreads();
+        if (tid < n) queue[tid] = keep;
     }
-    if (tid == 0) partial[(size_t)p * nchunk + chunk] = make_double2(sc[0], ss[0]);
-}
-
-__global__ void k_ftrho_final(const double2 *partial, int nchunk, int npairs, double *re, double *im) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npairs) return;
-    double c = 0.0, s = 0.0;
-    for (int k = 0; k < nchunk; ++k) {
-        const double2 v = partial[(size_t)p * nchunk + k];
-        c += v.x;
-        s += v.y;
+    // results: column lane % 16, rows lane / 16 + 4 r
+    const int qp = FT_TILE * nt;
+    double *out = part + (size_t)blockIdx.x * 2 * qp * qp;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const size_t o = (size_t)(FT_TILE * ti + wi + (lane >> 4) + 4 * r) * qp + FT_TILE * tj + wj + (lane & 15);
+        out[o] = re[r];
+        out[(size_t)qp * qp + o] = im[r];
     }
-    re[p] = c;
-    im[p] = s;
 }
 
-// chunks of at least FT_THREADS * FT_PER_THREAD positions, at most FT_MAX_CHUNKS
-static void ftrho_split(const bdk_t *h, int &nchunk, int &per) {
-    nchunk = std::min((int)nblk(h->g.N, FT_THREADS * FT_PER_THREAD), FT_MAX_CHUNKS);
-    per = (int)nblk(h->g.N, nchunk * FT_THREADS) * FT_THREADS;
-    nchunk = std::max(1, (int)nblk(h->g.N, per));
+// parts of the list (a multiple of 64 positions each) such that about 1024
+// blocks run; side of the padded square of index pairs
+FtPlan ftrho_plan(const bdk_t *h, int qbins) {
+    FtPlan f;
+    const int nt = (int)nblk(qbins, FT_TILE);
+    f.side = FT_TILE * nt;
+    const int want = std::max(1, std::min(256, 1024 / (nt * nt)));
+    f.per = (int)nblk(nblk(h->g.N, want), 64) * 64;
+    f.parts = (int)nblk(h->g.N, f.per);
+    return f;
 }
 
-hipError_t launch_ftrho(bdk_t *h, const int2 *ij, int npairs, int species, double dq, double2 *partial, double *re,
-                        double *im) {
-    int nchunk, per;
-    ftrho_split(h, nchunk, per);
-    hipLaunchKernelGGL(k_ftrho, dim3(nchunk, npairs), dim3(FT_THREADS), 0, h->stream, h->g, h->d, ij, species,
-                       h->p.ftrho_fix ? 1 : 0, dq, partial, nchunk, per);
-    hipLaunchKernelGGL(k_ftrho_final, dim3(nblk(npairs, 256)), dim3(256), 0, h->stream, partial, nchunk, npairs, re,
-                       im);
+// sums of the species: out[2][side][side] = cos and sin sums of (i, j); part
+// [parts][2][side][side].  Entries outside the quarter circle hold nothing.
+hipError_t launch_ftrho(bdk_t *h, const FtPlan &f, int qbins, int species, double dq, double *part, double *out) {
+    const int nt = f.side / FT_TILE;
+    const long double c = (long double)dq / 3.14159265358979323846264338327950288L;
+    const double ch = (double)c, cl = (double)(c - (long double)ch);
+    hipLaunchKernelGGL(k_ftrho, dim3(f.parts, nt * nt), dim3(FT_THREADS), 0, h->stream, h->g, h->d, species,
+                       h->p.ftrho_fix ? 1 : 0, qbins, nt, ch, cl, f.per, part);
+    launch_sum_rows(part, f.parts, 2 * f.side * f.side, out, h->stream);
     return hipGetLastError();
-}
-
-int ftrho_chunks(const bdk_t *h) {
-    int nchunk, per;
-    ftrho_split(h, nchunk, per);
-    return nchunk;
 }
 
 }  // namespace bdkx

@@ -337,8 +337,8 @@ int bdk_density_stats(bdk_t *h, int32_t m, int32_t nbins, double dbin, const dou
    species 1 the reference takes y = git_y B + rel_x (au:333), kept here
    unless bd_params.ftrho_fix is set (then rel_y, as species 2 uses).
    re/im receive *npairs (<= qbins^2) entries; the shells by i^2 + j^2 are
-   the caller's (init_ftrho, au:262-300).  Device scratch: npairs x at most
-   64 partial sums (16 B each), allocated for the call. */
+   the caller's (init_ftrho, au:262-300).  Device scratch: at most 18 MB of
+   partial sums, kept with the handle. */
 int bdk_ftrho_sums(bdk_t *h, int32_t species, int32_t qbins, double dq_ft, double *re, double *im, int32_t *npairs);
 
 /* ---------------------------------------------------------------- batches

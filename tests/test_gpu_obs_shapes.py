@@ -117,3 +117,24 @@ def test_snapshot_tiles(m, outside):
         hr, orf = density_stats_ref(r1, r2, nbins, dbin, th, dth)
         assert np.array_equal(hist, hr) and np.array_equal(over, orf)
     s.close()
+
+
+@pytest.mark.parametrize("n1,n2", [(1, 1), (31, 33), (257, 64), (900, 4000)])
+@pytest.mark.parametrize("qbins", [1, 16, 17, 32, 33, 70])
+def test_ftrho_tiles(n1, n2, qbins):
+    """Tiles of 32 x 32 index pairs with remainders, species of fewer and more
+    particles than a batch of 32, list parts without the species.  Bound: the
+    numpy side rounds each angle (up to 2 pi 2 qbins sqrt 2) three times."""
+    print("case: ftrho tiles n=%d+%d qbins=%d" % (n1, n2, qbins), flush=True)
+    L = 90.0
+    s = random_sim(n1, n2, L, 37 + n1, ftrho_fix=1)
+    x, dq = s.absolute(), 4.0 * np.pi / L
+    pairs = np.array([(i, j) for i in range(qbins) for j in range(qbins) if i * i + j * j <= qbins * qbins])
+    for sp, xs in ((1, x[:n1]), (2, x[n1:])):
+        re, im = s.ftrho_sums(sp, qbins, dq)
+        assert len(re) == len(pairs)
+        a = dq * (pairs @ xs.T)
+        tol = len(xs) * (4 * math.pi * qbins * math.sqrt(2.0) * 3 * 2.0 ** -53 + 1e-15)
+        assert np.abs(re - np.cos(a).sum(1)).max() <= tol and np.abs(im - np.sin(a).sum(1)).max() <= tol
+        assert re[0] == len(xs) and im[0] == 0.0
+    s.close()
