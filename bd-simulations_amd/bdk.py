@@ -301,24 +301,23 @@ class RunDynamik:
     init = set_positions  # RunDynamik::init builds lists from the current positions (am:361-364)
 
     def positions(self):
-        out_g, out_r = [], []
-        for sp, n in ((1, self.p.n1), (2, self.p.n2)):
-            g = np.zeros((max(n, 1), 2), np.int32)
-            r = np.zeros((max(n, 1), 2))
-            self._chk(self.L.bdk_get_positions(self.h, sp, n, _p(g), _p(r)))
-            out_g.append(g[:n])
-            out_r.append(r[:n])
-        return np.concatenate(out_g), np.concatenate(out_r)
+        n1 = self.p.n1
+        g = np.empty((self.N, 2), np.int32)
+        r = np.empty((self.N, 2))
+        for sp, n, sl in ((1, n1, slice(0, n1)), (2, self.p.n2, slice(n1, self.N))):
+            self._chk(self.L.bdk_get_positions(self.h, sp, n, _p(g[sl]), _p(r[sl])))
+        return g, r
 
     def absolute(self):
         g, r = self.positions()
-        return r + self.B * g
+        for a in range(0, self.N, 1 << 15):  # in place, a part that fits the cache at a time
+            r[a:a + (1 << 15)] += self.B * g[a:a + (1 << 15)]
+        return r
 
     def _two(self, fn):
-        a = np.zeros((max(self.p.n1, 1), 2))
-        b = np.zeros((max(self.p.n2, 1), 2))
-        self._chk(fn(self.h, _p(a), _p(b)))
-        return np.concatenate([a[: self.p.n1], b[: self.p.n2]])
+        f, n1 = np.empty((self.N, 2)), self.p.n1
+        self._chk(fn(self.h, _p(f[:n1]), _p(f[n1:])))
+        return f
 
     # --- force entry points
     def berechne_WCA(self):

@@ -148,6 +148,9 @@ void free_dev(bdk_t *h) {
     if (h->ws) (void)hipFree(h->ws);
     h->ws = nullptr;
     h->ws_cap = 0;
+    if (h->pin) (void)hipHostFree(h->pin);
+    h->pin = nullptr;
+    h->pin_cap = 0;
     if (h->info_dev) (void)hipFree(h->info_dev);
     h->info_dev = nullptr;
     h->d = bdkx::DevBufs();
@@ -195,6 +198,28 @@ struct Scratch {
         return p;
     }
 };
+
+// Pinned host staging of the handle, for copies up to kPinned bytes: one
+// transfer without the runtime's own staging (at 4000 particles some 10 us
+// each).  Larger copies go to the caller's memory directly.  Null when the
+// request is larger or the allocation fails.  Every call that fills it waits
+// for its copies before it returns.
+constexpr size_t kPinned = 4u << 20;
+char *pinned(bdk_t *h, size_t bytes) {
+    if (bytes > kPinned) return nullptr;
+    if (bytes > h->pin_cap) {
+        if (h->pin) (void)hipHostFree(h->pin);
+        h->pin = nullptr;
+        h->pin_cap = 0;
+        if (hipHostMalloc((void **)&h->pin, bytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            h->pin = nullptr;
+            return nullptr;
+        }
+        h->pin_cap = bytes;
+    }
+    return h->pin;
+}
 
 // spectral tables (dm:578-594, dm:1384-1394), built in FP64 on the host
 int build_tables_host(bdk_t *h) {
@@ -280,8 +305,12 @@ hipError_t clear_flags(bdk_t *h) {
 // rebuild the cell lists (WCA_init, dm:459-526)
 int upload(bdk_t *h) {
     const int n1 = h->p.n1, n2 = h->p.n2, N = n1 + n2, nc = h->g.nc;
-    std::vector<int> cell(N);
-    std::vector<double> rel(2 * (size_t)N);
+    // storage order: grouped by cell, ascending id.  A counting sort, unless
+    // the cells by far outnumber the particles (2M particles in 1.6M cells: 35
+    // instead of 180 ms; 1000 particles in 16M cells would pay for the cells).
+    const size_t ncell = (size_t)nc * nc;
+    const bool counting = ncell <= 32 * (size_t)N + 65536;
+    std::vector<int> cell(N), at(counting ? ncell + 1 : 0, 0), order;
     for (int sp = 0; sp < 2; ++sp) {
         const int n = sp == 0 ? n1 : n2, off = sp == 0 ? 0 : n1;
         for (int i = 0; i < n; ++i) {
@@ -294,29 +323,41 @@ int upload(bdk_t *h) {
                 return fail(h, BDK_ERR_NONFINITE, "non-finite rel for species " + std::to_string(sp + 1) +
                                                       " particle " + std::to_string(i));
             cell[off + i] = gx * nc + gy;
-            if (h->g.pos_mode) {  // FP32 storage of the in-cell positions
-                rx = (double)(float)rx;
-                ry = (double)(float)ry;
-            }
-            rel[2 * (size_t)(off + i)] = rx;
-            rel[2 * (size_t)(off + i) + 1] = ry;
+            if (counting) ++at[cell[off + i] + 1];
         }
     }
-    std::vector<int> order(N);
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cell[a] < cell[b]; });
-    std::vector<int> scell(N), spid(N);
-    std::vector<double> srel(2 * (size_t)N);
-    for (int s = 0; s < N; ++s) {
-        int p = order[s];
+    if (counting) {
+        for (size_t c = 1; c < at.size(); ++c) at[c] += at[c - 1];
+    } else {
+        order.resize(N);
+        std::iota(order.begin(), order.end(), 0);
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cell[a] < cell[b]; });
+    }
+    // offsets, cells and ids in storage order, staged for one transfer each
+    std::vector<char> own;
+    char *stage = pinned(h, (size_t)N * 24);
+    if (!stage) {
+        own.resize((size_t)N * 24);
+        stage = own.data();
+    }
+    double *srel = (double *)stage;
+    int *scell = (int *)(stage + (size_t)N * 16), *spid = scell + N;
+    for (int k = 0; k < N; ++k) {
+        const int p = counting ? k : order[k], s = counting ? at[cell[p]]++ : k;
+        const int sp = p < n1 ? 0 : 1, i = sp ? p - n1 : p;
+        double rx = h->hrel[sp][2 * (size_t)i], ry = h->hrel[sp][2 * (size_t)i + 1];
+        if (h->g.pos_mode) {  // FP32 storage of the in-cell positions
+            rx = (double)(float)rx;
+            ry = (double)(float)ry;
+        }
         scell[s] = cell[p];
         spid[s] = p;
-        srel[2 * (size_t)s] = rel[2 * (size_t)p];
-        srel[2 * (size_t)s + 1] = rel[2 * (size_t)p + 1];
+        srel[2 * (size_t)s] = rx;
+        srel[2 * (size_t)s + 1] = ry;
     }
-    HIPCHK(h, hipMemcpyAsync(h->d.cell, scell.data(), (size_t)N * 4, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(h, hipMemcpyAsync(h->d.pid, spid.data(), (size_t)N * 4, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(h, hipMemcpyAsync(h->d.rel, srel.data(), (size_t)N * 16, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, hipMemcpyAsync(h->d.cell, scell, (size_t)N * 4, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, hipMemcpyAsync(h->d.pid, spid, (size_t)N * 4, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, hipMemcpyAsync(h->d.rel, srel, (size_t)N * 16, hipMemcpyHostToDevice, h->stream));
     if (h->d.comp) HIPCHK(h, hipMemsetAsync(h->d.comp, 0, (size_t)N * 8, h->stream));
     HIPCHK(h, hipMemsetAsync(h->d.count, 0, (size_t)h->g.ncell * 4, h->stream));
     HIPCHK(h, clear_flags(h));
@@ -346,26 +387,23 @@ int ensure_forces(bdk_t *h) {
 }
 
 // list-ordered device array of real2 -> per-species [n][2] doubles
-template <typename R>
-int download_r2(bdk_t *h, const void *src, double *f1, double *f2) {
-    const int N = h->g.N, n1 = h->p.n1;
-    std::vector<R> buf(2 * (size_t)N);
-    std::vector<int> pid(N);
-    HIPCHK(h, hipMemcpyAsync(buf.data(), src, buf.size() * sizeof(R), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(pid.data(), h->d.lpid, (size_t)N * 4, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (int s = 0; s < N; ++s) {
-        int p = pid[s];
-        double *dst = p < n1 ? (f1 ? f1 + 2 * (size_t)p : nullptr) : (f2 ? f2 + 2 * (size_t)(p - n1) : nullptr);
-        if (!dst) continue;
-        dst[0] = (double)buf[2 * (size_t)s];
-        dst[1] = (double)buf[2 * (size_t)s + 1];
-    }
-    return BDK_OK;
-}
-
 int download_forces(bdk_t *h, const void *src, double *f1, double *f2) {
-    return h->p.precision != BDK_FP64 ? download_r2<float>(h, src, f1, f2) : download_r2<double>(h, src, f1, f2);
+    const size_t n1 = h->p.n1, n2 = h->p.n2, N = n1 + n2;
+    Scratch ws(h);
+    HIPCHK(h, ws.reserve(Scratch::pad(N * 16)));
+    double2 *out = ws.take<double2>(N);
+    HIPCHK(h, bdkx::launch_force_by_id(h, src, out));
+    if (char *stage = pinned(h, N * 16)) {
+        HIPCHK(h, hipMemcpyAsync(stage, out, N * 16, hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        if (f1 && n1) std::memcpy(f1, stage, n1 * 16);
+        if (f2 && n2) std::memcpy(f2, stage + n1 * 16, n2 * 16);
+        return BDK_OK;
+    }
+    if (f1 && n1) HIPCHK(h, hipMemcpyAsync(f1, out, n1 * 16, hipMemcpyDeviceToHost, h->stream));
+    if (f2 && n2) HIPCHK(h, hipMemcpyAsync(f2, out + n1, n2 * 16, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    return BDK_OK;
 }
 
 // steps per replay of the multi-step graph
@@ -789,28 +827,32 @@ int bdk_get_positions(bdk_t *h, int species, int32_t n, int32_t *git, double *re
     int rc = ensure(h);
     if (rc) return rc;
     if (species != 1 && species != 2) return fail(h, BDK_ERR_ARG, "species must be 1 or 2");
-    const int n1 = h->p.n1, N = h->g.N, nc = h->g.nc;
+    const int n1 = h->p.n1;
     if (n != (species == 1 ? n1 : h->p.n2)) return fail(h, BDK_ERR_ARG, "n does not match");
-    std::vector<int> cell(N), pid(N);
-    std::vector<double> r(2 * (size_t)N);
-    HIPCHK(h, hipMemcpyAsync(cell.data(), h->d.cell, (size_t)N * 4, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(pid.data(), h->d.pid, (size_t)N * 4, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(r.data(), h->d.rel, (size_t)N * 16, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (int s = 0; s < N; ++s) {
-        int p = pid[s];
-        int i = species == 1 ? p : p - n1;
-        if ((species == 1) != (p < n1)) continue;
-        if (git) {
-            git[2 * (size_t)i] = cell[s] / nc;
-            git[2 * (size_t)i + 1] = cell[s] % nc;
-        }
-        if (rel) {
-            rel[2 * (size_t)i] = r[2 * (size_t)s];
-            rel[2 * (size_t)i + 1] = r[2 * (size_t)s + 1];
-        }
+    // [flags | offsets | cells], in id order
+    const size_t head = sizeof(bdkx::ByIdHead), bytes = head + (size_t)n * 24;
+    Scratch ws(h);
+    HIPCHK(h, ws.reserve(Scratch::pad(bytes)));
+    char *out = ws.take<char>(bytes);
+    double2 *orel = (double2 *)(out + head);
+    int2 *ogit = (int2 *)(out + head + (size_t)n * 16);
+    HIPCHK(h, bdkx::launch_by_id(h, species == 1 ? 0 : n1, n, (bdkx::ByIdHead *)out, ogit, orel));
+    bdkx::ByIdHead flags;
+    if (char *stage = pinned(h, bytes)) {
+        HIPCHK(h, hipMemcpyAsync(stage, out, bytes, hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        std::memcpy(&flags, stage, head);
+        if (rel && n) std::memcpy(rel, stage + head, (size_t)n * 16);
+        if (git && n) std::memcpy(git, stage + head + (size_t)n * 16, (size_t)n * 8);
+    } else {
+        HIPCHK(h, hipMemcpyAsync(&flags, out, head, hipMemcpyDeviceToHost, h->stream));
+        if (rel) HIPCHK(h, hipMemcpyAsync(rel, orel, (size_t)n * 16, hipMemcpyDeviceToHost, h->stream));
+        if (git) HIPCHK(h, hipMemcpyAsync(git, ogit, (size_t)n * 8, hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(h, hipStreamSynchronize(h->stream));
     }
-    return check_nonfinite(h);
+    std::string m;
+    rc = flag_status(flags.flags, &m);
+    return rc ? fail(h, rc, m) : BDK_OK;
 }
 
 int bdk_compute_wca(bdk_t *h, double *f1, double *f2) {

@@ -202,6 +202,8 @@ struct bdk {
     bdkx::StepInfoDev *info_dev = nullptr;  // step counters (bdk_step_info), allocated on first use
     void *ws = nullptr;            // scratch of the observables (bdk_api.cpp: Scratch), kept up to kKeepScratch
     size_t ws_cap = 0;
+    char *pin = nullptr;           // pinned host staging (bdk_api.cpp: pinned), at most kPinned bytes
+    size_t pin_cap = 0;
     bdkx::PosWriter writer;
 };
 
@@ -212,6 +214,13 @@ hipError_t launch_wca(bdk_t *h, hipStream_t st = nullptr);  // WCA forces -> fwc
 hipError_t launch_deposit(bdk_t *h, int reset, int slot = 0, hipStream_t st = nullptr);  // charges -> rho
                                                   // (reset: re-arm per-step scalars; slot: during a rebuild)
 hipError_t launch_species_deposit(bdk_t *h, int species);  // number density of one species -> rho
+// cells and offsets of ids id0 .. id0 + n - 1 in id order, and the error flags
+struct ByIdHead {
+    int flags;
+    int pad[63];
+};
+hipError_t launch_by_id(bdk_t *h, int id0, int n, ByIdHead *head, int2 *git, double2 *rel);
+hipError_t launch_force_by_id(bdk_t *h, const void *f, double2 *out);  // list-ordered forces -> [N] by id
 hipError_t launch_zero_ints(int *p, int n, hipStream_t st);
 hipError_t launch_rearm(bdk_t *h);                // per-step scalars when no deposit runs
 size_t deposit_lds_bytes(const bdk_t *h);          // LDS of one deposit block

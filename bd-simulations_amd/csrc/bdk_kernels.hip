@@ -1264,6 +1264,30 @@ __global__ void k_noise_out(Geo g, DevBufs d) {
     d.noise_out[p] = particle_noise(g, d, p, d.sc->step);
 }
 
+// Cells and offsets of one species (ids id0 .. id0 + n - 1) in id order, for
+// the host, after a header with the error flags: the scatter by id that a
+// host thread would do over the whole state runs here (a random 24 B write
+// per particle; 20 us at 2M particles against 15 ms), and only the species
+// asked for crosses to the host.
+__global__ void k_by_id(Geo g, DevBufs d, int id0, int n, ByIdHead *head, int2 *git, double2 *rel) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0) head->flags = d.sc->nonfinite;
+    if (s >= g.N) return;
+    const int i = d.pid[s] - id0;
+    if ((unsigned)i >= (unsigned)n) return;
+    const int c = d.cell[s], gx = div_nc(c, g);
+    git[i] = make_int2(gx, c - gx * g.nc);
+    rel[i] = d.rel[s];
+}
+
+// list-ordered forces as doubles in id order
+template <typename R>
+__global__ void k_force_by_id(Geo g, DevBufs d, const typename V2<R>::T *__restrict__ f, double2 *out) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= g.N) return;
+    out[d.lpid[q]] = make_double2((double)f[q].x, (double)f[q].y);
+}
+
 // ------------------------------------------------------------------ scan + fill
 // Full recount of bcount from the cell counts (after an upload or a
 // refresh; during steps the update keeps bcount current).
@@ -1914,6 +1938,20 @@ hipError_t launch_species_deposit(bdk_t *h, int species) {
     case 1: f32 ? launch_deposit_t<float, 1>(h, pl, st) : launch_deposit_t<double, 1>(h, pl, st); break;
     default: f32 ? launch_deposit_t<float, 2>(h, pl, st) : launch_deposit_t<double, 2>(h, pl, st); break;
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_by_id(bdk_t *h, int id0, int n, ByIdHead *head, int2 *git, double2 *rel) {
+    hipLaunchKernelGGL(k_by_id, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d, id0, n, head, git, rel);
+    return hipGetLastError();
+}
+
+hipError_t launch_force_by_id(bdk_t *h, const void *f, double2 *out) {
+    const dim3 grid(nblk(h->g.N, 256)), blk(256);
+    if (h->p.precision != BDK_FP64)
+        hipLaunchKernelGGL(k_force_by_id<float>, grid, blk, 0, h->stream, h->g, h->d, (const float2 *)f, out);
+    else
+        hipLaunchKernelGGL(k_force_by_id<double>, grid, blk, 0, h->stream, h->g, h->d, (const double2 *)f, out);
     return hipGetLastError();
 }
 
