@@ -289,6 +289,26 @@ __device__ __forceinline__ bool wca_pair(double xa, double ya, double xb, double
     return true;
 }
 
+// End of a step: step counter + 1, and the per-step scalars of the next
+// update re-armed (dt minimum and the 64 slots of dt candidates, excursion
+// slot, displacement bound).  Run by threads 0..63 of one block of the
+// step's last mesh pass (k_c2r_rows), which follows every reader of these
+// scalars in the step.
+__device__ __forceinline__ void step_end_body(const Geo &g, const DevBufs &d) {
+    const int t = threadIdx.x;
+    if (t < 64) {
+        d.exo[t * 16] = 0ull;
+        d.dts[t * 16] = ~0ull;
+    }
+    if (t == 0) {
+        const unsigned long long s = d.sc->step;
+        d.sc->dt_bits = bitsd(g.dt_max);
+        d.sc->exc_bits[s & 1] = 0ull;  // filled by the update of step s + 1
+        d.sc->step = s + 1;
+    }
+}
+
+
 // ------------------------------------------------------------------ block scan
 // exclusive scan of a[0..n) in LDS (n <= 4*blockDim.x, blockDim.x <= 1024),
 // returns the total; all threads must call it
@@ -324,6 +344,36 @@ static __device__ int block_exscan4(int *a, int n, int *wsum) {
     }
     __syncthreads();
     return total;
+}
+
+// ------------------------------------------------------------------ batches
+// Every batched kernel walks its stage's block map: one map entry per block,
+// or in the persistent form (a grid smaller than the map) each block takes
+// the entries blockIdx.x, blockIdx.x + gridDim.x, ...  Kernels whose bodies
+// use LDS end every entry with a barrier, so the next entry may refill it.
+// A member's results do not depend on the grid or on the WCA block size
+// (per-particle sums, integer deposit sums, order-free min/max reductions).
+// P (persistent) selects the form at compile time: without it a kernel
+// handles exactly its own entry (no loop, so the code and its register use
+// are those of a plain one-entry kernel).
+template <bool P, bool SYNC, typename F> __device__ __forceinline__ void for_entries(int nmap, F &&f) {
+    if (!P) {
+        f((int)blockIdx.x);
+        return;
+    }
+    for (int e = blockIdx.x; e < nmap; e += gridDim.x) {
+        f(e);
+        if (SYNC) __syncthreads();
+    }
+}
+
+static inline bool zp2(int Z) { return (Z & (Z - 1)) == 0; }
+static inline unsigned nblk(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
+
+// blocks of a launch over a map of n entries (the persistent form caps them)
+static inline unsigned stage_grid(const BatchPlan &bp, int n) {
+    const int p = bp.tune.persist;
+    return (unsigned)std::max(1, p > 0 ? std::min(n, p) : n);
 }
 
 }  // namespace bdkx

@@ -1,0 +1,796 @@
+// The three FFT passes of the mesh force (gfx950), for one simulation and for
+// batches:
+//   r2c rows   row transforms of the real mesh, transposed half spectrum out;
+//   columns    column transform, Green's function x gradient (dm:1210-1216),
+//              two inverse column transforms (Fx, Fy);
+//   c2r rows   inverse row transform of Fx + i Fy -> the real force mesh.
+// Power-of-two meshes: rows in registers (RowFft), sizes known at compile
+// time.  Other even meshes: rows in LDS, any length 2^a 3^b 5^c 7^d.
+//
+// The power-of-two passes in one place (us, r2c / columns / c2r; before, rows
+// went through LDS for the load, every pass, the product and the store, with
+// block barriers, and blocks of 256 threads took up to 16 rows of a small
+// mesh): 128^2 FP64 6.6 / 12.9 / 8.9 -> 3.3 / 5.8 / 3.1, 512^2 FP32 6.9 /
+// 11.2 / 8.1 -> 3.4 / 4.2 / 3.6, 1024^2 FP64 8.4 / 19.3 / 13.1 -> 5.7 / 10.7 /
+// 9.0, 2048^2 FP32 14.3 / 21 / 19 -> 10.1 / 15.4 / 14.9, 4096^2 FP32 104 / 120
+// / 86 -> 32 / 52 / 49.  The largest meshes are now bound by memory (134, 201
+// and 268 MB at 4096^2: 3.9 to 5.5 TB/s), 2048^2 by memory and LDS about
+// equally, the small ones by the chain of one global read, the passes and one
+// global write.
+#pragma clang fp contract(off)
+
+#include "bdk_device.hpp"
+#include "bdk_fft.hpp"
+
+namespace bdkx {
+
+constexpr int FFT_MAX_THREADS = 512;  // power-of-two passes
+
+// G(j, m') = 1/((lap[j] + lap[m']) + 1/lambda^2) (dm:585-593, dm:1384-1394)
+template <typename R> __device__ __forceinline__ R green(R lapj, R lapm, bool zero, R lam2inv) {
+    if (zero) return (R)0.0;
+    if (sizeof(R) == 4)  // FP32: the hardware reciprocal (1 ulp) instead of a correctly rounded division
+        return (R)__builtin_amdgcn_rcpf((float)((lapj + lapm) + lam2inv));
+    return (R)1.0 / ((lapj + lapm) + lam2inv);
+}
+
+// spectral factors of one (j, m') pair: gx = sq[j] G / Z / Z, gy = sq[m'] G / Z / Z
+template <typename R>
+__device__ __forceinline__ void symbols(int j, int mm, const Geo &g, const R *sq, const R *lap, R &gx, R &gy) {
+    const R G = green<R>(lap[j], lap[mm], j == 0 && mm == 0 && g.zero_mode_g, (R)g.lam2inv);
+    // x / Z / Z == x * 2^(-2 log2 Z) exactly where Z is a power of two
+    const R izz = (R)1.0 / ((R)g.Z * (R)g.Z);
+    gx = sq[j] * G * izz;
+    gy = sq[mm] * G * izz;
+}
+
+// The packed (DC, Nyquist) column at j, from P = S[j] and Q = S[Z - j]:
+// i g(., 0) S_dc + i (i g(., Z/2) S_ny) for x and y
+template <typename R, typename C>
+__device__ __forceinline__ void packed_column(int j, C P, C Q, const Geo &g, const R *sq, const R *lap, C &fx, C &fy) {
+    const C Sdc = cscale(cadd(P, cconj(Q)), (R)0.5);
+    const C Sny = cmul_mi(cscale(csub(P, cconj(Q)), (R)0.5));
+    R gx0, gy0, gxN, gyN;
+    symbols<R>(j, 0, g, sq, lap, gx0, gy0);
+    symbols<R>(j, g.Z >> 1, g, sq, lap, gxN, gyN);
+    fx = cadd(cmul_i(cscale(Sdc, gx0)), cmul_i(cmul_i(cscale(Sny, gxN))));
+    fy = cadd(cmul_i(cscale(Sdc, gy0)), cmul_i(cmul_i(cscale(Sny, gyN))));
+}
+
+// half spectrum X[m] of a real row from its packed transform: a = z[m],
+// b = z[n - m], w = exp(-2 pi i m / Z)
+template <typename C> __device__ __forceinline__ C split_real(C a, C b, C w) {
+    using R = decltype(C::x);
+    const C bc = cconj(b);
+    const C E = cscale(cadd(a, bc), (R)0.5);
+    const C O = cmul_mi(cscale(csub(a, bc), (R)0.5));
+    return cadd(E, cmul(w, O));
+}
+
+// ------------------------------------------------------------------ power-of-two meshes
+template <typename R, int LOGZ> struct P2Pass {
+    using C = typename V2<R>::T;
+    static constexpr int Z = 1 << LOGZ, E = fft_ept(Z, sizeof(R) == 4);
+    static constexpr int ER = E < Z / 2 ? E : Z / 2;  // of the r2c rows
+    static constexpr int per = 256 / (int)sizeof(C);  // elements that fill all LDS banks once
+    using Row = RowFft<R, LOGZ - 1, ER, LOGZ>;        // r2c rows: Z/2 complex points
+    using Col = RowFft<R, LOGZ, E, LOGZ>;             // columns and c2r rows
+    static constexpr int col_stride = 2 * (Z + Z / E) + 2;
+};
+
+// LDS bytes of a block of `rows` rows; pass 0 r2c, 1 columns, 2 c2r
+template <typename R, int LOGZ> static size_t p2_lds(int pass, int rows) {
+    using P = P2Pass<R, LOGZ>;
+    const size_t c = sizeof(typename P::C);
+    if (pass == 0) return (size_t)rows * row_stride(P::Z / 2, P::ER, rows, P::per) * c;
+    if (pass == 1) return (size_t)rows * P::col_stride * c;
+    return (size_t)rows * row_stride(P::Z, P::E, rows, P::per) * c;
+}
+template <typename R, int LOGZ> static int p2_threads(int pass, int rows) {
+    using P = P2Pass<R, LOGZ>;
+    return rows * (pass == 0 ? P::Row::T : P::Col::T);
+}
+
+// Row r2c: rows k0..k0+rows-1 of the real mesh -> half spectrum X[m], m<Z/2,
+// with X[0] packing (DC, Nyquist) (both real), written transposed:
+// ht[m*Z + k].  Length-Z/2 complex transform of (x[2n], x[2n+1]) + split.
+// The stores take the rows of the block together (rows x 8 or 16 bytes).
+template <typename R, int LOGZ>
+__device__ __forceinline__ void r2c_p2(const R *__restrict__ rho, typename V2<R>::T *__restrict__ ht,
+                                       const typename V2<R>::T *__restrict__ tw, int rows, int blk) {
+    using P = P2Pass<R, LOGZ>;
+    using F = typename P::Row;
+    using C = typename P::C;
+    constexpr int Z = P::Z, E = P::ER, N = F::N, T = F::T;
+    extern __shared__ unsigned char smem_raw[];
+    C *s = (C *)smem_raw;
+    const int tid = threadIdx.x, row = tid / T, t = tid % T, k0 = blk * rows, na = rows * T;
+    const int stride = row_stride(N, E, rows, P::per), lrows = __ffs(rows) - 1;
+    C *sr = s + row * stride;
+    const bool act = tid < na;
+    if (act || !F::WAVE) {
+        const C *p = (const C *)(rho + (size_t)(k0 + row) * Z) + t;
+        C v[1][E];
+#pragma unroll
+        for (int u = 0; u < E; ++u) v[0][u] = p[T * u];
+        F f;
+        f.load(tw, t);
+        f.template run<1, false, true>(v, sr, t);
+        if (F::NP > 1) row_sync<F::WAVE>();
+#pragma unroll
+        for (int u = 0; u < E; ++u) sr[T % E == 0 ? lpe<E>(t) + u * lpe<E>(T) : lpe<E>(t + T * u)] = v[0][u];
+    }
+    C w[E];
+#pragma unroll
+    for (int u = 0; u < E; ++u) w[u] = tw[((tid + u * na) >> lrows) & (N - 1)];
+    __syncthreads();
+    if (!act) return;
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+        const int i = tid + u * na, m = i >> lrows, r = i & (rows - 1);
+        const C *p = s + r * stride;
+        const C a = p[lpe<E>(m)];
+        C o;
+        if (m == 0)
+            o = cm<C>(a.x + a.y, a.x - a.y);
+        else
+            o = split_real(a, p[lpe<E>(N - m)], w[u]);
+        ht[(size_t)m * Z + k0 + r] = o;
+    }
+}
+
+// Column pass: rows m0..m0+rows-1 of ht (length Z along x), forward
+// transform, times i*gx and i*gy, inverse transform of both together, out
+// gt[m*Z+k] = (Fx, Fy).  The spectrum stays in registers in between.
+template <typename R, int LOGZ>
+__device__ __forceinline__ void col_p2(const typename V2<R>::T *__restrict__ ht, typename V4<R>::T *__restrict__ gt,
+                                       const typename V2<R>::T *__restrict__ tw, const R *__restrict__ sq,
+                                       const R *__restrict__ lap, const Geo &g, int rows, int blk) {
+    using P = P2Pass<R, LOGZ>;
+    using F = typename P::Col;
+    using C = typename P::C;
+    using C4 = typename V4<R>::T;
+    constexpr int Z = P::Z, E = P::E, T = F::T;
+    extern __shared__ unsigned char smem_raw[];
+    C *s = (C *)smem_raw;
+    const int tid = threadIdx.x, row = tid / T, t = tid % T, m0 = blk * rows, m = m0 + row;
+    const bool act = tid < rows * T;
+    C *sr = s + row * P::col_stride;
+    F f;
+    C v[1][E], xy[2][E];
+    if (act || !F::WAVE) {
+        const C *p = ht + (size_t)m * Z + t;
+#pragma unroll
+        for (int u = 0; u < E; ++u) v[0][u] = p[T * u];
+        f.load(tw, t);
+        f.template run<1, false, true>(v, sr, t);
+    }
+    if (m0 == 0) {
+        // the packed column pairs j with Z - j, held by other threads
+        __syncthreads();
+        if (act && m == 0)
+#pragma unroll
+            for (int u = 0; u < E; ++u) sr[t + T * u] = v[0][u];
+        __syncthreads();
+        if (act && m == 0)
+#pragma unroll
+            for (int u = 0; u < E; ++u) {
+                const int j = t + T * u;
+                packed_column<R, C>(j, v[0][u], sr[(Z - j) & (Z - 1)], g, sq, lap, xy[0][u], xy[1][u]);
+            }
+        __syncthreads();
+    }
+    if (!act && F::WAVE) return;
+    if (m != 0) {
+        const R sqm = sq[m], lapm = lap[m], l2 = (R)g.lam2inv, izz = (R)1.0 / ((R)Z * (R)Z);
+#pragma unroll
+        for (int u = 0; u < E; ++u) {
+            const int j = t + T * u;
+            const R G = green<R>(lap[j], lapm, false, l2);
+            const R gx = sq[j] * G * izz, gy = sqm * G * izz;
+            const C S = v[0][u];
+            xy[0][u] = cm<C>(-gx * S.y, gx * S.x);
+            xy[1][u] = cm<C>(-gy * S.y, gy * S.x);
+        }
+    }
+    f.template run<2, true, F::NP == 1>(xy, sr, t);
+    C4 *o = gt + (size_t)m * Z + t;
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+        C4 q;
+        q.x = xy[0][u].x;
+        q.y = xy[0][u].y;
+        q.z = xy[1][u].x;
+        q.w = xy[1][u].y;
+        o[T * u] = q;
+    }
+}
+
+// Row c2r of the two real signals Fx, Fy: rows k0..k0+rows-1, spectrum
+// C[m] = X[m] + i Y[m] completed by Hermitian symmetry, inverse transform of
+// length Z, out fmesh[k*Z + l] = (Re, Im) = (Fx, Fy).
+template <typename R, int LOGZ>
+__device__ __forceinline__ void c2r_p2(const typename V4<R>::T *__restrict__ gt, typename V2<R>::T *__restrict__ fm,
+                                       const typename V2<R>::T *__restrict__ tw, int rows, int blk) {
+    using P = P2Pass<R, LOGZ>;
+    using F = typename P::Col;
+    using C = typename P::C;
+    using C4 = typename V4<R>::T;
+    constexpr int Z = P::Z, E = P::E, T = F::T;
+    extern __shared__ unsigned char smem_raw[];
+    C *s = (C *)smem_raw;
+    const int tid = threadIdx.x, row = tid / T, t = tid % T, k0 = blk * rows, na = rows * T;
+    const int stride = row_stride(Z, E, rows, P::per), lrows = __ffs(rows) - 1;
+    const bool act = tid < na;
+    F f;
+    if (act) {
+        C4 q[E / 2];
+#pragma unroll
+        for (int u = 0; u < E / 2; ++u) {
+            const int i = tid + u * na;
+            q[u] = gt[(size_t)(i >> lrows) * Z + k0 + (i & (rows - 1))];
+        }
+        f.load(tw, t);
+#pragma unroll
+        for (int u = 0; u < E / 2; ++u) {
+            const int i = tid + u * na, m = i >> lrows;
+            C *p = s + (i & (rows - 1)) * stride;
+            if (m == 0) {
+                p[0] = cm<C>(q[u].x, q[u].z);
+                p[lpe<E>(Z / 2)] = cm<C>(q[u].y, q[u].w);
+            } else {
+                p[lpe<E>(m)] = cm<C>(q[u].x - q[u].w, q[u].y + q[u].z);
+                p[lpe<E>(Z - m)] = cm<C>(q[u].x + q[u].w, -q[u].y + q[u].z);
+            }
+        }
+    }
+    __syncthreads();
+    if (!act && F::WAVE) return;
+    C *sr = s + row * stride;
+    C v[1][E];
+    F::template gather<1>(v, sr, t);
+    f.template run<1, true, false>(v, sr, t);
+    C *o = fm + (size_t)(k0 + row) * Z + t;
+#pragma unroll
+    for (int u = 0; u < E; ++u) o[T * u] = v[0][u];
+}
+
+template <typename R, int LOGZ>
+__global__ __launch_bounds__(FFT_MAX_THREADS) void k_r2c_rows(const R *__restrict__ rho,
+                                                              typename V2<R>::T *__restrict__ ht,
+                                                              const typename V2<R>::T *__restrict__ tw, int rows,
+                                                              int remap) {
+    r2c_p2<R, LOGZ>(rho, ht, tw, rows, xcd_block(remap));
+}
+
+template <typename R, int LOGZ>
+__global__ __launch_bounds__(FFT_MAX_THREADS) void k_col(const typename V2<R>::T *__restrict__ ht,
+                                                         typename V4<R>::T *__restrict__ gt,
+                                                         const typename V2<R>::T *__restrict__ tw,
+                                                         const R *__restrict__ sq, const R *__restrict__ lap, Geo g,
+                                                         int rows) {
+    col_p2<R, LOGZ>(ht, gt, tw, sq, lap, g, rows, blockIdx.x);
+}
+
+template <typename R, int LOGZ>
+__global__ __launch_bounds__(FFT_MAX_THREADS) void k_c2r_rows(const typename V4<R>::T *__restrict__ gt,
+                                                              typename V2<R>::T *__restrict__ fm,
+                                                              const typename V2<R>::T *__restrict__ tw, int rows,
+                                                              int remap, Geo g, DevBufs d, int end_step) {
+    if (end_step && blockIdx.x == 0) step_end_body(g, d);
+    c2r_p2<R, LOGZ>(gt, fm, tw, rows, xcd_block(remap));
+}
+
+// ------------------------------------------------------------------ other meshes
+// Rows in LDS: the block's rows are read, transformed in place and written.
+template <typename R, int EPT>
+__device__ __forceinline__ void r2c_any(const R *__restrict__ rho, typename V2<R>::T *__restrict__ ht,
+                                        const typename V2<R>::T *__restrict__ tw, int Z, int RB, int stride, int blk) {
+    using C = typename V2<R>::T;
+    extern __shared__ unsigned char smem_raw[];
+    C *s = (C *)smem_raw;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int n = Z >> 1;
+    const Dv dn(n), drb(RB);
+    const int k0 = blk * RB;
+    for (int idx = tid; idx < RB * n; idx += nt) {
+        const int row = dn.q(idx), m = dn.r(idx);
+        s[row * stride + lp(m)] = ((const C *)(rho + (size_t)(k0 + row) * Z))[m];
+    }
+    __syncthreads();
+    lds_fft_g<R, EPT>(s, n, RB, stride, tw, Z, false);
+    for (int idx = tid; idx < RB * n; idx += nt) {
+        const int m = drb.q(idx), row = drb.r(idx);
+        const C *p = s + row * stride;
+        const C a = p[lp(m)];
+        ht[(size_t)m * Z + k0 + row] = m == 0 ? cm<C>(a.x + a.y, a.x - a.y) : split_real(a, p[lp(n - m)], tw[m]);
+    }
+}
+
+template <typename R, int EPT>
+__device__ __forceinline__ void col_any(const typename V2<R>::T *__restrict__ ht, typename V4<R>::T *__restrict__ gt,
+                                        const typename V2<R>::T *__restrict__ tw, const R *__restrict__ sq,
+                                        const R *__restrict__ lap, const Geo &g, int RC, int stride, int blk) {
+    using C = typename V2<R>::T;
+    using C4 = typename V4<R>::T;
+    extern __shared__ unsigned char smem_raw[];
+    C *s = (C *)smem_raw;
+    C *sB = s + RC * stride;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int Z = g.Z, Zh = Z >> 1;
+    const Dv dz(Z);
+    const int m0 = blk * RC;
+    for (int idx = tid; idx < RC * Z; idx += nt) {
+        const int row = dz.q(idx), k = dz.r(idx);
+        s[row * stride + lp(k)] = ht[(size_t)(m0 + row) * Z + k];
+    }
+    __syncthreads();
+    lds_fft_g<R, EPT>(s, Z, RC, stride, tw, Z, false);
+    for (int idx = tid; idx < RC * Z; idx += nt) {
+        const int row = dz.q(idx), j = dz.r(idx);
+        const int m = m0 + row;
+        if (m == 0) {
+            // packed (DC, Nyquist) column: pairs (j, Z-j) by one thread
+            if (j > Zh) continue;
+            const int jn = j == 0 ? 0 : Z - j;
+            const C P = s[lp(j)], Q = s[lp(jn)];
+            C fx, fy, gx, gy;
+            packed_column<R, C>(j, P, Q, g, sq, lap, fx, fy);
+            packed_column<R, C>(jn, Q, P, g, sq, lap, gx, gy);
+            s[lp(j)] = fx;
+            sB[lp(j)] = fy;
+            if (jn != j) {
+                s[lp(jn)] = gx;
+                sB[lp(jn)] = gy;
+            }
+        } else {
+            R gx, gy;
+            symbols<R>(j, m, g, sq, lap, gx, gy);
+            const int o = row * stride + lp(j);
+            const C S = s[o];
+            s[o] = cm<C>(-gx * S.y, gx * S.x);
+            sB[o] = cm<C>(-gy * S.y, gy * S.x);
+        }
+    }
+    __syncthreads();
+    lds_fft_g<R, EPT>(s, Z, 2 * RC, stride, tw, Z, true);
+    for (int idx = tid; idx < RC * Z; idx += nt) {
+        const int row = dz.q(idx), k = dz.r(idx);
+        const int so = row * stride + lp(k);
+        const C a = s[so], b = sB[so];
+        C4 o;
+        o.x = a.x;
+        o.y = a.y;
+        o.z = b.x;
+        o.w = b.y;
+        gt[(size_t)(m0 + row) * Z + k] = o;
+    }
+}
+
+template <typename R, int EPT>
+__device__ __forceinline__ void c2r_any(const typename V4<R>::T *__restrict__ gt, typename V2<R>::T *__restrict__ fm,
+                                        const typename V2<R>::T *__restrict__ tw, int Z, int RB2, int stride,
+                                        int blk) {
+    using C = typename V2<R>::T;
+    using C4 = typename V4<R>::T;
+    extern __shared__ unsigned char smem_raw[];
+    C *s = (C *)smem_raw;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int Zh = Z >> 1;
+    const Dv dz(Z), drb(RB2);
+    const int k0 = blk * RB2;
+    for (int idx = tid; idx < RB2 * Zh; idx += nt) {
+        const int m = drb.q(idx), row = drb.r(idx);
+        const C4 v = gt[(size_t)m * Z + k0 + row];
+        C *p = s + row * stride;
+        if (m == 0) {
+            p[0] = cm<C>(v.x, v.z);
+            p[lp(Zh)] = cm<C>(v.y, v.w);
+        } else {
+            p[lp(m)] = cm<C>(v.x - v.w, v.y + v.z);
+            p[lp(Z - m)] = cm<C>(v.x + v.w, -v.y + v.z);
+        }
+    }
+    __syncthreads();
+    lds_fft_g<R, EPT>(s, Z, RB2, stride, tw, Z, true);
+    for (int idx = tid; idx < RB2 * Z; idx += nt) {
+        const int row = dz.q(idx), l = dz.r(idx);
+        fm[(size_t)(k0 + row) * Z + l] = s[row * stride + lp(l)];
+    }
+}
+
+template <typename R, int EPT>
+__global__ __launch_bounds__(FFT_THREADS) void k_r2c_any(const R *__restrict__ rho, typename V2<R>::T *__restrict__ ht,
+                                                         const typename V2<R>::T *__restrict__ tw, int Z, int RB,
+                                                         int stride, int remap) {
+    r2c_any<R, EPT>(rho, ht, tw, Z, RB, stride, xcd_block(remap));
+}
+
+template <typename R, int EPT>
+__global__ __launch_bounds__(FFT_THREADS) void k_col_any(const typename V2<R>::T *__restrict__ ht,
+                                                         typename V4<R>::T *__restrict__ gt,
+                                                         const typename V2<R>::T *__restrict__ tw,
+                                                         const R *__restrict__ sq, const R *__restrict__ lap, Geo g,
+                                                         int RC, int stride) {
+    col_any<R, EPT>(ht, gt, tw, sq, lap, g, RC, stride, blockIdx.x);
+}
+
+template <typename R, int EPT>
+__global__ __launch_bounds__(FFT_THREADS) void k_c2r_any(const typename V4<R>::T *__restrict__ gt,
+                                                         typename V2<R>::T *__restrict__ fm,
+                                                         const typename V2<R>::T *__restrict__ tw, int Z, int RB2,
+                                                         int stride, int remap, Geo g, DevBufs d, int end_step) {
+    if (end_step && blockIdx.x == 0) step_end_body(g, d);
+    c2r_any<R, EPT>(gt, fm, tw, Z, RB2, stride, xcd_block(remap));
+}
+
+// ------------------------------------------------------------------ batched
+// One map entry per block; the size is the member's, so one launch serves
+// every power-of-two mesh with the same points per thread.
+#define BDK_LOGZ_LOW(CALL) \
+    case 3: CALL(3); break;   \
+    case 4: CALL(4); break;   \
+    case 5: CALL(5); break;   \
+    case 6: CALL(6); break;   \
+    case 7: CALL(7); break;   \
+    case 8: CALL(8); break;   \
+    case 9: CALL(9); break;
+#define BDK_LOGZ_HIGH(CALL) \
+    case 10: CALL(10); break; \
+    case 11: CALL(11); break; \
+    default: CALL(12); break;
+
+// H: FP32 meshes of 1024 points and more (16 points per thread)
+template <typename R, bool P, bool H>
+__global__ __launch_bounds__(FFT_MAX_THREADS) void kb_r2c(const RepDev *m, const int2 *map, int nmap) {
+    using C = typename V2<R>::T;
+    for_entries<P, true>(nmap, [&](int e_) {
+        const int2 t = map[e_];
+        const RepDev &r = m[t.x];
+#define CALL(LZ) r2c_p2<R, LZ>((const R *)r.d.rho, (C *)r.d.ht, (const C *)r.d.tw, r.rb, t.y)
+        if constexpr (H) {
+            switch (r.g.logZ) { BDK_LOGZ_HIGH(CALL) }
+        } else if constexpr (sizeof(R) == 4) {
+            switch (r.g.logZ) { BDK_LOGZ_LOW(CALL) }
+        } else {
+            switch (r.g.logZ) { BDK_LOGZ_LOW(CALL) BDK_LOGZ_HIGH(CALL) }
+        }
+#undef CALL
+    });
+}
+
+template <typename R, bool P, bool H>
+__global__ __launch_bounds__(FFT_MAX_THREADS) void kb_col(const RepDev *m, const int2 *map, int nmap) {
+    using C = typename V2<R>::T;
+    using C4 = typename V4<R>::T;
+    for_entries<P, true>(nmap, [&](int e_) {
+        const int2 t = map[e_];
+        const RepDev &r = m[t.x];
+        const R *sq = std::is_same<R, float>::value ? (const R *)r.d.sqf : (const R *)r.d.sq;
+        const R *lap = std::is_same<R, float>::value ? (const R *)r.d.lapf : (const R *)r.d.lap;
+#define CALL(LZ) col_p2<R, LZ>((const C *)r.d.ht, (C4 *)r.d.gt, (const C *)r.d.tw, sq, lap, r.g, r.rc, t.y)
+        if constexpr (H) {
+            switch (r.g.logZ) { BDK_LOGZ_HIGH(CALL) }
+        } else if constexpr (sizeof(R) == 4) {
+            switch (r.g.logZ) { BDK_LOGZ_LOW(CALL) }
+        } else {
+            switch (r.g.logZ) { BDK_LOGZ_LOW(CALL) BDK_LOGZ_HIGH(CALL) }
+        }
+#undef CALL
+    });
+}
+
+template <typename R, bool P, bool H>
+__global__ __launch_bounds__(FFT_MAX_THREADS) void kb_c2r(const RepDev *m, const int2 *map, int nmap, int end_step) {
+    using C = typename V2<R>::T;
+    using C4 = typename V4<R>::T;
+    for_entries<P, true>(nmap, [&](int e_) {
+        const int2 t = map[e_];
+        const RepDev &r = m[t.x];
+        if (end_step && t.y == 0) step_end_body(r.g, r.d);
+#define CALL(LZ) c2r_p2<R, LZ>((const C4 *)r.d.gt, (C *)r.d.fmesh, (const C *)r.d.tw, r.rb2, t.y)
+        if constexpr (H) {
+            switch (r.g.logZ) { BDK_LOGZ_HIGH(CALL) }
+        } else if constexpr (sizeof(R) == 4) {
+            switch (r.g.logZ) { BDK_LOGZ_LOW(CALL) }
+        } else {
+            switch (r.g.logZ) { BDK_LOGZ_LOW(CALL) BDK_LOGZ_HIGH(CALL) }
+        }
+#undef CALL
+    });
+}
+
+template <typename R, int EPT, bool P>
+__global__ __launch_bounds__(FFT_THREADS) void kb_r2c_any(const RepDev *m, const int2 *map, int nmap) {
+    using C = typename V2<R>::T;
+    for_entries<P, true>(nmap, [&](int e_) {
+        const int2 t = map[e_];
+        const RepDev &r = m[t.x];
+        r2c_any<R, EPT>((const R *)r.d.rho, (C *)r.d.ht, (const C *)r.d.tw, r.g.Z, r.rb, r.sR1, t.y);
+    });
+}
+
+template <typename R, int EPT, bool P>
+__global__ __launch_bounds__(FFT_THREADS) void kb_col_any(const RepDev *m, const int2 *map, int nmap) {
+    using C = typename V2<R>::T;
+    using C4 = typename V4<R>::T;
+    for_entries<P, true>(nmap, [&](int e_) {
+        const int2 t = map[e_];
+        const RepDev &r = m[t.x];
+        const R *sq = std::is_same<R, float>::value ? (const R *)r.d.sqf : (const R *)r.d.sq;
+        const R *lap = std::is_same<R, float>::value ? (const R *)r.d.lapf : (const R *)r.d.lap;
+        col_any<R, EPT>((const C *)r.d.ht, (C4 *)r.d.gt, (const C *)r.d.tw, sq, lap, r.g, r.rc, r.sC, t.y);
+    });
+}
+
+template <typename R, int EPT, bool P>
+__global__ __launch_bounds__(FFT_THREADS) void kb_c2r_any(const RepDev *m, const int2 *map, int nmap, int end_step) {
+    using C = typename V2<R>::T;
+    using C4 = typename V4<R>::T;
+    for_entries<P, true>(nmap, [&](int e_) {
+        const int2 t = map[e_];
+        const RepDev &r = m[t.x];
+        if (end_step && t.y == 0) step_end_body(r.g, r.d);
+        c2r_any<R, EPT>((const C4 *)r.d.gt, (C *)r.d.fmesh, (const C *)r.d.tw, r.g.Z, r.rb2, r.sR2, t.y);
+    });
+}
+
+// ------------------------------------------------------------------ launchers
+// the largest divisor of m not above cap (at least 1)
+static int div_at_most(int m, int cap) {
+    cap = std::max(1, std::min(m, cap));
+    while (m % cap) --cap;
+    return cap;
+}
+
+// rows of a pass (of its batch or single launch)
+static int pass_rows(int pass, int Z) { return pass == 1 ? Z / 2 : Z; }
+// complex values a row of the pass keeps in a block
+static int pass_need(int pass, int Z) { return pass == 0 ? Z / 2 : (pass == 1 ? 2 * Z : Z); }
+
+static size_t p2_lds_bytes(bool f32, int Z, int pass, int rows) {
+#define CALL(LZ) return f32 ? p2_lds<float, LZ>(pass, rows) : p2_lds<double, LZ>(pass, rows)
+    switch (__builtin_ctz(Z)) { BDK_LOGZ_LOW(CALL) BDK_LOGZ_HIGH(CALL) }
+#undef CALL
+    return 0;
+}
+static int p2_block(bool f32, int Z, int pass, int rows) {
+#define CALL(LZ) return f32 ? p2_threads<float, LZ>(pass, rows) : p2_threads<double, LZ>(pass, rows)
+    switch (__builtin_ctz(Z)) { BDK_LOGZ_LOW(CALL) BDK_LOGZ_HIGH(CALL) }
+#undef CALL
+    return 0;
+}
+
+// Rows per block of a power-of-two pass.  The columns need no company (one per
+// block).  The r2c rows are stored and the c2r rows read across rows, so 4
+// rows of a block make 32 or 64 consecutive bytes; below 1024 points, where
+// the mesh lies in the caches, more blocks count for more.  Measured (us, rows
+// 1 / 2 / 4 / 8): r2c 2048^2 FP32 15.6 / 11.8 / 10.1 / 10.3, 4096^2 80 / 45 /
+// 32 / -, 1024^2 FP64 6.7 / 6.4 / 5.7 / 6.7, 512^2 FP32 3.4 / 3.8 / 3.7 / 4.1;
+// c2r 2048^2 18.1 / 15.4 / 14.9 / 15.0, 4096^2 76 / 49 / 49 / -, 1024^2 FP64
+// 9.6 / 9.0 / 9.3 / 9.3, 512^2 3.6 / 4.2 / 4.1 / 4.3; columns at 2 instead of
+// 1: 15.4 to 15.6, 10.7 to 11.6 and 4.2 to 5.0.  At least a wave per block.
+static int p2_rows(bool f32, int Z, int pass) {
+    const int all = pass_rows(pass, Z), t = p2_block(f32, Z, pass, 1);
+    const int want = pass == 1 || Z < 1024 ? 1 : (pass == 2 && Z < 2048 ? 2 : 4);
+    int rows = 1;
+    while (rows < all && (rows < want || rows * t < 64)) rows *= 2;
+    while (rows > 1 && rows * t > FFT_MAX_THREADS) rows /= 2;
+    return rows;
+}
+
+// Threads and elements per thread of a pass over a mesh of another size:
+// 128 threads of 8 elements where a row fits (384^2 FP64: 17.2 / 11.8 us for
+// the columns and c2r rows at 256 threads of 16, 11.0 / 7.1 so), else 256
+// threads of as many as the row needs.
+struct AnyCfg {
+    int ept, threads, rows, stride;
+    size_t lds;
+};
+static AnyCfg any_cfg(int pass, int Z, size_t csz) {
+    const int need = pass_need(pass, Z);
+    AnyCfg c;
+    c.threads = need <= 8 * 128 ? 128 : FFT_THREADS;
+    c.ept = ept_for(8, need);
+    c.rows = div_at_most(pass_rows(pass, Z), c.ept * c.threads / need);
+    c.stride = lds_row(pass == 0 ? Z / 2 : Z);
+    c.lds = (size_t)(pass == 1 ? 2 : 1) * c.rows * c.stride * csz;
+    return c;
+}
+
+template <typename R> static void launch_pass_p2(bdk_t *h, int pass, hipStream_t st, int end_step) {
+    using C = typename V2<R>::T;
+    using C4 = typename V4<R>::T;
+    constexpr bool f32 = sizeof(R) == 4;
+    const int Z = h->g.Z, rows = p2_rows(f32, Z, pass);
+    const dim3 grid(pass_rows(pass, Z) / rows), blk(std::max(64, p2_block(f32, Z, pass, rows)));
+    const size_t lds = p2_lds_bytes(f32, Z, pass, rows);
+    const R *sq = f32 ? (const R *)h->d.sqf : (const R *)h->d.sq, *lap = f32 ? (const R *)h->d.lapf : (const R *)h->d.lap;
+    const C *tw = (const C *)h->d.tw;
+#define R2C(LZ) \
+    hipLaunchKernelGGL((k_r2c_rows<R, LZ>), grid, blk, lds, st, (const R *)h->d.rho, (C *)h->d.ht, tw, rows, h->g.xcd)
+#define COL(LZ)                                                                                                   \
+    hipLaunchKernelGGL((k_col<R, LZ>), grid, blk, lds, st, (const C *)h->d.ht, (C4 *)h->d.gt, tw, sq, lap, h->g, \
+                       rows)
+#define C2R(LZ)                                                                                               \
+    hipLaunchKernelGGL((k_c2r_rows<R, LZ>), grid, blk, lds, st, (const C4 *)h->d.gt, (C *)h->d.fmesh, tw, rows, \
+                       h->g.xcd, h->g, h->d, end_step)
+    if (pass == 0)
+        switch (h->g.logZ) { BDK_LOGZ_LOW(R2C) BDK_LOGZ_HIGH(R2C) }
+    else if (pass == 1)
+        switch (h->g.logZ) { BDK_LOGZ_LOW(COL) BDK_LOGZ_HIGH(COL) }
+    else
+        switch (h->g.logZ) { BDK_LOGZ_LOW(C2R) BDK_LOGZ_HIGH(C2R) }
+#undef R2C
+#undef COL
+#undef C2R
+}
+
+template <typename R> static void launch_pass_any(bdk_t *h, int pass, hipStream_t st, int end_step) {
+    using C = typename V2<R>::T;
+    using C4 = typename V4<R>::T;
+    const int Z = h->g.Z;
+    const AnyCfg c = any_cfg(pass, Z, sizeof(C));
+    const dim3 grid(pass_rows(pass, Z) / c.rows), blk(c.threads);
+    const R *sq = sizeof(R) == 4 ? (const R *)h->d.sqf : (const R *)h->d.sq;
+    const R *lap = sizeof(R) == 4 ? (const R *)h->d.lapf : (const R *)h->d.lap;
+    const C *tw = (const C *)h->d.tw;
+#define R2C(E)                                                                                                        \
+    hipLaunchKernelGGL((k_r2c_any<R, E>), grid, blk, c.lds, st, (const R *)h->d.rho, (C *)h->d.ht, tw, Z, c.rows,       \
+                       c.stride, h->g.xcd)
+#define COL(E)                                                                                                        \
+    hipLaunchKernelGGL((k_col_any<R, E>), grid, blk, c.lds, st, (const C *)h->d.ht, (C4 *)h->d.gt, tw, sq, lap, h->g,   \
+                       c.rows, c.stride)
+#define C2R(E)                                                                                                        \
+    hipLaunchKernelGGL((k_c2r_any<R, E>), grid, blk, c.lds, st, (const C4 *)h->d.gt, (C *)h->d.fmesh, tw, Z, c.rows,    \
+                       c.stride, h->g.xcd, h->g, h->d, end_step)
+    if (pass == 0)
+        BDK_EPT_SWITCH(c.ept, R2C)
+    else if (pass == 1)
+        BDK_EPT_SWITCH(c.ept, COL)
+    else
+        BDK_EPT_SWITCH(c.ept, C2R)
+#undef R2C
+#undef COL
+#undef C2R
+}
+
+hipError_t launch_fft_pass(bdk_t *h, int pass, hipStream_t st, int end_step) {
+    if (!st) st = h->stream;
+    const bool f32 = h->p.precision != BDK_FP64;
+    if (zp2(h->g.Z))
+        f32 ? launch_pass_p2<float>(h, pass, st, end_step) : launch_pass_p2<double>(h, pass, st, end_step);
+    else
+        f32 ? launch_pass_any<float>(h, pass, st, end_step) : launch_pass_any<double>(h, pass, st, end_step);
+    return hipGetLastError();
+}
+
+hipError_t launch_fft(bdk_t *h) {
+    hipError_t e = hipSuccess;
+    for (int p = 0; p < 3 && e == hipSuccess; ++p) e = launch_fft_pass(h, p);
+    return e;
+}
+
+int batch_min_ept(int stage, int zmax) { return ept_for(8, pass_need(stage, zmax)); }
+
+// rows per block of a member's passes for the batch's elements per thread
+// (ept x FFT_THREADS complex values per block), and the LDS its launches need
+void fft_member(RepDev &r, int Z, const int ept[3], BatchPlan &bp) {
+    int rows[3];
+    for (int k = 0; k < 3; ++k) {
+        const int cap = ept[k] * FFT_THREADS / pass_need(k, Z);
+        size_t lds;
+        int kind;
+        if (zp2(Z)) {
+            rows[k] = 1;
+            while (2 * rows[k] <= std::min(cap, pass_rows(k, Z)) &&
+                   p2_block(bp.f32, Z, k, 2 * rows[k]) <= FFT_MAX_THREADS)
+                rows[k] *= 2;
+            lds = p2_lds_bytes(bp.f32, Z, k, rows[k]);
+            kind = fft_ept(Z, bp.f32) == 16 ? 0 : 1;
+            bp.fft_threads[kind][k] = std::max(bp.fft_threads[kind][k], std::max(64, p2_block(bp.f32, Z, k, rows[k])));
+        } else {
+            rows[k] = div_at_most(pass_rows(k, Z), cap);
+            lds = (size_t)(k == 1 ? 2 : 1) * rows[k] * lds_row(k == 0 ? Z / 2 : Z) * (bp.f32 ? 8 : 16);
+            kind = 2;
+            bp.fft_threads[kind][k] = FFT_THREADS;
+        }
+        bp.fft_lds[kind][k] = std::max(bp.fft_lds[kind][k], lds);
+    }
+    r.rb = rows[0];
+    r.rc = rows[1];
+    r.rb2 = rows[2];
+    r.sR1 = lds_row(Z / 2);
+    r.sC = lds_row(Z);
+    r.sR2 = lds_row(Z);
+}
+
+// stage 2 r2c, 3 columns, 4 c2r, 12 c2r + step end: one launch per kind of
+// mesh present (16 points per thread, other powers of two, other sizes)
+template <typename R, bool P> static void batch_fft_t(const BatchPlan &bp, int stage, hipStream_t st) {
+    const int pass = stage == 2 ? 0 : (stage == 3 ? 1 : 2), S = pass == 0 ? BS_R2C : (pass == 1 ? BS_COL : BS_C2R);
+    const int cut[4] = {0, bp.nblk16[S], bp.nblk2[S], bp.nblk[S]};
+    const RepDev *m = bp.reps;
+    for (int kind = 0; kind < 3; ++kind) {
+        const int n = cut[kind + 1] - cut[kind];
+        if (n <= 0) continue;
+        const int2 *map = bp.map[S] + cut[kind];
+        const dim3 grid(stage_grid(bp, n)), blk(bp.fft_threads[kind][pass]);
+        const size_t lds = bp.fft_lds[kind][pass];
+        const int end = stage == 12 ? 1 : 0;
+        if (kind < 2) {
+            auto go = [&](auto h) {
+                constexpr bool H = decltype(h)::value && sizeof(R) == 4;
+                if (pass == 0)
+                    hipLaunchKernelGGL((kb_r2c<R, P, H>), grid, blk, lds, st, m, map, n);
+                else if (pass == 1)
+                    hipLaunchKernelGGL((kb_col<R, P, H>), grid, blk, lds, st, m, map, n);
+                else
+                    hipLaunchKernelGGL((kb_c2r<R, P, H>), grid, blk, lds, st, m, map, n, end);
+            };
+            if (kind == 0)
+                go(std::true_type());
+            else
+                go(std::false_type());
+        } else {
+#define R2C(E) hipLaunchKernelGGL((kb_r2c_any<R, E, P>), grid, blk, lds, st, m, map, n)
+#define COL(E) hipLaunchKernelGGL((kb_col_any<R, E, P>), grid, blk, lds, st, m, map, n)
+#define C2R(E) hipLaunchKernelGGL((kb_c2r_any<R, E, P>), grid, blk, lds, st, m, map, n, end)
+            if (pass == 0)
+                BDK_EPT_SWITCH(bp.ept[0], R2C)
+            else if (pass == 1)
+                BDK_EPT_SWITCH(bp.ept[1], COL)
+            else
+                BDK_EPT_SWITCH(bp.ept[2], C2R)
+#undef R2C
+#undef COL
+#undef C2R
+        }
+    }
+}
+
+void batch_fft_stage(const BatchPlan &bp, int stage, hipStream_t st) {
+    const bool p = bp.tune.persist > 0;
+    if (bp.f32)
+        p ? batch_fft_t<float, true>(bp, stage, st) : batch_fft_t<float, false>(bp, stage, st);
+    else
+        p ? batch_fft_t<double, true>(bp, stage, st) : batch_fft_t<double, false>(bp, stage, st);
+}
+
+// dynamic LDS above the default limit
+hipError_t fft_set_attributes() {
+    hipError_t e = hipSuccess;
+    auto big = [&](const void *k) {
+        if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    };
+#define ONE(R, LZ)                          \
+    big((const void *)k_r2c_rows<R, LZ>); \
+    big((const void *)k_col<R, LZ>);      \
+    big((const void *)k_c2r_rows<R, LZ>);
+#define BOTH(LZ) ONE(float, LZ) ONE(double, LZ)
+    BOTH(3) BOTH(4) BOTH(5) BOTH(6) BOTH(7) BOTH(8) BOTH(9) BOTH(10) BOTH(11) BOTH(12)
+#undef BOTH
+#undef ONE
+#define ANY(R, E)                              \
+    big((const void *)k_r2c_any<R, E>);      \
+    big((const void *)k_col_any<R, E>);      \
+    big((const void *)k_c2r_any<R, E>);      \
+    big((const void *)kb_r2c_any<R, E, false>); \
+    big((const void *)kb_col_any<R, E, false>); \
+    big((const void *)kb_c2r_any<R, E, false>); \
+    big((const void *)kb_r2c_any<R, E, true>);  \
+    big((const void *)kb_col_any<R, E, true>);  \
+    big((const void *)kb_c2r_any<R, E, true>);
+    ANY(float, 8) ANY(float, 16) ANY(float, 32) ANY(double, 8) ANY(double, 16) ANY(double, 32)
+#undef ANY
+#define KB(R, P, H)                       \
+    big((const void *)kb_r2c<R, P, H>); \
+    big((const void *)kb_col<R, P, H>); \
+    big((const void *)kb_c2r<R, P, H>);
+    KB(float, false, false) KB(float, true, false) KB(float, false, true) KB(float, true, true)
+    KB(double, false, false) KB(double, true, false)
+#undef KB
+    return e;
+}
+
+}  // namespace bdkx

@@ -1,4 +1,5 @@
-// Stockham transforms of rows held in LDS (device code).
+// Stockham transforms of mesh rows (device code): rows of 2^n points in
+// registers, rows of other lengths in LDS.
 #pragma once
 #include "bdk_device.hpp"
 
@@ -82,125 +83,171 @@ __device__ __forceinline__ void dft16(const C *v, C *y, bool inv) {
     }
 }
 
-// LDS layout of the FFT rows: element i of a row sits at lp(i), one padding
-// element after every 8.  The output strides of the first Stockham passes
-// (8 and 64 elements) then spread over the banks instead of piling onto a
-// few (measured: half the LDS cycles of the unpadded passes were bank
-// conflicts).  A row of n elements takes n + n/8 + 1 (odd) elements.
+// ------------------------------------------------------------------ rows of 2^LOGN points
+// Sync between the LDS writes and reads of one row: in-order LDS and a fence
+// where one wave holds the whole row, else the block's barrier.
+template <bool WAVE> __device__ __forceinline__ void row_sync() {
+    if (WAVE) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+        __syncthreads();
+    }
+}
+
+// Elements per thread of a power-of-two mesh: 16 in FP32 from 1024 points on
+// (radix-16 passes, a 1024-point row in one wave), else 8.  It fixes the
+// passes and so the rounding: the mesh decides, not the launch, so a
+// simulation transforms alike alone and in a batch.
+__host__ __device__ constexpr int fft_ept(int Z, bool f32) { return f32 && Z >= 1024 ? 16 : 8; }
+
+// LDS index of element i of a row, one padding element after every E: the
+// writes of a pass (strides E, E^2, ...) and the consecutive reads then touch
+// every bank once per 32 lanes (8-byte elements) or 16 lanes (16-byte ones).
+template <int E> __host__ __device__ __forceinline__ constexpr int lpe(int i) {
+    return i + (i >> (E == 16 ? 4 : (E == 8 ? 3 : 2)));
+}
+// A row of 2^LOGN points, transformed by T = 2^LOGN / E threads with E points
+// each in registers: thread t always holds the points t + T u, u < E.
+// Stockham passes of radix E (the last one smaller if need be): butterfly
+// j = t + T e takes the points j + (N/r) i, which are the thread's own, and
+// its outputs k + (j - k) r + Ns i (k = j mod Ns) go through LDS to the
+// threads that hold them next; after the last pass they are the thread's own
+// points again.  So the first pass reads and the last pass writes global
+// memory directly (consecutive threads, consecutive points), and a forward
+// transform, a product and an inverse transform need no exchange between them.
+// tw[k] = exp(-2 pi i k / Z), Z = 2^LOGZ; the powers a pass needs (1, 2, 4, 8;
+// the others as products, up to three roundings deeper) are loaded once by
+// load(), ahead of the passes, and serve both directions.
+template <typename R, int LOGN, int E, int LOGZ> struct RowFft {
+    using C = typename V2<R>::T;
+    static constexpr int LE = E == 16 ? 4 : (E == 8 ? 3 : 2);
+    static constexpr int N = 1 << LOGN, T = N / E, NP = (LOGN + LE - 1) / LE;
+    static constexpr bool WAVE = T <= 64;
+    static constexpr int logr(int p) { return p + 1 < NP ? LE : LOGN - LE * (NP - 1); }
+
+    C tb[NP][8];  // base twiddles of pass p: [butterfly][power 1, 2, 4, 8] (tb[0] unused)
+
+    __device__ __forceinline__ void load(const C *__restrict__ tw, int t) {
+#pragma unroll
+        for (int p = 1; p < NP; ++p) {
+            const int lr = logr(p), nb = E >> lr, ns = 1 << (LE * p);
+#pragma unroll
+            for (int e = 0; e < nb; ++e) {
+                const int k = (t + e * T) & (ns - 1);
+#pragma unroll
+                for (int i = 0; i < lr; ++i) tb[p][e * lr + i] = tw[(k << i) << (LOGZ - LE * p - lr)];
+            }
+        }
+    }
+
+    // pass P on A rows at once (their twiddle products are shared)
+    template <int P, int A, bool INV> __device__ __forceinline__ void pass(C (&v)[A][E]) const {
+        constexpr int LR = logr(P), RAD = 1 << LR, NB = E / RAD;
+#pragma unroll
+        for (int e = 0; e < NB; ++e) {
+            C w[RAD];
+            if (P > 0) {
+                const C *b = &tb[P][e * LR];
+                w[1] = b[0];
+                if (RAD >= 4) {
+                    w[2] = b[1];
+                    w[3] = cmul(w[1], w[2]);
+                }
+                if (RAD >= 8) {
+                    w[4] = b[2];
+                    w[5] = cmul(w[4], w[1]);
+                    w[6] = cmul(w[4], w[2]);
+                    w[7] = cmul(w[4], w[3]);
+                }
+                if (RAD == 16) {
+                    w[8] = b[3];
+#pragma unroll
+                    for (int i = 9; i < 16; ++i) w[i] = cmul(w[8], w[i - 8]);
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < A; ++a) {
+                C x[RAD], y[RAD];
+#pragma unroll
+                for (int i = 0; i < RAD; ++i) {
+                    x[i] = v[a][e + i * NB];
+                    if (P > 0 && i > 0) x[i] = cmul(x[i], INV ? cconj(w[i]) : w[i]);
+                }
+                if constexpr (RAD == 2) {
+                    y[0] = cadd(x[0], x[1]);
+                    y[1] = csub(x[0], x[1]);
+                } else if constexpr (RAD == 4) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) y[i] = x[i];
+                    dft4(y, INV);
+                } else if constexpr (RAD == 8) {
+                    dft8(x, y, INV);
+                } else {
+                    dft16(x, y, INV);
+                }
+#pragma unroll
+                for (int i = 0; i < RAD; ++i) v[a][e + i * NB] = y[i];
+            }
+        }
+    }
+
+    // the outputs of pass P through LDS to the inputs of pass P + 1; s: A
+    // values per element, the row's own part of LDS
+    template <int P, int A> __device__ __forceinline__ static void exchange(C (&v)[A][E], C *s, int t) {
+        constexpr int LR = logr(P), RAD = 1 << LR, NB = E / RAD, NS = 1 << (LE * P);
+#pragma unroll
+        for (int e = 0; e < NB; ++e) {
+            const int j = t + e * T, k = j & (NS - 1);
+            const int base = lpe<E>(((j - k) << LR) + k);
+#pragma unroll
+            for (int i = 0; i < RAD; ++i) {
+                // NS = 1: the E outputs of a butterfly fill one padded group
+                C *q = s + A * (base + i * (NS == 1 ? 1 : lpe<E>(NS)));
+#pragma unroll
+                for (int a = 0; a < A; ++a) q[a] = v[a][e + i * NB];
+            }
+        }
+        row_sync<WAVE>();
+        gather<A>(v, s, t);
+    }
+    // the thread's points t + T u from LDS
+    template <int A> __device__ __forceinline__ static void gather(C (&v)[A][E], const C *s, int t) {
+#pragma unroll
+        for (int u = 0; u < E; ++u) {
+            const C *q = s + A * (T % E == 0 ? lpe<E>(t) + u * lpe<E>(T) : lpe<E>(t + T * u));
+#pragma unroll
+            for (int a = 0; a < A; ++a) v[a][u] = q[a];
+        }
+    }
+
+    // whole transform of the points in v; every thread of the block calls it.
+    // s holds no values still to be read by another thread (FRESH), or may
+    // (the previous use ends with reads): then a sync comes first.
+    template <int A, bool INV, bool FRESH, int P = 0>
+    __device__ __forceinline__ void run(C (&v)[A][E], C *s, int t) const {
+        pass<P, A, INV>(v);
+        if constexpr (P + 1 < NP) {
+            if (P > 0 || !FRESH) row_sync<WAVE>();
+            exchange<P, A>(v, s, t);
+            run<A, INV, FRESH, P + 1>(v, s, t);
+        }
+    }
+};
+
+// LDS elements from row to row of a block with `rows` rows of n points
+// (padded after every E), such that the accesses across rows (row index
+// fastest) spread over the banks: `per` elements fill all banks once
+__host__ __device__ constexpr int row_stride(int n, int E, int rows, int per) {
+    return (n + n / E + per - 1) / per * per + (rows < per ? per / rows : 1);
+}
+
+// ------------------------------------------------------------------ rows of any length
+// LDS layout of these rows: element i sits at lp(i), one padding element
+// after every 8; a row of n elements takes n + n/8 + 1 (odd) elements.
 __device__ __forceinline__ int lp(int i) { return i + (i >> 3); }
 __host__ __device__ __forceinline__ int lds_row(int n) { return n + n / 8 + 1; }
-
-// One Stockham pass of radix RAD (2, 4 or 8) over nrows rows of length
-// n = 2^logn held in LDS (row stride `stride`, layout lp), in place: every thread reads
-// its butterflies' inputs (and, for small register footprints, their
-// twiddles: powers 1, 2, 4 from the FP64-built table, 3, 5, 6, 7 as
-// products) before the barrier and writes the outputs after it.  Twiddle of input t of butterfly j: tw[(t k) << twsh],
-// k = j mod Ns (conjugated for the inverse transform).
-// Output index ((j - k) << LR) + k + t Ns with Ns a power of 8 maps to
-// lp(base) + t (Ns + Ns/8); input index j + t nb to lp(j) + t (nb + nb/8)
-// when nb is a multiple of 8 (SMALL: nb < 8, mapped per element).
-template <typename R, int EPT, int RAD, bool SMALL>
-__device__ __forceinline__ void fft_pass(typename V2<R>::T *buf, int logn, int nrows, int stride, int logNs,
-                                         const typename V2<R>::T *__restrict__ tw, int logZ, bool inv) {
-    using C = typename V2<R>::T;
-    constexpr int LR = RAD == 16 ? 4 : (RAD == 8 ? 3 : (RAD == 4 ? 2 : 1));
-    // butterflies per thread (radix 16 at 8 elements per thread: one, on half
-    // of the threads)
-    constexpr int NB = EPT >= RAD ? EPT / RAD : 1;
-    constexpr bool PRE = sizeof(R) == 4 && NB * (RAD - 1) <= 16;  // twiddles fetched before the barrier
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int lognb = logn - LR, nb = 1 << lognb;
-    const int tot = nb * nrows;
-    const int Ns = 1 << logNs;
-    const int twsh = logZ - (logNs + LR);
-    const int nbp = nb + (nb >> 3), Nsp = Ns + (Ns >> 3);
-    C v[NB][RAD];
-    C w[PRE ? NB : 1][RAD - 1];
-    // twiddles of butterfly k: tw^1, tw^2, tw^4 (and tw^8) from the table,
-    // the other powers as products (one to three roundings deeper; 3 loads
-    // instead of 7 for radix 8, 4 instead of 15 for radix 16).  Every tiling
-    // forms them the same way -- before the barrier when the registers allow
-    // (PRE), else after it -- so the transform's rounding does not depend on
-    // the elements per thread.
-    auto twiddles = [&](int k, C *ww) {
-        ww[0] = tw[k << twsh];
-        if (RAD >= 4) {
-            ww[1] = tw[(2 * k) << twsh];
-            ww[2] = cmul(ww[0], ww[1]);
-        }
-        if (RAD >= 8) {
-            ww[3] = tw[(4 * k) << twsh];
-            ww[4] = cmul(ww[3], ww[0]);
-            ww[5] = cmul(ww[3], ww[1]);
-            ww[6] = cmul(ww[3], ww[2]);
-        }
-        if (RAD == 16) {
-            ww[7] = tw[(8 * k) << twsh];
-#pragma unroll
-            for (int t = 8; t < 15; ++t) ww[t] = cmul(ww[7], ww[t - 8]);
-        }
-    };
-#pragma unroll
-    for (int e = 0; e < NB; ++e) {
-        const int b = tid + e * nt;
-        if (b < tot) {
-            const int row = b >> lognb, j = b & (nb - 1);
-            const C *p = buf + row * stride;
-            if (SMALL) {
-#pragma unroll
-                for (int t = 0; t < RAD; ++t) v[e][t] = p[lp(j + t * nb)];
-            } else {
-                p += lp(j);
-#pragma unroll
-                for (int t = 0; t < RAD; ++t) v[e][t] = p[t * nbp];
-            }
-            if (PRE) twiddles(j & (Ns - 1), w[PRE ? e : 0]);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < NB; ++e) {
-        const int b = tid + e * nt;
-        if (b < tot) {
-            const int row = b >> lognb, j = b & (nb - 1);
-            const int k = j & (Ns - 1);
-            C wl[RAD - 1];
-            if (!PRE) twiddles(k, wl);
-#pragma unroll
-            for (int t = 1; t < RAD; ++t) {
-                C ww = PRE ? w[PRE ? e : 0][t - 1] : wl[t - 1];
-                if (inv) ww.y = -ww.y;
-                v[e][t] = cmul(v[e][t], ww);
-            }
-            C y[RAD];
-            if (RAD == 2) {
-                y[0] = cadd(v[e][0], v[e][1]);
-                y[1] = csub(v[e][0], v[e][1]);
-            } else if (RAD == 4) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) y[t] = v[e][t];
-                dft4(y, inv);
-            } else if (RAD == 8) {
-                dft8(v[e], y, inv);
-            } else {
-                dft16(v[e], y, inv);
-            }
-            if (RAD == 16 && Ns < 8) {
-                // the first radix-16 pass (Ns = 1): outputs 16 j + t straddle a
-                // padding element, so each takes its own padded index
-                C *q = buf + row * stride;
-                const int base = (j - k) << LR;
-#pragma unroll
-                for (int t = 0; t < RAD; ++t) q[lp(base + k + t * Ns)] = y[t];
-            } else {
-                C *q = buf + row * stride + lp(((j - k) << LR) + k);
-#pragma unroll
-                for (int t = 0; t < RAD; ++t) q[t * Nsp] = y[t];
-            }
-        }
-    }
-    __syncthreads();
-}
 
 // radix-3 butterfly, y = DFT3(v): W = exp(-+2 pi i / 3) = -1/2 -+ i sqrt(3)/2
 template <typename C>
@@ -237,9 +284,8 @@ __device__ __forceinline__ void dftp(const C *v, C *y, const C *__restrict__ tw,
 }
 
 // One Stockham pass of radix RAD (2, 3, 4, 5, 7 or 8) over rows of any
-// length n divisible by RAD (the meshes whose size is not a power of two).
-// The same butterflies as fft_pass, with per-element LDS addresses (lp of
-// every index), exact integer division for the butterfly and row indices,
+// length n divisible by RAD (the meshes whose size is not a power of two),
+// with per-element LDS addresses (lp of every index), exact integer division for the butterfly and row indices,
 // and every twiddle power loaded from the table: tw[t k Z / (Ns RAD)].
 // Inputs are read before the barrier, outputs written after it (in place).
 template <typename R, int EPT, int RAD>
@@ -301,8 +347,7 @@ __device__ __forceinline__ void fft_pass_g(typename V2<R>::T *buf, int n, int nr
 
 // Transform of rows of length n = 2^p 3^c 5^d 7^f: radix-8 passes over the
 // factor 2^p, one radix-4 or radix-2 pass for its remaining bits, then one
-// radix-3, -5 or -7 pass per odd factor.  A power-of-two n takes fft_pass
-// (below).
+// radix-3, -5 or -7 pass per odd factor.
 template <typename R, int EPT>
 __device__ __forceinline__ void lds_fft_g(typename V2<R>::T *buf, int n, int nrows, int stride,
                                           const typename V2<R>::T *__restrict__ tw, int Z, bool inv) {
@@ -343,90 +388,6 @@ __device__ __forceinline__ void lds_fft_g(typename V2<R>::T *buf, int n, int nro
     for (; c7 > 0; --c7) {
         fft_pass_g<R, EPT, 7>(buf, n, nrows, stride, Ns, tw, Z, inv);
         Ns *= 7;
-    }
-}
-
-// rows of length n: the power-of-two passes below, or lds_fft_g when n has an
-// odd factor (tw holds exp(-2 pi i k / Z), k < Z; n divides Z).  R16: the
-// kernel's power-of-two rows take radix-16 passes (FP32); a kernel's choice
-// does not depend on its elements per thread, so neither does its rounding.
-template <typename R, int EPT, bool R16 = false, bool R16T = false>
-__device__ __forceinline__ void lds_fft_pow2(typename V2<R>::T *buf, int logn, int nrows, int stride,
-                                             const typename V2<R>::T *__restrict__ tw, int logZ, bool inv);
-template <typename R, int EPT>
-__device__ __forceinline__ void lds_fft(typename V2<R>::T *buf, int n, int nrows, int stride,
-                                        const typename V2<R>::T *__restrict__ tw, int Z, bool inv) {
-    if ((n & (n - 1)) == 0 && (Z & (Z - 1)) == 0)
-        lds_fft_pow2<R, EPT>(buf, __ffs(n) - 1, nrows, stride, tw, __ffs(Z) - 1, inv);
-    else
-        lds_fft_g<R, EPT>(buf, n, nrows, stride, tw, Z, inv);
-}
-// the same with the mesh kind known at compile time (P2: n and Z powers of two)
-template <typename R, int EPT, bool P2, bool R16 = false, bool R16T = false>
-__device__ __forceinline__ void lds_fft_t(typename V2<R>::T *buf, int n, int nrows, int stride,
-                                          const typename V2<R>::T *__restrict__ tw, int Z, bool inv) {
-    if (P2)
-        lds_fft_pow2<R, EPT, R16, R16T>(buf, __ffs(n) - 1, nrows, stride, tw, __ffs(Z) - 1, inv);
-    else
-        lds_fft_g<R, EPT>(buf, n, nrows, stride, tw, Z, inv);
-}
-
-// radix-8 passes (radix-16 passes with R16), then one pass of a smaller radix
-// for the remaining bits
-template <typename R, int EPT, bool R16, bool R16T>
-__device__ __forceinline__ void lds_fft_pow2(typename V2<R>::T *buf, int logn, int nrows, int stride,
-                                             const typename V2<R>::T *__restrict__ tw, int logZ, bool inv) {
-    int logNs = 0;
-    if constexpr (R16T && sizeof(R) == 4) {
-        // radix-8 passes, with the last 4 bits (when radix 8 would leave one
-        // bit for a radix-2 pass) in one radix-16 pass: 1024 points in passes
-        // of 8, 8 and 16
-        if (logn >= 7 && logn % 3 == 1) {
-            while (logn - logNs > 4) {
-                fft_pass<R, EPT, 8, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-                logNs += 3;
-            }
-            fft_pass<R, EPT, 16, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-            return;
-        }
-    }
-    if constexpr (R16 && sizeof(R) == 4) {
-        // FP32 rows of at least 128: radix-16 passes, then one pass of radix
-        // 8, 4 or 2 for the remaining bits (2048 points in 3 passes instead
-        // of 4)
-        if (logn >= 7) {
-            while (logn - logNs >= 4) {
-                fft_pass<R, EPT, 16, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-                logNs += 4;
-            }
-            const int rem = logn - logNs;
-            if (rem == 3)
-                fft_pass<R, EPT, 8, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-            else if (rem == 2)
-                fft_pass<R, EPT, 4, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-            else if (rem == 1)
-                fft_pass<R, EPT, 2, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-            return;
-        }
-    }
-    const bool small8 = logn - 3 < 3;  // nb = n/8 below 8
-    while (logn - logNs >= 3) {
-        if (small8)
-            fft_pass<R, EPT, 8, true>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-        else
-            fft_pass<R, EPT, 8, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-        logNs += 3;
-    }
-    if (logn - logNs == 2) {
-        if (logn - 2 < 3)
-            fft_pass<R, EPT, 4, true>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-        else
-            fft_pass<R, EPT, 4, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-    } else if (logn - logNs == 1) {
-        if (logn - 1 < 3)
-            fft_pass<R, EPT, 2, true>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
-        else
-            fft_pass<R, EPT, 2, false>(buf, logn, nrows, stride, logNs, tw, logZ, inv);
     }
 }
 

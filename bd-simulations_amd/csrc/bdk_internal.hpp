@@ -167,10 +167,13 @@ struct BatchPlan {
     int2 *map[BS_COUNT] = {};        // device maps
     int nblk[BS_COUNT] = {};
     int nblk2[BS_COUNT] = {};        // leading entries of members with a power-of-two mesh
-    int nblk16[BS_COUNT] = {};       // of those, the leading entries whose column and c2r passes are radix 16
+    int nblk16[BS_COUNT] = {};       // of those, the leading entries with 16 mesh points per FFT thread
     BatchTuning tune;
     int ept[3] = {8, 8, 8};          // the FFT elements per thread in use (at least the members' minimum)
-    size_t dep_lds = 0, l1 = 0, lc = 0, l2 = 0;
+    size_t dep_lds = 0;
+    // FFT launches by kind of mesh (16 points per thread, other powers of two, other sizes) and pass
+    size_t fft_lds[3][3] = {};
+    int fft_threads[3][3] = {};
 };
 
 }  // namespace bdkx
@@ -269,6 +272,9 @@ hipError_t build_tables(bdk_t *h);                // spectral tables in device m
 
 // batches (a batch is a view over member handles, each with its own buffers)
 int batch_min_ept(int stage, int zmax);
+void fft_member(RepDev &r, int Z, const int ept[3], BatchPlan &bp);
+void batch_fft_stage(const BatchPlan &bp, int stage, hipStream_t st);
+hipError_t fft_set_attributes();
 hipError_t batch_build(const std::vector<bdk_t *> &mem, const BatchTuning &tune, BatchPlan &bp,
                        std::vector<RepDev> &reps, std::vector<int2> maps[BS_COUNT]);
 hipError_t batch_stage(const BatchPlan &bp, int stage, hipStream_t st);

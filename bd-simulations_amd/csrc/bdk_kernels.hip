@@ -20,9 +20,7 @@
 //   k_col       column FFT, Green's function x gradient (dm:1210-1216), two
 //               inverse column FFTs (Fx, Fy);
 //   k_c2r_rows  inverse row FFT of (Fx + i Fy) -> real Fx, Fy mesh
-//               (Stockham passes in LDS: radix 8, radix 16 for the column
-//               and c2r passes of FP32 meshes of 1024 points and more, whose
-//               r2c rows end in one radix-16 pass instead of radix 8 and 2).
+//               (the three passes: bdk_fft.hip).
 // Every force, gather and update kernel runs over list positions q and
 // reads the list-ordered state; k_update writes the new state to slot q.
 // The slots are therefore re-sorted by cell every step: consecutive threads
@@ -34,9 +32,6 @@
 // compiled without FP contraction so it rounds like the reference's x86-64
 // build; cell indices are therefore bit-exact.
 #pragma clang fp contract(off)
-
-#include <cstdio>
-#include <cstdlib>
 
 #include "bdk_device.hpp"
 #include "bdk_fft.hpp"
@@ -647,25 +642,6 @@ __global__ __launch_bounds__(DP_THREADS) void k_deposit(Geo g, DevBufs d, DepArg
     deposit_body<R, SCHEME, P2>(g, d, a, blockIdx.x + blockIdx.y * gridDim.x, gridDim.x);
 }
 
-// End of a step: step counter + 1, and the per-step scalars of the next
-// update re-armed (dt minimum and the 64 slots of dt candidates, excursion
-// slot, displacement bound).  Run by threads 0..63 of one block of the
-// step's last mesh pass (k_c2r_rows), which follows every reader of these
-// scalars in the step.
-__device__ __forceinline__ void step_end_body(const Geo &g, const DevBufs &d) {
-    const int t = threadIdx.x;
-    if (t < 64) {
-        d.exo[t * 16] = 0ull;
-        d.dts[t * 16] = ~0ull;
-    }
-    if (t == 0) {
-        const unsigned long long s = d.sc->step;
-        d.sc->dt_bits = bitsd(g.dt_max);
-        d.sc->exc_bits[s & 1] = 0ull;  // filled by the update of step s + 1
-        d.sc->step = s + 1;
-    }
-}
-
 // per-step scalar re-arm when no deposit runs (ideal-gas runs), at the start
 // of the step; one wave
 __global__ void k_rearm(Geo g, DevBufs d) {
@@ -675,199 +651,6 @@ __global__ void k_rearm(Geo g, DevBufs d) {
         d.sc->dt_bits = bitsd(g.dt_max);
         d.sc->exc_bits[(step + 1) & 1] = 0ull;
     }
-}
-
-// Row r2c: rows k0..k0+RB-1 of the real mesh -> half spectrum X[m], m<Z/2,
-// with X[0] packing (DC, Nyquist) (both real), written transposed:
-// ht[m*Z + k].  Length-Z/2 complex FFT of (x[2n], x[2n+1]) + split; with
-// R16 (FP32) a row length of 2^(3m+1) ends in one radix-16 pass.
-template <typename R, int EPT, bool P2, bool R16 = false>
-__device__ __forceinline__ void r2c_rows_body(const R *__restrict__ rho, typename V2<R>::T *__restrict__ ht,
-                                              const typename V2<R>::T *__restrict__ tw, int Z, int RB,
-                                              int stride, int blk) {
-    using C = typename V2<R>::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int n = Z >> 1;
-    const DvT<P2> dn(n), drb(RB);  // RB divides Z: a power of two with Z
-    const int k0 = blk * RB;
-    for (int idx = tid; idx < RB * n; idx += nt) {
-        const int row = dn.q(idx), m = dn.r(idx);
-        s[row * stride + lp(m)] = ((const C *)(rho + (size_t)(k0 + row) * Z))[m];
-    }
-    __syncthreads();
-    lds_fft_t<R, EPT, P2, false, R16>(s, n, RB, stride, tw, Z, false);
-    const int half = n >> 1;
-    for (int idx = tid; idx < RB * (half + 1); idx += nt) {
-        const int row = idx / (half + 1), m = idx - row * (half + 1);
-        C *p = s + row * stride;
-        if (m == 0) {
-            C z = p[0];
-            p[0] = cm<C>(z.x + z.y, z.x - z.y);
-        } else {
-            C a = p[lp(m)], bc = cconj(p[lp(n - m)]);
-            C E = cscale(cadd(a, bc), (R)0.5);
-            C O = cmul_mi(cscale(csub(a, bc), (R)0.5));
-            C WO = cmul(tw[m], O);
-            p[lp(m)] = cadd(E, WO);
-            if (m != n - m) p[lp(n - m)] = cconj(csub(E, WO));
-        }
-    }
-    __syncthreads();
-    for (int idx = tid; idx < RB * n; idx += nt) {
-        const int m = drb.q(idx), row = drb.r(idx);
-        ht[(size_t)m * Z + k0 + row] = s[row * stride + lp(m)];
-    }
-}
-
-template <typename R, int EPT, bool P2, bool R16 = false>
-__global__ __launch_bounds__(FFT_THREADS) void k_r2c_rows(const R *__restrict__ rho, typename V2<R>::T *__restrict__ ht,
-                                                          const typename V2<R>::T *__restrict__ tw, int Z,
-                                                          int RB, int stride, int remap) {
-    r2c_rows_body<R, EPT, P2, R16>(rho, ht, tw, Z, RB, stride, xcd_block(remap));
-}
-
-// spectral factors of one (j, m') pair: gx = sq[j] G / Z / Z, gy = sq[m'] G / Z / Z,
-// G = 1/((lap[j] + lap[m']) + 1/lambda^2) (dm:585-593, dm:1384-1394)
-template <typename R>
-__device__ __forceinline__ void symbols(int j, int mm, const Geo &g, const R *sq, const R *lap, R &gx, R &gy) {
-    R G;
-    if (j == 0 && mm == 0 && g.zero_mode_g)
-        G = (R)0.0;
-    else if (sizeof(R) == 4)  // FP32: the hardware reciprocal (1 ulp) instead of a correctly rounded division
-        G = (R)__builtin_amdgcn_rcpf((float)((lap[j] + lap[mm]) + (R)g.lam2inv));
-    else
-        G = (R)1.0 / ((lap[j] + lap[mm]) + (R)g.lam2inv);
-    // x / Z / Z == x * 2^(-2 log2 Z) exactly (Z is a power of two)
-    const R izz = (R)1.0 / ((R)g.Z * (R)g.Z);
-    gx = sq[j] * G * izz;
-    gy = sq[mm] * G * izz;
-}
-
-// Column pass: rows m0..m0+RC-1 of ht (length Z along x), forward FFT,
-// multiply by i*gx and i*gy, inverse FFT of both, out gt[m*Z+k] = (Fx, Fy).
-template <typename R, int EPT, bool P2, bool R16 = false>
-__device__ __forceinline__ void col_body(const typename V2<R>::T *__restrict__ ht, typename V4<R>::T *__restrict__ gt,
-                                         const typename V2<R>::T *__restrict__ tw, const R *__restrict__ sq,
-                                         const R *__restrict__ lap, const Geo &g, int RC, int stride, int blk) {
-    using C = typename V2<R>::T;
-    using C4 = typename V4<R>::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    C *sB = s + RC * stride;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int Z = g.Z, Zh = Z >> 1;
-    const DvT<P2> dz(Z);
-    const int m0 = blk * RC;
-    for (int idx = tid; idx < RC * Z; idx += nt) {
-        const int row = dz.q(idx), k = dz.r(idx);
-        s[row * stride + lp(k)] = ht[(size_t)(m0 + row) * Z + k];
-    }
-    __syncthreads();
-    lds_fft_t<R, EPT, P2, R16>(s, Z, RC, stride, tw, Z, false);
-    for (int idx = tid; idx < RC * Z; idx += nt) {
-        const int row = dz.q(idx), j = dz.r(idx);
-        const int m = m0 + row;
-        if (m == 0) {
-            // packed (DC, Nyquist) column: pairs (j, Z-j) by one thread
-            if (j > Zh) continue;
-            const int jn = P2 ? ((Z - j) & (Z - 1)) : (j == 0 ? 0 : Z - j);
-            C P = s[lp(j)], Q = s[lp(jn)];
-            C Sdc = cscale(cadd(P, cconj(Q)), (R)0.5);
-            C Sny = cmul_mi(cscale(csub(P, cconj(Q)), (R)0.5));
-            R gx0, gy0, gxN, gyN, hx0, hy0, hxN, hyN;
-            symbols<R>(j, 0, g, sq, lap, gx0, gy0);
-            symbols<R>(j, Zh, g, sq, lap, gxN, gyN);
-            symbols<R>(jn, 0, g, sq, lap, hx0, hy0);
-            symbols<R>(jn, Zh, g, sq, lap, hxN, hyN);
-            // packed = i g(.,0) S_dc + i (i g(.,Z/2) S_ny)
-            C fxj = cadd(cmul_i(cscale(Sdc, gx0)), cmul_i(cmul_i(cscale(Sny, gxN))));
-            C fyj = cadd(cmul_i(cscale(Sdc, gy0)), cmul_i(cmul_i(cscale(Sny, gyN))));
-            C fxn = cadd(cmul_i(cscale(cconj(Sdc), hx0)), cmul_i(cmul_i(cscale(cconj(Sny), hxN))));
-            C fyn = cadd(cmul_i(cscale(cconj(Sdc), hy0)), cmul_i(cmul_i(cscale(cconj(Sny), hyN))));
-            s[lp(j)] = fxj;
-            sB[lp(j)] = fyj;
-            if (jn != j) {
-                s[lp(jn)] = fxn;
-                sB[lp(jn)] = fyn;
-            }
-        } else {
-            R gx, gy;
-            symbols<R>(j, m, g, sq, lap, gx, gy);
-            const int o = row * stride + lp(j);
-            C S = s[o];
-            s[o] = cm<C>(-gx * S.y, gx * S.x);
-            sB[o] = cm<C>(-gy * S.y, gy * S.x);
-        }
-    }
-    __syncthreads();
-    lds_fft_t<R, EPT, P2, R16>(s, Z, 2 * RC, stride, tw, Z, true);
-    for (int idx = tid; idx < RC * Z; idx += nt) {
-        const int row = dz.q(idx), k = dz.r(idx);
-        const int so = row * stride + lp(k);
-        C a = s[so], b = sB[so];
-        C4 o;
-        o.x = a.x;
-        o.y = a.y;
-        o.z = b.x;
-        o.w = b.y;
-        gt[(size_t)(m0 + row) * Z + k] = o;
-    }
-}
-
-template <typename R, int EPT, bool P2, bool R16 = false>
-__global__ __launch_bounds__(FFT_THREADS) void k_col(const typename V2<R>::T *__restrict__ ht,
-                                                     typename V4<R>::T *__restrict__ gt,
-                                                     const typename V2<R>::T *__restrict__ tw, const R *__restrict__ sq,
-                                                     const R *__restrict__ lap, Geo g, int RC, int stride) {
-    col_body<R, EPT, P2, R16>(ht, gt, tw, sq, lap, g, RC, stride, blockIdx.x);
-}
-
-// Row c2r of the two real signals Fx, Fy: rows k0..k0+RB2-1, spectrum
-// C[m] = X[m] + i Y[m] completed by Hermitian symmetry, inverse FFT of
-// length Z, out fmesh[k*Z + l] = (Re, Im) = (Fx, Fy).
-template <typename R, int EPT, bool P2, bool R16 = false>
-__device__ __forceinline__ void c2r_rows_body(const typename V4<R>::T *__restrict__ gt,
-                                              typename V2<R>::T *__restrict__ fm,
-                                              const typename V2<R>::T *__restrict__ tw, int Z, int RB2,
-                                              int stride, int blk) {
-    using C = typename V2<R>::T;
-    using C4 = typename V4<R>::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int Zh = Z >> 1;
-    const DvT<P2> dz(Z), drb(RB2);  // RB2 divides Z: a power of two with Z
-    const int k0 = blk * RB2;
-    for (int idx = tid; idx < RB2 * Zh; idx += nt) {
-        const int m = drb.q(idx), row = drb.r(idx);
-        C4 v = gt[(size_t)m * Z + k0 + row];
-        C *p = s + row * stride;
-        if (m == 0) {
-            p[0] = cm<C>(v.x, v.z);
-            p[lp(Zh)] = cm<C>(v.y, v.w);
-        } else {
-            p[lp(m)] = cm<C>(v.x - v.w, v.y + v.z);
-            p[lp(Z - m)] = cm<C>(v.x + v.w, -v.y + v.z);
-        }
-    }
-    __syncthreads();
-    lds_fft_t<R, EPT, P2, R16>(s, Z, RB2, stride, tw, Z, true);
-    for (int idx = tid; idx < RB2 * Z; idx += nt) {
-        const int row = dz.q(idx), l = dz.r(idx);
-        fm[(size_t)(k0 + row) * Z + l] = s[row * stride + lp(l)];
-    }
-}
-
-template <typename R, int EPT, bool P2, bool R16 = false>
-__global__ __launch_bounds__(FFT_THREADS) void k_c2r_rows(const typename V4<R>::T *__restrict__ gt,
-                                                          typename V2<R>::T *__restrict__ fm,
-                                                          const typename V2<R>::T *__restrict__ tw, int Z,
-                                                          int RB2, int stride, int remap, Geo g, DevBufs d,
-                                                          int end_step) {
-    if (end_step && blockIdx.x == 0) step_end_body(g, d);
-    c2r_rows_body<R, EPT, P2, R16>(gt, fm, tw, Z, RB2, stride, xcd_block(remap));
 }
 
 // ------------------------------------------------------------------ gather, update
@@ -1512,26 +1295,6 @@ __global__ void k_sort_cells(Geo g, DevBufs d, int moved_ranks) { sort_cells_bod
 // single-simulation kernel on that member's geometry and buffers, so every
 // member's results are bit-identical alone and in a batch.
 
-// Every batched kernel walks its stage's block map: one map entry per block,
-// or in the persistent form (a grid smaller than the map) each block takes
-// the entries blockIdx.x, blockIdx.x + gridDim.x, ...  Kernels whose bodies
-// use LDS end every entry with a barrier, so the next entry may refill it.
-// A member's results do not depend on the grid or on the WCA block size
-// (per-particle sums, integer deposit sums, order-free min/max reductions).
-// P (persistent) selects the form at compile time: without it a kernel
-// handles exactly its own entry (no loop, so the code and its register use
-// are those of a plain one-entry kernel).
-template <bool P, bool SYNC, typename F> __device__ __forceinline__ void for_entries(int nmap, F &&f) {
-    if (!P) {
-        f((int)blockIdx.x);
-        return;
-    }
-    for (int e = blockIdx.x; e < nmap; e += gridDim.x) {
-        f(e);
-        if (SYNC) __syncthreads();
-    }
-}
-
 template <typename R, bool P>
 __global__ __launch_bounds__(512) void kb_wca(const RepDev *m, const int2 *map, int nmap) {
     constexpr int S = std::is_same<R, float>::value ? WCA_STAGE + 1 : 1;  // FP64 members read the list directly
@@ -1567,42 +1330,6 @@ __global__ __launch_bounds__(DP_THREADS) void kb_deposit(const RepDev *m, const 
         case 1: deposit_body<R, 1, P2>(r.g, r.d, a, t.y, r.dep_tx); break;
         default: deposit_body<R, 2, P2>(r.g, r.d, a, t.y, r.dep_tx); break;
         }
-    });
-}
-
-template <typename R, int EPT, bool P, bool P2, bool R16 = false>
-__global__ __launch_bounds__(FFT_THREADS) void kb_r2c(const RepDev *m, const int2 *map, int nmap) {
-    using C = typename V2<R>::T;
-    for_entries<P, true>(nmap, [&](int e_) {
-        const int2 t = map[e_];
-        const RepDev &r = m[t.x];
-        r2c_rows_body<R, EPT, P2, R16>((const R *)r.d.rho, (C *)r.d.ht, (const C *)r.d.tw, r.g.Z, r.rb, r.sR1, t.y);
-    });
-}
-
-template <typename R, int EPT, bool P, bool P2, bool R16 = false>
-__global__ __launch_bounds__(FFT_THREADS) void kb_col(const RepDev *m, const int2 *map, int nmap) {
-    using C = typename V2<R>::T;
-    using C4 = typename V4<R>::T;
-    for_entries<P, true>(nmap, [&](int e_) {
-        const int2 t = map[e_];
-        const RepDev &r = m[t.x];
-        const R *sq = std::is_same<R, float>::value ? (const R *)r.d.sqf : (const R *)r.d.sq;
-        const R *lap = std::is_same<R, float>::value ? (const R *)r.d.lapf : (const R *)r.d.lap;
-        col_body<R, EPT, P2, R16>((const C *)r.d.ht, (C4 *)r.d.gt, (const C *)r.d.tw, sq, lap, r.g, r.rc, r.sC, t.y);
-    });
-}
-
-template <typename R, int EPT, bool P, bool P2, bool R16 = false>
-__global__ __launch_bounds__(FFT_THREADS) void kb_c2r(const RepDev *m, const int2 *map, int nmap, int end_step) {
-    using C = typename V2<R>::T;
-    using C4 = typename V4<R>::T;
-    for_entries<P, true>(nmap, [&](int e_) {
-        const int2 t = map[e_];
-        const RepDev &r = m[t.x];
-        if (end_step && t.y == 0) step_end_body(r.g, r.d);
-        c2r_rows_body<R, EPT, P2, R16>((const C4 *)r.d.gt, (C *)r.d.fmesh, (const C *)r.d.tw, r.g.Z, r.rb2,
-                                       r.sR2, t.y);
     });
 }
 
@@ -1678,127 +1405,8 @@ __global__ __launch_bounds__(256) void kb_sort_cells(const RepDev *m, const int2
 }
 
 // ------------------------------------------------------------------ launchers
-static inline unsigned nblk(int n, int b) { return (unsigned)((n + b - 1) / b); }
-
-// Elements per thread (EPT) of the three FFT kernels; a block of
-// FFT_THREADS threads holds EPT * FFT_THREADS complex values.  The defaults
-// (8, 16, 16) were the fastest of {8, 16, 32} per kernel at Z = 2048 (FP32):
-// 2 rows per r2c block (1024 blocks), one column per k_col block (1024),
-// 2 rows per c2r block (1024).  Each EPT is raised to the smallest value
-// whose block still holds one transform.  BDK_FFT_EPT="a,b,c" (8, 16 or 32)
-// overrides them.
-struct FftCfg {
-    int e1, e2, e3;      // EPT of r2c rows, columns, c2r rows
-    int RB, RC, RB2;     // rows per block
-    int sR1, sC, sR2;    // LDS row strides (padded)
-    size_t l1, lc, l2;   // LDS bytes
-};
-
-static const int *fft_ept_default() {
-    static int v[3] = {0, 0, 0};
-    if (!v[0]) {
-        int a = 8, b = 16, c = 16;
-        if (const char *e = getenv("BDK_FFT_EPT")) {
-            int x, y, z;
-            if (sscanf(e, "%d,%d,%d", &x, &y, &z) == 3) {
-                auto ok = [](int t) { return t == 8 || t == 16 || t == 32; };
-                if (ok(x) && ok(y) && ok(z)) a = x, b = y, c = z;
-            }
-        }
-        v[1] = b;
-        v[2] = c;
-        v[0] = a;
-    }
-    return v;
-}
-
-// the largest divisor of m not above cap (at least 1)
-static int div_at_most(int m, int cap) {
-    cap = std::max(1, std::min(m, cap));
-    while (m % cap) --cap;
-    return cap;
-}
-
-// FFT rows per block for elements-per-thread (e1, e2, e3) at mesh size Z:
-// as many rows as the block's elements hold, a divisor of the row count
-// (for a power-of-two Z the element count itself)
-static void fft_rows(int Z, const int e[3], int &rb, int &rc, int &rb2) {
-    rb = div_at_most(Z, e[0] * FFT_THREADS / (Z / 2));
-    rc = div_at_most(Z / 2, e[1] * FFT_THREADS / (2 * Z));
-    rb2 = div_at_most(Z, e[2] * FFT_THREADS / Z);
-}
-
-template <typename R> static FftCfg fft_cfg(int Z) {
-    using C = typename V2<R>::T;
-    const int *w = fft_ept_default();
-    FftCfg c;
-    c.e1 = ept_for(w[0], Z / 2);
-    c.e2 = ept_for(w[1], 2 * Z);
-    c.e3 = ept_for(w[2], Z);
-    const int e[3] = {c.e1, c.e2, c.e3};
-    fft_rows(Z, e, c.RB, c.RC, c.RB2);
-    c.sR1 = lds_row(Z / 2);
-    c.sC = lds_row(Z);
-    c.sR2 = lds_row(Z);
-    c.l1 = (size_t)c.RB * c.sR1 * sizeof(C);
-    c.lc = (size_t)2 * c.RC * c.sC * sizeof(C);
-    c.l2 = (size_t)c.RB2 * c.sR2 * sizeof(C);
-    return c;
-}
-
 hipError_t set_kernel_attributes() {
-    const int big = 160 * 1024;
-    hipError_t e = hipSuccess;
-#define BDK_ATTR(K)                                                                            \
-    if (e == hipSuccess) e = hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-#define BDK_ATTR_E(E, Q)                \
-    BDK_ATTR((k_r2c_rows<float, E, Q>))  \
-    BDK_ATTR((k_r2c_rows<double, E, Q>)) \
-    BDK_ATTR((k_col<float, E, Q>))       \
-    BDK_ATTR((k_col<double, E, Q>))      \
-    BDK_ATTR((k_c2r_rows<float, E, Q>))  \
-    BDK_ATTR((k_c2r_rows<double, E, Q>))
-    BDK_ATTR_E(8, true)
-    BDK_ATTR_E(16, true)
-    BDK_ATTR_E(32, true)
-    BDK_ATTR_E(8, false)
-    BDK_ATTR_E(16, false)
-    BDK_ATTR_E(32, false)
-#undef BDK_ATTR_E
-    // the radix-16 column and c2r passes (FP32, power-of-two meshes)
-#define BDK_ATTR_16(E)                         \
-    BDK_ATTR((k_r2c_rows<float, E, true, true>)) \
-    BDK_ATTR((kb_r2c<float, E, false, true, true>)) \
-    BDK_ATTR((kb_r2c<float, E, true, true, true>))  \
-    BDK_ATTR((k_col<float, E, true, true>))      \
-    BDK_ATTR((k_c2r_rows<float, E, true, true>)) \
-    BDK_ATTR((kb_col<float, E, false, true, true>)) \
-    BDK_ATTR((kb_col<float, E, true, true, true>))  \
-    BDK_ATTR((kb_c2r<float, E, false, true, true>)) \
-    BDK_ATTR((kb_c2r<float, E, true, true, true>))
-    BDK_ATTR_16(8)
-    BDK_ATTR_16(16)
-    BDK_ATTR_16(32)
-#undef BDK_ATTR_16
-#define BDK_ATTR_B(E, P, Q)            \
-    BDK_ATTR((kb_r2c<float, E, P, Q>))  \
-    BDK_ATTR((kb_r2c<double, E, P, Q>)) \
-    BDK_ATTR((kb_col<float, E, P, Q>))  \
-    BDK_ATTR((kb_col<double, E, P, Q>)) \
-    BDK_ATTR((kb_c2r<float, E, P, Q>))  \
-    BDK_ATTR((kb_c2r<double, E, P, Q>))
-#define BDK_ATTR_BQ(Q)           \
-    BDK_ATTR_B(8, false, Q)  \
-    BDK_ATTR_B(16, false, Q) \
-    BDK_ATTR_B(32, false, Q) \
-    BDK_ATTR_B(8, true, Q)   \
-    BDK_ATTR_B(16, true, Q)  \
-    BDK_ATTR_B(32, true, Q)
-    BDK_ATTR_BQ(true)
-    BDK_ATTR_BQ(false)
-#undef BDK_ATTR_BQ
-#undef BDK_ATTR_B
-#undef BDK_ATTR
+    hipError_t e = fft_set_attributes();
     // the deposit also has a little static LDS: ask for 128 KB of dynamic LDS
 #define BDK_ATTR_D(K)                                                                          \
     if (e == hipSuccess) e = hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
@@ -1895,16 +1503,6 @@ static DepPlan dep_plan(const bdk_t *h, int reset, int tile_pts = 38) {
 
 size_t deposit_lds_bytes(const bdk_t *h) { return dep_plan(h, 0).lds; }
 
-static bool zp2(int Z) { return (Z & (Z - 1)) == 0; }
-
-// FP32 power-of-two meshes of at least FFT_R16_MIN points per side run the
-// column and c2r passes in radix-16 kernels and the r2c rows with a radix-16
-// last pass where radix 8 would leave one bit (fewer LDS passes); smaller
-// meshes keep the radix-8 kernels, whose registers the radix-16 code would
-// raise.  The choice depends on the mesh only, so a simulation takes the same
-// kernels alone and in a batch.
-constexpr int FFT_R16_MIN = 1024;
-static bool fft_r16(int Z) { return zp2(Z) && Z >= FFT_R16_MIN; }
 
 template <typename R, int SCHEME> static void launch_deposit_t(bdk_t *h, const DepPlan &pl, hipStream_t st) {
     if (zp2(h->g.Z))
@@ -1962,61 +1560,6 @@ hipError_t launch_zero_ints(int *p, int n, hipStream_t st) {
 
 hipError_t launch_rearm(bdk_t *h) {
     hipLaunchKernelGGL(k_rearm, dim3(1), dim3(64), 0, h->stream, h->g, h->d);
-    return hipGetLastError();
-}
-
-template <typename R, bool Q, bool R16> static void launch_fft_tq(bdk_t *h, int only, hipStream_t st, int end_step) {
-    using C = typename V2<R>::T;
-    using C4 = typename V4<R>::T;
-    const int Z = h->g.Z;
-    const FftCfg c = fft_cfg<R>(Z);
-    const R *sq = std::is_same<R, float>::value ? (const R *)h->d.sqf : (const R *)h->d.sq;
-    const R *lap = std::is_same<R, float>::value ? (const R *)h->d.lapf : (const R *)h->d.lap;
-#define R2C(E)                                                                                              \
-    hipLaunchKernelGGL((k_r2c_rows<R, E, Q, R16>), dim3(Z / c.RB), dim3(FFT_THREADS), c.l1, st,     \
-                       (const R *)h->d.rho, (C *)h->d.ht, (const C *)h->d.tw, Z, c.RB, c.sR1, h->g.xcd)
-#define COL(E)                                                                                              \
-    hipLaunchKernelGGL((k_col<R, E, Q, R16>), dim3((Z / 2) / c.RC), dim3(FFT_THREADS), c.lc, st,    \
-                       (const C *)h->d.ht, (C4 *)h->d.gt, (const C *)h->d.tw, sq, lap, h->g, c.RC, c.sC)
-#define C2R(E)                                                                                              \
-    hipLaunchKernelGGL((k_c2r_rows<R, E, Q, R16>), dim3(Z / c.RB2), dim3(FFT_THREADS), c.l2, st,    \
-                       (const C4 *)h->d.gt, (C *)h->d.fmesh, (const C *)h->d.tw, Z, c.RB2, c.sR2, h->g.xcd, h->g, h->d,  \
-                       end_step)
-    if (only < 0 || only == 0) BDK_EPT_SWITCH(c.e1, R2C)
-    if (only < 0 || only == 1) BDK_EPT_SWITCH(c.e2, COL)
-    if (only < 0 || only == 2) BDK_EPT_SWITCH(c.e3, C2R)
-#undef R2C
-#undef COL
-#undef C2R
-}
-
-template <typename R> static void launch_fft_t(bdk_t *h, int only = -1, hipStream_t st = nullptr, int end_step = 0) {
-    if (!st) st = h->stream;
-    if constexpr (std::is_same<R, float>::value) {
-        if (fft_r16(h->g.Z)) {
-            launch_fft_tq<R, true, true>(h, only, st, end_step);
-            return;
-        }
-    }
-    if (zp2(h->g.Z))
-        launch_fft_tq<R, true, false>(h, only, st, end_step);
-    else
-        launch_fft_tq<R, false, false>(h, only, st, end_step);
-}
-
-hipError_t launch_fft_pass(bdk_t *h, int pass, hipStream_t st, int end_step) {
-    if (h->p.precision != BDK_FP64)
-        launch_fft_t<float>(h, pass, st, end_step);
-    else
-        launch_fft_t<double>(h, pass, st, end_step);
-    return hipGetLastError();
-}
-
-hipError_t launch_fft(bdk_t *h) {
-    if (h->p.precision != BDK_FP64)
-        launch_fft_t<float>(h);
-    else
-        launch_fft_t<double>(h);
     return hipGetLastError();
 }
 
@@ -2313,11 +1856,6 @@ hipError_t enqueue_step(bdk_t *h, std::vector<std::string> *names, std::vector<h
 
 // ------------------------------------------------------------------ batch plans
 
-int batch_min_ept(int stage, int zmax) {
-    const int need = stage == 0 ? zmax / 2 : (stage == 1 ? 2 * zmax : zmax);
-    return ept_for(8, need);
-}
-
 hipError_t batch_build(const std::vector<bdk_t *> &mem, const BatchTuning &tune, BatchPlan &bp,
                        std::vector<RepDev> &reps, std::vector<int2> maps[BS_COUNT]) {
     const int n = (int)mem.size();
@@ -2334,13 +1872,13 @@ hipError_t batch_build(const std::vector<bdk_t *> &mem, const BatchTuning &tune,
     for (const bdk_t *h : mem) zmax = std::max(zmax, h->g.Z);
     for (int k = 0; k < 3; ++k) bp.ept[k] = std::max(tune.ept[k], batch_min_ept(k, zmax));
     const int *ept = bp.ept;
-    bp.dep_lds = bp.l1 = bp.lc = bp.l2 = 0;
-    const size_t csz = bp.f32 ? 8 : 16;
-    // entries of the members with a power-of-two mesh first, those with
-    // radix-16 column and c2r passes (FP32) before the others: the mesh
-    // stages launch once per mesh kind present (the kind is a template
-    // parameter)
-    auto cls = [&](const bdk_t *h) { return bp.f32 && fft_r16(h->g.Z) ? 0 : (zp2(h->g.Z) ? 1 : 2); };
+    bp.dep_lds = 0;
+    std::fill(&bp.fft_lds[0][0], &bp.fft_lds[0][0] + 9, (size_t)0);
+    std::fill(&bp.fft_threads[0][0], &bp.fft_threads[0][0] + 9, 0);
+    // entries of the members with a power-of-two mesh first, those with 16
+    // mesh points per FFT thread (FP32) before the others: the mesh stages
+    // launch once per mesh kind present (the kind is a template parameter)
+    auto cls = [&](const bdk_t *h) { return zp2(h->g.Z) ? (fft_ept(h->g.Z, bp.f32) == 16 ? 0 : 1) : 2; };
     std::vector<int> order;
     for (int pass = 0; pass < 3; ++pass)
         for (int i = 0; i < n; ++i)
@@ -2356,13 +1894,7 @@ hipError_t batch_build(const std::vector<bdk_t *> &mem, const BatchTuning &tune,
         r.dep_tx = (int)pl.grid.x;
         bp.dep_lds = std::max(bp.dep_lds, pl.lds);
         const int Z = h->g.Z;
-        fft_rows(Z, ept, r.rb, r.rc, r.rb2);
-        r.sR1 = lds_row(Z / 2);
-        r.sC = lds_row(Z);
-        r.sR2 = lds_row(Z);
-        bp.l1 = std::max(bp.l1, (size_t)r.rb * r.sR1 * csz);
-        bp.lc = std::max(bp.lc, (size_t)2 * r.rc * r.sC * csz);
-        bp.l2 = std::max(bp.l2, (size_t)r.rb2 * r.sR2 * csz);
+        fft_member(r, Z, ept, bp);
         r.scan_nb = (int)nblk(h->g.ncell, SCAN_BLOCK);
         r.unit = h->p.sigma11_22 == 1.0 && h->p.sigma11_12 == 1.0 && h->p.eps22_11 == 1.0 && h->p.eps12_11 == 1.0;
         const int ad = h->g.adaptive ? 1 : 0;
@@ -2380,19 +1912,6 @@ hipError_t batch_build(const std::vector<bdk_t *> &mem, const BatchTuning &tune,
     return hipSuccess;
 }
 
-#define BDK_EPT_SWITCH2(E, CALL) \
-    switch (E) {                 \
-    case 8: CALL(8); break;      \
-    case 16: CALL(16); break;    \
-    default: CALL(32); break;    \
-    }
-
-// blocks of a launch over a map of n entries (the persistent form caps them)
-static unsigned stage_grid(const BatchPlan &bp, int n) {
-    const int p = bp.tune.persist;
-    return (unsigned)std::max(1, p > 0 ? std::min(n, p) : n);
-}
-
 template <typename R, bool P> static void batch_stage_tp(const BatchPlan &bp, int stage, hipStream_t st) {
     const RepDev *m = bp.reps;
     // f(kind, map, entries) once per mesh kind present in stage S's map
@@ -2400,14 +1919,6 @@ template <typename R, bool P> static void batch_stage_tp(const BatchPlan &bp, in
         const int n2 = bp.nblk2[S], nall = bp.nblk[S];
         if (n2 > 0) f(std::true_type(), (const int2 *)bp.map[S], n2);
         if (nall > n2) f(std::false_type(), (const int2 *)bp.map[S] + n2, nall - n2);
-    };
-    // the same for the column and c2r passes, with the radix-16 members
-    // (leading) apart: f(kind, radix 16, map, entries)
-    auto kinds16 = [&](int S, auto &&f) {
-        const int n16 = std::is_same<R, float>::value ? bp.nblk16[S] : 0, n2 = bp.nblk2[S], nall = bp.nblk[S];
-        if (n16 > 0) f(std::true_type(), std::true_type(), (const int2 *)bp.map[S], n16);
-        if (n2 > n16) f(std::true_type(), std::false_type(), (const int2 *)bp.map[S] + n16, n2 - n16);
-        if (nall > n2) f(std::false_type(), std::false_type(), (const int2 *)bp.map[S] + n2, nall - n2);
     };
 #define BDK_G(S) dim3(stage_grid(bp, bp.nblk[S]))
     switch (stage) {
@@ -2424,38 +1935,10 @@ template <typename R, bool P> static void batch_stage_tp(const BatchPlan &bp, in
         });
         break;
     case 2:
-        kinds16(BS_R2C, [&](auto q, auto r16, const int2 *mp, int nm) {
-            constexpr bool Q = decltype(q)::value;
-            constexpr bool R16 = decltype(r16)::value && std::is_same<R, float>::value;
-#define R2C(E)                                                                                                 \
-    hipLaunchKernelGGL((kb_r2c<R, E, P, Q, R16>), dim3(stage_grid(bp, nm)), dim3(FFT_THREADS), bp.l1, st, m, mp, \
-                       nm)
-            BDK_EPT_SWITCH2(bp.ept[0], R2C)
-#undef R2C
-        });
-        break;
     case 3:
-        kinds16(BS_COL, [&](auto q, auto r16, const int2 *mp, int nm) {
-            constexpr bool Q = decltype(q)::value;
-            constexpr bool R16 = decltype(r16)::value && std::is_same<R, float>::value;
-#define COL(E)                                                                                                 \
-    hipLaunchKernelGGL((kb_col<R, E, P, Q, R16>), dim3(stage_grid(bp, nm)), dim3(FFT_THREADS), bp.lc, st, m, mp, \
-                       nm)
-            BDK_EPT_SWITCH2(bp.ept[1], COL)
-#undef COL
-        });
-        break;
     case 4:
-    case 12:  // 12: also the end of the step
-        kinds16(BS_C2R, [&](auto q, auto r16, const int2 *mp, int nm) {
-            constexpr bool Q = decltype(q)::value;
-            constexpr bool R16 = decltype(r16)::value && std::is_same<R, float>::value;
-#define C2R(E)                                                                                                  \
-    hipLaunchKernelGGL((kb_c2r<R, E, P, Q, R16>), dim3(stage_grid(bp, nm)), dim3(FFT_THREADS), bp.l2, st, m, mp, \
-                       nm, stage == 12 ? 1 : 0)
-            BDK_EPT_SWITCH2(bp.ept[2], C2R)
-#undef C2R
-        });
+    case 12:  // 12: c2r, also the end of the step
+        batch_fft_stage(bp, stage, st);
         break;
     case 5:
         kinds(BS_PART, [&](auto q, const int2 *mp, int nm) {

@@ -7,8 +7,6 @@
 
 namespace bdkx {
 
-static inline unsigned nblk(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
-
 // Column sums of part[nrow][ncol] in a fixed order: 32 columns x 32 threads
 // per block, thread y adds rows y, y + 32, ..., then its 32 sums are added in
 // order.
@@ -60,17 +58,10 @@ __device__ __forceinline__ int shell_begin(int b, double m2, double dqr, int Zh)
     return a;
 }
 
-template <typename R, int EPT>
-__global__ __launch_bounds__(FFT_THREADS) void k_col_rhok(const typename V2<R>::T *__restrict__ ht,
-                                                          const typename V2<R>::T *__restrict__ tw, int Z,
-                                                          double dqr, int nbins, double *part) {
-    using C = typename V2<R>::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    const int m = blockIdx.x, tid = threadIdx.x, Zh = Z >> 1;
-    for (int k = tid; k < Z; k += blockDim.x) s[lp(k)] = ht[(size_t)m * Z + k];
-    __syncthreads();
-    lds_fft<R, EPT>(s, Z, 1, lds_row(Z), tw, Z, false);
+// the shells of column m's transform, point i at s[at(i)]
+template <typename C, typename F>
+__device__ __forceinline__ void shell_sums(const C *s, F &&at, int m, int Z, double dqr, int nbins, double *part) {
+    const int tid = threadIdx.x, Zh = Z >> 1;
     // column m > 0, or the DC (col = 0) and Nyquist (col = Z/2) columns that
     // share the packed column 0
     for (int t = tid; t < (m == 0 ? 2 : 1) * nbins; t += blockDim.x) {
@@ -81,7 +72,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_col_rhok(const typename V2<R>::
         for (int a = a0; a < a1; ++a) {
             // |j| = a: j = a and Z - a (one of them for a = 0 and Z/2)
             const bool two = a > 0 && a < Zh;
-            const C P = s[lp(a)], Q = s[lp(a == 0 ? 0 : Z - a)];
+            const C P = s[at(a)], Q = s[at(a == 0 ? 0 : Z - a)];
             double w = two ? (double)P.x + (double)Q.x : (double)P.x;
             if (m > 0)
                 w *= 2.0;
@@ -98,18 +89,85 @@ __global__ __launch_bounds__(FFT_THREADS) void k_col_rhok(const typename V2<R>::
     }
 }
 
+// power-of-two meshes: one column per block, the transform by its first Z/E
+// threads (all of them where several waves take part)
+template <typename R, int LOGZ>
+__global__ __launch_bounds__(512) void k_col_rhok(const typename V2<R>::T *__restrict__ ht,
+                                                  const typename V2<R>::T *__restrict__ tw, double dqr, int nbins,
+                                                  double *part) {
+    using C = typename V2<R>::T;
+    constexpr int Z = 1 << LOGZ, E = fft_ept(Z, sizeof(R) == 4);
+    using F = RowFft<R, LOGZ, E, LOGZ>;
+    extern __shared__ unsigned char smem_raw[];
+    C *s = (C *)smem_raw;
+    const int m = blockIdx.x, t = threadIdx.x;
+    if (t < F::T) {
+        C v[1][E];
+#pragma unroll
+        for (int u = 0; u < E; ++u) v[0][u] = ht[(size_t)m * Z + t + F::T * u];
+        F f;
+        f.load(tw, t);
+        f.template run<1, false, true>(v, s, t);
+        if (F::NP > 1) row_sync<F::WAVE>();
+#pragma unroll
+        for (int u = 0; u < E; ++u) s[lpe<E>(t + F::T * u)] = v[0][u];
+    }
+    __syncthreads();
+    shell_sums(s, [](int i) { return lpe<E>(i); }, m, Z, dqr, nbins, part);
+}
+
+// other meshes
+template <typename R, int EPT>
+__global__ __launch_bounds__(FFT_THREADS) void k_col_rhok_any(const typename V2<R>::T *__restrict__ ht,
+                                                              const typename V2<R>::T *__restrict__ tw, int Z,
+                                                              double dqr, int nbins, double *part) {
+    using C = typename V2<R>::T;
+    extern __shared__ unsigned char smem_raw[];
+    C *s = (C *)smem_raw;
+    const int m = blockIdx.x;
+    for (int k = threadIdx.x; k < Z; k += blockDim.x) s[lp(k)] = ht[(size_t)m * Z + k];
+    __syncthreads();
+    lds_fft_g<R, EPT>(s, Z, 1, lds_row(Z), tw, Z, false);
+    shell_sums(s, [](int i) { return lp(i); }, m, Z, dqr, nbins, part);
+}
+
 template <typename R> static void launch_rhok_t(bdk_t *h, double dqr, int nbins, double *part, double *out) {
     using C = typename V2<R>::T;
     const int Z = h->g.Z;
-    const int ept = ept_for(8, Z);
-    const size_t lds = (size_t)lds_row(Z) * sizeof(C);
-#define RHOK(E)                                                                                              \
-    (void)hipFuncSetAttribute((const void *)k_col_rhok<R, E>, hipFuncAttributeMaxDynamicSharedMemorySize,      \
-                              160 * 1024);                                                                     \
-    hipLaunchKernelGGL((k_col_rhok<R, E>), dim3(Z / 2), dim3(FFT_THREADS), lds, h->stream, (const C *)h->d.ht, \
-                       (const C *)h->d.tw, Z, dqr, nbins, part)
-    BDK_EPT_SWITCH(ept, RHOK)
+    const C *ht = (const C *)h->d.ht, *tw = (const C *)h->d.tw;
+    const size_t lds = (size_t)(Z + Z / 8 + 1) * sizeof(C);
+    auto big = [](const void *k) {
+        (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    };
+    if (zp2(Z)) {
+        // blocks whose barriers every thread reaches: exactly the row's
+        // threads where they are more than a wave
+        const int T = Z / fft_ept(Z, sizeof(R) == 4), nt = T > 64 ? T : 256;
+#define RHOK(LZ)                                                                                                 \
+    big((const void *)k_col_rhok<R, LZ>);                                                                        \
+    hipLaunchKernelGGL((k_col_rhok<R, LZ>), dim3(Z / 2), dim3(nt), lds, h->stream, ht, tw, dqr, nbins, part)
+        switch (h->g.logZ) {
+        case 3: RHOK(3); break;
+        case 4: RHOK(4); break;
+        case 5: RHOK(5); break;
+        case 6: RHOK(6); break;
+        case 7: RHOK(7); break;
+        case 8: RHOK(8); break;
+        case 9: RHOK(9); break;
+        case 10: RHOK(10); break;
+        case 11: RHOK(11); break;
+        default: RHOK(12); break;
+        }
 #undef RHOK
+    } else {
+        const int ept = ept_for(8, Z);
+#define RHOK(E)                                                                                                    \
+    big((const void *)k_col_rhok_any<R, E>);                                                                       \
+    hipLaunchKernelGGL((k_col_rhok_any<R, E>), dim3(Z / 2), dim3(FFT_THREADS), lds, h->stream, ht, tw, Z, dqr, nbins, \
+                       part)
+        BDK_EPT_SWITCH(ept, RHOK)
+#undef RHOK
+    }
     launch_sum_rows(part, Z / 2 + 1, 2 * nbins, out, h->stream);
 }
 
