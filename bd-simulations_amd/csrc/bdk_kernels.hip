@@ -6,8 +6,8 @@
 //               (dm:116-157), refresh (dm:216-325); the cell counts are
 //               updated by the particles that change cell;
 // then on two streams side by side:
-//   k_rank_scan rank of each particle that stayed in its cell (no atomics)
-//               beside the exclusive scan of the cell counts;
+//   k_scan      exclusive scan of the cell counts (the update ranked the
+//               particles that stay in their cell, without atomics);
 //   k_fill      cell list = slots grouped by cell, species in bit 31, and
 //               the particle state in list order (lcell, lrel, lpid, lrelf);
 //   k_sort_cells  the arrivals of each cell in slot order;
@@ -47,8 +47,11 @@ namespace bdkx {
 // grouping of dm:617-702 + dm:973-1059.
 constexpr unsigned LIST_SLOT = 0x7fffffffu;
 // rank of a particle that changed cell during the step: its arrival index
-// in the new cell, marked (ranks stay below 2^30)
+// in the new cell, marked (ranks stay below 2^30).  RANK_OPEN marks the rank
+// of a stayer whose cell begins before its wave's first list position: the
+// stayers there are still to be added.
 constexpr int RANK_MOVED = 1 << 30;
+constexpr int RANK_OPEN = 1 << 31;
 // Scan of the cell counts: blocks of SCAN_BLOCK cells, SCAN_PER_THREAD
 // consecutive cells per thread; bcount[c >> SCAN_SHIFT] is the particle count
 // of the block holding cell c
@@ -937,8 +940,9 @@ __device__ __forceinline__ double fmod_cell(double y, double B) {
 // position s (written to slot s).  Returns how far the stored new position
 // (cell and offset) lies outside the particle's previous cell (<= 0 inside).
 // FUSED: capillary force gathered here (fixed dt); else read from fkap.
+// cell: the particle's previous cell if it stays there, else -1 - that cell.
 template <typename R, int SCHEME, bool FUSED, bool P2>
-__device__ __forceinline__ double update_one(const Geo &g, const DevBufs &d, int s, double dt) {
+__device__ __forceinline__ double update_one(const Geo &g, const DevBufs &d, int s, double dt, int &cell) {
     using R2 = typename V2<R>::T;
     const unsigned long long step = d.sc->step;
     const int c = d.lcell[s];
@@ -1044,7 +1048,7 @@ __device__ __forceinline__ double update_one(const Geo &g, const DevBufs &d, int
     if (nc_new != c) {
         // a cell change (a few percent of the particles per step): the
         // counts follow, and the rank among the new cell's arrivals comes
-        // from arr; particles that stay are ranked by k_rank without atomics
+        // from arr; particles that stay are ranked without atomics
         atomicSub(&d.count[c], 1);
         atomicAdd(&d.count[nc_new], 1);
         if ((c >> SCAN_SHIFT) != (nc_new >> SCAN_SHIFT)) {
@@ -1053,6 +1057,7 @@ __device__ __forceinline__ double update_one(const Geo &g, const DevBufs &d, int
         }
         d.rank[s] = RANK_MOVED | atomicAdd(&d.arr[nc_new], 1);
     }
+    cell = nc_new == c ? c : -1 - c;
     double ex = fmax(fmax(-rn.x, rn.x - B), fmax(-rn.y, rn.y - B));
     if (ex > 0.0) atomicMax(&d.sc->exc_bits[(step + 1) & 1], bitsd(ex));
     if (s == 0) d.sc->dt_last = bitsd(dt);
@@ -1091,7 +1096,22 @@ __device__ __forceinline__ void update_body(const Geo &g, const DevBufs &d, int 
         }
     }
     double m = 0.0;
-    if (s < g.N) m = update_one<R, SCHEME, FUSED, P2>(g, d, s, dt);
+    int cell = -1 - g.ncell;  // (no particle: a cell of its own, not a stayer)
+    if (s < g.N) m = update_one<R, SCHEME, FUSED, P2>(g, d, s, dt, cell);
+    // Rank of a particle that stays: the stayers of its cell before it.  A
+    // wave holds 64 consecutive list positions, so the cell's entries are
+    // neighbouring lanes; the fill adds the stayers before the wave for the
+    // wave's first cell.  (A pass of its own that compared the cells of each
+    // particle's predecessors took 16 us at 2M particles.)
+    {
+        const int lane = threadIdx.x & 63, c = cell >= 0 ? cell : -1 - cell;
+        const int prev = __shfl_up(c, 1, 64);
+        const unsigned long long heads = __ballot(lane == 0 || prev != c), stay = __ballot(cell >= 0);
+        const unsigned long long upto = ~0ull >> (63 - lane);
+        const int first = 63 - __clzll((long long)(heads & upto));  // the cell's first lane
+        const int r = __popcll(stay & (upto >> 1) & (~0ull << first));
+        if (cell >= 0) d.rank[s] = first == 0 ? r | RANK_OPEN : r;
+    }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
     if ((threadIdx.x & 63) == 0 && m > 0.0) {
@@ -1287,32 +1307,9 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan(const int *__restrict__ c
     scan_body(count, bcount, start, ncell, nb, nmax, sc, inc_step, blockIdx.x);
 }
 
-// Rank of a particle that stayed in its cell during the step: its position
-// among the cell's previous entries, minus the entries before it that left.
-// Reads the previous starts from the update's copy, so it runs beside the
-// scan that overwrites start.
-__device__ __forceinline__ void rank_body(const Geo &g, const DevBufs &d, int blk) {
-    const int q = blk * blockDim.x + threadIdx.x;
-    if (q >= g.N) return;
-    const int c = d.lcell[q];
-    if (d.cell[q] != c) return;  // moved: ranked among the arrivals
-    const int b = d.start_old[c];
-    int r = q - b;
-    for (int p = b; p < q; ++p) r -= d.cell[p] != d.lcell[p];
-    d.rank[q] = r;
-}
-
-// the ranks and the scan of the new counts as one launch: blocks [0, nrank)
-// rank, the others scan
-__global__ __launch_bounds__(256) void k_rank_scan(Geo g, DevBufs d, int nrank, int nb, int inc_step) {
-    if ((int)blockIdx.x < nrank)
-        rank_body(g, d, blockIdx.x);
-    else
-        scan_body(d.count, d.bcount, d.start, g.ncell, nb, g.N, d.sc, inc_step, blockIdx.x - nrank);
-}
 // List entries and the list-ordered state from the ranks.  After a step
-// (moved_ranks) a cell holds its stayers first (ascending slot, from
-// k_rank), then its arrivals (marked ranks, ordered by k_sort_cells); after
+// (moved_ranks) a cell holds its stayers first (ascending slot, ranked by
+// the update), then its arrivals (marked ranks, ordered by k_sort_cells); after
 // a full binning every rank is the position in the cell (ordered by
 // k_sort_cells).
 __device__ __forceinline__ void fill_body(const Geo &g, const DevBufs &d, int moved_ranks, int blk) {
@@ -1322,7 +1319,11 @@ __device__ __forceinline__ void fill_body(const Geo &g, const DevBufs &d, int mo
     const int c = d.cell[s];
     const int rk = d.rank[s];
     int pos = d.start[c] + (rk & (RANK_MOVED - 1));
-    if (moved_ranks && (rk & RANK_MOVED)) pos += d.start[c + 1] - d.start[c] - d.arr[c];
+    if (moved_ranks) {
+        if (rk & RANK_MOVED) pos += d.start[c + 1] - d.start[c] - d.arr[c];
+        if (rk & RANK_OPEN)  // the stayers of the cell before the update's wave
+            for (int p = d.start_old[c]; p < (s & ~63); ++p) pos += d.cell[p] == c;
+    }
     if ((unsigned)pos >= (unsigned)g.N) {  // inconsistent counts: flagged, nothing written
         atomicOr(&d.sc->nonfinite, 2);
         return;
@@ -1487,19 +1488,12 @@ __global__ __launch_bounds__(256) void kb_gather(const RepDev *m, const int2 *ma
     });
 }
 
-// entries [0, nrank): ranks (map mp); entries [nrank, nrank + nscan): scans (map ms)
 template <bool P>
-__global__ __launch_bounds__(256) void kb_rank_scan(const RepDev *m, const int2 *mp, int nrank, const int2 *ms,
-                                                    int nscan) {
-    for_entries<P, true>(nrank + nscan, [&](int e_) {
-        if (e_ < nrank) {
-            const int2 t = mp[e_];
-            rank_body(m[t.x].g, m[t.x].d, t.y);
-        } else {
-            const int2 t = ms[e_ - nrank];
-            const RepDev &r = m[t.x];
-            scan_body(r.d.count, r.d.bcount, r.d.start, r.g.ncell, r.scan_nb, r.g.N, r.d.sc, 0, t.y);
-        }
+__global__ __launch_bounds__(SCAN_THREADS) void kb_scan(const RepDev *m, const int2 *map, int nmap) {
+    for_entries<P, true>(nmap, [&](int e_) {
+        const int2 t = map[e_];
+        const RepDev &r = m[t.x];
+        scan_body(r.d.count, r.d.bcount, r.d.start, r.g.ncell, r.scan_nb, r.g.N, r.d.sc, 0, t.y);
     });
 }
 
@@ -1897,7 +1891,7 @@ hipError_t enqueue_forces(bdk_t *h, std::vector<std::string> *names, std::vector
 // One step from a state whose forces are ready: the update (gather, noise,
 // Euler step, refresh), then the two halves that only need its output side
 // by side:
-//   main stream: the list rebuild (rank, scan, fill, sort), then the WCA
+//   main stream: the list rebuild (scan, fill, sort), then the WCA
 //                forces of the new lists;
 //   second stream: the deposit from the slot arrays (grouped by the previous
 //                starts, which the update kept; halo widened by the
@@ -1951,11 +1945,10 @@ hipError_t enqueue_step(bdk_t *h, std::vector<std::string> *names, std::vector<h
         }
         if (fork) m.chk(hipEventRecord(h->ev_join, side));
     }
-    // bcount is current (the update adjusted it with the counts); the ranks
-    // read the previous starts that the update kept
-    const int nrank = (int)nblk(h->g.N, 256);
-    hipLaunchKernelGGL(k_rank_scan, dim3(nrank + nb), dim3(256), 0, h->stream, h->g, h->d, nrank, nb, !kap);
-    m.mark("k_rank_scan");
+    // bcount is current (the update adjusted it with the counts)
+    hipLaunchKernelGGL(k_scan, dim3(nb), dim3(SCAN_THREADS), 0, h->stream, h->d.count, h->d.bcount, h->d.start, ncell,
+                       nb, h->g.N, h->d.sc, kap ? 0 : 1);
+    m.mark("k_scan");
     hipLaunchKernelGGL(k_fill, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d, 1);
     m.mark("k_fill");
     hipLaunchKernelGGL(k_sort_cells, dim3(nblk(ncell, 256)), dim3(256), 0, h->stream, h->g, h->d, 1);
@@ -2070,8 +2063,7 @@ template <typename R, bool P> static void batch_stage_tp(const BatchPlan &bp, in
         }
         break;
     case 6:
-        hipLaunchKernelGGL(kb_rank_scan<P>, dim3(stage_grid(bp, bp.nblk[BS_PART] + bp.nblk[BS_SCAN])), dim3(256), 0, st,
-                           m, bp.map[BS_PART], bp.nblk[BS_PART], bp.map[BS_SCAN], bp.nblk[BS_SCAN]);
+        hipLaunchKernelGGL(kb_scan<P>, BDK_G(BS_SCAN), dim3(SCAN_THREADS), 0, st, m, bp.map[BS_SCAN], bp.nblk[BS_SCAN]);
         break;
     default: {  // 11: fill, sort
         hipLaunchKernelGGL(kb_fill<P>, BDK_G(BS_PART), dim3(256), 0, st, m, bp.map[BS_PART], bp.nblk[BS_PART]);
@@ -2090,7 +2082,7 @@ template <typename R> static void batch_stage_t(const BatchPlan &bp, int stage, 
 }
 
 // stage 0 WCA, 1 deposit (list order), 2 r2c, 3 col, 4 c2r, 5 update,
-// 6 rank + scan, 8 deposit (slot arrays), 11 fill + sort, 12 c2r + step end,
+// 6 scan, 8 deposit (slot arrays), 11 fill + sort, 12 c2r + step end,
 // 13 gather (forces and dt candidates) of the adaptive members
 hipError_t batch_stage(const BatchPlan &bp, int stage, hipStream_t st) {
     if (bp.f32)
