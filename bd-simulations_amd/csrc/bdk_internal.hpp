@@ -123,11 +123,10 @@ struct DevBufs {
 
 // Deposit launch arguments (one tile per block).
 struct DepArgs {
-    int tc;        // list cells per tile side
-    int seg_cap;   // staged list segments (rows, two per row when y wraps)
-    int win_cap;   // owned mesh points per tile (capacity)
-    int win_fast;  // FP32: points of the stencil window of a tile (0: no windowed path)
-    float scale_f; // FP32 windowed path: 2^S with |charge| 2^S < 2^31
+    int tcx, tcy;  // list cells per tile
+    int ty;        // tiles along y
+    int win_cap;   // mesh points of a tile's window (capacity)
+    float scale_f; // FP32: 2^S with |charge| 2^S < 2^31
     double iscale_f;
     double scale_hi, scale_lo;      // 2^S1, 2^S2
     double iscale_hi, iscale_lo;    // 2^-S1, 2^-S2
@@ -141,7 +140,6 @@ struct RepDev {
     Geo g;
     DevBufs d;
     DepArgs dep;
-    int dep_tx;                      // deposit tiles per row
     int rb, rc, rb2, sR1, sC, sR2;   // FFT rows per block and LDS row strides
     int scan_nb;                     // scan blocks
     int unit;                        // all sigma/epsilon ratios 1

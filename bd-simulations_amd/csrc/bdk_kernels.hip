@@ -445,17 +445,33 @@ __global__ __launch_bounds__(256) void k_wca_f32(Geo g, DevBufs d) {
 }
 
 // ------------------------------------------------------------------ deposit
-// Charge assignment (gr:31-547) per tile of tc x tc list cells.  A mesh
+// Charge assignment (gr:31-547) per tile of tcx x tcy list cells.  A mesh
 // point belongs to the tile whose cells contain its centre,
-// owner(k) = floor((k+1/2)h/B).  Every particle of the tile's cells and of
-// a halo of hx cells adds its (up to 9) weighted charges to the tile's own
-// mesh points in LDS.  The additions are integer (fixed point, scale 2^S),
-// so the sums do not depend on the order of the atomics: the deposit is
-// deterministic without floating-point atomics.  FP64 mode splits every
+// owner(k) = floor((k+1/2)h/B).  Every particle near enough adds its (up to
+// 9) weighted charges in LDS to a window of the tile's own points and two
+// more on every side, so a particle has one base index and fixed offsets: one
+// whose stencil misses the own points is skipped, and what falls beside them
+// is not written out.  The particles come row by row of list cells (each
+// row's cells are one range of the list, two where y wraps), DP_LANES lanes
+// per row.
+//
+// The additions are integer (fixed point, scale 2^S), so the sums do not
+// depend on the order of the atomics: the deposit is deterministic without
+// floating-point atomics.  FP32 charges are truncated to 32-bit fixed point
+// (|charge| 2^S < 2^31: a truncation error of 2^-31 of the largest charge,
+// far below FP32 resolution) and summed in 64 bits.  FP64 mode splits every
 // charge into a coarse and a fine integer part (two accumulators), which
 // keeps the sum exact to ~2^-(S+40).
+//
+// Bound by its phases' latency (bounds, list starts, particles, write-out)
+// and the 64-bit LDS atomics.  Before (square tiles, a window over all that the
+// staged cells could reach, particles through a prefix sum and a segment
+// table): 26.3 us at 2M particles on 2048^2, now 22.6; 4M on 4096^2 74.6 ->
+// 53.4; 64,000 on 512^2 8.2 -> 6.0; 200,000 FP64 on 1024^2 14.9 -> 13.0.  With 8,
+// 32 or 64 lanes per row: 25.8, 21.7 and 23.0 us on 2048^2, 63, 55 and 55 on
+// 4096^2, 9.0, 7.1 and 7.5 on 512^2; 512 threads: 26.1, 69 and 6.8.
 constexpr int DP_THREADS = 256;
-constexpr int DP_SEG_TAB = 1536;  // staged particles with a segment table entry
+constexpr int DP_LANES = 16;     // lanes per row of list cells
 
 __device__ int first_owned(int c, const Geo &g) {
     if (c <= 0) return 0;
@@ -474,276 +490,187 @@ __global__ void k_own(Geo g, int *own) {
     if (c <= g.nc) own[c] = first_owned(c, g);
 }
 
-// FP32 deposit into a window that holds the whole stencil of every staged
-// particle (mesh rows kw0 .. kw0 + nwx - 1, columns lw0 .., unwrapped): one
-// base index per particle and nine fixed offsets, no per-point bounds.  The
-// charges are truncated to 32-bit fixed point (scale 2^S, |charge| 2^S <
-// 2^31: a truncation error of 2^-31 of the largest charge, far below FP32
-// resolution) and summed in 64 bits, so the sums stay exact and independent
-// of the order of the atomics.  dqs: the particle's charge drho q times 2^S
-// (exact: a power of two), so a point's fixed-point value is
-// (int)((wx wy) dqs).
-template <int SCHEME, bool P2>
-__device__ __forceinline__ void deposit_particle_win(const Geo &g, const DevBufs &d, float dqs, int gx, int gy,
-                                                     double2 rr, int kw0, int lw0, int nwx, int nwy,
-                                                     unsigned long long *acc) {
-    const double x = gx * g.B + rr.x, y = gy * g.B + rr.y;
-    int kp, lp;
-    float wx[3], wy[3];
-    weights_r<float, SCHEME>(x, g, kp, wx);
-    weights_r<float, SCHEME>(y, g, lp, wy);
-    const int kb = wrapz<P2>(kp - 1 - kw0, g.Z), lb = wrapz<P2>(lp - 1 - lw0, g.Z);
-    if (kb > nwx - 3 || lb > nwy - 3) {  // outside the window: not reachable, flagged
-        atomicOr(&d.sc->nonfinite, 4);
-        return;
+// one mesh point's charge into the accumulators at w
+template <typename R>
+__device__ __forceinline__ void deposit_add(const DepArgs &a, float cf, double cd, int w, unsigned long long *hi,
+                                            unsigned long long *lo) {
+    if (std::is_same<R, float>::value) {
+        atomicAdd(&hi[w], (unsigned long long)(long long)(int)cf);
+    } else {
+        const long long Xh = __double2ll_rn(cd * a.scale_hi);
+        const double rem = cd - (double)Xh * a.iscale_hi;
+        const long long Xl = __double2ll_rn(rem * a.scale_lo);
+        atomicAdd(&hi[w], (unsigned long long)Xh);
+        atomicAdd(&lo[w], (unsigned long long)Xl);
     }
-    unsigned long long *p = acc + kb * nwy + lb;
-    if (SCHEME == 0) {
-        atomicAdd(&p[nwy + 1], (unsigned long long)(long long)(int)dqs);
-        return;
-    }
-#pragma unroll
-    for (int ia = 0; ia < 3; ++ia)
-#pragma unroll
-        for (int ib = 0; ib < 3; ++ib) {
-            const int X = (int)((wx[ia] * wy[ib]) * dqs);
-            atomicAdd(&p[ia * nwy + ib], (unsigned long long)(long long)X);
-        }
 }
 
+// The window of a tile: mesh rows kw0 .. kw0 + nwx - 1, columns lw0 ..
+// (unwrapped), its own points klo .. khi - 1, llo .. lhi - 1; and the points
+// that a particle of the visited cells may reach (kr0, nrx, ...), beyond
+// which the displacement bound was wrong.
+struct DepWin {
+    int klo, khi, llo, lhi, kw0, lw0, nwx, nwy, kr0, nrx, lr0, nry;
+    bool win;  // the window's points are distinct (else only own points, tested one by one)
+    bool chk;  // the reachable points are well short of the whole mesh
+};
+
+// one particle at (x, y) with fixed-point charge dqs (FP32: drho q 2^S) or q (FP64)
 template <typename R, int SCHEME, bool P2>
-__device__ __forceinline__ void deposit_particle(const Geo &g, const DevBufs &d, const DepArgs &a, float dqs, int gx,
-                                                 int gy, double2 rr, bool s2, int klo, int khi, int llo, int lhi,
-                                                 unsigned long long *acc_hi, unsigned long long *acc_lo) {
-    const double x = gx * g.B + rr.x, y = gy * g.B + rr.y;
+__device__ __forceinline__ void deposit_particle(const Geo &g, const DevBufs &d, const DepArgs &a, const DepWin &v,
+                                                 float dqs, double q, double x, double y, unsigned long long *hi,
+                                                 unsigned long long *lo) {
     int kp, lp;
     R wx[3], wy[3];
     weights_r<R, SCHEME>(x, g, kp, wx);
     weights_r<R, SCHEME>(y, g, lp, wy);
-    const int Z = g.Z, nl = lhi - llo;
+    constexpr bool F32 = std::is_same<R, float>::value;
+    auto charge = [&](int ia, int ib, float &cf, double &cd) {
+        if (F32)
+            cf = SCHEME == 0 ? dqs : ((float)wx[ia] * (float)wy[ib]) * dqs;
+        else
+            cd = SCHEME == 0 ? g.drho * q : (double)wx[ia] * (double)wy[ib] * g.drho * q;
+    };
+    if (v.win) {
+        const int kb = wrapz<P2>(kp - 1 - v.kw0, g.Z), lb = wrapz<P2>(lp - 1 - v.lw0, g.Z);
+        if (kb > v.nwx - 3 || lb > v.nwy - 3) {  // none of the own points
+            if (v.chk && (wrapz<P2>(kp - v.kr0, g.Z) >= v.nrx || wrapz<P2>(lp - v.lr0, g.Z) >= v.nry))
+                atomicOr(&d.sc->nonfinite, 4);
+            return;
+        }
+        const int w = kb * v.nwy + lb;
+#pragma unroll
+        for (int ia = 0; ia < 3; ++ia) {
+            if (SCHEME == 0 && ia != 1) continue;
+            if (SCHEME == 1 && wx[ia] == 0) continue;
+#pragma unroll
+            for (int ib = 0; ib < 3; ++ib) {
+                if (SCHEME == 0 && ib != 1) continue;
+                if (SCHEME == 1 && wy[ib] == 0) continue;
+                float cf = 0.f;
+                double cd = 0.0;
+                charge(ia, ib, cf, cd);
+                deposit_add<R>(a, cf, cd, w + ia * v.nwy + ib, hi, lo);
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int ia = 0; ia < 3; ++ia) {
         if (SCHEME == 0 && ia != 1) continue;
-        if (wx[ia] == 0.0) continue;
-        const int k = wrapz<P2>(kp + ia - 1, Z);
-        if (k < klo || k >= khi) continue;
+        const int k = wrapz<P2>(kp + ia - 1, g.Z);
+        if (k < v.klo || k >= v.khi) continue;
 #pragma unroll
         for (int ib = 0; ib < 3; ++ib) {
             if (SCHEME == 0 && ib != 1) continue;
-            if (wy[ib] == 0.0) continue;
-            const int l = wrapz<P2>(lp + ib - 1, Z);
-            if (l < llo || l >= lhi) continue;
-            const int w = (k - klo) * nl + (l - llo);
-            if (std::is_same<R, float>::value) {
-                // the charge and its fixed point exactly as in the window path,
-                // so the mesh does not depend on which path a tile takes
-                const float cf = SCHEME == 0 ? dqs : ((float)wx[ia] * (float)wy[ib]) * dqs;
-                atomicAdd(&acc_hi[w], (unsigned long long)(long long)(int)cf);
-            } else {
-                double cd;
-                if (SCHEME == 0)
-                    cd = g.drho * (s2 ? a.q2 : a.q1);
-                else {
-                    cd = wx[ia] * wy[ib] * g.drho;
-                    cd = cd * (s2 ? a.q2 : a.q1);
-                }
-                const long long Xh = __double2ll_rn(cd * a.scale_hi);
-                const double rem = cd - (double)Xh * a.iscale_hi;
-                const long long Xl = __double2ll_rn(rem * a.scale_lo);
-                atomicAdd(&acc_hi[w], (unsigned long long)Xh);
-                atomicAdd(&acc_lo[w], (unsigned long long)Xl);
-            }
+            const int l = wrapz<P2>(lp + ib - 1, g.Z);
+            if (l < v.llo || l >= v.lhi) continue;
+            float cf = 0.f;
+            double cd = 0.0;
+            charge(ia, ib, cf, cd);
+            deposit_add<R>(a, cf, cd, (k - v.kw0) * v.nwy + (l - v.lw0), hi, lo);
         }
     }
 }
 
-// lb: tile index, tiles numbered x fastest over tx tiles per row
+// list cells that hold every particle which can reach mesh points [p0, p1) of
+// an axis: those of x / h in [p0 - 1, p1 + 1), widened by the bound e on how
+// far a particle lies outside its cell; c0 in [-nc, nc), n <= nc
+__device__ __forceinline__ void deposit_span(int p0, int p1, double e, const Geo &g, int &c0, int &n) {
+    const int lo = (int)floor(((p0 - 1) * g.h - e) / g.B), hi = (int)floor(((p1 + 1) * g.h + e) / g.B);
+    c0 = lo;
+    n = hi - lo + 1;
+    if (n >= g.nc) {
+        c0 = 0;
+        n = g.nc;
+    }
+}
+
+// lb: tile index, tiles numbered y fastest over a.ty tiles per row
 template <typename R, int SCHEME, bool P2>
-__device__ __forceinline__ void deposit_body(const Geo &g, const DevBufs &d, const DepArgs &a, int lb, int tx) {
+__device__ __forceinline__ void deposit_body(const Geo &g, const DevBufs &d, const DepArgs &a, int lb) {
     extern __shared__ unsigned char smem_raw[];
-    unsigned long long *acc_hi = (unsigned long long *)smem_raw;
-    unsigned long long *acc_lo = acc_hi + a.win_cap;
-    const int acc_n = max(a.win_cap * (std::is_same<R, double>::value ? 2 : 1), a.win_fast);
-    int *seg_q = (int *)(acc_hi + acc_n);
-    int *seg_pre = seg_q + a.seg_cap;       // [seg_cap + 1]
-    int *seg_row = seg_pre + a.seg_cap + 1;
-    unsigned short *seg_of = (unsigned short *)(seg_row + a.seg_cap);  // [DP_SEG_TAB]
-    __shared__ int info[4];
-    __shared__ int wsum[16];
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int nc = g.nc, tc = a.tc;
-    const int cx0 = (lb % tx) * tc, cy0 = (lb / tx) * tc;
-    const int nx = min(tc, nc - cx0), ny = min(tc, nc - cy0);
+    constexpr bool F32 = std::is_same<R, float>::value;
+    unsigned long long *hi = (unsigned long long *)smem_raw, *lo = hi + a.win_cap;
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63;
+    const int nc = g.nc;
+    const int cx0 = (lb / a.ty) * a.tcx, cy0 = (lb % a.ty) * a.tcy;
+    const int nx = min(a.tcx, nc - cx0), ny = min(a.tcy, nc - cy0);
     const unsigned long long step = d.sc->step;
-    // bound on how far a staged particle lies outside its staging cell: the
+    // bound on how far a particle lies outside the cell it is listed in: the
     // excursion of rel outside [0, B] (list order), or during a rebuild the
     // distance of the new positions outside their previous cells
-    __shared__ double e_sh;
-    if (a.slot) {
-        if (tid < 64) {
-            double m = dbits(d.exo[tid * 16]);
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
-            if (tid == 0) e_sh = m;
-        }
-    } else if (tid == 0) {
-        e_sh = dbits(d.sc->exc_bits[step & 1]);
+    double e = a.slot ? dbits(d.exo[lane * 16]) : dbits(d.sc->exc_bits[step & 1]);
+    DepWin v;
+    v.klo = d.own[cx0];
+    v.khi = d.own[cx0 + nx];
+    v.llo = d.own[cy0];
+    v.lhi = d.own[cy0 + ny];
+    v.win = v.khi - v.klo + 4 <= g.Z && v.lhi - v.llo + 4 <= g.Z;
+    const int rim = v.win ? 2 : 0;
+    v.kw0 = v.klo - rim;
+    v.lw0 = v.llo - rim;
+    v.nwx = v.khi - v.klo + 2 * rim;
+    v.nwy = v.lhi - v.llo + 2 * rim;
+    for (int w = tid; w < v.nwx * v.nwy; w += nt) {
+        hi[w] = 0ull;
+        if (!F32) lo[w] = 0ull;
     }
-    const int *st = a.slot ? d.start_old : d.start;
     if (a.reset && lb == 0 && tid == 0) {
         // per-step scalars for the kernels that follow this one
         d.sc->dt_bits = bitsd(g.dt_max);
         d.sc->exc_bits[(step + 1) & 1] = 0ull;
     }
-    if (tid < 4) info[tid] = d.own[tid == 0 ? cx0 : tid == 1 ? cx0 + nx : tid == 2 ? cy0 : cy0 + ny];
-    __syncthreads();
-    const int klo = info[0], khi = info[1], llo = info[2], lhi = info[3];
+    if (a.slot) {
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) e = fmax(e, __shfl_xor(e, o, 64));
+    }
+    e += 1e-9 * g.L;
+    int rx0, nrows, ry0, ncols;
+    deposit_span(v.klo, v.khi, e, g, rx0, nrows);
+    deposit_span(v.llo, v.lhi, e, g, ry0, ncols);
+    // mesh indices of the visited cells' particles (with a margin of one)
+    v.kr0 = (int)floor((rx0 * g.B - e) * g.hinv) - 1;
+    v.nrx = (int)floor(((rx0 + nrows) * g.B + e) * g.hinv) + 2 - v.kr0;
+    v.lr0 = (int)floor((ry0 * g.B - e) * g.hinv) - 1;
+    v.nry = (int)floor(((ry0 + ncols) * g.B + e) * g.hinv) + 2 - v.lr0;
+    v.chk = nrows < nc && ncols < nc && 2 * v.nrx <= g.Z && 2 * v.nry <= g.Z;
+    rx0 = wrapc(rx0, nc);
+    ry0 = wrapc(ry0, nc);
+    const int *st = a.slot ? d.start_old : d.start;
     // FP32: the species charges in fixed point, drho q 2^S (2^S exact)
     const float dqs1 = ((float)g.drho * (float)a.q1) * a.scale_f, dqs2 = ((float)g.drho * (float)a.q2) * a.scale_f;
-    const double e = e_sh + 1e-9 * g.L;
-    int hx = (int)floor((1.5 * g.h + e) / g.B) + 1;
-    if (hx < 1) hx = 1;
-    // staged cells: the tile plus hx halo cells, each distinct cell once (a
-    // halo that would wrap onto the tile itself stages the whole axis)
-    const bool allx = nx + 2 * hx >= nc, ally = ny + 2 * hx >= nc;
-    const int SX = allx ? nc : nx + 2 * hx, SY = ally ? nc : ny + 2 * hx;
-    const int sx0 = allx ? 0 : cx0 - hx, sy0 = ally ? 0 : cy0 - hx;
-    // FP32: the window of mesh points reachable from the staged cells (their
-    // positions lie within e of them; margins cover the index rounding)
-    const int kw0 = (int)floor((sx0 * g.B - e) * g.hinv) - 3, lw0 = (int)floor((sy0 * g.B - e) * g.hinv) - 3;
-    const int nwx = (int)floor(((sx0 + SX) * g.B + e) * g.hinv) + 4 - kw0;
-    const int nwy = (int)floor(((sy0 + SY) * g.B + e) * g.hinv) + 4 - lw0;
-    const bool win = std::is_same<R, float>::value && !allx && !ally && nwx <= g.Z && nwy <= g.Z &&
-                     nwx * nwy <= a.win_fast;
-    const int nwin = win ? nwx * nwy : (khi - klo) * (lhi - llo);
-    for (int w = tid; w < nwin; w += nt) {
-        acc_hi[w] = 0ull;
-        if (std::is_same<R, double>::value) acc_lo[w] = 0ull;
-    }
-    // The list holds the particles in cell order, so the staged cells of one
-    // row (fixed x) are one contiguous list range, or two when the y range
-    // wraps: segments of consecutive list positions.
-    const int ywrap = (sy0 < 0 || sy0 + SY > nc) ? 1 : 0;
-    const int nsr = 1 + ywrap, nseg = SX * nsr;
+    const int *cells = a.slot ? d.cell : d.lcell, *ids = a.slot ? d.pid : d.lpid;
+    const double2 *rels = a.slot ? d.rel : d.lrel;
+    const int yend = ry0 + ncols, ye = min(yend, nc), wrapped = max(yend - nc, 0);
     __syncthreads();  // accumulators cleared before the first atomic
-    if (nseg <= a.seg_cap) {
-        for (int i = tid; i < nseg; i += nt) {
-            const int r = i / nsr, part = i - r * nsr;
-            const int gx = wrap1(sx0 + r, nc), row = gx * nc;
-            int ya, yb;
-            if (!ywrap) {
-                ya = sy0;
-                yb = sy0 + SY;
-            } else if (sy0 < 0) {
-                ya = part == 0 ? sy0 + nc : 0;
-                yb = part == 0 ? nc : sy0 + SY;
-            } else {
-                ya = part == 0 ? sy0 : 0;
-                yb = part == 0 ? nc : sy0 + SY - nc;
-            }
-            const int qa = st[row + ya];
-            seg_q[i] = qa;
-            seg_pre[i] = max(st[row + yb] - qa, 0);
-            seg_row[i] = gx;
-        }
-        __syncthreads();
-        const int total = block_exscan4(seg_pre, nseg, wsum);
-        if (tid == 0) seg_pre[nseg] = total;
-        __syncthreads();
-        // the segment of every staged particle, written once per segment
-        // (a table lookup per particle instead of a binary search)
-        const bool tab = total <= DP_SEG_TAB;
-        if (tab) {
-            for (int i = tid; i < nseg; i += nt)
-                for (int t = seg_pre[i], te = seg_pre[i + 1]; t < te; ++t) seg_of[t] = (unsigned short)i;
-            __syncthreads();
-        }
-        for (int t = tid; t < total; t += nt) {
-            int lo = 0, hi = nseg - 1;  // last segment with seg_pre <= t
-            if (tab)
-                lo = seg_of[t];
-            else
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (seg_pre[mid] <= t) lo = mid;
-                    else hi = mid - 1;
-                }
-            const int q = seg_q[lo] + (t - seg_pre[lo]);
-            int gx, gy;
-            double2 rr;
-            bool s2;
-            if (a.slot) {  // the particle's new cell, not its staging row
-                const int c = d.cell[q];
-                gx = div_nc(c, g);
-                gy = c - gx * nc;
-                rr = d.rel[q];
-                s2 = d.pid[q] >= g.n1;
-            } else {
-                gx = seg_row[lo];
-                gy = d.lcell[q] - gx * nc;
-                rr = d.lrel[q];
-                s2 = (((const unsigned *)d.list)[q] >> 31) != 0;
-            }
-            const float dqs = s2 ? dqs2 : dqs1;
-            if (win)
-                deposit_particle_win<SCHEME, P2>(g, d, dqs, gx, gy, rr, kw0, lw0, nwx, nwy, acc_hi);
-            else
-                deposit_particle<R, SCHEME, P2>(g, d, a, dqs, gx, gy, rr, s2, klo, khi, llo, lhi, acc_hi, acc_lo);
-        }
-    } else {
-        for (int idx = tid; idx < SX * SY; idx += nt) {
-            const int ia = idx / SY, ib = idx - ia * SY;
-            const int gx = wrap1(sx0 + ia, nc), gy = wrap1(sy0 + ib, nc);
-            const int c = gx * nc + gy;
-            for (int q = st[c]; q < st[c + 1]; ++q) {
-                int px = gx, py = gy;
-                double2 rr;
-                bool s2;
-                if (a.slot) {
-                    const int cq = d.cell[q];
-                    px = div_nc(cq, g);
-                    py = cq - px * nc;
-                    rr = d.rel[q];
-                    s2 = d.pid[q] >= g.n1;
-                } else {
-                    rr = d.lrel[q];
-                    s2 = (((const unsigned *)d.list)[q] >> 31) != 0;
-                }
-                const float dqs = s2 ? dqs2 : dqs1;
-                if (win)
-                    deposit_particle_win<SCHEME, P2>(g, d, dqs, px, py, rr, kw0, lw0, nwx, nwy, acc_hi);
-                else
-                    deposit_particle<R, SCHEME, P2>(g, d, a, dqs, px, py, rr, s2, klo, khi, llo, lhi, acc_hi,
-                                                    acc_lo);
-            }
+    for (int r = tid / DP_LANES; r < nrows; r += nt / DP_LANES) {
+        const int *row = st + wrap1(rx0 + r, nc) * nc;
+        const int qa = row[ry0], na = row[ye] - qa, qb = row[0], nb = wrapped ? row[wrapped] - qb : 0;
+        for (int k = tid & (DP_LANES - 1); k < na + nb; k += DP_LANES) {
+            const int q = k < na ? qa + k : qb + (k - na);
+            const int c = cells[q];  // during a rebuild the new cell, not that of the row
+            const double2 rr = rels[q];
+            const bool s2 = ids[q] >= g.n1;
+            const int gx = div_nc(c, g), gy = c - gx * nc;
+            deposit_particle<R, SCHEME, P2>(g, d, a, v, s2 ? dqs2 : dqs1, s2 ? a.q2 : a.q1, gx * g.B + rr.x,
+                                            gy * g.B + rr.y, hi, lo);
         }
     }
     __syncthreads();
+    // the own points, a wave per mesh row
     R *rho = (R *)d.rho;
-    const int nl = lhi - llo, nown = (khi - klo) * nl;
-    // w / nl from a float reciprocal, corrected to the exact quotient
-    // (w < 2^24): an integer division per point cost more than the point
-    const float rnl = nl > 0 ? 1.0f / (float)nl : 0.0f;
-    for (int w = tid; w < nown; w += nt) {
-        int qk = (int)((float)w * rnl);
-        int rl = w - qk * nl;
-        if (rl >= nl) {
-            ++qk;
-            rl -= nl;
-        } else if (rl < 0) {
-            --qk;
-            rl += nl;
+    const int nl = v.lhi - v.llo;
+    for (int k = v.klo + (tid >> 6); k < v.khi; k += nt >> 6) {
+        const int w = (k - v.kw0) * v.nwy + rim;
+        for (int l = lane; l < nl; l += 64) {
+            double val;
+            if (F32)
+                val = (double)(long long)hi[w + l] * a.iscale_f;
+            else
+                val = (double)(long long)hi[w + l] * a.iscale_hi + (double)(long long)lo[w + l] * a.iscale_lo;
+            rho[(size_t)k * g.Z + v.llo + l] = (R)val;
         }
-        const int k = klo + qk, l = llo + rl;
-        double v;
-        if (win) {
-            v = (double)(long long)acc_hi[wrapz<P2>(k - kw0, g.Z) * nwy + wrapz<P2>(l - lw0, g.Z)] * a.iscale_f;
-        } else if (std::is_same<R, float>::value) {
-            v = (double)(long long)acc_hi[w] * a.iscale_f;
-        } else {
-            v = (double)(long long)acc_hi[w] * a.iscale_hi + (double)(long long)acc_lo[w] * a.iscale_lo;
-        }
-        rho[(size_t)k * g.Z + l] = (R)v;
     }
 }
 
@@ -752,7 +679,7 @@ __device__ __forceinline__ void deposit_body(const Geo &g, const DevBufs &d, con
 // scalar registers of the power-of-two path as they were)
 template <typename R, int SCHEME, bool P2>
 __global__ __launch_bounds__(DP_THREADS) void k_deposit(Geo g, DevBufs d, DepArgs a) {
-    deposit_body<R, SCHEME, P2>(g, d, a, blockIdx.x + blockIdx.y * gridDim.x, gridDim.x);
+    deposit_body<R, SCHEME, P2>(g, d, a, blockIdx.x);
 }
 
 // per-step scalar re-arm when no deposit runs (ideal-gas runs), at the start
@@ -1442,9 +1369,9 @@ __global__ __launch_bounds__(DP_THREADS) void kb_deposit(const RepDev *m, const 
             a.reset = 0;
         }
         switch (r.g.scheme) {
-        case 0: deposit_body<R, 0, P2>(r.g, r.d, a, t.y, r.dep_tx); break;
-        case 1: deposit_body<R, 1, P2>(r.g, r.d, a, t.y, r.dep_tx); break;
-        default: deposit_body<R, 2, P2>(r.g, r.d, a, t.y, r.dep_tx); break;
+        case 0: deposit_body<R, 0, P2>(r.g, r.d, a, t.y); break;
+        case 1: deposit_body<R, 1, P2>(r.g, r.d, a, t.y); break;
+        default: deposit_body<R, 2, P2>(r.g, r.d, a, t.y); break;
         }
     });
 }
@@ -1516,9 +1443,8 @@ __global__ __launch_bounds__(256) void kb_sort_cells(const RepDev *m, const int2
 // ------------------------------------------------------------------ launchers
 hipError_t set_kernel_attributes() {
     hipError_t e = fft_set_attributes();
-    // the deposit also has a little static LDS: ask for 128 KB of dynamic LDS
-#define BDK_ATTR_D(K)                                                                          \
-    if (e == hipSuccess) e = hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+#define BDK_ATTR_D(K) \
+    if (e == hipSuccess) e = hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
 #define BDK_ATTR_DQ(Q)                      \
     BDK_ATTR_D((k_deposit<float, 0, Q>))    \
     BDK_ATTR_D((k_deposit<float, 1, Q>))    \
@@ -1557,26 +1483,37 @@ hipError_t launch_wca(bdk_t *h, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Deposit tiling: tile side tc (list cells) such that a tile owns at most
-// about tile_pts x tile_pts mesh points (38 unless a batch tuned it); fixed-point scales chosen so that no sum of
-// N charges can overflow 63 bits.
+// Deposit tiling: tcx x tcy list cells such that a tile owns about tile_pts^2
+// mesh points; fixed-point scales chosen so that no sum of N charges can
+// overflow 63 bits.  Without a batch's choice the side is 38 points, less on
+// meshes below 532 points, so that there are some 200 tiles.  Deposit alone
+// (us) at sides 16 / 24 / 30 / 38 / 46: 128^2 FP64 5.0 / 5.2 / 6.4 / 6.8 / 8.5,
+// 384^2 FP64 6.8 / 6.2 / 5.2 / 6.9 / 7.9, 512^2 6.0 / 6.0 / 6.0 / 6.5 / 9.3,
+// 1024^2 FP64 20.6 / 17.7 / 14.0 / 13.0 / 15.3, 2048^2 45 / 29 / 24.8 / 22.6 /
+// 23.8, 4096^2 156 / 82 / 68 / 53 / 60; square tiles of side 38: 7.0, 8.4, 8.2,
+// 16.9, 25.6 and 66.
 struct DepPlan {
     DepArgs a;
     dim3 grid;
     size_t lds;
 };
 
-static DepPlan dep_plan(const bdk_t *h, int reset, int tile_pts = 38) {
+static DepPlan dep_plan(const bdk_t *h, int reset, int tile_pts = 0) {
     const Geo &g = h->g;
     const bool f64 = h->p.precision == BDK_FP64;
     DepPlan pl;
-    int tc = (int)std::floor(tile_pts * g.h / g.B);
-    if (tc < 1) tc = 1;
-    if (tc > g.nc) tc = g.nc;
-    const int side = (int)std::floor(tc * g.B / g.h) + 2;
-    pl.a.tc = tc;
-    pl.a.win_cap = side * side;
-    pl.a.seg_cap = std::min(2 * (tc + 6), 4 * DP_THREADS);  // block_exscan4 limit
+    if (tile_pts <= 0) tile_pts = std::max(16, std::min(38, g.Z / 14));
+    // 1.6 times the side along y, so that a wave's lanes cover a row of the
+    // tile and the rows of cells make longer ranges, but at most a wave's 64
+    const double py = std::min(62.0, 1.6 * tile_pts), px = (double)tile_pts * tile_pts / py;
+    auto cells = [&](double pts) { return std::max(1, std::min(g.nc, (int)std::floor(pts * g.h / g.B))); };
+    pl.a.tcx = cells(px);
+    pl.a.tcy = cells(py);
+    auto points = [&](int tc) { return (int)std::floor(tc * g.B / g.h) + 2 + 4; };  // with the rim
+    // the window stays below 64 KB of LDS
+    while (pl.a.tcx > 1 && (size_t)points(pl.a.tcx) * points(pl.a.tcy) * (f64 ? 16 : 8) > 64 * 1024) --pl.a.tcx;
+    while (pl.a.tcy > 1 && (size_t)points(pl.a.tcx) * points(pl.a.tcy) * (f64 ? 16 : 8) > 64 * 1024) --pl.a.tcy;
+    pl.a.win_cap = points(pl.a.tcx) * points(pl.a.tcy);
     const double cmax = g.drho * std::max(1.0, std::fabs(g.f2_f1));
     const double nlog = std::log2((double)g.N * cmax + 1.0);
     int s1 = (int)std::floor(62.0 - nlog);
@@ -1591,22 +1528,16 @@ static DepPlan dep_plan(const bdk_t *h, int reset, int tile_pts = 38) {
     pl.a.q1 = 1.0;  // species charges of the capillary deposit (gr:31-547)
     pl.a.q2 = g.f2_f1;
     pl.a.slot = 0;
-    // FP32 stencil window, sized for halos of up to 2 cells and excursions
-    // up to B/4 (larger ones take the bounds-checked path): the staged span
-    // plus the excursion on both sides and the index margins
-    pl.a.win_fast = 0;
     pl.a.scale_f = 1.0f;
     pl.a.iscale_f = 1.0;
     if (!f64) {
-        const int wside = (int)std::ceil((tc + 4.5) * g.B / g.h) + 8;
-        pl.a.win_fast = wside * wside;
         const int sf = (int)std::floor(30.0 - std::log2(cmax));
         pl.a.scale_f = std::ldexp(1.0f, sf);
         pl.a.iscale_f = std::ldexp(1.0, -sf);
     }
-    pl.grid = dim3(nblk(g.nc, tc), nblk(g.nc, tc));
-    pl.lds = (size_t)std::max(pl.a.win_cap * (f64 ? 2 : 1), pl.a.win_fast) * 8 + (size_t)(3 * pl.a.seg_cap + 1) * 4 +
-             (size_t)DP_SEG_TAB * 2;
+    pl.a.ty = (int)nblk(g.nc, pl.a.tcy);
+    pl.grid = dim3(nblk(g.nc, pl.a.tcx) * pl.a.ty);
+    pl.lds = (size_t)pl.a.win_cap * (f64 ? 16 : 8);
     return pl;
 }
 
@@ -1999,7 +1930,6 @@ hipError_t batch_build(const std::vector<bdk_t *> &mem, const BatchTuning &tune,
         r.d = h->d;
         const DepPlan pl = dep_plan(h, 1, tune.dep_tile);
         r.dep = pl.a;
-        r.dep_tx = (int)pl.grid.x;
         bp.dep_lds = std::max(bp.dep_lds, pl.lds);
         const int Z = h->g.Z;
         fft_member(r, Z, ept, bp);
@@ -2007,7 +1937,7 @@ hipError_t batch_build(const std::vector<bdk_t *> &mem, const BatchTuning &tune,
         r.unit = h->p.sigma11_22 == 1.0 && h->p.sigma11_12 == 1.0 && h->p.eps22_11 == 1.0 && h->p.eps12_11 == 1.0;
         const int ad = h->g.adaptive ? 1 : 0;
         const int nb[BS_COUNT] = {(int)nblk(h->g.N, 256), (int)nblk(h->g.ncell, 256), r.scan_nb,
-                                  (int)(pl.grid.x * pl.grid.y), Z / r.rb, (Z / 2) / r.rc, Z / r.rb2,
+                                  (int)pl.grid.x, Z / r.rb, (Z / 2) / r.rc, Z / r.rb2,
                                   ad * (int)nblk(h->g.N, 256), (int)nblk(h->g.N, tune.wca_block)};
         for (int k = 0; k < BS_COUNT; ++k)
             for (int b = 0; b < nb[k]; ++b) maps[k].push_back(make_int2(i, b));
