@@ -24,7 +24,7 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contra
 
 # device sources, compiled side by side and joined (ld -r) into one object,
 # bdk_kernels.hip.o; then the rest
-KERNELS = ("bdk_kernels.hip", "bdk_fft.hip", "bdk_obs.hip")
+KERNELS = ("bdk_kernels.hip", "bdk_fft.hip", "bdk_pairs.hip", "bdk_obs.hip")
 SOURCES = KERNELS + ("bdk_noalloc.hip", "bdk_api.cpp", "bdk_serve.cpp")
 
 

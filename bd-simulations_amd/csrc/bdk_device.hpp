@@ -108,13 +108,36 @@ __device__ __forceinline__ double2 philox_noise_f32(unsigned long long seed, uin
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own
 // L2.  Renumbered so that every XCD runs one contiguous range of the logical
 // grid, neighbouring tiles (whose inputs overlap) share an L2.
-__device__ __forceinline__ int xcd_block(int on) {
-    const int b = blockIdx.x + blockIdx.y * gridDim.x;
+__device__ __forceinline__ int xcd_of(int b, int nb, int on) {  // block b of nb
     if (!on) return b;
-    const int nb = gridDim.x * gridDim.y;
     const int x = b & 7, i = b >> 3, base = nb >> 3, rem = nb & 7;
     return x < rem ? x * (base + 1) + i : rem * (base + 1) + (x - rem) * base + i;
 }
+__device__ __forceinline__ int xcd_block(int on) {
+    return xcd_of(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y, on);
+}
+
+// Two kinds of work in one launch: na blocks of the first and nb of the
+// second, interleaved evenly in groups of eight, so that block i of either
+// kind runs on XCD i mod 8 as in a launch of its own.
+struct PairGrid {
+    int na, nb;
+    unsigned long long share;  // groups of the first kind per group, 32 fractional bits
+    PairGrid(int na_, int nb_) : na(na_), nb(nb_) {
+        const unsigned long long ga = (na + 7) / 8, all = groups();
+        share = ((ga << 32) + all - 1) / all;
+    }
+    unsigned long long groups() const { return (na + 7) / 8 + (nb + 7) / 8; }
+    unsigned blocks() const { return (unsigned)(8 * groups()); }
+    // the block's kind and number there; false: nothing to do
+    __device__ __forceinline__ bool mine(bool &first, int &i) const {
+        const unsigned long long grp = blockIdx.x >> 3;
+        const int a0 = (int)((grp * share) >> 32), a1 = (int)(((grp + 1) * share) >> 32);
+        first = a1 > a0;
+        i = (first ? a0 : (int)grp - a0) * 8 + (int)(blockIdx.x & 7);
+        return i < (first ? na : nb);
+    }
+};
 
 // ------------------------------------------------------------------ geometry
 __device__ __forceinline__ int wrapc(int u, int n) {

@@ -24,60 +24,6 @@
 
 namespace bdkx {
 
-constexpr int FFT_MAX_THREADS = 512;  // power-of-two passes
-
-// G(j, m') = 1/((lap[j] + lap[m']) + 1/lambda^2) (dm:585-593, dm:1384-1394)
-template <typename R> __device__ __forceinline__ R green(R lapj, R lapm, bool zero, R lam2inv) {
-    if (zero) return (R)0.0;
-    if (sizeof(R) == 4)  // FP32: the hardware reciprocal (1 ulp) instead of a correctly rounded division
-        return (R)__builtin_amdgcn_rcpf((float)((lapj + lapm) + lam2inv));
-    return (R)1.0 / ((lapj + lapm) + lam2inv);
-}
-
-// spectral factors of one (j, m') pair: gx = sq[j] G / Z / Z, gy = sq[m'] G / Z / Z
-template <typename R>
-__device__ __forceinline__ void symbols(int j, int mm, const Geo &g, const R *sq, const R *lap, R &gx, R &gy) {
-    const R G = green<R>(lap[j], lap[mm], j == 0 && mm == 0 && g.zero_mode_g, (R)g.lam2inv);
-    // x / Z / Z == x * 2^(-2 log2 Z) exactly where Z is a power of two
-    const R izz = (R)1.0 / ((R)g.Z * (R)g.Z);
-    gx = sq[j] * G * izz;
-    gy = sq[mm] * G * izz;
-}
-
-// The packed (DC, Nyquist) column at j, from P = S[j] and Q = S[Z - j]:
-// i g(., 0) S_dc + i (i g(., Z/2) S_ny) for x and y
-template <typename R, typename C>
-__device__ __forceinline__ void packed_column(int j, C P, C Q, const Geo &g, const R *sq, const R *lap, C &fx, C &fy) {
-    const C Sdc = cscale(cadd(P, cconj(Q)), (R)0.5);
-    const C Sny = cmul_mi(cscale(csub(P, cconj(Q)), (R)0.5));
-    R gx0, gy0, gxN, gyN;
-    symbols<R>(j, 0, g, sq, lap, gx0, gy0);
-    symbols<R>(j, g.Z >> 1, g, sq, lap, gxN, gyN);
-    fx = cadd(cmul_i(cscale(Sdc, gx0)), cmul_i(cmul_i(cscale(Sny, gxN))));
-    fy = cadd(cmul_i(cscale(Sdc, gy0)), cmul_i(cmul_i(cscale(Sny, gyN))));
-}
-
-// half spectrum X[m] of a real row from its packed transform: a = z[m],
-// b = z[n - m], w = exp(-2 pi i m / Z)
-template <typename C> __device__ __forceinline__ C split_real(C a, C b, C w) {
-    using R = decltype(C::x);
-    const C bc = cconj(b);
-    const C E = cscale(cadd(a, bc), (R)0.5);
-    const C O = cmul_mi(cscale(csub(a, bc), (R)0.5));
-    return cadd(E, cmul(w, O));
-}
-
-// ------------------------------------------------------------------ power-of-two meshes
-template <typename R, int LOGZ> struct P2Pass {
-    using C = typename V2<R>::T;
-    static constexpr int Z = 1 << LOGZ, E = fft_ept(Z, sizeof(R) == 4);
-    static constexpr int ER = E < Z / 2 ? E : Z / 2;  // of the r2c rows
-    static constexpr int per = 256 / (int)sizeof(C);  // elements that fill all LDS banks once
-    using Row = RowFft<R, LOGZ - 1, ER, LOGZ>;        // r2c rows: Z/2 complex points
-    using Col = RowFft<R, LOGZ, E, LOGZ>;             // columns and c2r rows
-    static constexpr int col_stride = 2 * (Z + Z / E) + 2;
-};
-
 // LDS bytes of a block of `rows` rows; pass 0 r2c, 1 columns, 2 c2r
 template <typename R, int LOGZ> static size_t p2_lds(int pass, int rows) {
     using P = P2Pass<R, LOGZ>;
@@ -89,170 +35,6 @@ template <typename R, int LOGZ> static size_t p2_lds(int pass, int rows) {
 template <typename R, int LOGZ> static int p2_threads(int pass, int rows) {
     using P = P2Pass<R, LOGZ>;
     return rows * (pass == 0 ? P::Row::T : P::Col::T);
-}
-
-// Row r2c: rows k0..k0+rows-1 of the real mesh -> half spectrum X[m], m<Z/2,
-// with X[0] packing (DC, Nyquist) (both real), written transposed:
-// ht[m*Z + k].  Length-Z/2 complex transform of (x[2n], x[2n+1]) + split.
-// The stores take the rows of the block together (rows x 8 or 16 bytes).
-template <typename R, int LOGZ>
-__device__ __forceinline__ void r2c_p2(const R *__restrict__ rho, typename V2<R>::T *__restrict__ ht,
-                                       const typename V2<R>::T *__restrict__ tw, int rows, int blk) {
-    using P = P2Pass<R, LOGZ>;
-    using F = typename P::Row;
-    using C = typename P::C;
-    constexpr int Z = P::Z, E = P::ER, N = F::N, T = F::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    const int tid = threadIdx.x, row = tid / T, t = tid % T, k0 = blk * rows, na = rows * T;
-    const int stride = row_stride(N, E, rows, P::per), lrows = __ffs(rows) - 1;
-    C *sr = s + row * stride;
-    const bool act = tid < na;
-    if (act || !F::WAVE) {
-        const C *p = (const C *)(rho + (size_t)(k0 + row) * Z) + t;
-        C v[1][E];
-#pragma unroll
-        for (int u = 0; u < E; ++u) v[0][u] = p[T * u];
-        F f;
-        f.load(tw, t);
-        f.template run<1, false, true>(v, sr, t);
-        if (F::NP > 1) row_sync<F::WAVE>();
-#pragma unroll
-        for (int u = 0; u < E; ++u) sr[T % E == 0 ? lpe<E>(t) + u * lpe<E>(T) : lpe<E>(t + T * u)] = v[0][u];
-    }
-    C w[E];
-#pragma unroll
-    for (int u = 0; u < E; ++u) w[u] = tw[((tid + u * na) >> lrows) & (N - 1)];
-    __syncthreads();
-    if (!act) return;
-#pragma unroll
-    for (int u = 0; u < E; ++u) {
-        const int i = tid + u * na, m = i >> lrows, r = i & (rows - 1);
-        const C *p = s + r * stride;
-        const C a = p[lpe<E>(m)];
-        C o;
-        if (m == 0)
-            o = cm<C>(a.x + a.y, a.x - a.y);
-        else
-            o = split_real(a, p[lpe<E>(N - m)], w[u]);
-        ht[(size_t)m * Z + k0 + r] = o;
-    }
-}
-
-// Column pass: rows m0..m0+rows-1 of ht (length Z along x), forward
-// transform, times i*gx and i*gy, inverse transform of both together, out
-// gt[m*Z+k] = (Fx, Fy).  The spectrum stays in registers in between.
-template <typename R, int LOGZ>
-__device__ __forceinline__ void col_p2(const typename V2<R>::T *__restrict__ ht, typename V4<R>::T *__restrict__ gt,
-                                       const typename V2<R>::T *__restrict__ tw, const R *__restrict__ sq,
-                                       const R *__restrict__ lap, const Geo &g, int rows, int blk) {
-    using P = P2Pass<R, LOGZ>;
-    using F = typename P::Col;
-    using C = typename P::C;
-    using C4 = typename V4<R>::T;
-    constexpr int Z = P::Z, E = P::E, T = F::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    const int tid = threadIdx.x, row = tid / T, t = tid % T, m0 = blk * rows, m = m0 + row;
-    const bool act = tid < rows * T;
-    C *sr = s + row * P::col_stride;
-    F f;
-    C v[1][E], xy[2][E];
-    if (act || !F::WAVE) {
-        const C *p = ht + (size_t)m * Z + t;
-#pragma unroll
-        for (int u = 0; u < E; ++u) v[0][u] = p[T * u];
-        f.load(tw, t);
-        f.template run<1, false, true>(v, sr, t);
-    }
-    if (m0 == 0) {
-        // the packed column pairs j with Z - j, held by other threads
-        __syncthreads();
-        if (act && m == 0)
-#pragma unroll
-            for (int u = 0; u < E; ++u) sr[t + T * u] = v[0][u];
-        __syncthreads();
-        if (act && m == 0)
-#pragma unroll
-            for (int u = 0; u < E; ++u) {
-                const int j = t + T * u;
-                packed_column<R, C>(j, v[0][u], sr[(Z - j) & (Z - 1)], g, sq, lap, xy[0][u], xy[1][u]);
-            }
-        __syncthreads();
-    }
-    if (!act && F::WAVE) return;
-    if (m != 0) {
-        const R sqm = sq[m], lapm = lap[m], l2 = (R)g.lam2inv, izz = (R)1.0 / ((R)Z * (R)Z);
-#pragma unroll
-        for (int u = 0; u < E; ++u) {
-            const int j = t + T * u;
-            const R G = green<R>(lap[j], lapm, false, l2);
-            const R gx = sq[j] * G * izz, gy = sqm * G * izz;
-            const C S = v[0][u];
-            xy[0][u] = cm<C>(-gx * S.y, gx * S.x);
-            xy[1][u] = cm<C>(-gy * S.y, gy * S.x);
-        }
-    }
-    f.template run<2, true, F::NP == 1>(xy, sr, t);
-    C4 *o = gt + (size_t)m * Z + t;
-#pragma unroll
-    for (int u = 0; u < E; ++u) {
-        C4 q;
-        q.x = xy[0][u].x;
-        q.y = xy[0][u].y;
-        q.z = xy[1][u].x;
-        q.w = xy[1][u].y;
-        o[T * u] = q;
-    }
-}
-
-// Row c2r of the two real signals Fx, Fy: rows k0..k0+rows-1, spectrum
-// C[m] = X[m] + i Y[m] completed by Hermitian symmetry, inverse transform of
-// length Z, out fmesh[k*Z + l] = (Re, Im) = (Fx, Fy).
-template <typename R, int LOGZ>
-__device__ __forceinline__ void c2r_p2(const typename V4<R>::T *__restrict__ gt, typename V2<R>::T *__restrict__ fm,
-                                       const typename V2<R>::T *__restrict__ tw, int rows, int blk) {
-    using P = P2Pass<R, LOGZ>;
-    using F = typename P::Col;
-    using C = typename P::C;
-    using C4 = typename V4<R>::T;
-    constexpr int Z = P::Z, E = P::E, T = F::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    const int tid = threadIdx.x, row = tid / T, t = tid % T, k0 = blk * rows, na = rows * T;
-    const int stride = row_stride(Z, E, rows, P::per), lrows = __ffs(rows) - 1;
-    const bool act = tid < na;
-    F f;
-    if (act) {
-        C4 q[E / 2];
-#pragma unroll
-        for (int u = 0; u < E / 2; ++u) {
-            const int i = tid + u * na;
-            q[u] = gt[(size_t)(i >> lrows) * Z + k0 + (i & (rows - 1))];
-        }
-        f.load(tw, t);
-#pragma unroll
-        for (int u = 0; u < E / 2; ++u) {
-            const int i = tid + u * na, m = i >> lrows;
-            C *p = s + (i & (rows - 1)) * stride;
-            if (m == 0) {
-                p[0] = cm<C>(q[u].x, q[u].z);
-                p[lpe<E>(Z / 2)] = cm<C>(q[u].y, q[u].w);
-            } else {
-                p[lpe<E>(m)] = cm<C>(q[u].x - q[u].w, q[u].y + q[u].z);
-                p[lpe<E>(Z - m)] = cm<C>(q[u].x + q[u].w, -q[u].y + q[u].z);
-            }
-        }
-    }
-    __syncthreads();
-    if (!act && F::WAVE) return;
-    C *sr = s + row * stride;
-    C v[1][E];
-    F::template gather<1>(v, sr, t);
-    f.template run<1, true, false>(v, sr, t);
-    C *o = fm + (size_t)(k0 + row) * Z + t;
-#pragma unroll
-    for (int u = 0; u < E; ++u) o[T * u] = v[0][u];
 }
 
 template <typename R, int LOGZ>
@@ -279,124 +61,6 @@ __global__ __launch_bounds__(FFT_MAX_THREADS) void k_c2r_rows(const typename V4<
                                                               int remap, Geo g, DevBufs d, int end_step) {
     if (end_step && blockIdx.x == 0) step_end_body(g, d);
     c2r_p2<R, LOGZ>(gt, fm, tw, rows, xcd_block(remap));
-}
-
-// ------------------------------------------------------------------ other meshes
-// Rows in LDS: the block's rows are read, transformed in place and written.
-template <typename R, int EPT>
-__device__ __forceinline__ void r2c_any(const R *__restrict__ rho, typename V2<R>::T *__restrict__ ht,
-                                        const typename V2<R>::T *__restrict__ tw, int Z, int RB, int stride, int blk) {
-    using C = typename V2<R>::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int n = Z >> 1;
-    const Dv dn(n), drb(RB);
-    const int k0 = blk * RB;
-    for (int idx = tid; idx < RB * n; idx += nt) {
-        const int row = dn.q(idx), m = dn.r(idx);
-        s[row * stride + lp(m)] = ((const C *)(rho + (size_t)(k0 + row) * Z))[m];
-    }
-    __syncthreads();
-    lds_fft_g<R, EPT>(s, n, RB, stride, tw, Z, false);
-    for (int idx = tid; idx < RB * n; idx += nt) {
-        const int m = drb.q(idx), row = drb.r(idx);
-        const C *p = s + row * stride;
-        const C a = p[lp(m)];
-        ht[(size_t)m * Z + k0 + row] = m == 0 ? cm<C>(a.x + a.y, a.x - a.y) : split_real(a, p[lp(n - m)], tw[m]);
-    }
-}
-
-template <typename R, int EPT>
-__device__ __forceinline__ void col_any(const typename V2<R>::T *__restrict__ ht, typename V4<R>::T *__restrict__ gt,
-                                        const typename V2<R>::T *__restrict__ tw, const R *__restrict__ sq,
-                                        const R *__restrict__ lap, const Geo &g, int RC, int stride, int blk) {
-    using C = typename V2<R>::T;
-    using C4 = typename V4<R>::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    C *sB = s + RC * stride;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int Z = g.Z, Zh = Z >> 1;
-    const Dv dz(Z);
-    const int m0 = blk * RC;
-    for (int idx = tid; idx < RC * Z; idx += nt) {
-        const int row = dz.q(idx), k = dz.r(idx);
-        s[row * stride + lp(k)] = ht[(size_t)(m0 + row) * Z + k];
-    }
-    __syncthreads();
-    lds_fft_g<R, EPT>(s, Z, RC, stride, tw, Z, false);
-    for (int idx = tid; idx < RC * Z; idx += nt) {
-        const int row = dz.q(idx), j = dz.r(idx);
-        const int m = m0 + row;
-        if (m == 0) {
-            // packed (DC, Nyquist) column: pairs (j, Z-j) by one thread
-            if (j > Zh) continue;
-            const int jn = j == 0 ? 0 : Z - j;
-            const C P = s[lp(j)], Q = s[lp(jn)];
-            C fx, fy, gx, gy;
-            packed_column<R, C>(j, P, Q, g, sq, lap, fx, fy);
-            packed_column<R, C>(jn, Q, P, g, sq, lap, gx, gy);
-            s[lp(j)] = fx;
-            sB[lp(j)] = fy;
-            if (jn != j) {
-                s[lp(jn)] = gx;
-                sB[lp(jn)] = gy;
-            }
-        } else {
-            R gx, gy;
-            symbols<R>(j, m, g, sq, lap, gx, gy);
-            const int o = row * stride + lp(j);
-            const C S = s[o];
-            s[o] = cm<C>(-gx * S.y, gx * S.x);
-            sB[o] = cm<C>(-gy * S.y, gy * S.x);
-        }
-    }
-    __syncthreads();
-    lds_fft_g<R, EPT>(s, Z, 2 * RC, stride, tw, Z, true);
-    for (int idx = tid; idx < RC * Z; idx += nt) {
-        const int row = dz.q(idx), k = dz.r(idx);
-        const int so = row * stride + lp(k);
-        const C a = s[so], b = sB[so];
-        C4 o;
-        o.x = a.x;
-        o.y = a.y;
-        o.z = b.x;
-        o.w = b.y;
-        gt[(size_t)(m0 + row) * Z + k] = o;
-    }
-}
-
-template <typename R, int EPT>
-__device__ __forceinline__ void c2r_any(const typename V4<R>::T *__restrict__ gt, typename V2<R>::T *__restrict__ fm,
-                                        const typename V2<R>::T *__restrict__ tw, int Z, int RB2, int stride,
-                                        int blk) {
-    using C = typename V2<R>::T;
-    using C4 = typename V4<R>::T;
-    extern __shared__ unsigned char smem_raw[];
-    C *s = (C *)smem_raw;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int Zh = Z >> 1;
-    const Dv dz(Z), drb(RB2);
-    const int k0 = blk * RB2;
-    for (int idx = tid; idx < RB2 * Zh; idx += nt) {
-        const int m = drb.q(idx), row = drb.r(idx);
-        const C4 v = gt[(size_t)m * Z + k0 + row];
-        C *p = s + row * stride;
-        if (m == 0) {
-            p[0] = cm<C>(v.x, v.z);
-            p[lp(Zh)] = cm<C>(v.y, v.w);
-        } else {
-            p[lp(m)] = cm<C>(v.x - v.w, v.y + v.z);
-            p[lp(Z - m)] = cm<C>(v.x + v.w, -v.y + v.z);
-        }
-    }
-    __syncthreads();
-    lds_fft_g<R, EPT>(s, Z, RB2, stride, tw, Z, true);
-    for (int idx = tid; idx < RB2 * Z; idx += nt) {
-        const int row = dz.q(idx), l = dz.r(idx);
-        fm[(size_t)(k0 + row) * Z + l] = s[row * stride + lp(l)];
-    }
 }
 
 template <typename R, int EPT>
@@ -427,19 +91,6 @@ __global__ __launch_bounds__(FFT_THREADS) void k_c2r_any(const typename V4<R>::T
 // ------------------------------------------------------------------ batched
 // One map entry per block; the size is the member's, so one launch serves
 // every power-of-two mesh with the same points per thread.
-#define BDK_LOGZ_LOW(CALL) \
-    case 3: CALL(3); break;   \
-    case 4: CALL(4); break;   \
-    case 5: CALL(5); break;   \
-    case 6: CALL(6); break;   \
-    case 7: CALL(7); break;   \
-    case 8: CALL(8); break;   \
-    case 9: CALL(9); break;
-#define BDK_LOGZ_HIGH(CALL) \
-    case 10: CALL(10); break; \
-    case 11: CALL(11); break; \
-    default: CALL(12); break;
-
 // H: FP32 meshes of 1024 points and more (16 points per thread)
 template <typename R, bool P, bool H>
 __global__ __launch_bounds__(FFT_MAX_THREADS) void kb_r2c(const RepDev *m, const int2 *map, int nmap) {
@@ -598,13 +249,30 @@ static AnyCfg any_cfg(int pass, int Z, size_t csz) {
     return c;
 }
 
+FftLaunch fft_launch(const bdk_t *h, int pass) {
+    const bool f32 = h->p.precision != BDK_FP64;
+    const int Z = h->g.Z;
+    FftLaunch l = {};
+    if (zp2(Z)) {
+        l.rows = p2_rows(f32, Z, pass);
+        l.threads = std::max(64, p2_block(f32, Z, pass, l.rows));
+        l.lds = p2_lds_bytes(f32, Z, pass, l.rows);
+    } else {
+        const AnyCfg c = any_cfg(pass, Z, f32 ? 8 : 16);
+        l = {c.rows, c.threads, 0, c.ept, c.stride, c.lds};
+    }
+    l.blocks = pass_rows(pass, Z) / l.rows;
+    return l;
+}
+
 template <typename R> static void launch_pass_p2(bdk_t *h, int pass, hipStream_t st, int end_step) {
     using C = typename V2<R>::T;
     using C4 = typename V4<R>::T;
     constexpr bool f32 = sizeof(R) == 4;
-    const int Z = h->g.Z, rows = p2_rows(f32, Z, pass);
-    const dim3 grid(pass_rows(pass, Z) / rows), blk(std::max(64, p2_block(f32, Z, pass, rows)));
-    const size_t lds = p2_lds_bytes(f32, Z, pass, rows);
+    const FftLaunch l = fft_launch(h, pass);
+    const int rows = l.rows;
+    const dim3 grid(l.blocks), blk(l.threads);
+    const size_t lds = l.lds;
     const R *sq = f32 ? (const R *)h->d.sqf : (const R *)h->d.sq, *lap = f32 ? (const R *)h->d.lapf : (const R *)h->d.lap;
     const C *tw = (const C *)h->d.tw;
 #define R2C(LZ) \
@@ -630,8 +298,8 @@ template <typename R> static void launch_pass_any(bdk_t *h, int pass, hipStream_
     using C = typename V2<R>::T;
     using C4 = typename V4<R>::T;
     const int Z = h->g.Z;
-    const AnyCfg c = any_cfg(pass, Z, sizeof(C));
-    const dim3 grid(pass_rows(pass, Z) / c.rows), blk(c.threads);
+    const FftLaunch c = fft_launch(h, pass);
+    const dim3 grid(c.blocks), blk(c.threads);
     const R *sq = sizeof(R) == 4 ? (const R *)h->d.sqf : (const R *)h->d.sq;
     const R *lap = sizeof(R) == 4 ? (const R *)h->d.lapf : (const R *)h->d.lap;
     const C *tw = (const C *)h->d.tw;

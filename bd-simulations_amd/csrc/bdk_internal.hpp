@@ -225,6 +225,17 @@ hipError_t launch_force_by_id(bdk_t *h, const void *f, double2 *out);  // list-o
 hipError_t launch_zero_ints(int *p, int n, hipStream_t st);
 hipError_t launch_rearm(bdk_t *h);                // per-step scalars when no deposit runs
 size_t deposit_lds_bytes(const bdk_t *h);          // LDS of one deposit block
+// the deposit beside a rebuild, as a part of a paired launch
+struct DepLaunch {
+    DepArgs a;
+    int blocks;
+    size_t lds;
+};
+DepLaunch deposit_launch(const bdk_t *h);
+// the mesh chain and the list rebuild after the update, paired stage by stage
+bool pairs_apply(const bdk_t *h);
+hipError_t launch_pairs(bdk_t *h);
+hipError_t pairs_set_attributes();
 hipError_t launch_fft(bdk_t *h);                  // rho -> fmesh (r2c, multiply, c2r)
 // 0 r2c rows, 1 columns, 2 c2r rows (end_step: the c2r pass also ends the step)
 hipError_t launch_fft_pass(bdk_t *h, int pass, hipStream_t st = nullptr, int end_step = 0);
