@@ -100,6 +100,7 @@ struct DevBufs {
     unsigned long long *dts = nullptr; // [64 x 16] adaptive dt: minima of the candidates by block (double bits;
                                        // all ones = none), reduced by the step's update (by k_dt_fold for
                                        // bdk_optimal_dt), re-armed at the end of the step
+    double *hdt = nullptr;    // adaptive dt of single steps: host memory that the update writes dt to (else null)
     double *dtlog = nullptr;  // [kDtLog] adaptive dt of step s at s mod kDtLog (written by the update)
     int *list = nullptr;      // [N] slots grouped by cell (slot | species << 31)
     // the state in list order (k_fill): cell, rel and particle id of list entry q
@@ -203,6 +204,8 @@ struct bdk {
     bdkx::StepInfoDev *info_dev = nullptr;  // step counters (bdk_step_info), allocated on first use
     void *ws = nullptr;            // scratch of the observables (bdk_api.cpp: Scratch), kept up to kKeepScratch
     size_t ws_cap = 0;
+    double *hdt = nullptr;         // pinned host copy of a single step's adaptive dt, and the event after its update
+    hipEvent_t ev_dt = nullptr;
     char *pin = nullptr;           // pinned host staging (bdk_api.cpp: pinned), at most kPinned bytes
     size_t pin_cap = 0;
     bdkx::PosWriter writer;
@@ -273,7 +276,7 @@ struct FtPlan {
 };
 FtPlan ftrho_plan(const bdk_t *h, int qbins);
 hipError_t launch_ftrho(bdk_t *h, const FtPlan &f, int qbins, int species, double dq, double *part, double *out);
-hipError_t set_kernel_attributes();
+hipError_t set_kernel_attributes(int dev);
 // device address of the allocation-free entry's scratch array on device
 // `dev` (current), looked up once per device (bdk_noalloc.hip)
 hipError_t noalloc_setup(int dev);
@@ -311,8 +314,9 @@ struct StepInfoDev {
 // needed once after the state was set from the host; every step leaves the
 // forces of its new state behind (h->forces_ready).
 hipError_t enqueue_forces(bdk_t *h, std::vector<std::string> *names = nullptr, std::vector<hipEvent_t> *ev = nullptr);
-// One step from a state whose forces are ready.
+// One step from a state whose forces are ready.  dt_known (if non-null) is
+// recorded once the update has taken the step's dt.
 hipError_t enqueue_step(bdk_t *h, std::vector<std::string> *names, std::vector<hipEvent_t> *ev,
-                        StepInfoDev *info = nullptr);
+                        StepInfoDev *info = nullptr, hipEvent_t dt_known = nullptr);
 
 }  // namespace bdkx

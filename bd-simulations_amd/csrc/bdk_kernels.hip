@@ -33,6 +33,8 @@
 // build; cell indices are therefore bit-exact.
 #pragma clang fp contract(off)
 
+#include <mutex>
+
 #include "bdk_device.hpp"
 #include "bdk_fft.hpp"
 #include "bdk_particles.hpp"
@@ -421,6 +423,7 @@ __device__ __forceinline__ void update_body(const Geo &g, const DevBufs &d, int 
         if (blk == 0 && threadIdx.x == 0) {
             d.sc->dt_bits = bitsd(dt);
             d.dtlog[d.sc->step & (kDtLog - 1)] = dt;
+            if (d.hdt) __hip_atomic_store(d.hdt, dt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
     double m = 0.0;
@@ -688,7 +691,13 @@ __global__ __launch_bounds__(256) void kb_sort_cells(const RepDev *m, const int2
 }
 
 // ------------------------------------------------------------------ launchers
-hipError_t set_kernel_attributes() {
+// Dynamic LDS above the default limit, once per device: some 200 kernels, 1 us
+// each, which every bdk_create paid.
+hipError_t set_kernel_attributes(int dev) {
+    static std::mutex mu;
+    static std::vector<char> done;
+    std::lock_guard<std::mutex> lock(mu);
+    if (dev < (int)done.size() && done[dev]) return hipSuccess;
     hipError_t e = fft_set_attributes();
     if (e == hipSuccess) e = pairs_set_attributes();
 #define BDK_ATTR_D(K) \
@@ -708,6 +717,10 @@ hipError_t set_kernel_attributes() {
     BDK_ATTR_DQ(false)
 #undef BDK_ATTR_DQ
 #undef BDK_ATTR_D
+    if (e == hipSuccess) {
+        if (dev >= (int)done.size()) done.resize(dev + 1, 0);
+        done[dev] = 1;
+    }
     return e;
 }
 
@@ -1085,7 +1098,7 @@ hipError_t enqueue_forces(bdk_t *h, std::vector<std::string> *names, std::vector
 // joined.  The new state leaves with its forces ready.  Without forces (an
 // ideal gas) the scan ends the step.
 hipError_t enqueue_step(bdk_t *h, std::vector<std::string> *names, std::vector<hipEvent_t> *ev,
-                        StepInfoDev *info) {
+                        StepInfoDev *info, hipEvent_t dt_known) {
     Marks m{h, names, ev};
     if (ev) m.mark("begin");
     const bool kap = !h->g.idgas;
@@ -1114,6 +1127,7 @@ hipError_t enqueue_step(bdk_t *h, std::vector<std::string> *names, std::vector<h
         m.chk(launch_update(h, kap ? 1 : 0));
     }
     m.mark("k_update");
+    if (dt_known) m.chk(hipEventRecord(dt_known, h->stream));
     if (info) hipLaunchKernelGGL(k_info_moves, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d, info);
     if (kap && !ev && pairs_apply(h)) {
         m.chk(launch_pairs(h));
