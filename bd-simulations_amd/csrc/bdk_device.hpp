@@ -379,9 +379,14 @@ static __device__ int block_exscan4(int *a, int n, int *wsum) {
 // P (persistent) selects the form at compile time: without it a kernel
 // handles exactly its own entry (no loop, so the code and its register use
 // are those of a plain one-entry kernel).
-template <bool P, bool SYNC, typename F> __device__ __forceinline__ void for_entries(int nmap, F &&f) {
+// XCD: the entries in contiguous ranges per XCD, as the single-simulation
+// kernels run, so a member's blocks share an L2 between the particle stages
+// and the FFT passes. 32 members of 16,384 particles on 512^2: 176 -> 167 us
+// per step. The stages whose single kernels run in plain order (scan, sort,
+// column pass) or order their tiles themselves (deposit) pass false.
+template <bool P, bool SYNC, bool XCD, typename F> __device__ __forceinline__ void for_entries(int nmap, F &&f) {
     if (!P) {
-        f((int)blockIdx.x);
+        f(XCD ? xcd_of((int)blockIdx.x, nmap, 1) : (int)blockIdx.x);
         return;
     }
     for (int e = blockIdx.x; e < nmap; e += gridDim.x) {

@@ -95,7 +95,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_c2r_any(const typename V4<R>::T
 template <typename R, bool P, bool H>
 __global__ __launch_bounds__(FFT_MAX_THREADS) void kb_r2c(const RepDev *m, const int2 *map, int nmap) {
     using C = typename V2<R>::T;
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, true>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
 #define CALL(LZ) r2c_p2<R, LZ>((const R *)r.d.rho, (C *)r.d.ht, (const C *)r.d.tw, r.rb, t.y)
@@ -114,7 +114,7 @@ template <typename R, bool P, bool H>
 __global__ __launch_bounds__(FFT_MAX_THREADS) void kb_col(const RepDev *m, const int2 *map, int nmap) {
     using C = typename V2<R>::T;
     using C4 = typename V4<R>::T;
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, false>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         const R *sq = std::is_same<R, float>::value ? (const R *)r.d.sqf : (const R *)r.d.sq;
@@ -135,7 +135,7 @@ template <typename R, bool P, bool H>
 __global__ __launch_bounds__(FFT_MAX_THREADS) void kb_c2r(const RepDev *m, const int2 *map, int nmap, int end_step) {
     using C = typename V2<R>::T;
     using C4 = typename V4<R>::T;
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, true>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         if (end_step && t.y == 0) step_end_body(r.g, r.d);
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(FFT_MAX_THREADS) void kb_c2r(const RepDev *m, const
 template <typename R, int EPT, bool P>
 __global__ __launch_bounds__(FFT_THREADS) void kb_r2c_any(const RepDev *m, const int2 *map, int nmap) {
     using C = typename V2<R>::T;
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, true>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         r2c_any<R, EPT>((const R *)r.d.rho, (C *)r.d.ht, (const C *)r.d.tw, r.g.Z, r.rb, r.sR1, t.y);
@@ -165,7 +165,7 @@ template <typename R, int EPT, bool P>
 __global__ __launch_bounds__(FFT_THREADS) void kb_col_any(const RepDev *m, const int2 *map, int nmap) {
     using C = typename V2<R>::T;
     using C4 = typename V4<R>::T;
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, false>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         const R *sq = std::is_same<R, float>::value ? (const R *)r.d.sqf : (const R *)r.d.sq;
@@ -178,7 +178,7 @@ template <typename R, int EPT, bool P>
 __global__ __launch_bounds__(FFT_THREADS) void kb_c2r_any(const RepDev *m, const int2 *map, int nmap, int end_step) {
     using C = typename V2<R>::T;
     using C4 = typename V4<R>::T;
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, true>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         if (end_step && t.y == 0) step_end_body(r.g, r.d);

@@ -589,7 +589,7 @@ __global__ __launch_bounds__(512) void kb_wca(const RepDev *m, const int2 *map, 
     __shared__ float2 sp[S];
     __shared__ unsigned se[S];
     __shared__ int hdr[8];
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, true>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         if (std::is_same<R, float>::value && r.g.fast_wca) {
@@ -610,7 +610,7 @@ __global__ __launch_bounds__(512) void kb_wca(const RepDev *m, const int2 *map, 
 
 template <typename R, bool P, bool P2>
 __global__ __launch_bounds__(DP_THREADS) void kb_deposit(const RepDev *m, const int2 *map, int nmap, int slot) {
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, false>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         DepArgs a = r.dep;
@@ -631,7 +631,7 @@ __global__ __launch_bounds__(DP_THREADS) void kb_deposit(const RepDev *m, const 
 // candidates, as their single-simulation steps do.
 template <typename R, bool P, bool P2>
 __global__ __launch_bounds__(256) void kb_update(const RepDev *m, const int2 *map, int nmap) {
-    for_entries<P, false>(nmap, [&](int e_) {
+    for_entries<P, false, true>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         if (r.g.adaptive) {
@@ -654,7 +654,7 @@ __global__ __launch_bounds__(256) void kb_update(const RepDev *m, const int2 *ma
 // particle blocks only)
 template <typename R, bool P, bool P2>
 __global__ __launch_bounds__(256) void kb_gather(const RepDev *m, const int2 *map, int nmap) {
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, true>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         switch (r.g.scheme) {
@@ -667,7 +667,7 @@ __global__ __launch_bounds__(256) void kb_gather(const RepDev *m, const int2 *ma
 
 template <bool P>
 __global__ __launch_bounds__(SCAN_THREADS) void kb_scan(const RepDev *m, const int2 *map, int nmap) {
-    for_entries<P, true>(nmap, [&](int e_) {
+    for_entries<P, true, false>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         scan_body(r.d.count, r.d.bcount, r.d.start, r.g.ncell, r.scan_nb, r.g.N, r.d.sc, 0, t.y);
@@ -676,7 +676,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void kb_scan(const RepDev *m, const i
 
 template <bool P>
 __global__ __launch_bounds__(256) void kb_fill(const RepDev *m, const int2 *map, int nmap) {
-    for_entries<P, false>(nmap, [&](int e_) {
+    for_entries<P, false, true>(nmap, [&](int e_) {
         const int2 t = map[e_];
         fill_body(m[t.x].g, m[t.x].d, 1, t.y);
     });
@@ -684,7 +684,7 @@ __global__ __launch_bounds__(256) void kb_fill(const RepDev *m, const int2 *map,
 
 template <bool P>
 __global__ __launch_bounds__(256) void kb_sort_cells(const RepDev *m, const int2 *map, int nmap) {
-    for_entries<P, false>(nmap, [&](int e_) {
+    for_entries<P, false, false>(nmap, [&](int e_) {
         const int2 t = map[e_];
         sort_cells_body(m[t.x].g, m[t.x].d, 1, t.y);
     });
