@@ -225,6 +225,40 @@ char *pinned(bdk_t *h, size_t bytes) {
     return h->pin;
 }
 
+// `bytes` of device memory (16-byte aligned, readable to the next multiple of
+// 16) in host memory once the stream has come to them, valid until the
+// handle's next call that stages.  A kernel writes them into the pinned
+// staging: the copy engine's start and its completion signal cost more than
+// a short copy itself (behind a kernel: 24 us for 125 KB and 27 for 312, by
+// a kernel 16.5 and 20; a pageable 16 KB 29 us against 14).
+hipError_t fetch(bdk_t *h, const void *dev, size_t bytes, std::vector<char> &own, const char **out) {
+    hipError_t e;
+    if (char *stage = pinned(h, Scratch::pad(bytes))) {
+        *out = stage;
+        e = bdkx::launch_to_host(dev, bytes, stage, h->stream);
+    } else {
+        own.resize(bytes);
+        *out = own.data();
+        e = hipMemcpyAsync(own.data(), dev, bytes, hipMemcpyDeviceToHost, h->stream);
+    }
+    const hipError_t es = hipStreamSynchronize(h->stream);
+    return e == hipSuccess ? es : e;
+}
+
+hipError_t fetch_scalars(bdk_t *h, DevScalars &sc) {
+    std::vector<char> own;
+    const char *p = nullptr;
+    const hipError_t e = fetch(h, h->d.sc, sizeof(sc), own, &p);
+    if (e == hipSuccess) std::memcpy(&sc, p, sizeof(sc));
+    return e;
+}
+
+// particles up to which the kernels that put results in id order write them
+// straight to the staging (16-byte writes over the bus): 16 KB in 11.6 us
+// against 14 in two kernels, 125 KB in 16.2 against 16.5, 312 KB in 30
+// against 20
+constexpr int kDirectIds = 4096;
+
 // spectral tables (dm:578-594, dm:1384-1394), built in FP64 on the host
 int build_tables_host(bdk_t *h) {
     const bd_params &p = h->p;
@@ -292,8 +326,7 @@ int flag_status(int flags, std::string *msg) {
 
 int check_nonfinite(bdk_t *h) {
     DevScalars sc;
-    HIPCHK(h, hipMemcpyAsync(&sc, h->d.sc, sizeof(sc), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    HIPCHK(h, fetch_scalars(h, sc));
     std::string m;
     const int rc = flag_status(sc.nonfinite, &m);
     return rc ? fail(h, rc, m) : BDK_OK;
@@ -396,14 +429,16 @@ int download_forces(bdk_t *h, const void *src, double *f1, double *f2) {
     Scratch ws(h);
     HIPCHK(h, ws.reserve(Scratch::pad(N * 16)));
     double2 *out = ws.take<double2>(N);
-    HIPCHK(h, bdkx::launch_force_by_id(h, src, out));
-    if (char *stage = pinned(h, N * 16)) {
-        HIPCHK(h, hipMemcpyAsync(stage, out, N * 16, hipMemcpyDeviceToHost, h->stream));
+    if (char *stage = pinned(h, Scratch::pad(N * 16))) {
+        const bool direct = N <= (size_t)kDirectIds;
+        HIPCHK(h, bdkx::launch_force_by_id(h, src, direct ? (double2 *)stage : out));
+        if (!direct) HIPCHK(h, bdkx::launch_to_host(out, N * 16, stage, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
         if (f1 && n1) std::memcpy(f1, stage, n1 * 16);
         if (f2 && n2) std::memcpy(f2, stage + n1 * 16, n2 * 16);
         return BDK_OK;
     }
+    HIPCHK(h, bdkx::launch_force_by_id(h, src, out));
     if (f1 && n1) HIPCHK(h, hipMemcpyAsync(f1, out, n1 * 16, hipMemcpyDeviceToHost, h->stream));
     if (f2 && n2) HIPCHK(h, hipMemcpyAsync(f2, out + n1, n2 * 16, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -838,12 +873,15 @@ int bdk_get_positions(bdk_t *h, int species, int32_t n, int32_t *git, double *re
     Scratch ws(h);
     HIPCHK(h, ws.reserve(Scratch::pad(bytes)));
     char *out = ws.take<char>(bytes);
-    double2 *orel = (double2 *)(out + head);
-    int2 *ogit = (int2 *)(out + head + (size_t)n * 16);
-    HIPCHK(h, bdkx::launch_by_id(h, species == 1 ? 0 : n1, n, (bdkx::ByIdHead *)out, ogit, orel));
+    char *stage = pinned(h, Scratch::pad(bytes));
+    const bool direct = stage && n <= kDirectIds;
+    char *to = direct ? stage : out;
+    double2 *orel = (double2 *)(to + head);
+    int2 *ogit = (int2 *)(to + head + (size_t)n * 16);
+    HIPCHK(h, bdkx::launch_by_id(h, species == 1 ? 0 : n1, n, (bdkx::ByIdHead *)to, ogit, orel));
     bdkx::ByIdHead flags;
-    if (char *stage = pinned(h, bytes)) {
-        HIPCHK(h, hipMemcpyAsync(stage, out, bytes, hipMemcpyDeviceToHost, h->stream));
+    if (stage) {
+        if (!direct) HIPCHK(h, bdkx::launch_to_host(out, bytes, stage, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
         std::memcpy(&flags, stage, head);
         if (rel && n) std::memcpy(rel, stage + head, (size_t)n * 16);
@@ -926,8 +964,7 @@ int bdk_optimal_dt(bdk_t *h, double *dt) {
     }
     HIPCHK(h, bdkx::launch_gather(h, 1));
     DevScalars sc;
-    HIPCHK(h, hipMemcpyAsync(&sc, h->d.sc, sizeof(sc), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    HIPCHK(h, fetch_scalars(h, sc));
     *dt = dt_from_bits(sc.dt_bits);
     return BDK_OK;
 }
@@ -1022,11 +1059,12 @@ static int run_logged(bdk_t *h, int64_t k, long double *t) {
     int64_t i = 0;
     for (; i + kGraphSteps <= k; i += kGraphSteps) HIPCHK(h, hipGraphLaunch(h->gexec_multi, h->stream));
     for (; i < k; ++i) HIPCHK(h, hipGraphLaunch(h->gexec, h->stream));
-    std::vector<double> log(bdkx::kDtLog);
     DevScalars sc;
-    HIPCHK(h, hipMemcpyAsync(log.data(), h->d.dtlog, bdkx::kDtLog * 8, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(&sc, h->d.sc, sizeof(sc), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    std::vector<char> own;
+    const char *got = nullptr;
+    HIPCHK(h, fetch_scalars(h, sc));
+    HIPCHK(h, fetch(h, h->d.dtlog, bdkx::kDtLog * 8, own, &got));
+    const double *log = (const double *)got;
     h->host_step += k;
     const unsigned long long s0 = sc.step - (unsigned long long)k;
     for (int64_t j = 0; j < k; ++j) *t += (long double)log[(s0 + (unsigned long long)j) & (bdkx::kDtLog - 1)];
@@ -1061,9 +1099,8 @@ int bdk_run_steps(bdk_t *h, int64_t k, double *t_out) {
             t += (long double)dt;
         }
     }
-    HIPCHK(h, hipStreamSynchronize(h->stream));
     if (t_out) *t_out = (double)t;
-    return check_nonfinite(h);
+    return check_nonfinite(h);  // waits for the steps
 }
 
 int bdk_set_max_travel(bdk_t *h, double max_travel) {
@@ -1862,16 +1899,17 @@ int bdk_radial_profile(bdk_t *h, int32_t nbins, double dr, double *centers, doub
     const size_t np = (size_t)bdkx::radial_blocks(h) * 8, ncnt = (size_t)6 * nbins, ncopy = (size_t)bdkx::radial_copies(nbins);
     Scratch ws(h);
     hipError_t e = ws.reserve(Scratch::pad(np * 8) + Scratch::pad(6 * 8 + ncopy * ncnt * 4));
-    std::vector<char> got(6 * 8 + ncopy * ncnt * 4);  // centres, then the copies of the counts
+    const size_t bytes = 6 * 8 + ncopy * ncnt * 4;  // centres, then the copies of the counts
+    std::vector<char> own;
+    const char *got = nullptr;
     if (e == hipSuccess) {
-        double *part = ws.take<double>(np), *cen = (double *)ws.take<char>(got.size());
+        double *part = ws.take<double>(np), *cen = (double *)ws.take<char>(bytes);
         e = bdkx::launch_radial(h, nbins, dr, part, cen, (int *)(cen + 6));
-        if (e == hipSuccess) e = hipMemcpyAsync(got.data(), cen, got.size(), hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        if (e == hipSuccess) e = fetch(h, cen, bytes, own, &got);
     }
     if (e != hipSuccess) return hipfail(h, e, "bdk_radial_profile");
-    const double *c6 = (const double *)got.data();
-    const int *copies = (const int *)(got.data() + 6 * 8);
+    const double *c6 = (const double *)got;
+    const int *copies = (const int *)(got + 6 * 8);
     std::vector<int> cnt(copies, copies + ncnt);
     for (size_t k = 1; k < ncopy; ++k)
         for (size_t i = 0; i < ncnt; ++i) cnt[i] += copies[k * ncnt + i];
@@ -1893,15 +1931,16 @@ int bdk_pair_correlation(bdk_t *h, int32_t nbins, double dr, double *g11, double
     const size_t hb = (size_t)3 * nbins * sizeof(unsigned long long);
     Scratch ws(h);
     hipError_t e = ws.reserve(Scratch::pad(hb));
-    std::vector<unsigned long long> cnt((size_t)3 * nbins);
+    std::vector<char> own;
+    const char *got = nullptr;
     if (e == hipSuccess) {
         unsigned long long *hist = ws.take<unsigned long long>((size_t)3 * nbins);
         e = hipMemsetAsync(hist, 0, hb, h->stream);
         if (e == hipSuccess) e = bdkx::launch_pair_hist(h, nbins, dr, hist);
-        if (e == hipSuccess) e = hipMemcpyAsync(cnt.data(), hist, hb, hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        if (e == hipSuccess) e = fetch(h, hist, hb, own, &got);
     }
     if (e != hipSuccess) return hipfail(h, e, "bdk_pair_correlation");
+    const unsigned long long *cnt = (const unsigned long long *)got;
     // auswertung.cpp:120-121, 149-150, 173-174 (g12 keeps the reference's N1-1)
     const double L = h->p.L, n1 = h->p.n1, n2 = h->p.n2;
     const double v11 = n1 > 1 ? 2.0 / ((n1 - 1) * M_PI * (n1 / L / L) * dr * dr) : 0.0;
@@ -1936,7 +1975,8 @@ static int density_snapshot(bdk_t *h, int32_t m, double *rho1, double *rho2, int
     const bool grid = rho1 || rho2;
     Scratch ws(h);
     hipError_t e = ws.reserve(Scratch::pad(grid ? 2 * mm * 8 : 0) + Scratch::pad(ncopy * nc * sizeof(unsigned int)));
-    std::vector<unsigned int> c(ncopy * nc);
+    std::vector<char> own;
+    const char *got = nullptr;
     if (e == hipSuccess) {
         double *rho = grid ? ws.take<double>(2 * mm) : nullptr;
         unsigned int *cnt = stats ? ws.take<unsigned int>(ncopy * nc) : nullptr;
@@ -1944,13 +1984,14 @@ static int density_snapshot(bdk_t *h, int32_t m, double *rho1, double *rho2, int
         if (e == hipSuccess) e = bdkx::launch_snap(h, m, rho, stats, nbins, dbin, th, cnt);
         if (e == hipSuccess && rho1) e = hipMemcpyAsync(rho1, rho, mm * 8, hipMemcpyDeviceToHost, h->stream);
         if (e == hipSuccess && rho2) e = hipMemcpyAsync(rho2, rho + mm, mm * 8, hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess && stats)
-            e = hipMemcpyAsync(c.data(), cnt, c.size() * sizeof(unsigned int), hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess && stats) e = fetch(h, cnt, ncopy * nc * sizeof(unsigned int), own, &got);
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     }
     if (e != hipSuccess) return hipfail(h, e, what);
+    const unsigned int *copies = (const unsigned int *)got;
+    std::vector<unsigned int> c(copies, copies + nc);
     for (size_t k = 1; k < ncopy; ++k)
-        for (size_t i = 0; i < nc; ++i) c[i] += c[k * nc + i];
+        for (size_t i = 0; i < nc; ++i) c[i] += copies[k * nc + i];
     if (stats) {
         const double pre = 1.0 / (double)mm;  // main_auswertung.cpp:328
         if (hist)
@@ -1982,14 +2023,16 @@ int bdk_ftrho_sums(bdk_t *h, int32_t species, int32_t qbins, double dq_ft, doubl
     const size_t sq = (size_t)f.side * f.side;
     Scratch ws(h);
     hipError_t e = ws.reserve(Scratch::pad(f.parts * 2 * sq * 8) + Scratch::pad(2 * sq * 8));
-    std::vector<double> sums(2 * sq);
+    std::vector<char> own;
+    const char *got = nullptr;
     if (e == hipSuccess) {
         double *part = ws.take<double>(f.parts * 2 * sq), *out = ws.take<double>(2 * sq);
-        e = bdkx::launch_ftrho(h, f, qbins, species, dq_ft, part, out);
-        if (e == hipSuccess) e = hipMemcpyAsync(sums.data(), out, sums.size() * 8, hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        char *stage = pinned(h, 2 * sq * 8);  // the last kernel's sums go straight to it
+        e = bdkx::launch_ftrho(h, f, qbins, species, dq_ft, part, stage ? (double *)stage : out);
+        if (e == hipSuccess) e = stage ? (got = stage, hipStreamSynchronize(h->stream)) : fetch(h, out, 2 * sq * 8, own, &got);
     }
     if (e != hipSuccess) return hipfail(h, e, "bdk_ftrho_sums");
+    const double *sums = (const double *)got;
     // the reference's loop order: the inner loop stops at the first j beyond the quarter circle
     int np = 0;
     for (int i = 0; i < qbins; ++i)
@@ -2010,15 +2053,18 @@ int bdk_rho_k(bdk_t *h, int32_t species, double dq_ratio, int32_t nbins, double 
     const size_t np = (size_t)(Z / 2 + 1) * 2 * nbins;
     Scratch ws(h);
     hipError_t e = ws.reserve(Scratch::pad(np * 8) + Scratch::pad((size_t)2 * nbins * 8));
-    std::vector<double> sum((size_t)2 * nbins);  // shell sums, then lattice points per shell (auswertung.cpp:497-510)
+    std::vector<char> own;
+    const char *got = nullptr;
     if (e == hipSuccess) {
         double *part = ws.take<double>(np), *out = ws.take<double>((size_t)2 * nbins);
-        e = bdkx::launch_rhok(h, species, dq_ratio, nbins, part, out);
-        if (e == hipSuccess) e = hipMemcpyAsync(sum.data(), out, sum.size() * 8, hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        char *stage = pinned(h, (size_t)2 * nbins * 8);  // the last kernel's sums go straight to it
+        e = bdkx::launch_rhok(h, species, dq_ratio, nbins, part, stage ? (double *)stage : out);
+        if (e == hipSuccess)
+            e = stage ? (got = stage, hipStreamSynchronize(h->stream)) : fetch(h, out, (size_t)2 * nbins * 8, own, &got);
     }
     if (e != hipSuccess) return hipfail(h, e, "bdk_rho_k");
-    const double L = h->p.L, *cnt = sum.data() + nbins;
+    // shell sums, then lattice points per shell (auswertung.cpp:497-510)
+    const double L = h->p.L, *sum = (const double *)got, *cnt = sum + nbins;
     for (int b = 0; b < nbins; ++b) {  // auswertung.cpp:572-576
         re[b] = cnt[b] > 0.0 ? sum[b] * (L * L / ((double)Z * Z)) / cnt[b] : 0.0;
         if (im) im[b] = 0.0;

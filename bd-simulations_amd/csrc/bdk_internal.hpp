@@ -225,6 +225,8 @@ struct ByIdHead {
 };
 hipError_t launch_by_id(bdk_t *h, int id0, int n, ByIdHead *head, int2 *git, double2 *rel);
 hipError_t launch_force_by_id(bdk_t *h, const void *f, double2 *out);  // list-ordered forces -> [N] by id
+// bytes (up to the next multiple of 16) of device memory into pinned host memory
+hipError_t launch_to_host(const void *src, size_t bytes, void *dst, hipStream_t st);
 hipError_t launch_zero_ints(int *p, int n, hipStream_t st);
 hipError_t launch_rearm(bdk_t *h);                // per-step scalars when no deposit runs
 size_t deposit_lds_bytes(const bdk_t *h);          // LDS of one deposit block

@@ -524,6 +524,12 @@ __global__ void k_by_id(Geo g, DevBufs d, int id0, int n, ByIdHead *head, int2 *
     rel[i] = d.rel[s];
 }
 
+// n 16-byte words into pinned host memory, a wave's 1 KB per store; bound by
+// the bus (2.7 MB: 60 us, 46 GB/s)
+__global__ __launch_bounds__(256) void k_to_host(const uint4 *__restrict__ src, uint4 *__restrict__ dst, int n) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dst[i] = src[i];
+}
+
 // list-ordered forces as doubles in id order
 template <typename R>
 __global__ void k_force_by_id(Geo g, DevBufs d, const typename V2<R>::T *__restrict__ f, double2 *out) {
@@ -857,6 +863,13 @@ hipError_t launch_force_by_id(bdk_t *h, const void *f, double2 *out) {
         hipLaunchKernelGGL(k_force_by_id<float>, grid, blk, 0, h->stream, h->g, h->d, (const float2 *)f, out);
     else
         hipLaunchKernelGGL(k_force_by_id<double>, grid, blk, 0, h->stream, h->g, h->d, (const double2 *)f, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_to_host(const void *src, size_t bytes, void *dst, hipStream_t st) {
+    const int n = (int)((bytes + 15) / 16);
+    hipLaunchKernelGGL(k_to_host, dim3(std::max(1u, std::min(256u, nblk(n, 256)))), dim3(256), 0, st,
+                       (const uint4 *)src, (uint4 *)dst, n);
     return hipGetLastError();
 }
 
