@@ -206,12 +206,16 @@ struct Scratch {
 // Pinned host staging of the handle, for copies up to kPinned bytes: one
 // transfer without the runtime's own staging (at 4000 particles some 10 us
 // each).  Larger copies go to the caller's memory directly.  Null when the
-// request is larger or the allocation fails.  Every call that fills it waits
-// for its copies before it returns.
+// request is larger or the allocation fails.  What the device writes there is
+// waited for by the call that reads it; what it reads (an upload, pin_read) may
+// still be on its way when the call returns, so the next host write or a new
+// allocation waits first.
 constexpr size_t kPinned = 4u << 20;
 char *pinned(bdk_t *h, size_t bytes) {
     if (bytes > kPinned) return nullptr;
     if (bytes > h->pin_cap) {
+        if (h->pin_read) (void)hipStreamSynchronize(h->stream);
+        h->pin_read = false;
         if (h->pin) (void)hipHostFree(h->pin);
         h->pin = nullptr;
         h->pin_cap = 0;
@@ -242,6 +246,7 @@ hipError_t fetch(bdk_t *h, const void *dev, size_t bytes, std::vector<char> &own
         e = hipMemcpyAsync(own.data(), dev, bytes, hipMemcpyDeviceToHost, h->stream);
     }
     const hipError_t es = hipStreamSynchronize(h->stream);
+    if (es == hipSuccess) h->pin_read = false;
     return e == hipSuccess ? es : e;
 }
 
@@ -338,68 +343,55 @@ hipError_t clear_flags(bdk_t *h) {
     return hipMemsetAsync(&h->d.sc->nonfinite, 0, sizeof(int), h->stream);
 }
 
-// upload both species in storage order (grouped by cell, ascending id) and
-// rebuild the cell lists (WCA_init, dm:459-526)
+// Upload both species and rebuild the cell lists (WCA_init, dm:459-526).  The
+// host checks the positions and stages them as they are, in id order; k_place
+// writes the state and counts, and the list stages put it in order.  (With a
+// counting sort on the host, three copies and three fills the upload of 4000
+// particles in 71,289 cells took 90 us; it takes 30.)
 int upload(bdk_t *h) {
     const int n1 = h->p.n1, n2 = h->p.n2, N = n1 + n2, nc = h->g.nc;
-    // storage order: grouped by cell, ascending id.  A counting sort, unless
-    // the cells by far outnumber the particles (2M particles in 1.6M cells: 35
-    // instead of 180 ms; 1000 particles in 16M cells would pay for the cells).
-    const size_t ncell = (size_t)nc * nc;
-    const bool counting = ncell <= 32 * (size_t)N + 65536;
-    std::vector<int> cell(N), at(counting ? ncell + 1 : 0, 0), order;
     for (int sp = 0; sp < 2; ++sp) {
-        const int n = sp == 0 ? n1 : n2, off = sp == 0 ? 0 : n1;
-        for (int i = 0; i < n; ++i) {
-            int gx = h->hgit[sp][2 * i], gy = h->hgit[sp][2 * i + 1];
-            if (gx < 0 || gx >= nc || gy < 0 || gy >= nc)
-                return fail(h, BDK_ERR_ARG, "git out of range [0, nachList_Zellen) for species " +
-                                                std::to_string(sp + 1) + " particle " + std::to_string(i));
-            double rx = h->hrel[sp][2 * i], ry = h->hrel[sp][2 * i + 1];
-            if (!(std::fabs(rx) < 1e9 && std::fabs(ry) < 1e9))
-                return fail(h, BDK_ERR_NONFINITE, "non-finite rel for species " + std::to_string(sp + 1) +
-                                                      " particle " + std::to_string(i));
-            cell[off + i] = gx * nc + gy;
-            if (counting) ++at[cell[off + i] + 1];
+        const int n = sp == 0 ? n1 : n2;
+        const int *git = h->hgit[sp].data();
+        const double *rel = h->hrel[sp].data();
+        int bad = 0;
+        for (int i = 0; i < 2 * n; ++i) bad |= (unsigned)git[i] >= (unsigned)nc;
+        for (int i = 0; i < 2 * n; ++i) bad |= !(std::fabs(rel[i]) < 1e9);
+        for (int i = 0; bad && i < n; ++i) {
+            const std::string who =
+                " for species " + std::to_string(sp + 1) + " particle " + std::to_string(i);
+            if ((unsigned)git[2 * i] >= (unsigned)nc || (unsigned)git[2 * i + 1] >= (unsigned)nc)
+                return fail(h, BDK_ERR_ARG, "git out of range [0, nachList_Zellen)" + who);
+            if (!(std::fabs(rel[2 * i]) < 1e9 && std::fabs(rel[2 * i + 1]) < 1e9))
+                return fail(h, BDK_ERR_NONFINITE, "non-finite rel" + who);
         }
     }
-    if (counting) {
-        for (size_t c = 1; c < at.size(); ++c) at[c] += at[c - 1];
+    // [rel | git], both by id.  Up to kPinned bytes the kernel reads the pinned
+    // staging itself and the upload does not wait; more is copied first.
+    const size_t relb = (size_t)N * 16, bytes = (size_t)N * 24;
+    Scratch ws(h);
+    char *from = pinned(h, bytes);
+    if (from) {
+        if (h->pin_read) HIPCHK(h, hipStreamSynchronize(h->stream));  // the last upload's kernel
+        for (int sp = 0; sp < 2; ++sp) {
+            const size_t n = sp == 0 ? n1 : n2, off = sp == 0 ? 0 : n1;
+            if (n) std::memcpy(from + off * 16, h->hrel[sp].data(), n * 16);
+            if (n) std::memcpy(from + relb + off * 8, h->hgit[sp].data(), n * 8);
+        }
+        h->pin_read = true;
     } else {
-        order.resize(N);
-        std::iota(order.begin(), order.end(), 0);
-        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cell[a] < cell[b]; });
-    }
-    // offsets, cells and ids in storage order, staged for one transfer each
-    std::vector<char> own;
-    char *stage = pinned(h, (size_t)N * 24);
-    if (!stage) {
-        own.resize((size_t)N * 24);
-        stage = own.data();
-    }
-    double *srel = (double *)stage;
-    int *scell = (int *)(stage + (size_t)N * 16), *spid = scell + N;
-    for (int k = 0; k < N; ++k) {
-        const int p = counting ? k : order[k], s = counting ? at[cell[p]]++ : k;
-        const int sp = p < n1 ? 0 : 1, i = sp ? p - n1 : p;
-        double rx = h->hrel[sp][2 * (size_t)i], ry = h->hrel[sp][2 * (size_t)i + 1];
-        if (h->g.pos_mode) {  // FP32 storage of the in-cell positions
-            rx = (double)(float)rx;
-            ry = (double)(float)ry;
+        HIPCHK(h, ws.reserve(Scratch::pad(bytes)));
+        from = ws.take<char>(bytes);
+        for (int sp = 0; sp < 2; ++sp) {
+            const size_t n = sp == 0 ? n1 : n2, off = sp == 0 ? 0 : n1;
+            if (!n) continue;
+            HIPCHK(h, hipMemcpyAsync(from + off * 16, h->hrel[sp].data(), n * 16, hipMemcpyHostToDevice, h->stream));
+            HIPCHK(h, hipMemcpyAsync(from + relb + off * 8, h->hgit[sp].data(), n * 8, hipMemcpyHostToDevice,
+                                     h->stream));
         }
-        scell[s] = cell[p];
-        spid[s] = p;
-        srel[2 * (size_t)s] = rx;
-        srel[2 * (size_t)s + 1] = ry;
     }
-    HIPCHK(h, hipMemcpyAsync(h->d.cell, scell, (size_t)N * 4, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(h, hipMemcpyAsync(h->d.pid, spid, (size_t)N * 4, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(h, hipMemcpyAsync(h->d.rel, srel, (size_t)N * 16, hipMemcpyHostToDevice, h->stream));
-    if (h->d.comp) HIPCHK(h, hipMemsetAsync(h->d.comp, 0, (size_t)N * 8, h->stream));
-    HIPCHK(h, hipMemsetAsync(h->d.count, 0, (size_t)h->g.ncell * 4, h->stream));
-    HIPCHK(h, clear_flags(h));
-    HIPCHK(h, bdkx::launch_bin(h));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    HIPCHK(h, bdkx::launch_place(h, (const int2 *)(from + relb), (const double2 *)from));
+    if (from != h->pin) HIPCHK(h, hipStreamSynchronize(h->stream));
     h->dev_valid = true;
     h->forces_ready = false;
     return BDK_OK;
@@ -434,6 +426,7 @@ int download_forces(bdk_t *h, const void *src, double *f1, double *f2) {
         HIPCHK(h, bdkx::launch_force_by_id(h, src, direct ? (double2 *)stage : out));
         if (!direct) HIPCHK(h, bdkx::launch_to_host(out, N * 16, stage, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
+        h->pin_read = false;
         if (f1 && n1) std::memcpy(f1, stage, n1 * 16);
         if (f2 && n2) std::memcpy(f2, stage + n1 * 16, n2 * 16);
         return BDK_OK;

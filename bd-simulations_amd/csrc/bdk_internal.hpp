@@ -208,6 +208,7 @@ struct bdk {
     hipEvent_t ev_dt = nullptr;
     char *pin = nullptr;           // pinned host staging (bdk_api.cpp: pinned), at most kPinned bytes
     size_t pin_cap = 0;
+    bool pin_read = false;         // a kernel that reads the staging may be in flight
     bdkx::PosWriter writer;
 };
 
@@ -246,7 +247,8 @@ hipError_t launch_fft(bdk_t *h);                  // rho -> fmesh (r2c, multiply
 hipError_t launch_fft_pass(bdk_t *h, int pass, hipStream_t st = nullptr, int end_step = 0);
 hipError_t launch_gather(bdk_t *h, int with_dt, int fold = 1);  // fkap (+ dt candidates; + their fold)
 hipError_t launch_update(bdk_t *h, int fused);    // noise, Euler step, refresh, counting
-hipError_t launch_bin(bdk_t *h);                  // counting after an upload/refresh
+hipError_t launch_place(bdk_t *h, const int2 *git, const double2 *rel);  // a new state, by id, and its lists
+hipError_t launch_bin(bdk_t *h);                  // counting after a state's load
 hipError_t launch_own(bdk_t *h);                  // owned-mesh-index table of the deposit tiles
 hipError_t launch_scan_fill(bdk_t *h);            // exclusive scan + fill of the cell list
 hipError_t launch_refresh(bdk_t *h);              // refresh only (no motion)

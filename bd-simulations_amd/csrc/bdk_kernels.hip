@@ -486,16 +486,45 @@ __global__ void k_refresh(Geo g, DevBufs d) {
     if (ex > 0.0) atomicMax(&d.sc->exc_bits[d.sc->step & 1], bitsd(ex));
 }
 
-// counting only (after an upload): rank and excursion
-__global__ void k_bin(Geo g, DevBufs d) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= g.N) return;
-    const int c = d.cell[s];
+// counting: rank and excursion of a particle in slot s
+__device__ __forceinline__ void bin_slot(const Geo &g, const DevBufs &d, int s, int c, double2 rn) {
     d.rank[s] = atomicAdd(&d.count[c], 1);
-    const double2 rn = d.rel[s];
     const double B = g.B;
     double ex = fmax(fmax(-rn.x, rn.x - B), fmax(-rn.y, rn.y - B));
     if (ex > 0.0) atomicMax(&d.sc->exc_bits[d.sc->step & 1], bitsd(ex));
+}
+
+// counting only (after a state's load)
+__global__ void k_bin(Geo g, DevBufs d) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < g.N) bin_slot(g, d, s, d.cell[s], d.rel[s]);
+}
+
+// A new state: cells and offsets by id (device memory, or the pinned staging
+// read over the bus) into the slots of the same number, counted on the way.
+// The flags and counters start cleared (k_place_clear).
+__global__ __launch_bounds__(256) void k_place(Geo g, DevBufs d, const int2 *__restrict__ git,
+                                               const double2 *__restrict__ rel) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= g.N) return;
+    const int2 gi = git[s];
+    double2 r = rel[s];
+    if (g.pos_mode) r = make_double2((double)(float)r.x, (double)(float)r.y);  // FP32 storage of the in-cell positions
+    const int c = gi.x * g.nc + gi.y;
+    d.cell[s] = c;
+    d.pid[s] = s;
+    d.rel[s] = r;
+    if (d.comp) d.comp[s] = make_float2(0.f, 0.f);
+    bin_slot(g, d, s, c, r);
+}
+
+__global__ __launch_bounds__(256) void k_place_clear(int *count, int ncell, DevScalars *sc) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < ncell) count[i] = 0;
+    if (i == 0) {
+        sc->exc_bits[sc->step & 1] = 0ull;
+        sc->nonfinite = 0;  // the flags describe a run from the state before
+    }
 }
 
 // clears the excursion slot that k_bin / k_refresh fill
@@ -948,6 +977,14 @@ hipError_t launch_own(bdk_t *h) {
 hipError_t launch_bin(bdk_t *h) {
     hipLaunchKernelGGL(k_reset_exc, dim3(1), dim3(1), 0, h->stream, h->d.sc);
     hipLaunchKernelGGL(k_bin, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d);
+    launch_scan_fill_inner(h, 0);
+    return hipGetLastError();
+}
+
+hipError_t launch_place(bdk_t *h, const int2 *git, const double2 *rel) {
+    hipLaunchKernelGGL(k_place_clear, dim3(nblk(h->g.ncell, 256)), dim3(256), 0, h->stream, h->d.count, h->g.ncell,
+                       h->d.sc);
+    hipLaunchKernelGGL(k_place, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d, git, rel);
     launch_scan_fill_inner(h, 0);
     return hipGetLastError();
 }

@@ -42,3 +42,25 @@ def test_read_back_in_id_order(n1, n2):
     push = f[:, 1, 0][np.argsort(gap)]
     assert np.all(push > 0.0) and np.all(np.diff(push) < 0.0)
     s.close()
+
+
+@pytest.mark.parametrize("precision", [bdk.FP64, bdk.FP32, bdk.FP32_POS32, bdk.FP32_POS32K])
+@pytest.mark.parametrize("n1,n2", [(1, 0), (255, 2), (3000, 1000), (150000, 60000)])
+def test_a_state_replaced_before_it_was_waited_for(precision, n1, n2):
+    print("case: replaced state, %d + %d particles, precision %d" % (n1, n2, precision), flush=True)
+    n, L = n1 + n2, max(8.0, 1.6 * math.sqrt(n1 + n2))
+    bp, _ = params(n1=n1, n2=n2, L=L, Z=64, precision=precision)
+    d, rng = bdk.derived(bp), np.random.default_rng(n)
+    states = [to_git_rel(rng.uniform(0.0, L, (n, 2)), d["B"], d["nc"]) for _ in range(3)]
+    s, fresh = bdk.RunDynamik(bp), bdk.RunDynamik(bp)
+    for git, rel in states:
+        s.set_positions(git, rel)
+        s.prepare()  # enqueues the lists and forces
+    fresh.set_positions(*states[-1])
+    for got, want in zip(s.positions() + s.cells(), fresh.positions() + fresh.cells()):
+        assert np.array_equal(got, want)
+    assert np.array_equal(s.positions()[0], states[-1][0])
+    assert np.array_equal(s.berechne_WCA(), fresh.berechne_WCA())
+    assert np.array_equal(s.berechne_kapkraefte(), fresh.berechne_kapkraefte())
+    s.close()
+    fresh.close()
