@@ -683,6 +683,7 @@ int bdk_create(const bd_params *p, bdk_t **out) {
     g.ncell = dv.nc * dv.nc;
     g.Z = p->Z;
     g.logZ = ilog2(p->Z);
+    bdkx::mix_plans(p->Z, h->mixr, h->mixc);
     g.scheme = p->scheme;
     g.idgas = p->idgas_only != 0;
     g.nowca = p->no_wca != 0;

@@ -5,7 +5,8 @@
 //              two inverse column transforms (Fx, Fy);
 //   c2r rows   inverse row transform of Fx + i Fy -> the real force mesh.
 // Power-of-two meshes: rows in registers (RowFft), sizes known at compile
-// time.  Other even meshes: rows in LDS, any length 2^a 3^b 5^c 7^d.
+// time.  Other even meshes: a plan of radices, a butterfly per thread and pass
+// (bdk_fftmix.hpp), or rows in LDS, any length 2^a 3^b 5^c 7^d.
 //
 // The power-of-two passes in one place (us, r2c / columns / c2r; before, rows
 // went through LDS for the load, every pass, the product and the store, with
@@ -21,6 +22,7 @@
 
 #include "bdk_device.hpp"
 #include "bdk_fft.hpp"
+#include "bdk_fftmix.hpp"
 
 namespace bdkx {
 
@@ -66,8 +68,8 @@ __global__ __launch_bounds__(FFT_MAX_THREADS) void k_c2r_rows(const typename V4<
 template <typename R, int EPT>
 __global__ __launch_bounds__(FFT_THREADS) void k_r2c_any(const R *__restrict__ rho, typename V2<R>::T *__restrict__ ht,
                                                          const typename V2<R>::T *__restrict__ tw, int Z, int RB,
-                                                         int stride, int remap) {
-    r2c_any<R, EPT>(rho, ht, tw, Z, RB, stride, xcd_block(remap));
+                                                         int stride, int remap, MixPlan mp) {
+    r2c_other<R, EPT>(rho, ht, tw, Z, mp, RB, stride, xcd_block(remap));
 }
 
 template <typename R, int EPT>
@@ -75,17 +77,18 @@ __global__ __launch_bounds__(FFT_THREADS) void k_col_any(const typename V2<R>::T
                                                          typename V4<R>::T *__restrict__ gt,
                                                          const typename V2<R>::T *__restrict__ tw,
                                                          const R *__restrict__ sq, const R *__restrict__ lap, Geo g,
-                                                         int RC, int stride) {
-    col_any<R, EPT>(ht, gt, tw, sq, lap, g, RC, stride, blockIdx.x);
+                                                         int RC, int stride, MixPlan mp) {
+    col_other<R, EPT>(ht, gt, tw, sq, lap, g, mp, RC, stride, blockIdx.x);
 }
 
 template <typename R, int EPT>
 __global__ __launch_bounds__(FFT_THREADS) void k_c2r_any(const typename V4<R>::T *__restrict__ gt,
                                                          typename V2<R>::T *__restrict__ fm,
                                                          const typename V2<R>::T *__restrict__ tw, int Z, int RB2,
-                                                         int stride, int remap, Geo g, DevBufs d, int end_step) {
+                                                         int stride, int remap, Geo g, DevBufs d, int end_step,
+                                                         MixPlan mp) {
     if (end_step && blockIdx.x == 0) step_end_body(g, d);
-    c2r_any<R, EPT>(gt, fm, tw, Z, RB2, stride, xcd_block(remap));
+    c2r_other<R, EPT>(gt, fm, tw, Z, mp, RB2, stride, xcd_block(remap));
 }
 
 // ------------------------------------------------------------------ batched
@@ -157,7 +160,10 @@ __global__ __launch_bounds__(FFT_THREADS) void kb_r2c_any(const RepDev *m, const
     for_entries<P, true, true>(nmap, [&](int e_) {
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
-        r2c_any<R, EPT>((const R *)r.d.rho, (C *)r.d.ht, (const C *)r.d.tw, r.g.Z, r.rb, r.sR1, t.y);
+        if (r.mixr.rad)
+            r2c_mix<R>((const R *)r.d.rho, (C *)r.d.ht, (const C *)r.d.tw, r.g.Z, r.mixr, r.rb, r.sR1, t.y);
+        else
+            r2c_any<R, EPT>((const R *)r.d.rho, (C *)r.d.ht, (const C *)r.d.tw, r.g.Z, r.rb, r.sR1, t.y);
     });
 }
 
@@ -170,7 +176,10 @@ __global__ __launch_bounds__(FFT_THREADS) void kb_col_any(const RepDev *m, const
         const RepDev &r = m[t.x];
         const R *sq = std::is_same<R, float>::value ? (const R *)r.d.sqf : (const R *)r.d.sq;
         const R *lap = std::is_same<R, float>::value ? (const R *)r.d.lapf : (const R *)r.d.lap;
-        col_any<R, EPT>((const C *)r.d.ht, (C4 *)r.d.gt, (const C *)r.d.tw, sq, lap, r.g, r.rc, r.sC, t.y);
+        if (r.mixc.rad)
+            col_mix<R>((const C *)r.d.ht, (C4 *)r.d.gt, (const C *)r.d.tw, sq, lap, r.g, r.mixc, r.rc, r.sC, t.y);
+        else
+            col_any<R, EPT>((const C *)r.d.ht, (C4 *)r.d.gt, (const C *)r.d.tw, sq, lap, r.g, r.rc, r.sC, t.y);
     });
 }
 
@@ -182,7 +191,10 @@ __global__ __launch_bounds__(FFT_THREADS) void kb_c2r_any(const RepDev *m, const
         const int2 t = map[e_];
         const RepDev &r = m[t.x];
         if (end_step && t.y == 0) step_end_body(r.g, r.d);
-        c2r_any<R, EPT>((const C4 *)r.d.gt, (C *)r.d.fmesh, (const C *)r.d.tw, r.g.Z, r.rb2, r.sR2, t.y);
+        if (r.mixc.rad)
+            c2r_mix<R>((const C4 *)r.d.gt, (C *)r.d.fmesh, (const C *)r.d.tw, r.g.Z, r.mixc, r.rb2, r.sR2, t.y);
+        else
+            c2r_any<R, EPT>((const C4 *)r.d.gt, (C *)r.d.fmesh, (const C *)r.d.tw, r.g.Z, r.rb2, r.sR2, t.y);
     });
 }
 
@@ -230,6 +242,39 @@ static int p2_rows(bool f32, int Z, int pass) {
     return rows;
 }
 
+// The cheapest passes over n points, a pass of radix r taken to cost r + 4 (its
+// chain of loads, products and sums, and its trip through LDS), with at most
+// FFT_THREADS / 2 butterflies each (so 15 and 16 never pay).  Largest radix first.  r2c / c2r of 192^2
+// FP64 with r + 1.6, r + 4 and r + 8: 6.6 / 7.0, 5.3 / 5.9 and 5.7 / 5.9 us.  A
+// wave's worth of threads per block: with two, r2c of 600^2 takes 8.2 instead of
+// 7.0.
+static void mix_search(int n, int left, int top, unsigned rad, int np, double cost, unsigned &best, double &best_cost) {
+    static const int radices[] = {14, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+    if (left == 1 && np >= 2 && cost < best_cost) {
+        best = rad;
+        best_cost = cost;
+    }
+    if (np == 4) return;
+    for (int r : radices)
+        if (r <= top && left % r == 0 && n / r <= FFT_THREADS / 2)
+            mix_search(n, left / r, r, rad | (unsigned)r << (8 * np), np + 1, cost + r + 4.0, best, best_cost);
+}
+static MixPlan mix_plan(int n) {
+    unsigned best = 0;
+    double cost = 1e9;
+    mix_search(n, n, 14, 0, 0, 0.0, best, cost);
+    int least = 14;
+    for (unsigned r = best; r; r >>= 8) least = std::min(least, (int)(r & 255));
+    return {best, best ? n / least : 0};
+}
+void mix_plans(int Z, MixPlan &r, MixPlan &c) {
+    r = c = {0, 0};
+    if (zp2(Z)) return;
+    r = mix_plan(Z / 2);
+    c = mix_plan(Z);
+    if (!r.rad || !c.rad) r = c = {0, 0};
+}
+
 // Threads and elements per thread of a pass over a mesh of another size:
 // 128 threads of 8 elements where a row fits (384^2 FP64: 17.2 / 11.8 us for
 // the columns and c2r rows at 256 threads of 16, 11.0 / 7.1 so), else 256
@@ -258,8 +303,18 @@ FftLaunch fft_launch(const bdk_t *h, int pass) {
         l.threads = std::max(64, p2_block(f32, Z, pass, l.rows));
         l.lds = p2_lds_bytes(f32, Z, pass, l.rows);
     } else {
-        const AnyCfg c = any_cfg(pass, Z, f32 ? 8 : 16);
-        l = {c.rows, c.threads, 0, c.ept, c.stride, c.lds};
+        l.mix = pass == 0 ? h->mixr : h->mixc;
+        if (l.mix.rad) {
+            const int per = (pass == 1 ? 2 : 1) * l.mix.tpr;  // threads per row
+            l.rows = div_at_most(pass_rows(pass, Z), 64 / per);
+            l.threads = 64;
+            while (l.threads < l.rows * per) l.threads *= 2;
+            l.stride = lds_row(pass == 0 ? Z / 2 : Z);
+            l.lds = (size_t)(pass == 1 ? 2 : 1) * l.rows * l.stride * (f32 ? 8 : 16);
+        } else {
+            const AnyCfg c = any_cfg(pass, Z, f32 ? 8 : 16);
+            l = {c.rows, c.threads, 0, c.ept, c.stride, c.lds, {0, 0}};
+        }
     }
     l.blocks = pass_rows(pass, Z) / l.rows;
     return l;
@@ -305,19 +360,20 @@ template <typename R> static void launch_pass_any(bdk_t *h, int pass, hipStream_
     const C *tw = (const C *)h->d.tw;
 #define R2C(E)                                                                                                        \
     hipLaunchKernelGGL((k_r2c_any<R, E>), grid, blk, c.lds, st, (const R *)h->d.rho, (C *)h->d.ht, tw, Z, c.rows,       \
-                       c.stride, h->g.xcd)
+                       c.stride, h->g.xcd, c.mix)
 #define COL(E)                                                                                                        \
     hipLaunchKernelGGL((k_col_any<R, E>), grid, blk, c.lds, st, (const C *)h->d.ht, (C4 *)h->d.gt, tw, sq, lap, h->g,   \
-                       c.rows, c.stride)
+                       c.rows, c.stride, c.mix)
 #define C2R(E)                                                                                                        \
     hipLaunchKernelGGL((k_c2r_any<R, E>), grid, blk, c.lds, st, (const C4 *)h->d.gt, (C *)h->d.fmesh, tw, Z, c.rows,    \
-                       c.stride, h->g.xcd, h->g, h->d, end_step)
-    if (pass == 0)
-        BDK_EPT_SWITCH(c.ept, R2C)
-    else if (pass == 1)
-        BDK_EPT_SWITCH(c.ept, COL)
-    else
-        BDK_EPT_SWITCH(c.ept, C2R)
+                       c.stride, h->g.xcd, h->g, h->d, end_step, c.mix)
+    if (pass == 0) {
+        BDK_OTHER_SWITCH(c.ept, R2C)
+    } else if (pass == 1) {
+        BDK_OTHER_SWITCH(c.ept, COL)
+    } else {
+        BDK_OTHER_SWITCH(c.ept, C2R)
+    }
 #undef R2C
 #undef COL
 #undef C2R
@@ -358,7 +414,8 @@ void fft_member(RepDev &r, int Z, const int ept[3], BatchPlan &bp) {
             kind = fft_ept(Z, bp.f32) == 16 ? 0 : 1;
             bp.fft_threads[kind][k] = std::max(bp.fft_threads[kind][k], std::max(64, p2_block(bp.f32, Z, k, rows[k])));
         } else {
-            rows[k] = div_at_most(pass_rows(k, Z), cap);
+            const MixPlan &mp = k == 0 ? r.mixr : r.mixc;
+            rows[k] = div_at_most(pass_rows(k, Z), mp.rad ? std::min(cap, FFT_THREADS / ((k == 1 ? 2 : 1) * mp.tpr)) : cap);
             lds = (size_t)(k == 1 ? 2 : 1) * rows[k] * lds_row(k == 0 ? Z / 2 : Z) * (bp.f32 ? 8 : 16);
             kind = 2;
             bp.fft_threads[kind][k] = FFT_THREADS;
@@ -439,10 +496,12 @@ hipError_t fft_set_attributes() {
     BOTH(3) BOTH(4) BOTH(5) BOTH(6) BOTH(7) BOTH(8) BOTH(9) BOTH(10) BOTH(11) BOTH(12)
 #undef BOTH
 #undef ONE
-#define ANY(R, E)                              \
+#define ONE(R, E)                              \
     big((const void *)k_r2c_any<R, E>);      \
     big((const void *)k_col_any<R, E>);      \
-    big((const void *)k_c2r_any<R, E>);      \
+    big((const void *)k_c2r_any<R, E>);
+#define ANY(R, E)                              \
+    ONE(R, E)                                  \
     big((const void *)kb_r2c_any<R, E, false>); \
     big((const void *)kb_col_any<R, E, false>); \
     big((const void *)kb_c2r_any<R, E, false>); \
@@ -450,6 +509,8 @@ hipError_t fft_set_attributes() {
     big((const void *)kb_col_any<R, E, true>);  \
     big((const void *)kb_c2r_any<R, E, true>);
     ANY(float, 8) ANY(float, 16) ANY(float, 32) ANY(double, 8) ANY(double, 16) ANY(double, 32)
+    ONE(float, 0) ONE(double, 0)
+#undef ONE
 #undef ANY
 #define KB(R, P, H)                       \
     big((const void *)kb_r2c<R, P, H>); \

@@ -745,11 +745,13 @@ __device__ __forceinline__ void c2r_any(const typename V4<R>::T *__restrict__ gt
     }
 }
 
-// a pass over one mesh: rows per block, threads and LDS of a block; power-of-
-// two meshes (ept = 0) or others (elements per thread, LDS row stride)
+// a pass over one mesh: rows per block, threads and LDS of a block; for meshes
+// whose size is not a power of two also the LDS row stride and the plan of the
+// row's passes (ept = 0) or the elements per thread
 struct FftLaunch {
     int rows, threads, blocks, ept, stride;
     size_t lds;
+    MixPlan mix;
 };
 FftLaunch fft_launch(const bdk_t *h, int pass);
 

@@ -137,11 +137,19 @@ struct DepArgs {
 };
 
 // One member of a batch, as the batched kernels read it (device memory).
+// Rows of a length that is not a power of two in two to four passes: the
+// radices (first in the low byte) and the threads per row; rad = 0: no plan.
+struct MixPlan {
+    unsigned rad;
+    int tpr;
+};
+
 struct RepDev {
     Geo g;
     DevBufs d;
     DepArgs dep;
     int rb, rc, rb2, sR1, sC, sR2;   // FFT rows per block and LDS row strides
+    MixPlan mixr, mixc;              // of the r2c rows and of the columns and c2r rows
     int scan_nb;                     // scan blocks
     int unit;                        // all sigma/epsilon ratios 1
 };
@@ -206,6 +214,7 @@ struct bdk {
     size_t ws_cap = 0;
     double *hdt = nullptr;         // pinned host copy of a single step's adaptive dt, and the event after its update
     hipEvent_t ev_dt = nullptr;
+    bdkx::MixPlan mixr = {0, 0}, mixc = {0, 0};  // of the mesh's rows (mix_plans)
     char *pin = nullptr;           // pinned host staging (bdk_api.cpp: pinned), at most kPinned bytes
     size_t pin_cap = 0;
     bool pin_read = false;         // a kernel that reads the staging may be in flight
@@ -248,6 +257,8 @@ hipError_t launch_fft_pass(bdk_t *h, int pass, hipStream_t st = nullptr, int end
 hipError_t launch_gather(bdk_t *h, int with_dt, int fold = 1);  // fkap (+ dt candidates; + their fold)
 hipError_t launch_update(bdk_t *h, int fused);    // noise, Euler step, refresh, counting
 hipError_t launch_place(bdk_t *h, const int2 *git, const double2 *rel);  // a new state, by id, and its lists
+// plans of mesh size Z's r2c rows and of its columns and c2r rows, both or none
+void mix_plans(int Z, MixPlan &r, MixPlan &c);
 hipError_t launch_bin(bdk_t *h);                  // counting after a state's load
 hipError_t launch_own(bdk_t *h);                  // owned-mesh-index table of the deposit tiles
 hipError_t launch_scan_fill(bdk_t *h);            // exclusive scan + fill of the cell list

@@ -1254,6 +1254,8 @@ hipError_t batch_build(const std::vector<bdk_t *> &mem, const BatchTuning &tune,
         r.dep = pl.a;
         bp.dep_lds = std::max(bp.dep_lds, pl.lds);
         const int Z = h->g.Z;
+        r.mixr = h->mixr;
+        r.mixc = h->mixc;
         fft_member(r, Z, ept, bp);
         r.scan_nb = (int)nblk(h->g.ncell, SCAN_BLOCK);
         r.unit = h->p.sigma11_22 == 1.0 && h->p.sigma11_12 == 1.0 && h->p.eps22_11 == 1.0 && h->p.eps12_11 == 1.0;

@@ -11,6 +11,7 @@
 
 #include "bdk_device.hpp"
 #include "bdk_fft.hpp"
+#include "bdk_fftmix.hpp"
 #include "bdk_particles.hpp"
 
 namespace bdkx {
@@ -26,10 +27,11 @@ __global__ __launch_bounds__(DP_THREADS) void k_deposit_scan(Geo g, DevBufs d, D
         scan_body(d.count, d.bcount, d.start, g.ncell, pg.nb, g.N, d.sc, 0, i);
 }
 
-// LZ: log2 of a power-of-two mesh, or 0: another size, EPT elements per thread
+// LZ: log2 of a power-of-two mesh, or 0: another size, by its plan (EPT = 0) or
+// with EPT elements per thread
 template <typename R, int LZ, int EPT>
 __global__ __launch_bounds__(LZ ? FFT_MAX_THREADS : FFT_THREADS) void k_r2c_fill(Geo g, DevBufs d, int rows, int stride,
-                                                                                 PairGrid pg) {
+                                                                                 MixPlan mp, PairGrid pg) {
     using C = typename V2<R>::T;
     bool mesh;
     int i;
@@ -42,12 +44,12 @@ __global__ __launch_bounds__(LZ ? FFT_MAX_THREADS : FFT_THREADS) void k_r2c_fill
     if constexpr (LZ > 0)
         r2c_p2<R, LZ>((const R *)d.rho, (C *)d.ht, (const C *)d.tw, rows, blk);
     else
-        r2c_any<R, EPT>((const R *)d.rho, (C *)d.ht, (const C *)d.tw, g.Z, rows, stride, blk);
+        r2c_other<R, EPT>((const R *)d.rho, (C *)d.ht, (const C *)d.tw, g.Z, mp, rows, stride, blk);
 }
 
 template <typename R, int LZ, int EPT>
 __global__ __launch_bounds__(LZ ? FFT_MAX_THREADS : FFT_THREADS) void k_col_sort(Geo g, DevBufs d, int rows, int stride,
-                                                                                 PairGrid pg) {
+                                                                                 MixPlan mp, PairGrid pg) {
     using C = typename V2<R>::T;
     using C4 = typename V4<R>::T;
     bool mesh;
@@ -62,13 +64,13 @@ __global__ __launch_bounds__(LZ ? FFT_MAX_THREADS : FFT_THREADS) void k_col_sort
     if constexpr (LZ > 0)
         col_p2<R, LZ>((const C *)d.ht, (C4 *)d.gt, (const C *)d.tw, sq, lap, g, rows, i);
     else
-        col_any<R, EPT>((const C *)d.ht, (C4 *)d.gt, (const C *)d.tw, sq, lap, g, rows, stride, i);
+        col_other<R, EPT>((const C *)d.ht, (C4 *)d.gt, (const C *)d.tw, sq, lap, g, mp, rows, stride, i);
 }
 
 // UNIT: FP32 with all sigma and epsilon ratios 1
 template <typename R, int LZ, int EPT, bool UNIT>
 __global__ __launch_bounds__(LZ ? FFT_MAX_THREADS : FFT_THREADS) void k_c2r_wca(Geo g, DevBufs d, int rows, int stride,
-                                                                                int stage, PairGrid pg) {
+                                                                                MixPlan mp, int stage, PairGrid pg) {
     using C = typename V2<R>::T;
     using C4 = typename V4<R>::T;
     bool mesh;
@@ -92,7 +94,7 @@ __global__ __launch_bounds__(LZ ? FFT_MAX_THREADS : FFT_THREADS) void k_c2r_wca(
     if constexpr (LZ > 0)
         c2r_p2<R, LZ>((const C4 *)d.gt, (C *)d.fmesh, (const C *)d.tw, rows, blk);
     else
-        c2r_any<R, EPT>((const C4 *)d.gt, (C *)d.fmesh, (const C *)d.tw, g.Z, rows, stride, blk);
+        c2r_other<R, EPT>((const C4 *)d.gt, (C *)d.fmesh, (const C *)d.tw, g.Z, mp, rows, stride, blk);
 }
 
 // candidates staged by a WCA block of `threads` particles, and its LDS
@@ -142,24 +144,24 @@ template <typename R, int LZ, int EPT> static void launch_mesh_pair(bdk_t *h, in
     if (pass == 0) {
         const PairGrid pg(l.blocks, (int)nblk(h->g.N, l.threads));
         hipLaunchKernelGGL((k_r2c_fill<R, LZ, EPT>), dim3(pg.blocks()), blk, l.lds, h->stream, h->g, h->d, l.rows, l.stride,
-                           pg);
+                           l.mix, pg);
     } else if (pass == 1) {
         const PairGrid pg(l.blocks, (int)nblk(h->g.ncell, l.threads * SORT_CELLS));
         hipLaunchKernelGGL((k_col_sort<R, LZ, EPT>), dim3(pg.blocks()), blk, l.lds, h->stream, h->g, h->d, l.rows, l.stride,
-                           pg);
+                           l.mix, pg);
     } else if constexpr (sizeof(R) == 4) {
         const PairGrid pg(l.blocks, (int)nblk(h->g.N, l.threads));
         const size_t lds = std::max(l.lds, wca_lds(l.threads, unit));
         if (unit)
             hipLaunchKernelGGL((k_c2r_wca<R, LZ, EPT, true>), dim3(pg.blocks()), blk, lds, h->stream, h->g, h->d, l.rows,
-                               l.stride, wca_stage(l.threads), pg);
+                               l.stride, l.mix, wca_stage(l.threads), pg);
         else
             hipLaunchKernelGGL((k_c2r_wca<R, LZ, EPT, false>), dim3(pg.blocks()), blk, lds, h->stream, h->g, h->d, l.rows,
-                               l.stride, wca_stage(l.threads), pg);
+                               l.stride, l.mix, wca_stage(l.threads), pg);
     } else {
         const PairGrid pg(l.blocks, (int)nblk(h->g.N, l.threads / WCA_LANES));
         hipLaunchKernelGGL((k_c2r_wca<R, LZ, EPT, true>), dim3(pg.blocks()), blk, l.lds, h->stream, h->g, h->d, l.rows,
-                           l.stride, 0, pg);
+                           l.stride, l.mix, 0, pg);
     }
 }
 
@@ -172,7 +174,7 @@ template <typename R> static void launch_mesh_pairs(bdk_t *h) {
 #undef CALL
         } else {
 #define CALL(E) launch_mesh_pair<R, 0, E>(h, pass, l)
-            BDK_EPT_SWITCH(l.ept, CALL)
+            BDK_OTHER_SWITCH(l.ept, CALL)
 #undef CALL
         }
     }
@@ -206,7 +208,7 @@ hipError_t pairs_set_attributes() {
 #define CALL(E)                                         \
     MESH(float, 0, E) MESH(double, 0, E)              \
     big((const void *)k_c2r_wca<float, 0, E, false>);
-    CALL(8) CALL(16) CALL(32)
+    CALL(0) CALL(8) CALL(16) CALL(32)
 #undef CALL
 #undef MESH
 #define DS(S, Q)                                          \
