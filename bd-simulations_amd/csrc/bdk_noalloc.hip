@@ -17,7 +17,7 @@
 
 namespace {
 
-constexpr int kMaxBins = 4096;   // bins per histogram (the LDS histogram of k_pair_hist holds 3 x 4096)
+constexpr int kMaxBins = 4096;   // bins per histogram (a block's LDS histogram holds 3 x 4096)
 constexpr int kMaxDevices = 64;
 
 // [3][kMaxBins] ordered-pair counts (11, 12, 22): 96 KiB per GPU

@@ -23,6 +23,7 @@ import argparse
 import csv
 import glob
 import json
+import statistics
 import os
 import re
 import sys
@@ -102,10 +103,12 @@ def kernels(directory, step_kernels=STEP_KERNELS):
 
 
 def per_kernel_counter(directory):
+    """The median over a kernel's dispatches: that of a step (the few after an
+    upload, whose state is not yet in cell order, move several times as much)."""
     acc = defaultdict(lambda: defaultdict(list))
     for r in rows(directory, "counter_collection.csv"):
         acc[short(r["Kernel_Name"])][r["Counter_Name"]].append(float(r["Counter_Value"]))
-    return {k: {c: sum(v) / len(v) for c, v in cs.items()} for k, cs in acc.items()}
+    return {k: {c: statistics.median(v) for c, v in cs.items()} for k, cs in acc.items()}
 
 
 def probe_copy(directory, counter, copies):
