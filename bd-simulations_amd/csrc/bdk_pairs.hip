@@ -112,7 +112,7 @@ static size_t wca_lds(int threads, bool unit) {
 // two streams / paired (us): 2000 on 128^2 FP64 37 / 27, 16,000 on 256^2 40 /
 // 28, 64,000 on 512^2 with travel cap 48.5 / 39.0, 64,000 on 512^2 FP64 44.2 /
 // 41.6 (24 MB), 256,000 on 512^2 50.9 / 46.7 (26 MB), 128,000 on 512^2 FP64
-// 52.5 / 53.6 (29 MB), 256,000 on 720^2 66.8 / 67.2 (35 MB), 500,000 on 512^2
+// 52.5 / 53.6 (29 MB), 500,000 on 512^2
 // 59.5 / 61.7 (41 MB), 128,000 on 1024^2 48.8 / 48.6 (46 MB), 200,000 on 1024^2
 // FP64 71 / 73, 2M on 2048^2 164 / 191.
 bool pairs_apply(const bdk_t *h) {
