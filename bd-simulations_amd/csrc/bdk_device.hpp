@@ -153,6 +153,12 @@ __device__ __forceinline__ int wrap1(int u, int n) { return u < 0 ? u + n : (u >
 __device__ __forceinline__ bool zpow2(int Z) { return (Z & (Z - 1)) == 0; }
 // mesh index u in [-Z, 2Z) into [0, Z)
 template <bool P2> __device__ __forceinline__ int wrapz(int u, int Z) { return P2 ? (u & (Z - 1)) : wrap1(u, Z); }
+// any mesh index into [0, Z): a state may hold offsets of many boxes (|rel| < 1e9)
+template <bool P2> __device__ __forceinline__ int foldz(int u, int Z) {
+    if (P2) return u & (Z - 1);
+    const int v = wrap1(u, Z);
+    return (unsigned)v < (unsigned)Z ? v : wrapc(u, Z);
+}
 // x / d and x % d for 0 <= x < 2^22: a shift when d is a power of two, else
 // the float reciprocal corrected to the exact quotient
 struct Dv {

@@ -455,6 +455,12 @@ __device__ __forceinline__ void deposit_particle(const Geo &g, const DevBufs &d,
     R wx[3], wy[3];
     weights_r<R, SCHEME>(x, g, kp, wx);
     weights_r<R, SCHEME>(y, g, lp, wy);
+    if (!P2) {
+        // before the window's origin is taken off, so that wrapz's range holds
+        // (P2: its mask takes any index)
+        kp = foldz<P2>(kp, g.Z);
+        lp = foldz<P2>(lp, g.Z);
+    }
     constexpr bool F32 = std::is_same<R, float>::value;
     auto charge = [&](int ia, int ib, float &cf, double &cd) {
         if (F32)
