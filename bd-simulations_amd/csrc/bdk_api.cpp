@@ -390,6 +390,7 @@ int upload(bdk_t *h) {
                                      h->stream));
         }
     }
+    h->running = true;
     HIPCHK(h, bdkx::launch_place(h, (const int2 *)(from + relb), (const double2 *)from));
     if (from != h->pin) HIPCHK(h, hipStreamSynchronize(h->stream));
     h->dev_valid = true;
@@ -410,6 +411,7 @@ int ensure_forces(bdk_t *h) {
     int rc = ensure(h);
     if (rc) return rc;
     if (h->forces_ready) return BDK_OK;
+    h->running = true;
     HIPCHK(h, bdkx::enqueue_forces(h));
     h->forces_ready = true;
     return BDK_OK;
@@ -553,14 +555,22 @@ struct bdk_batch {
         *g = gg;
         return hipGraphInstantiate(x, gg, nullptr, nullptr, 0);
     }
-    // a member's asynchronous pos write copies on the member's stream: the
-    // batch's steps wait for those copies
-    hipError_t wait_writers() {
-        for (bdk_t *h : mem)
+    // What a member's own calls left on its stream (an upload, which does not
+    // wait, bdk_prepare's forces) and the copies of an asynchronous pos write
+    // come before anything of the batch that reads or writes the member.
+    hipError_t await_members() {
+        for (bdk_t *h : mem) {
+            if (h->running) {
+                hipError_t e = hipEventRecord(ev_fork, h->stream);
+                if (e == hipSuccess) e = hipStreamWaitEvent(stream, ev_fork, 0);
+                if (e != hipSuccess) return e;
+                h->running = false;
+            }
             if (h->writer.pending) {
                 hipError_t e = hipStreamWaitEvent(stream, h->writer.ev, 0);
                 if (e != hipSuccess) return e;
             }
+        }
         return hipSuccess;
     }
     // members uploaded since their last step get their forces first.  When
@@ -569,11 +579,12 @@ struct bdk_batch {
     // FFT tiling: a member's forces depend only on its own state and the
     // tiling, so they equal what the whole batch would compute.
     hipError_t ensure_forces() {
+        hipError_t e = await_members();
+        if (e != hipSuccess) return e;
         std::vector<bdk_t *> need;
         for (bdk_t *h : mem)
             if (!h->forces_ready) need.push_back(h);
         if (need.empty()) return hipSuccess;
-        hipError_t e = hipSuccess;
         if (need.size() == mem.size()) {
             e = bdkx::batch_enqueue_forces(bp, stream, aux, ev_fork, ev_join);
         } else {
@@ -971,6 +982,7 @@ int bdk_step(bdk_t *h, double tmax, double *dt_out) {
     }
     int rc = ensure_forces(h);
     if (rc) return rc;
+    h->running = true;
     if (h->g.idgas) {
         HIPCHK(h, hipMemsetAsync(h->d.fmesh, 0, (size_t)h->g.Z * h->g.Z * 2 * real_size(h->p), h->stream));
     }
@@ -2089,6 +2101,7 @@ int bdk_batch_create(bdk_t *const *members, int32_t n, bdk_batch_t **out) {
         if (rc) return fail(nullptr, rc, who + h->err);
         if (hipStreamSynchronize(h->stream) != hipSuccess)
             return fail(nullptr, BDK_ERR_HIP, who + "stream synchronisation failed");
+        h->running = false;
         zmax = std::max(zmax, h->g.Z);
     }
     bdk_batch_t *b = new bdk_batch();
@@ -2134,7 +2147,6 @@ int bdk_batch_run_steps(bdk_batch_t *b, int64_t k) {
     hipError_t e = hipSetDevice(b->dev);
     if (e == hipSuccess) e = b->ensure_forces();
     if (e == hipSuccess) e = b->ensure_graphs();
-    if (e == hipSuccess) e = b->wait_writers();
     int64_t i = 0;
     for (; e == hipSuccess && i + kGraphSteps <= k; i += kGraphSteps) e = hipGraphLaunch(b->gexec_multi, b->stream);
     for (; e == hipSuccess && i < k; ++i) e = hipGraphLaunch(b->gexec, b->stream);
@@ -2145,7 +2157,8 @@ int bdk_batch_run_steps(bdk_batch_t *b, int64_t k) {
 
 int bdk_batch_sync(bdk_batch_t *b) {
     if (!b) return fail(nullptr, BDK_ERR_ARG, "null batch");
-    hipError_t e = hipStreamSynchronize(b->stream);
+    hipError_t e = b->await_members();
+    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
     if (e != hipSuccess) return b->fail(BDK_ERR_HIP, std::string("bdk_batch_sync: ") + hipGetErrorString(e));
     for (size_t i = 0; i < b->mem.size(); ++i) {
         DevScalars sc;
@@ -2161,7 +2174,8 @@ int bdk_batch_sync(bdk_batch_t *b) {
 int bdk_batch_status(bdk_batch_t *b, int32_t n, int32_t *status) {
     if (!b) return fail(nullptr, BDK_ERR_ARG, "null batch");
     if (!status || n != (int32_t)b->mem.size()) return b->fail(BDK_ERR_ARG, "status needs one entry per member");
-    hipError_t e = hipStreamSynchronize(b->stream);
+    hipError_t e = b->await_members();
+    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
     for (int32_t i = 0; i < n && e == hipSuccess; ++i) {
         DevScalars sc;
         e = hipMemcpy(&sc, b->mem[i]->d.sc, sizeof(sc), hipMemcpyDeviceToHost);
@@ -2181,10 +2195,7 @@ int bdk_batch_profile(bdk_batch_t *b, int32_t stage, int32_t reps, double *ms_pe
     if (e == hipSuccess) e = b->ensure_forces();
     if (e == hipSuccess) e = b->ensure_graphs();
     auto launch = [&]() -> hipError_t {
-        if (stage == 7) {
-            hipError_t w = b->wait_writers();
-            return w != hipSuccess ? w : hipGraphLaunch(b->gexec, b->stream);
-        }
+        if (stage == 7) return hipGraphLaunch(b->gexec, b->stream);
         return bdkx::batch_stage(b->bp, stage, b->stream);
     };
     hipEvent_t e0 = nullptr, e1 = nullptr;

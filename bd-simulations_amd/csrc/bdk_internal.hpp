@@ -200,6 +200,7 @@ struct bdk {
     bool pos_set[2] = {false, false};
     bool dev_valid = false;       // device particle state uploaded
     bool forces_ready = false;    // fwca / fmesh hold the forces of the current state
+    bool running = false;         // a call left work on `stream` that no batch has been ordered behind yet
     std::vector<int32_t> hgit[2];
     std::vector<double> hrel[2];
     int scan_blocks = 0;
