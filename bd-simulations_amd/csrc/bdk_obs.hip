@@ -80,7 +80,7 @@ __device__ __forceinline__ void shell_sums(const C *s, F &&at, int m, int Z, dou
                 w = (two ? 1.0 : 0.5) * ((double)P.x + (double)Q.x);
             else
                 w = (two ? 1.0 : 0.5) * ((double)P.y + (double)Q.y);
-            v += ((m > 0 ? a + m : a) & 1) ? -w : w;
+            v += ((a + col) & 1) ? -w : w;  // (-1)^(j + col), Z even
             n += two ? 2.0 : 1.0;
         }
         double *p = part + (size_t)col * 2 * nbins;
