@@ -138,6 +138,12 @@ void release_streams(bdk_t *h) {
     h->aux = h->stream = nullptr;
 }
 
+void drop_scratch(bdk_t *h) {
+    if (h->ws) (void)hipFree(h->ws);  // waits for the device
+    h->ws = nullptr;
+    h->ws_cap = 0;
+}
+
 void free_dev(bdk_t *h) {
     void *ptrs[] = {h->d.cell, h->d.rel, h->d.pid, h->d.fwca, h->d.fkap, h->d.noise_up, h->d.noise_out,
                     h->d.rank, h->d.count, h->d.arr, h->d.start, h->d.list, h->d.lcell, h->d.lrel, h->d.lpid, h->d.lrelf, h->d.bcount, h->d.own, h->d.start_old, h->d.exo, h->d.dts, h->d.dtlog, h->d.comp, h->d.lcomp, h->d.rho, h->d.ht,
@@ -145,9 +151,7 @@ void free_dev(bdk_t *h) {
                     h->d.qvf, h->d.sc};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
-    if (h->ws) (void)hipFree(h->ws);
-    h->ws = nullptr;
-    h->ws_cap = 0;
+    drop_scratch(h);
     if (h->pin) (void)hipHostFree(h->pin);
     h->pin = nullptr;
     h->pin_cap = 0;
@@ -169,35 +173,39 @@ template <typename T> hipError_t dalloc(T *&p, size_t n) {
 
 hipError_t dalloc_v(void *&p, size_t bytes) { return hipMalloc(&p, bytes > 0 ? bytes : 16); }
 
-// Device scratch of one observable call, taken from the handle.  It is kept
-// for the next call up to kKeepScratch (a hipMalloc and hipFree pair and the
-// synchronisation they imply cost more than a small observable's kernels);
-// more is given back when the call ends.
+// Device scratch of one observable call: the noise_out array (16 bytes per
+// particle, otherwise bdk_get_noise's), or where that is too small (the direct
+// rho(k) sums, shells or grids of few particles) an allocation, kept up to
+// kKeepScratch while observables are taken (a hipMalloc and hipFree pair and
+// the synchronisation they imply cost more than a small observable's kernels)
+// and given back by the next upload or step (drop_scratch): a handle that
+// steps holds what footprint_of counts.
 constexpr size_t kKeepScratch = 64u << 20;
 struct Scratch {
     bdk_t *h;
+    char *base = nullptr;
     size_t used = 0;
     explicit Scratch(bdk_t *h_) : h(h_) {}
     ~Scratch() {
-        if (h->ws_cap <= kKeepScratch) return;
-        (void)hipFree(h->ws);  // waits for the device
-        h->ws = nullptr;
-        h->ws_cap = 0;
+        if (h->ws_cap > kKeepScratch) drop_scratch(h);
     }
     static size_t pad(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
     // room for parts of `bytes` in all (each padded); then take() them in turn
     hipError_t reserve(size_t bytes) {
         used = 0;
-        if (bytes <= h->ws_cap) return hipSuccess;
-        if (h->ws) (void)hipFree(h->ws);
-        h->ws = nullptr;
-        h->ws_cap = 0;
-        const hipError_t e = hipMalloc(&h->ws, bytes);
-        if (e == hipSuccess) h->ws_cap = bytes;
-        return e;
+        base = (char *)h->d.noise_out;
+        if (bytes <= (size_t)h->g.N * 16) return hipSuccess;
+        if (bytes > h->ws_cap) {
+            drop_scratch(h);
+            const hipError_t e = hipMalloc(&h->ws, bytes);
+            if (e != hipSuccess) return e;
+            h->ws_cap = bytes;
+        }
+        base = (char *)h->ws;
+        return hipSuccess;
     }
     template <typename T> T *take(size_t n) {
-        T *p = (T *)((char *)h->ws + used);
+        T *p = (T *)(base + used);
         used += pad(n * sizeof(T));
         return p;
     }
@@ -366,12 +374,17 @@ int upload(bdk_t *h) {
                 return fail(h, BDK_ERR_NONFINITE, "non-finite rel" + who);
         }
     }
+    drop_scratch(h);
     // [rel | git], both by id.  Up to kPinned bytes the kernel reads the pinned
-    // staging itself and the upload does not wait; more is copied first.
+    // staging itself and the upload does not wait; more is copied first, into
+    // the arrays of the list order, which the lists are then built into.
     const size_t relb = (size_t)N * 16, bytes = (size_t)N * 24;
-    Scratch ws(h);
+    const double2 *rel = h->d.lrel;
+    const int2 *git = (const int2 *)h->d.lrelf;
     char *from = pinned(h, bytes);
     if (from) {
+        rel = (const double2 *)from;
+        git = (const int2 *)(from + relb);
         if (h->pin_read) HIPCHK(h, hipStreamSynchronize(h->stream));  // the last upload's kernel
         for (int sp = 0; sp < 2; ++sp) {
             const size_t n = sp == 0 ? n1 : n2, off = sp == 0 ? 0 : n1;
@@ -380,19 +393,16 @@ int upload(bdk_t *h) {
         }
         h->pin_read = true;
     } else {
-        HIPCHK(h, ws.reserve(Scratch::pad(bytes)));
-        from = ws.take<char>(bytes);
         for (int sp = 0; sp < 2; ++sp) {
             const size_t n = sp == 0 ? n1 : n2, off = sp == 0 ? 0 : n1;
             if (!n) continue;
-            HIPCHK(h, hipMemcpyAsync(from + off * 16, h->hrel[sp].data(), n * 16, hipMemcpyHostToDevice, h->stream));
-            HIPCHK(h, hipMemcpyAsync(from + relb + off * 8, h->hgit[sp].data(), n * 8, hipMemcpyHostToDevice,
-                                     h->stream));
+            HIPCHK(h, hipMemcpyAsync(h->d.lrel + off, h->hrel[sp].data(), n * 16, hipMemcpyHostToDevice, h->stream));
+            HIPCHK(h, hipMemcpyAsync(h->d.lrelf + off, h->hgit[sp].data(), n * 8, hipMemcpyHostToDevice, h->stream));
         }
     }
     h->running = true;
-    HIPCHK(h, bdkx::launch_place(h, (const int2 *)(from + relb), (const double2 *)from));
-    if (from != h->pin) HIPCHK(h, hipStreamSynchronize(h->stream));
+    HIPCHK(h, bdkx::launch_place(h, git, rel));
+    if (!from) HIPCHK(h, hipStreamSynchronize(h->stream));
     h->dev_valid = true;
     h->forces_ready = false;
     return BDK_OK;
@@ -410,6 +420,7 @@ int ensure(bdk_t *h) {
 int ensure_forces(bdk_t *h) {
     int rc = ensure(h);
     if (rc) return rc;
+    drop_scratch(h);
     if (h->forces_ready) return BDK_OK;
     h->running = true;
     HIPCHK(h, bdkx::enqueue_forces(h));
@@ -420,9 +431,7 @@ int ensure_forces(bdk_t *h) {
 // list-ordered device array of real2 -> per-species [n][2] doubles
 int download_forces(bdk_t *h, const void *src, double *f1, double *f2) {
     const size_t n1 = h->p.n1, n2 = h->p.n2, N = n1 + n2;
-    Scratch ws(h);
-    HIPCHK(h, ws.reserve(Scratch::pad(N * 16)));
-    double2 *out = ws.take<double2>(N);
+    double2 *out = h->d.noise_out;
     if (char *stage = pinned(h, Scratch::pad(N * 16))) {
         const bool direct = N <= (size_t)kDirectIds;
         HIPCHK(h, bdkx::launch_force_by_id(h, src, direct ? (double2 *)stage : out));
@@ -581,6 +590,7 @@ struct bdk_batch {
     hipError_t ensure_forces() {
         hipError_t e = await_members();
         if (e != hipSuccess) return e;
+        for (bdk_t *h : mem) drop_scratch(h);
         std::vector<bdk_t *> need;
         for (bdk_t *h : mem)
             if (!h->forces_ready) need.push_back(h);
@@ -873,32 +883,40 @@ int bdk_get_positions(bdk_t *h, int species, int32_t n, int32_t *git, double *re
     if (species != 1 && species != 2) return fail(h, BDK_ERR_ARG, "species must be 1 or 2");
     const int n1 = h->p.n1;
     if (n != (species == 1 ? n1 : h->p.n2)) return fail(h, BDK_ERR_ARG, "n does not match");
-    // [flags | offsets | cells], in id order
-    const size_t head = sizeof(bdkx::ByIdHead), bytes = head + (size_t)n * 24;
-    Scratch ws(h);
-    HIPCHK(h, ws.reserve(Scratch::pad(bytes)));
-    char *out = ws.take<char>(bytes);
-    char *stage = pinned(h, Scratch::pad(bytes));
-    const bool direct = stage && n <= kDirectIds;
-    char *to = direct ? stage : out;
-    double2 *orel = (double2 *)(to + head);
-    int2 *ogit = (int2 *)(to + head + (size_t)n * 16);
-    HIPCHK(h, bdkx::launch_by_id(h, species == 1 ? 0 : n1, n, (bdkx::ByIdHead *)to, ogit, orel));
-    bdkx::ByIdHead flags;
-    if (stage) {
-        if (!direct) HIPCHK(h, bdkx::launch_to_host(out, bytes, stage, h->stream));
-        HIPCHK(h, hipStreamSynchronize(h->stream));
-        std::memcpy(&flags, stage, head);
-        if (rel && n) std::memcpy(rel, stage + head, (size_t)n * 16);
-        if (git && n) std::memcpy(git, stage + head + (size_t)n * 16, (size_t)n * 8);
+    // [flags | offsets | cells] in id order.  On the device the offsets and
+    // cells share the noise_out array (16 bytes per particle of both species);
+    // those of one species alone go through it one after the other.
+    const size_t head = sizeof(bdkx::ByIdHead), relb = (size_t)n * 16, gitb = (size_t)n * 8;
+    const int id0 = species == 1 ? 0 : n1;
+    char *stage = pinned(h, Scratch::pad(head + relb + gitb));
+    char *first = stage ? stage : pinned(h, head);
+    bdkx::ByIdHead *flags = (bdkx::ByIdHead *)first;
+    double2 *orel = h->d.noise_out;
+    const bool both = relb + gitb <= (size_t)h->g.N * 16;
+    int2 *ogit = (int2 *)(both ? orel + n : orel);
+    if (stage && n <= kDirectIds) {
+        HIPCHK(h, bdkx::launch_by_id(h, id0, n, flags, (int2 *)(stage + head + relb), (double2 *)(stage + head)));
     } else {
-        HIPCHK(h, hipMemcpyAsync(&flags, out, head, hipMemcpyDeviceToHost, h->stream));
-        if (rel) HIPCHK(h, hipMemcpyAsync(rel, orel, (size_t)n * 16, hipMemcpyDeviceToHost, h->stream));
-        if (git) HIPCHK(h, hipMemcpyAsync(git, ogit, (size_t)n * 8, hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(h, hipStreamSynchronize(h->stream));
+        auto out = [&](const void *dev, size_t off, size_t bytes, void *dst) {
+            return stage ? bdkx::launch_to_host(dev, bytes, stage + head + off, h->stream)
+                         : hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, h->stream);
+        };
+        HIPCHK(h, bdkx::launch_by_id(h, id0, n, flags, both ? ogit : nullptr, orel));
+        if (stage && both) {
+            HIPCHK(h, out(orel, 0, relb + gitb, nullptr));
+        } else {
+            if (rel) HIPCHK(h, out(orel, 0, relb, rel));
+            if (git && !both) HIPCHK(h, bdkx::launch_by_id(h, id0, n, nullptr, ogit, nullptr));
+            if (git) HIPCHK(h, out(ogit, relb, gitb, git));
+        }
     }
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    h->pin_read = false;
+    if (stage && rel && n) std::memcpy(rel, stage + head, relb);
+    if (stage && git && n) std::memcpy(git, stage + head + relb, gitb);
+    if (!flags) return check_nonfinite(h);
     std::string m;
-    rc = flag_status(flags.flags, &m);
+    rc = flag_status(flags->flags, &m);
     return rc ? fail(h, rc, m) : BDK_OK;
 }
 

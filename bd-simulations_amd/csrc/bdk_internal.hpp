@@ -87,7 +87,8 @@ struct DevBufs {
     void *fwca = nullptr;     // [N] real2, list order
     void *fkap = nullptr;     // [N] real2, list order
     double2 *noise_up = nullptr; // [N] by particle id (upload mode)
-    double2 *noise_out = nullptr; // [N] by particle id (bdk_get_noise)
+    double2 *noise_out = nullptr; // [N] by particle id (bdk_get_noise); between calls scratch for results on their
+                                  // way to the host and for the observables
     int *rank = nullptr;      // [N] rank of the slot inside its cell
     // cell list
     int *count = nullptr;     // [ncell] particles per cell (kept current across steps)
@@ -211,7 +212,7 @@ struct bdk {
     std::string err;
     int64_t host_step = 0;
     bdkx::StepInfoDev *info_dev = nullptr;  // step counters (bdk_step_info), allocated on first use
-    void *ws = nullptr;            // scratch of the observables (bdk_api.cpp: Scratch), kept up to kKeepScratch
+    void *ws = nullptr;            // scratch of the observables beyond the handle's own arrays (bdk_api.cpp: Scratch)
     size_t ws_cap = 0;
     double *hdt = nullptr;         // pinned host copy of a single step's adaptive dt, and the event after its update
     hipEvent_t ev_dt = nullptr;
@@ -229,7 +230,7 @@ hipError_t launch_wca(bdk_t *h, hipStream_t st = nullptr);  // WCA forces -> fwc
 hipError_t launch_deposit(bdk_t *h, int reset, int slot = 0, hipStream_t st = nullptr);  // charges -> rho
                                                   // (reset: re-arm per-step scalars; slot: during a rebuild)
 hipError_t launch_species_deposit(bdk_t *h, int species);  // number density of one species -> rho
-// cells and offsets of ids id0 .. id0 + n - 1 in id order, and the error flags
+// cells and offsets of ids id0 .. id0 + n - 1 in id order, and the error flags (null: not wanted)
 struct ByIdHead {
     int flags;
     int pad[63];

@@ -538,19 +538,19 @@ __global__ void k_noise_out(Geo g, DevBufs d) {
 }
 
 // Cells and offsets of one species (ids id0 .. id0 + n - 1) in id order, for
-// the host, after a header with the error flags: the scatter by id that a
+// the host, and the error flags (null: not wanted): the scatter by id that a
 // host thread would do over the whole state runs here (a random 24 B write
 // per particle; 20 us at 2M particles against 15 ms), and only the species
 // asked for crosses to the host.
 __global__ void k_by_id(Geo g, DevBufs d, int id0, int n, ByIdHead *head, int2 *git, double2 *rel) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s == 0) head->flags = d.sc->nonfinite;
+    if (s == 0 && head) head->flags = d.sc->nonfinite;
     if (s >= g.N) return;
     const int i = d.pid[s] - id0;
     if ((unsigned)i >= (unsigned)n) return;
     const int c = d.cell[s], gx = div_nc(c, g);
-    git[i] = make_int2(gx, c - gx * g.nc);
-    rel[i] = d.rel[s];
+    if (git) git[i] = make_int2(gx, c - gx * g.nc);
+    if (rel) rel[i] = d.rel[s];
 }
 
 // n 16-byte words into pinned host memory, a wave's 1 KB per store; bound by

@@ -167,7 +167,11 @@ int bdk_get_cells(bdk_t *h, int32_t *start, int32_t *ids);
    BDK_MESH_RHO = rhox[..][0] (gr:31-547), FX/FY = Fx/Fy[..][0] (dm:1221-1222). */
 int bdk_get_mesh(bdk_t *h, int which, double *out);
 
-/* Device memory this parameter set needs, bytes (admission by footprint). */
+/* Device memory this parameter set needs, bytes (admission by footprint):
+   what a handle holds while it steps and its positions and forces are read.
+   The observables work in the same memory (16 bytes per particle of it) or,
+   where they need more, in an allocation of their own, which stays until the
+   next upload or step if it is at most 64 MB. */
 int bdk_footprint(const bd_params *p, uint64_t *bytes);
 
 /* Per-kernel timing of k steps with HIP events on the handle's stream.
@@ -338,7 +342,7 @@ int bdk_density_stats(bdk_t *h, int32_t m, int32_t nbins, double dbin, const dou
    unless bd_params.ftrho_fix is set (then rel_y, as species 2 uses).
    re/im receive *npairs (<= qbins^2) entries; the shells by i^2 + j^2 are
    the caller's (init_ftrho, au:262-300).  Device scratch: at most 18 MB of
-   partial sums, kept with the handle. */
+   partial sums. */
 int bdk_ftrho_sums(bdk_t *h, int32_t species, int32_t qbins, double dq_ft, double *re, double *im, int32_t *npairs);
 
 /* ---------------------------------------------------------------- batches
