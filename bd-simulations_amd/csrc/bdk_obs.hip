@@ -737,17 +737,29 @@ hipError_t launch_snap(bdk_t *h, int m, double *rho, int stats, int nbins, doubl
 // [-pi, pi] before the sine and cosine without rounding (i u - 2 rint(i u / 2)
 // with u = x dq / pi kept in two doubles), so the sums come out nearer to
 // exact arithmetic than with one rounded angle per pair (against extended
-// precision: 1e-16 to 7e-16 of their norm, before 3e-15 to 2e-14).
+// precision: at most 4e-16 of their norm, the other way up to 3e-14).
 //
-// A block takes a tile of 32 x 32 index pairs and a part of the list: it
-// queues the species' particles in list order, and for every 32 of them
-// writes both factors to LDS and each of its four waves multiplies a 16 x 16
-// quarter.  The parts are added in order (k_sum_rows).  Bound by the FP64
-// sine/cosine evaluations.  20,000 particles, 30 x 30: 2 x 58 -> 2 x 15 us.
-constexpr int FT_THREADS = 256, FT_TILE = 32, FT_K = 32;
-// LDS row of one particle's factors: 32 cosines, 32 sines, padded so that two
-// consecutive rows' quarters read by half a wave lie in different banks
-constexpr int FT_ROW = 80;
+// A block takes a tile of P x P index pairs (P = 32; 16 or 8 for qbins up to
+// that) and a part of the list: it queues the species' particles in list order,
+// writes both factors of every FtTile::K of them to LDS, and its four waves
+// multiply: a 16 x 16 quarter each (P = 32), or every fourth of the particles
+// each (P = 16: real and imaginary parts as two products; P = 8: one product
+// of [cos | sin] by [cos | sin]), added in order of the waves at the end.  The
+// parts are added in order (k_sum_rows).  Bound by the FP64 sine/cosine
+// evaluations, 2 P per particle.
+// Both species of 2 x 500,000 particles (us a pair of calls): 5 bins 112, 16
+// bins 181, 30 bins 375.  With P = 32 for all: 374 throughout; one sine/cosine
+// pair per particle and wave vector: 1 bin 176, 5 bins 250, 8 bins 414, 16 bins
+// 1236.  2 x 10,000: 47 / 51 / 57, P = 32 for all 55, one pair each 105 to 180.
+// (One factor per thread instead of both costs P = 32 a sixth: 438.)
+constexpr int FT_THREADS = 256, FT_TILE = 32;
+template <int P> struct FtTile {
+    static constexpr int K = P == 8 ? 64 : 32;  // particles per round
+    // LDS row of one particle's factors: P cosines, P sines, padded to 16 mod 32
+    // doubles, so that two consecutive rows' parts read by half a wave lie in
+    // different banks
+    static constexpr int ROW = P == 32 ? 80 : (P == 16 ? 48 : 16);
+};
 
 typedef double ft_acc __attribute__((ext_vector_type(4)));
 
@@ -757,13 +769,16 @@ __device__ __forceinline__ void ft_factor(int k, double uh, double ul, double *c
     sincospi((t - 2.0 * rint(0.5 * t)) + te, sn, cs);
 }
 
+template <int P>
 __global__ __launch_bounds__(FT_THREADS) void k_ftrho(Geo g, DevBufs d, int species, int fix, int qbins, int nt,
                                                       double ch, double cl, int per, double *part) {
-    __shared__ double X[FT_K * FT_ROW], Y[FT_K * FT_ROW];
-    __shared__ double2 queue[FT_THREADS + FT_K];
-    __shared__ int wcnt[FT_THREADS / 64];
+    constexpr int K = FtTile<P>::K, ROW = FtTile<P>::ROW, WAVES = FT_THREADS / 64;
+    __shared__ double S[2 * K * ROW];
+    __shared__ double2 queue[FT_THREADS + K];
+    __shared__ int wcnt[WAVES];
+    double *X = S, *Y = S + K * ROW;
     const int ti = (int)blockIdx.y / nt, tj = (int)blockIdx.y - ti * nt;
-    if (FT_TILE * FT_TILE * (ti * ti + tj * tj) > qbins * qbins) return;  // beyond the quarter circle
+    if (P * P * (ti * ti + tj * tj) > qbins * qbins) return;  // beyond the quarter circle
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wi = (wave >> 1) * 16, wj = (wave & 1) * 16;
     const int q0 = blockIdx.x * per, q1 = min(q0 + per, g.N);
@@ -785,7 +800,7 @@ __global__ __launch_bounds__(FT_THREADS) void k_ftrho(Geo g, DevBufs d, int spec
         if (lane == 0) wcnt[wave] = __popcll(mask);
         __syncthreads();
         int pos = n + __popcll(mask & ((1ull << lane) - 1ull));
-        for (int w = 0; w < FT_THREADS / 64; ++w) {
+        for (int w = 0; w < WAVES; ++w) {
             if (w < wave) pos += wcnt[w];
             n += wcnt[w];
         }
@@ -793,38 +808,70 @@ __global__ __launch_bounds__(FT_THREADS) void k_ftrho(Geo g, DevBufs d, int spec
         __syncthreads();
         int head = 0;
         const bool last = base + FT_THREADS >= q1;
-        while (n - head >= FT_K || (last && n > head)) {
-            const int m = min(FT_K, n - head);
-            // factors: index tid % 32, particles tid / 32 + 8 e
-            for (int e = 0; e < FT_K / 8; ++e) {
-                const int i = tid & 31, k = (tid >> 5) + 8 * e;
-                double cx = 0.0, sx = 0.0, cy = 0.0, sy = 0.0;
-                if (k < m) {
-                    const double2 p = queue[head + k];
-                    const double ux = p.x * ch, uy = p.y * ch;
-                    ft_factor(FT_TILE * ti + i, ux, fma(p.x, ch, -ux) + p.x * cl, &cx, &sx);
-                    ft_factor(FT_TILE * tj + i, uy, fma(p.y, ch, -uy) + p.y * cl, &cy, &sy);
+        while (n - head >= K || (last && n > head)) {
+            const int m = min(K, n - head);
+            if constexpr (P == 32) {
+                // both factors: index tid % 32, particles tid / 32 + 8 e
+                for (int e = 0; e < K / 8; ++e) {
+                    const int i = tid & 31, k = (tid >> 5) + 8 * e;
+                    double cx = 0.0, sx = 0.0, cy = 0.0, sy = 0.0;
+                    if (k < m) {
+                        const double2 p = queue[head + k];
+                        const double ux = p.x * ch, uy = p.y * ch;
+                        ft_factor(P * ti + i, ux, fma(p.x, ch, -ux) + p.x * cl, &cx, &sx);
+                        ft_factor(P * tj + i, uy, fma(p.y, ch, -uy) + p.y * cl, &cy, &sy);
+                    }
+                    X[k * ROW + i] = cx;
+                    X[k * ROW + P + i] = sx;
+                    Y[k * ROW + i] = cy;
+                    Y[k * ROW + P + i] = sy;
                 }
-                X[k * FT_ROW + i] = cx;
-                X[k * FT_ROW + 32 + i] = sx;
-                Y[k * FT_ROW + i] = cy;
-                Y[k * FT_ROW + 32 + i] = sy;
+            } else {
+                // one factor: of x by the first P of 2 P threads, of y by the others
+                const int i = tid & (P - 1), iy = (tid / P) & 1;
+                double *row = (iy ? Y : X) + i;
+                for (int k = tid / (2 * P); k < K; k += FT_THREADS / (2 * P)) {
+                    double c = 0.0, s = 0.0;
+                    if (k < m) {
+                        const double2 p = queue[head + k];
+                        const double v = iy ? p.y : p.x, u = v * ch;
+                        ft_factor(i, u, fma(v, ch, -u) + v * cl, &c, &s);
+                    }
+                    row[k * ROW] = c;
+                    row[k * ROW + P] = s;
+                }
             }
             __syncthreads();
+            // operands: row (column) lane % 16 of particle k + lane / 16
+            if constexpr (P == 32) {
 #pragma unroll
-            for (int k = 0; k < FT_K; k += 4) {
-                // operands: row (column) lane % 16 of particle k + lane / 16
-                const int o = (k + (lane >> 4)) * FT_ROW + (lane & 15);
-                const double xc = X[o + wi], xs = X[o + wi + 32], yc = Y[o + wj], ys = Y[o + wj + 32];
-                re = __builtin_amdgcn_mfma_f64_16x16x4f64(xc, yc, re, 0, 0, 0);
-                re = __builtin_amdgcn_mfma_f64_16x16x4f64(-xs, ys, re, 0, 0, 0);
-                im = __builtin_amdgcn_mfma_f64_16x16x4f64(xs, yc, im, 0, 0, 0);
-                im = __builtin_amdgcn_mfma_f64_16x16x4f64(xc, ys, im, 0, 0, 0);
+                for (int k = 0; k < K; k += 4) {
+                    const int o = (k + (lane >> 4)) * ROW + (lane & 15);
+                    const double xc = X[o + wi], xs = X[o + wi + P], yc = Y[o + wj], ys = Y[o + wj + P];
+                    re = __builtin_amdgcn_mfma_f64_16x16x4f64(xc, yc, re, 0, 0, 0);
+                    re = __builtin_amdgcn_mfma_f64_16x16x4f64(-xs, ys, re, 0, 0, 0);
+                    im = __builtin_amdgcn_mfma_f64_16x16x4f64(xs, yc, im, 0, 0, 0);
+                    im = __builtin_amdgcn_mfma_f64_16x16x4f64(xc, ys, im, 0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int k = 4 * wave; k < K; k += 4 * WAVES) {
+                    const int o = (k + (lane >> 4)) * ROW + (lane & 15);
+                    if constexpr (P == 16) {
+                        const double xc = X[o], xs = X[o + P], yc = Y[o], ys = Y[o + P];
+                        re = __builtin_amdgcn_mfma_f64_16x16x4f64(xc, yc, re, 0, 0, 0);
+                        re = __builtin_amdgcn_mfma_f64_16x16x4f64(-xs, ys, re, 0, 0, 0);
+                        im = __builtin_amdgcn_mfma_f64_16x16x4f64(xs, yc, im, 0, 0, 0);
+                        im = __builtin_amdgcn_mfma_f64_16x16x4f64(xc, ys, im, 0, 0, 0);
+                    } else {
+                        re = __builtin_amdgcn_mfma_f64_16x16x4f64(X[o], Y[o], re, 0, 0, 0);
+                    }
+                }
             }
             __syncthreads();
             head += m;
         }
-        // what is left (fewer than FT_K) moves to the front
+        // what is left (fewer than K) moves to the front
         n -= head;
         double2 keep;
         if (tid < n) keep = queue[head + tid];
@@ -832,23 +879,48 @@ __global__ __launch_bounds__(FT_THREADS) void k_ftrho(Geo g, DevBufs d, int spec
         if (tid < n) queue[tid] = keep;
     }
     // results: column lane % 16, rows lane / 16 + 4 r
-    const int qp = FT_TILE * nt;
+    const int qp = P * nt;
     double *out = part + (size_t)blockIdx.x * 2 * qp * qp;
+    if constexpr (P == 32) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const size_t o = (size_t)(FT_TILE * ti + wi + (lane >> 4) + 4 * r) * qp + FT_TILE * tj + wj + (lane & 15);
-        out[o] = re[r];
-        out[(size_t)qp * qp + o] = im[r];
+        for (int r = 0; r < 4; ++r) {
+            const size_t o = (size_t)(P * ti + wi + (lane >> 4) + 4 * r) * qp + P * tj + wj + (lane & 15);
+            out[o] = re[r];
+            out[(size_t)qp * qp + o] = im[r];
+        }
+    } else {
+        constexpr int TILE = P == 16 ? 512 : 256;  // values of a wave
+        static_assert(WAVES * TILE <= 2 * K * ROW, "the waves' sums lie where the factors were");
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int o = wave * TILE + ((lane >> 4) + 4 * r) * 16 + (lane & 15);
+            S[o] = re[r];
+            if (P == 16) S[o + 256] = im[r];
+        }
+        __syncthreads();
+        auto sum = [&](int o) { return ((S[o] + S[o + TILE]) + S[o + 2 * TILE]) + S[o + 3 * TILE]; };
+        if (P == 16) {
+            out[tid] = sum(tid);
+            out[256 + tid] = sum(256 + tid);
+        } else if (tid < 64) {
+            const int o = (tid >> 3) * 16 + (tid & 7);
+            out[tid] = sum(o) - sum(o + 8 * 16 + 8);
+            out[64 + tid] = sum(o + 8 * 16) + sum(o + 8);
+        }
     }
 }
 
-// parts of the list (a multiple of 64 positions each) such that about 1024
-// blocks run; side of the padded square of index pairs
+// the tile's side: one tile of 8 or 16 where that holds all indices, so that a
+// few wave vectors do not pay for 32 factors per axis; parts of the list (a
+// multiple of 64 positions each) such that about 1024 blocks run, 512 of a
+// small tile (5 / 16 bins, 2 x 500,000 and 2 x 100,000 particles, us: 256 parts
+// 132 / 223, 62 / 82; 512 111 / 182, 61 / 78; 1024 112 / 178, 68 / 86); side of
+// the padded square of index pairs
 FtPlan ftrho_plan(const bdk_t *h, int qbins) {
     FtPlan f;
-    const int nt = (int)nblk(qbins, FT_TILE);
-    f.side = FT_TILE * nt;
-    const int want = std::max(1, std::min(256, 1024 / (nt * nt)));
+    const int tile = qbins <= 8 ? 8 : (qbins <= 16 ? 16 : FT_TILE), nt = (int)nblk(qbins, tile);
+    f.side = tile * nt;
+    const int want = tile < FT_TILE ? 512 : std::max(1, std::min(256, 1024 / (nt * nt)));
     f.per = (int)nblk(nblk(h->g.N, want), 64) * 64;
     f.parts = (int)nblk(h->g.N, f.per);
     return f;
@@ -857,11 +929,20 @@ FtPlan ftrho_plan(const bdk_t *h, int qbins) {
 // sums of the species: out[2][side][side] = cos and sin sums of (i, j); part
 // [parts][2][side][side].  Entries outside the quarter circle hold nothing.
 hipError_t launch_ftrho(bdk_t *h, const FtPlan &f, int qbins, int species, double dq, double *part, double *out) {
-    const int nt = f.side / FT_TILE;
     const long double c = (long double)dq / 3.14159265358979323846264338327950288L;
     const double ch = (double)c, cl = (double)(c - (long double)ch);
-    hipLaunchKernelGGL(k_ftrho, dim3(f.parts, nt * nt), dim3(FT_THREADS), 0, h->stream, h->g, h->d, species,
-                       h->p.ftrho_fix ? 1 : 0, qbins, nt, ch, cl, f.per, part);
+    auto go = [&](auto tile) {
+        constexpr int P = decltype(tile)::value;
+        const int nt = f.side / P;
+        hipLaunchKernelGGL(k_ftrho<P>, dim3(f.parts, nt * nt), dim3(FT_THREADS), 0, h->stream, h->g, h->d, species,
+                           h->p.ftrho_fix ? 1 : 0, qbins, nt, ch, cl, f.per, part);
+    };
+    if (f.side == 8)
+        go(std::integral_constant<int, 8>());
+    else if (f.side == 16)
+        go(std::integral_constant<int, 16>());
+    else
+        go(std::integral_constant<int, FT_TILE>());
     launch_sum_rows(part, f.parts, 2 * f.side * f.side, out, h->stream);
     return hipGetLastError();
 }
