@@ -153,11 +153,21 @@ __device__ __forceinline__ int wrap1(int u, int n) { return u < 0 ? u + n : (u >
 __device__ __forceinline__ bool zpow2(int Z) { return (Z & (Z - 1)) == 0; }
 // mesh index u in [-Z, 2Z) into [0, Z)
 template <bool P2> __device__ __forceinline__ int wrapz(int u, int Z) { return P2 ? (u & (Z - 1)) : wrap1(u, Z); }
-// any mesh index into [0, Z): a state may hold offsets of many boxes (|rel| < 1e9)
-template <bool P2> __device__ __forceinline__ int foldz(int u, int Z) {
-    if (P2) return u & (Z - 1);
-    const int v = wrap1(u, Z);
-    return (unsigned)v < (unsigned)Z ? v : wrapc(u, Z);
+// any two mesh indices into [0, Z): a state may hold offsets of many boxes (|rel| < 1e9)
+template <bool P2> __device__ __forceinline__ void foldz(int &k, int &l, int Z) {
+    if (P2) {
+        k &= Z - 1;
+        l &= Z - 1;
+        return;
+    }
+    const int a = wrap1(k, Z), b = wrap1(l, Z);
+    if (__builtin_expect(max((unsigned)a, (unsigned)b) >= (unsigned)Z, 0)) {
+        k = wrapc(k, Z);
+        l = wrapc(l, Z);
+    } else {
+        k = a;
+        l = b;
+    }
 }
 // x / d and x % d for 0 <= x < 2^22: a shift when d is a power of two, else
 // the float reciprocal corrected to the exact quotient

@@ -106,8 +106,7 @@ __device__ __forceinline__ void gather_kap(double x, double y, bool s2, const ty
     R wx[3], wy[3];
     weights_r<R, SCHEME>(x, g, k, wx);
     weights_r<R, SCHEME>(y, g, l, wy);
-    k = foldz<P2>(k, Z);
-    l = foldz<P2>(l, Z);
+    foldz<P2>(k, l, Z);
     if (SCHEME == 0) {
         R2 f = fm[(size_t)k * Z + l];
         if (!s2) {
