@@ -275,10 +275,17 @@ void mix_plans(int Z, MixPlan &r, MixPlan &c) {
     if (!r.rad || !c.rad) r = c = {0, 0};
 }
 
-// Threads and elements per thread of a pass over a mesh of another size:
-// 128 threads of 8 elements where a row fits (384^2 FP64: 17.2 / 11.8 us for
-// the columns and c2r rows at 256 threads of 16, 11.0 / 7.1 so), else 256
-// threads of as many as the row needs.
+// Threads and elements per thread of a pass over a mesh without a plan of
+// radices (750 points a side and more): 128 threads of 8 elements where a row
+// fits, else 256 threads of as many as the row needs.  Two exceptions, where
+// rows side by side fill the lines that a block writes (r2c) or reads (c2r)
+// across rows: r2c takes 256 threads where they hold an even number of rows and
+// more than 128 do (us, 128 / 256 threads: 980^2 FP32 13.4 / 12.6, FP64 16.2 /
+// 14.4, 1500^2 16.9 / 15.0 and 21.9 / 19.4, 2000^2 22.0 / 19.2 and 28.0 / 25.4;
+// odd numbers 750^2 10.1 / 10.8, 1050^2 11.3 / 12.0), and c2r in FP32 from 1800
+// points on two rows, 16 elements per thread (one / two rows: 1500^2 21.7 /
+// 22.0, 1890^2 35.4 / 33.1, 2016^2 34.4 / 30.6; FP64 1500^2 30.1 / 35.1, 2000^2
+// 45.1 / 52.1).
 struct AnyCfg {
     int ept, threads, rows, stride;
     size_t lds;
@@ -287,8 +294,15 @@ static AnyCfg any_cfg(int pass, int Z, size_t csz) {
     const int need = pass_need(pass, Z);
     AnyCfg c;
     c.threads = need <= 8 * 128 ? 128 : FFT_THREADS;
-    c.ept = ept_for(8, need);
+    c.ept = ept_for(pass == 2 && csz == 8 && Z >= 1800 ? 16 : 8, need);
     c.rows = div_at_most(pass_rows(pass, Z), c.ept * c.threads / need);
+    if (pass == 0 && c.threads < FFT_THREADS) {
+        const int rows = div_at_most(pass_rows(pass, Z), c.ept * FFT_THREADS / need);
+        if (rows > c.rows && rows % 2 == 0) {
+            c.threads = FFT_THREADS;
+            c.rows = rows;
+        }
+    }
     c.stride = lds_row(pass == 0 ? Z / 2 : Z);
     c.lds = (size_t)(pass == 1 ? 2 : 1) * c.rows * c.stride * csz;
     return c;
