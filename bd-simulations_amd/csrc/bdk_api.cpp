@@ -738,7 +738,8 @@ int bdk_create(const bd_params *p, bdk_t **out) {
     g.pos_mode = p->precision == BDK_FP32_POS32 ? 1 : (p->precision == BDK_FP32_POS32K ? 2 : 0);
     g.hinv = 1.0 / g.h;
     {
-        // BDK_XCD_REMAP=0 keeps the hardware workgroup order (for comparison)
+        // BDK_XCD_REMAP=0 keeps the hardware workgroup order of a single
+        // simulation's kernels (for comparison; batches always renumber)
         const char *e = getenv("BDK_XCD_REMAP");
         g.xcd = (e && e[0] == '0') ? 0 : 1;
     }

@@ -150,7 +150,6 @@ __device__ __forceinline__ int wrap1(int u, int n) { return u < 0 ? u + n : (u >
 // masks and shifts) and the other even sizes.  The kind is a template
 // parameter of every mesh kernel, chosen by its launcher, so the
 // power-of-two instruction stream carries no test of the other.
-__device__ __forceinline__ bool zpow2(int Z) { return (Z & (Z - 1)) == 0; }
 // mesh index u in [-Z, 2Z) into [0, Z)
 template <bool P2> __device__ __forceinline__ int wrapz(int u, int Z) { return P2 ? (u & (Z - 1)) : wrap1(u, Z); }
 // any two mesh indices into [0, Z): a state may hold offsets of many boxes (|rel| < 1e9)
@@ -184,16 +183,6 @@ struct Dv {
         return v;
     }
     __device__ int r(int x) const { return sh >= 0 ? (x & (d - 1)) : x - q(x) * d; }
-};
-// the same with the kind of d known at compile time (P2: a power of two)
-template <bool P2> struct DvT : Dv {
-    __device__ explicit DvT(int d_) : Dv(d_) {}
-};
-template <> struct DvT<true> {
-    int d, sh;
-    __device__ explicit DvT(int d_) : d(d_), sh(__ffs(d_) - 1) {}
-    __device__ int q(int x) const { return x >> sh; }
-    __device__ int r(int x) const { return x & (d - 1); }
 };
 // c / nc for 0 <= c < 2^24 (float reciprocal, corrected to the exact quotient)
 __device__ __forceinline__ int div_nc(int c, const Geo &g) {

@@ -244,7 +244,7 @@ static int p2_rows(bool f32, int Z, int pass) {
 
 // The cheapest passes over n points, a pass of radix r taken to cost r + 4 (its
 // chain of loads, products and sums, and its trip through LDS), with at most
-// FFT_THREADS / 2 butterflies each (so 15 and 16 never pay).  Largest radix first.  r2c / c2r of 192^2
+// FFT_THREADS / 2 butterflies each (radices of 15 and 16 would never pay).  Largest radix first.  r2c / c2r of 192^2
 // FP64 with r + 1.6, r + 4 and r + 8: 6.6 / 7.0, 5.3 / 5.9 and 5.7 / 5.9 us.  A
 // wave's worth of threads per block: with two, r2c of 600^2 takes 8.2 instead of
 // 7.0.

@@ -259,7 +259,7 @@ template <typename R> struct MixRow {
 // memory, the columns' product and the passes around it stay in registers.  The
 // general passes (rows in LDS throughout, radices 8, 4, 2, 3, 5, 7) run the
 // others.  Bound by the chain of a few waves per CU, part of it the fetch of code
-// (radices 15 and 16, never chosen, cost every pass 0.3 to 1 us).  Before (the
+// (with radices 15 and 16 in the switch, never chosen, every pass took 0.3 to 1 us more).  Before (the
 // general passes) and now, us, r2c / columns / c2r: 144^2 FP32 7.1 / 10.4 / 7.4
 // -> 5.1 / 6.7 / 5.2, 250^2 FP64 7.2 / 9.3 / 6.5 -> 5.1 / 9.4 / 6.1, 384^2 FP64
 // 6.9 / 10.8 / 7.1 -> 5.4 / 9.7 / 6.2, 600^2 FP32 9.7 / 11.9 / 7.8 -> 6.2 / 9.6 /

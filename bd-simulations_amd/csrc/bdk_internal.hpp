@@ -204,7 +204,6 @@ struct bdk {
     bool running = false;         // a call left work on `stream` that no batch has been ordered behind yet
     std::vector<int32_t> hgit[2];
     std::vector<double> hrel[2];
-    int scan_blocks = 0;
     hipGraph_t graph = nullptr;           // one step
     hipGraphExec_t gexec = nullptr;
     hipGraph_t graph_multi = nullptr;     // kGraphSteps steps
@@ -241,7 +240,6 @@ hipError_t launch_force_by_id(bdk_t *h, const void *f, double2 *out);  // list-o
 hipError_t launch_to_host(const void *src, size_t bytes, void *dst, hipStream_t st);
 hipError_t launch_zero_ints(int *p, int n, hipStream_t st);
 hipError_t launch_rearm(bdk_t *h);                // per-step scalars when no deposit runs
-size_t deposit_lds_bytes(const bdk_t *h);          // LDS of one deposit block
 // the deposit beside a rebuild, as a part of a paired launch
 struct DepLaunch {
     DepArgs a;
@@ -263,7 +261,6 @@ hipError_t launch_place(bdk_t *h, const int2 *git, const double2 *rel);  // a ne
 void mix_plans(int Z, MixPlan &r, MixPlan &c);
 hipError_t launch_bin(bdk_t *h);                  // counting after a state's load
 hipError_t launch_own(bdk_t *h);                  // owned-mesh-index table of the deposit tiles
-hipError_t launch_scan_fill(bdk_t *h);            // exclusive scan + fill of the cell list
 hipError_t launch_refresh(bdk_t *h);              // refresh only (no motion)
 hipError_t launch_noise_out(bdk_t *h);            // noise of the next step, by pid
 // ordered-pair distance histograms [3][nbins] (11, 12, 22), zeroed by the caller
@@ -297,7 +294,6 @@ hipError_t set_kernel_attributes(int dev);
 // device address of the allocation-free entry's scratch array on device
 // `dev` (current), looked up once per device (bdk_noalloc.hip)
 hipError_t noalloc_setup(int dev);
-hipError_t build_tables(bdk_t *h);                // spectral tables in device memory
 
 // batches (a batch is a view over member handles, each with its own buffers)
 int batch_min_ept(int stage, int zmax);

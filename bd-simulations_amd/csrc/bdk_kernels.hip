@@ -836,8 +836,6 @@ static DepPlan dep_plan(const bdk_t *h, int reset, int tile_pts = 0) {
     return pl;
 }
 
-size_t deposit_lds_bytes(const bdk_t *h) { return dep_plan(h, 0).lds; }
-
 DepLaunch deposit_launch(const bdk_t *h) {
     DepPlan pl = dep_plan(h, 0);
     pl.a.slot = 1;
@@ -953,19 +951,14 @@ hipError_t launch_update(bdk_t *h, int fused) {
     return hipGetLastError();
 }
 
-static void launch_scan_fill_inner(bdk_t *h, int inc_step) {
+static void launch_scan_fill(bdk_t *h) {
     const int ncell = h->g.ncell;
     const int nb = (int)nblk(ncell, SCAN_BLOCK);
     hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(SCAN_THREADS), 0, h->stream, h->d.count, ncell, h->d.bcount);
     hipLaunchKernelGGL(k_scan, dim3(nb), dim3(SCAN_THREADS), 0, h->stream, h->d.count, h->d.bcount, h->d.start, ncell,
-                       nb, h->g.N, h->d.sc, inc_step);
+                       nb, h->g.N, h->d.sc, 0);
     hipLaunchKernelGGL(k_fill, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d, 0);
     hipLaunchKernelGGL(k_sort_cells, dim3(nblk(ncell, 256 * SORT_CELLS)), dim3(256), 0, h->stream, h->g, h->d, 0);
-}
-
-hipError_t launch_scan_fill(bdk_t *h) {
-    launch_scan_fill_inner(h, 1);
-    return hipGetLastError();
 }
 
 hipError_t launch_own(bdk_t *h) {
@@ -976,7 +969,7 @@ hipError_t launch_own(bdk_t *h) {
 hipError_t launch_bin(bdk_t *h) {
     hipLaunchKernelGGL(k_reset_exc, dim3(1), dim3(1), 0, h->stream, h->d.sc);
     hipLaunchKernelGGL(k_bin, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d);
-    launch_scan_fill_inner(h, 0);
+    launch_scan_fill(h);
     return hipGetLastError();
 }
 
@@ -984,7 +977,7 @@ hipError_t launch_place(bdk_t *h, const int2 *git, const double2 *rel) {
     hipLaunchKernelGGL(k_place_clear, dim3(nblk(h->g.ncell, 256)), dim3(256), 0, h->stream, h->d.count, h->g.ncell,
                        h->d.sc);
     hipLaunchKernelGGL(k_place, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d, git, rel);
-    launch_scan_fill_inner(h, 0);
+    launch_scan_fill(h);
     return hipGetLastError();
 }
 
@@ -992,7 +985,7 @@ hipError_t launch_refresh(bdk_t *h) {
     hipLaunchKernelGGL(k_reset_exc, dim3(1), dim3(1), 0, h->stream, h->d.sc);
     hipLaunchKernelGGL(k_zero_int, dim3(nblk(h->g.ncell, 256)), dim3(256), 0, h->stream, h->d.count, h->g.ncell);
     hipLaunchKernelGGL(k_refresh, dim3(nblk(h->g.N, 256)), dim3(256), 0, h->stream, h->g, h->d);
-    launch_scan_fill_inner(h, 0);
+    launch_scan_fill(h);
     return hipGetLastError();
 }
 
