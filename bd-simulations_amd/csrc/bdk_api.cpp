@@ -2262,8 +2262,8 @@ int bdk_batch_set_tuning(bdk_batch_t *b, const int32_t *choice) {
 
 // The project's autotuner.  Each knob is timed on the batch's own members
 // with the stages that leave the particles unchanged, one knob at a time in
-// this order, keeping the fastest value: the FFT elements per thread of each
-// pass (8, 16, 32; stages 2-4), the WCA block size (128, 256, 512; stage 0),
+// this order, keeping the fastest value: the FFT block size of each pass (8, 16,
+// 32 times FFT_THREADS mesh values; stages 2-4), the WCA block size (128, 256, 512; stage 0),
 // the deposit tile (mesh points per tile side 24, 32, 38, 48, 64, 80; stage 1:
 // fine meshes put few particles in a small tile), and
 // the persistent grid (one block per map entry, or 4 or 8 blocks per compute

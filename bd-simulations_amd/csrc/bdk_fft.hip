@@ -411,7 +411,7 @@ hipError_t launch_fft(bdk_t *h) {
 
 int batch_min_ept(int stage, int zmax) { return ept_for(8, pass_need(stage, zmax)); }
 
-// rows per block of a member's passes for the batch's elements per thread
+// rows per block of a member's passes for the batch's block sizes
 // (ept x FFT_THREADS complex values per block), and the LDS its launches need
 void fft_member(RepDev &r, int Z, const int ept[3], BatchPlan &bp) {
     int rows[3];

@@ -162,7 +162,7 @@ enum BatchStage { BS_PART = 0, BS_CELL, BS_SCAN, BS_DEP, BS_R2C, BS_COL, BS_C2R,
 
 // The choices of the batch autotuner (bdk_batch_tune); none changes a result.
 struct BatchTuning {
-    int ept[3] = {8, 8, 8};  // FFT elements per thread (r2c, col, c2r)
+    int ept[3] = {8, 8, 8};  // FFT block sizes (r2c, col, c2r) in units of FFT_THREADS mesh values
     int wca_block = 256;     // threads per block of the WCA stage (128, 256 or 512)
     int dep_tile = 38;       // deposit tile: list cells per side such that a tile owns <= dep_tile^2 mesh points
     int persist = 0;         // blocks per launch of every stage (0: one block per map entry)
@@ -177,7 +177,7 @@ struct BatchPlan {
     int nblk2[BS_COUNT] = {};        // leading entries of members with a power-of-two mesh
     int nblk16[BS_COUNT] = {};       // of those, the leading entries with 16 mesh points per FFT thread
     BatchTuning tune;
-    int ept[3] = {8, 8, 8};          // the FFT elements per thread in use (at least the members' minimum)
+    int ept[3] = {8, 8, 8};          // the FFT block sizes in use (at least the members' minimum)
     size_t dep_lds = 0;
     // FFT launches by kind of mesh (16 points per thread, other powers of two, other sizes) and pass
     size_t fft_lds[3][3] = {};

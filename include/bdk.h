@@ -361,8 +361,11 @@ int bdk_ftrho_sums(bdk_t *h, int32_t species, int32_t qbins, double dq_ft, doubl
    reference's long-double clock from its own logged dt's.  Each member's state
    stays in its own buffers: after bdk_batch_sync the ordinary per-handle
    calls (bdk_get_positions, bdk_write_pos, ...) read it, and each member's
-   trajectory is bit-identical to running that handle alone.  A member must
-   not be stepped through its own handle while it belongs to a live batch. */
+   trajectory is bit-identical to running that handle alone.  A member may get
+   a new state through its own handle (after bdk_batch_sync; put on the device
+   by bdk_prepare or any call that reads it): the batch's next call comes
+   after it.  A member must not be stepped through its own handle while it
+   belongs to a live batch. */
 typedef struct bdk_batch bdk_batch_t;
 
 int bdk_batch_create(bdk_t *const *members, int32_t n, bdk_batch_t **out);
@@ -379,7 +382,9 @@ int bdk_batch_sync(bdk_batch_t *b);
 int bdk_batch_status(bdk_batch_t *b, int32_t n, int32_t *status);
 /* Project autotuner: times each knob on the batch's own members (reps
    launches of the stages that leave the particles unchanged) and keeps the
-   fastest value: the FFT elements per thread of each pass (8, 16, 32), the
+   fastest value: the FFT block size of each pass (8, 16 or 32 times 256 mesh
+   values, which sets the rows of a block, and on meshes that are neither a
+   power of two nor split into radices up to 14 the elements per thread), the
    WCA block size (128, 256, 512 threads), the deposit tile (list cells per
    side such that a tile owns at most 24^2, 32^2, 38^2, 48^2, 64^2 or 80^2 mesh points),
    and the persistent grid (one block per work item, or 4 or 8 blocks per
@@ -392,7 +397,7 @@ enum bdk_tune_index {
 };
 int bdk_batch_tune(bdk_batch_t *b, int32_t reps, int32_t *choice_out);
 /* Apply a choice (e.g. one bdk_batch_tune made for the same mix): FFT
-   elements per thread 8, 16 or 32 (raised to the members' minimum), WCA
+   block size 8, 16 or 32 (raised to the members' minimum), WCA
    block size 128, 256 or 512, deposit tile 8..96 mesh points per side,
    persistent grid >= 0 (0: one block per work item).  No choice changes a
    result. */
