@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n1,n2", [(70, 3000), (2500, 1200)])
-@pytest.mark.parametrize("qbins", [2, 7, 8, 9, 15, 16, 17, 31, 32, 33, 70])
+@pytest.mark.parametrize("qbins", [2, 8, 9, 16, 17, 33, 70])
 @pytest.mark.parametrize("fix", [0, 1])
 def test_sums_against_extended_precision(n1, n2, qbins, fix):
     print("case: ftrho against extended precision n=%d+%d qbins=%d fix=%d" % (n1, n2, qbins, fix), flush=True)
